@@ -7,7 +7,7 @@
 //     v_mfma_f32_16x16x32: 256x256x64 tile, 512 threads, direct global -> LDS loads of whole 128-byte lines into two
 //     stages, transposing LDS reads for row-major B; also as 128x128 tiles (two or four stages) and 256x64 tiles, and
 //     with the A operand gathered from a channels-last image (implicit-GEMM convolution); see the comment at the kernel.
-//   * gemm16_mfma_kernel  - bf16 / fp16 inputs, any operand layout (used for transposed A), fp32 accumulation on v_mfma_f32_32x32x16_{bf16,f16}.
+//   * gemm16_mfma_kernel  - bf16 / fp16 inputs, transposed A with a chip full of 256x256 tiles, fp32 accumulation on v_mfma_f32_32x32x16_{bf16,f16}.
 //     256x256 block tile, 64-deep K step, 256 threads = 4 wavefronts in a 2x2 grid, each wavefront owning a
 //     128x128 tile (16 MFMA accumulator tiles = 256 accumulator registers).  Both operand tiles live in LDS
 //     as [row][k] with k contiguous, 128 bytes per row, double buffered (2 x 64 KiB of the 160 KiB per CU);
@@ -16,10 +16,9 @@
 //     in registers (8x8 blocks of 16-bit values) on their way into LDS.  Requires M%256 == N%256 == K%64 == 0.
 //   * gemm32_mfma_kernel  - fp32 on v_mfma_f32_32x32x2f32, 128x128 tile (64x64 when that is what fills the chip),
 //     for M%128 == N%128 == K%32 == 0.
-//   * gemm_generic_kernel - any shape / transpose / type (fp16, bf16, fp32, fp64): 64x64 LDS tile, FMA units.
-// Shapes the tile kernels do not take (ragged, or too few tiles to fill the chip) run on the bounds-checked MFMA
-// kernel of conv_nhwc_mfma.hip as a 1x1 convolution, after transposing copies of the operands that are not
-// K-contiguous (transpose2d_kernel); gemm_generic_kernel is left with K % (16 bytes) != 0 and fp64.
+//   * gemm_generic_kernel - any shape / transpose / type: 64x64 LDS tile, FMA units; for fp64.
+// Everything else - ragged extents, a transposed A, too few tiles to fill the chip - runs on the register-staged MFMA
+// kernel of gemm_flex.hip.
 #include <hip/hip_runtime.h>
 
 #include <atomic>
@@ -32,6 +31,7 @@
 
 #include "cinn_hip_runtime.h"
 #include "kernels/conv_nhwc.h"
+#include "kernels/gemm_flex.h"
 #include "runtime/hip_check.h"
 
 namespace {
@@ -1478,44 +1478,6 @@ gemm_generic_kernel(const T* __restrict__ A, const T* __restrict__ B, T* __restr
   }
 }
 
-// [rows][cols] -> [cols][rows] through a 32x32 LDS tile (odd pitch), blockIdx.z = batch.  Brings an operand whose
-// contiguous axis is not K into the K-contiguous form the bounds-checked MFMA path wants.
-template <typename T>
-__global__ void __launch_bounds__(256)
-transpose2d_kernel(const T* __restrict__ in, T* __restrict__ out, int rows, int cols, int64_t in_stride, int64_t out_stride) {
-  __shared__ T tile[32][33];
-  in += (int64_t)blockIdx.z * in_stride;
-  out += (int64_t)blockIdx.z * out_stride;
-  const int c0 = blockIdx.x * 32, r0 = blockIdx.y * 32;
-  const int tx = threadIdx.x, ty = threadIdx.y;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = r0 + ty + 8 * i, c = c0 + tx;
-    if (r < rows && c < cols) tile[ty + 8 * i][tx] = in[(int64_t)r * cols + c];
-  }
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int c = c0 + ty + 8 * i, r = r0 + tx;
-    if (r < rows && c < cols) out[(int64_t)c * rows + r] = tile[tx][ty + 8 * i];
-  }
-}
-
-void LaunchTranspose(const void* in, void* out, int rows, int cols, int batch, int64_t in_stride, int elem_bytes,
-                     hipStream_t stream) {
-  dim3 grid((cols + 31) / 32, (rows + 31) / 32, batch);
-  CINN_RT_CHECK(grid.y <= 65535, "gemm: operand with %d rows is too tall for the transposing copy", rows);
-  const int64_t out_stride = (int64_t)rows * cols;
-  if (elem_bytes == 2) {
-    hipLaunchKernelGGL((transpose2d_kernel<uint16_t>), grid, dim3(32, 8), 0, stream, static_cast<const uint16_t*>(in),
-                       static_cast<uint16_t*>(out), rows, cols, in_stride, out_stride);
-  } else {
-    hipLaunchKernelGGL((transpose2d_kernel<uint32_t>), grid, dim3(32, 8), 0, stream, static_cast<const uint32_t*>(in),
-                       static_cast<uint32_t*>(out), rows, cols, in_stride, out_stride);
-  }
-  CINN_HIP_CALL(hipGetLastError());
-}
-
 enum class GemmType { kF16, kBF16, kF32, kF64 };
 
 struct GemmProblem {
@@ -2007,10 +1969,13 @@ void RunGemm(const GemmProblem& p, hipStream_t stream) {
                 p.m, p.n, p.k, p.batch);
   CINN_RT_CHECK(p.a && p.b && p.c, "gemm: null operand");
   CINN_RT_CHECK(p.batch <= 65535, "gemm: batch %d exceeds the grid limit", p.batch);
-  const bool fast16 = !ForceGeneric() && p.m % kBM == 0 && p.n % kBN == 0 && p.k % kBK == 0;
   const bool aligned16 = reinterpret_cast<uintptr_t>(p.a) % 16 == 0 && reinterpret_cast<uintptr_t>(p.b) % 16 == 0 &&
-                         p.stride_a % 4 == 0 && p.stride_b % 4 == 0;
-  const bool fast32 = !ForceGeneric() && p.m % kF32Tile == 0 && p.n % kF32Tile == 0 && p.k % kF32K == 0 && aligned16;
+                         p.stride_a % 8 == 0 && p.stride_b % 8 == 0;
+  // 256x256 tiles with register staging take a transposed A that fills the chip with them: 4096^3 164 us (171 on the
+  // 128x128 tiles of gemm_flex.hip); with 64 such tiles, 2048^3, 75 against 26 us
+  const bool fast16 = !ForceGeneric() && aligned16 && p.m % kBM == 0 && p.n % kBN == 0 && p.k % kBK == 0 &&
+                      (UseRegisterStaging() || (int64_t)(p.m / kBM) * (p.n / kBN) * p.batch >= 192);
+  const bool fast32 = !ForceGeneric() && aligned16 && p.m % kF32Tile == 0 && p.n % kF32Tile == 0 && p.k % kF32K == 0;
   if (!ForceGeneric() && !UseRegisterStaging() && (p.type == GemmType::kBF16 || p.type == GemmType::kF16)) {
     const bool taken = p.type == GemmType::kBF16 ? TryDma16<__bf16>(p, stream) : TryDma16<_Float16>(p, stream);
     if (taken) {
@@ -2018,60 +1983,18 @@ void RunGemm(const GemmProblem& p, hipStream_t stream) {
       return;
     }
   }
-  // Shapes the big-tile kernels do not take (ragged, or so few tiles that most CUs would idle) go to the
-  // channels-last convolution kernels: a 1x1 convolution over m "pixels" is this GEMM with both operands
-  // K-contiguous (A [m,k], B stored [n,k]); those kernels bound-check every tile edge, use 64x64 tiles and split K
-  // when the grid is small.  An operand stored the other way round is transposed into scratch first, which costs one
-  // pass over that operand.
-  const int elem_bytes = p.type == GemmType::kF32 ? 4 : (p.type == GemmType::kF64 ? 8 : 2);
-  const bool tile_fit  = p.type == GemmType::kF32 ? fast32 : fast16;
-  const int64_t tiles  = p.type == GemmType::kF32 ? (int64_t)(p.m / 64) * (p.n / 64) * p.batch
-                                                  : (int64_t)(p.m / kBM) * (p.n / kBN) * p.batch;
-  const bool few_tiles = tile_fit && tiles < 64;
-  const bool flexible  = !ForceGeneric() && p.type != GemmType::kF64 && p.k % (16 / elem_bytes) == 0 &&
-                         reinterpret_cast<uintptr_t>(p.a) % 16 == 0 && reinterpret_cast<uintptr_t>(p.b) % 16 == 0;
-  if (flexible && (!tile_fit || few_tiles)) {
-    const char* a_base = static_cast<const char*>(p.a);
-    const char* b_base = static_cast<const char*>(p.b);
-    int64_t stride_a = p.stride_a, stride_b = p.stride_b;
-    if (p.trans_a || !p.trans_b) {
-      const int batch_a    = p.trans_a ? (p.stride_a == 0 ? 1 : p.batch) : 0;
-      const int batch_b    = !p.trans_b ? (p.stride_b == 0 ? 1 : p.batch) : 0;
-      const size_t bytes_a = (size_t)batch_a * p.m * p.k * elem_bytes;
-      const size_t bytes_b = (size_t)batch_b * p.k * p.n * elem_bytes;
-      char* scratch        = static_cast<char*>(cinn_hip_kernels::Scratch(cinn_hip_kernels::ScratchKind::kTranspose, bytes_a + bytes_b, stream));
-      if (p.trans_a) {  // stored [k][m]
-        LaunchTranspose(p.a, scratch, p.k, p.m, batch_a, p.stride_a, elem_bytes, stream);
-        a_base   = scratch;
-        stride_a = p.stride_a == 0 ? 0 : (int64_t)p.m * p.k;
-      }
-      if (!p.trans_b) {  // stored [k][n]
-        LaunchTranspose(p.b, scratch + bytes_a, p.k, p.n, batch_b, p.stride_b, elem_bytes, stream);
-        b_base   = scratch + bytes_a;
-        stride_b = p.stride_b == 0 ? 0 : (int64_t)p.k * p.n;
-      }
-    }
-    for (int b = 0; b < p.batch; ++b) {
-      cinn_hip_kernels::ConvNhwcArgs a;
-      a.x = a_base + (int64_t)b * stride_a * elem_bytes;
-      a.w = b_base + (int64_t)b * stride_b * elem_bytes;
-      a.y = static_cast<char*>(p.c) + (int64_t)b * p.stride_c * elem_bytes;
-      a.scale = a.shift = nullptr;
-      a.residual        = p.beta != 0.0f ? a.y : nullptr;
-      a.alpha           = p.alpha;
-      a.residual_scale  = p.beta;
-      a.relu            = false;
-      a.nchw_input      = false;
-      a.n = 1, a.h = 1, a.w_in = p.m, a.c = p.k;
-      a.oc = p.n, a.kh = 1, a.kw = 1, a.oh = 1, a.ow = p.m;
-      a.pad_h = a.pad_w = 0;
-      a.stride_h = a.stride_w = a.dil_h = a.dil_w = 1;
-      a.type.code  = p.type == GemmType::kBF16 ? cinn_type_bfloat : cinn_type_float;
-      a.type.bits  = static_cast<uint8_t>(elem_bytes * CHAR_BIT);
-      a.type.lanes = 1;
-      cinn_hip_kernels::RunConvNhwc(a, stream);
-    }
-    return;
+  if (!ForceGeneric() && p.type != GemmType::kF64 && !(p.type == GemmType::kF32 ? fast32 : fast16)) {
+    cinn_hip_kernels::FlexGemm g;
+    g.type = p.type == GemmType::kF16 ? cinn_hip_kernels::FlexType::kF16
+                                      : (p.type == GemmType::kBF16 ? cinn_hip_kernels::FlexType::kBF16 : cinn_hip_kernels::FlexType::kF32);
+    g.a = p.a, g.b = p.b, g.c = p.c;
+    g.m = p.m, g.n = p.n, g.k = p.k;
+    g.a_kc = !p.trans_a, g.b_kc = p.trans_b;
+    g.lda = p.trans_a ? p.m : p.k, g.ldb = p.trans_b ? p.k : p.n;
+    g.batch = p.batch, g.stride_a = p.stride_a, g.stride_b = p.stride_b, g.stride_c = p.stride_c;
+    g.alpha = p.alpha;
+    if (p.beta != 0.0f) g.residual = p.c, g.residual_scale = p.beta;
+    if (cinn_hip_kernels::TryFlexGemm(g, stream)) return;
   }
   switch (p.type) {
     case GemmType::kBF16:

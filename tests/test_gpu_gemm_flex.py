@@ -1,0 +1,63 @@
+"""Products that run on the register-staged MFMA kernel (gemm_flex.hip), at the edges of its tiles, K steps and chunks:
+one row, one column, one k; extents one below and above 64 and 128; operands whose rows are no multiple of a 16-byte
+chunk; enough tiles for the 128x128 forms; few tiles and a long K for the split reduction.
+
+Bounds: the inputs are exact in the type, sums are fp32: every rounding of a sum of k products is at most 2^-24 of the
+sum of their magnitudes, and a blocked sum has far fewer of them in a row than k, so 2^-24 * sqrt(k) + 2^-22 of that
+magnitude covers it; a 16-bit result adds half an ulp of itself (2^-11 fp16, 2^-8 bf16)."""
+import numpy as np
+import pytest
+
+from cinn_amd.common import bfloat16_bits_to_float32, float32_to_bfloat16_bits
+
+from test_gpu_gemm import call_cublas
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [
+    (1, 1, 1, 1), (1, 1, 7, 3), (1, 3, 1, 65), (1, 63, 65, 64), (1, 65, 63, 129), (1, 129, 127, 127), (5, 1, 215, 48),
+    (3, 48, 1, 215), (1, 17, 300, 172), (2, 1500, 1300, 33),  # two K steps on 128x128 tiles of one group
+    (1, 1290, 1540, 700),  # 128x128 tiles of two groups
+    (1, 70, 90, 3001),     # K split
+]
+
+
+def rounded(rng, shape, kind):
+    v = rng.standard_normal(shape).astype(np.float32)
+    if kind == "bfloat16":
+        bits = float32_to_bfloat16_bits(v)
+        return bits, bfloat16_bits_to_float32(bits).astype(np.float64)
+    v = v.astype(kind)
+    return v, v.astype(np.float64)
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
+@pytest.mark.parametrize("kind", ["float32", "float16", "bfloat16"])
+@pytest.mark.parametrize("batch,m,n,k", SHAPES)
+def test_edges(gpu, batch, m, n, k, kind, ta, tb):
+    rng = np.random.default_rng(m * 7 + n * 3 + k)
+    a, af = rounded(rng, (batch, k, m) if ta else (batch, m, k), kind)
+    b, bf = rounded(rng, (batch, n, k) if tb else (batch, k, n), kind)
+    c0, cf = rounded(rng, (batch, m, n), kind)
+    got = call_cublas(a, b, (batch, m, n), kind, ta, tb, alpha=0.5, beta=-1.0, c_init=c0)
+    got = (bfloat16_bits_to_float32(got) if kind == "bfloat16" else got).astype(np.float64)
+    am, bm = (np.swapaxes(af, 1, 2) if ta else af), (np.swapaxes(bf, 1, 2) if tb else bf)
+    want  = 0.5 * (am @ bm) - cf
+    scale = 0.5 * (np.abs(am) @ np.abs(bm)) + np.abs(cf)
+    ulp   = {"float32": 2.0 ** -24, "float16": 2.0 ** -11, "bfloat16": 2.0 ** -8}[kind]
+    assert np.all(np.abs(got - want) <= (2.0 ** -24 * np.sqrt(k) + 2.0 ** -22) * scale + ulp * np.abs(want) + 2.0 ** -25)
+
+
+@pytest.mark.parametrize("kind", ["float32", "float16"])
+@pytest.mark.parametrize("ta,tb", [(False, True), (True, False)])
+def test_what_lies_beyond_k_is_not_multiplied(gpu, kind, ta, tb):
+    """k = 65: the chunk that reaches beyond a row's k holds the next row's first values, which are infinite here; and
+    rows beyond a [k][row] operand's last full chunk neighbour the next k row"""
+    m, n, k = 67, 70, 65
+    rng = np.random.default_rng(5)
+    a, b = rng.standard_normal((m, k)).astype(kind), rng.standard_normal((n, k)).astype(kind)
+    a[1:, :] = np.inf
+    got = call_cublas(np.ascontiguousarray(a.T) if ta else a, b if tb else np.ascontiguousarray(b.T), (m, n), kind, ta, tb)
+    want = a[0].astype(np.float64) @ b.astype(np.float64).T
+    assert np.all(np.isfinite(got[0].astype(np.float64)))
+    np.testing.assert_allclose(got[0].astype(np.float64), want, rtol=2.0 ** -10, atol=2.0 ** -10)
