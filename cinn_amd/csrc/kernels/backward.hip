@@ -4,8 +4,9 @@
 // (0 = NCHW with [F][C][KH][KW] filters, 1 = NHWC with [F][KH][KW][C] filters), results
 // out = alpha * gradient + beta * out, fp32 accumulation for fp32 / fp16 / bf16 tensors, fp64 for fp64 tensors.
 //
-// These are the straightforward gather forms - one thread (or, for the filter gradient, one block) per gradient
-// element, summing its contributions in a fixed order - not tiled MFMA kernels: the inference path never calls them.
+// Convolution gradients without groups in fp32 / fp16 / bf16 run on the matrix cores (conv_backward_mfma.hip).  The
+// kernels here are the straightforward gather forms - one thread (or, for the filter gradient, one block) per gradient
+// element, summing its contributions in a fixed order: convolutions with groups, fp64, pooling and log-softmax.
 //   dx[n,c,iy,ix] = sum over f of the group, ky, kx with iy = oy * stride - pad + ky * dilation (same in x):
 //                   dy[n,f,oy,ox] * w[f,c',ky,kx]
 //   dw[f,c',ky,kx] = sum over n, oy, ox: x[n,c,oy * stride - pad + ky * dilation, ...] * dy[n,f,oy,ox]
@@ -21,6 +22,7 @@
 #include <cstdlib>
 
 #include "cinn_hip_runtime.h"
+#include "kernels/conv_backward.h"
 #include "runtime/hip_check.h"
 
 namespace {
@@ -279,6 +281,19 @@ ConvDims MakeConvDims(const char* what, int format, float alpha, float beta, int
   return p;
 }
 
+cinn_hip_kernels::ConvBackwardArgs MatrixArgs(const ConvDims& p, const cinn_buffer_t* out) {
+  cinn_hip_kernels::ConvBackwardArgs a;
+  a.x = a.w = a.dy = nullptr;
+  a.out  = out->memory;
+  a.nhwc = p.nhwc != 0;
+  a.n = p.n, a.c = p.c, a.h = p.ih, a.w_in = p.iw;
+  a.f = p.f, a.kh = p.kh, a.kw = p.kw, a.oh = p.oh, a.ow = p.ow;
+  a.pad_h = p.ph, a.pad_w = p.pw, a.stride_h = p.sh, a.stride_w = p.sw, a.dil_h = p.dh, a.dil_w = p.dw;
+  a.alpha = p.alpha, a.beta = p.beta;
+  a.type = out->type;
+  return a;
+}
+
 }  // namespace
 
 extern "C" {
@@ -296,6 +311,11 @@ void cinn_call_cudnn_conv2d_backward_data(void* v_args, int num_args, int format
   cinn_buffer_t* w  = Arg(v_args, 0);
   cinn_buffer_t* dy = Arg(v_args, 1);
   cinn_buffer_t* dx = Arg(v_args, 2);
+  if (p.groups == 1) {
+    cinn_hip_kernels::ConvBackwardArgs a = MatrixArgs(p, dx);
+    a.w = w->memory, a.dy = dy->memory;
+    if (cinn_hip_kernels::TryConvBackwardData(a, static_cast<hipStream_t>(stream))) return;
+  }
   const int64_t total = (int64_t)p.n * p.c * p.ih * p.iw;
   dim3 grid((unsigned)((total + 255) / 256));
   auto s = static_cast<hipStream_t>(stream);
@@ -335,6 +355,11 @@ void cinn_call_cudnn_conv2d_backward_filter(void* v_args, int num_args, int form
   cinn_buffer_t* dw = Arg(v_args, 2);
   const int64_t total = (int64_t)p.f * p.fc * p.kh * p.kw;
   CINN_RT_CHECK(total < INT_MAX, "conv2d_backward_filter: filter too large");
+  if (p.groups == 1) {
+    cinn_hip_kernels::ConvBackwardArgs a = MatrixArgs(p, dw);
+    a.x = x->memory, a.dy = dy->memory;
+    if (cinn_hip_kernels::TryConvBackwardFilter(a, static_cast<hipStream_t>(stream))) return;
+  }
   dim3 grid((unsigned)total);
   auto s = static_cast<hipStream_t>(stream);
   switch (ElemOf(dw)) {

@@ -1,0 +1,578 @@
+// Gradients of a convolution on the MFMA units (gfx950), fp16 / bf16 / fp32, channels last inside.
+//
+// Both gradients are matrix products over tensors whose channels are contiguous:
+//   dx[pixel][c]      = sum over (tap, f)  dy[pixel - tap][f] * w[f][tap][c]
+//   dw[f][(tap, c)]   = sum over pixels    dy[pixel][f] * x[pixel + tap][c]
+//
+//   * dx at stride 1 is a forward convolution of dy with the filter turned round, [c][tap'][f]: it runs on the forward
+//     kernels (RunConvNhwc) after one small kernel has rearranged the filter.
+//   * dx at a larger stride: the input pixels of one remainder class (iy mod stride, ix mod stride) see the same taps,
+//     every stride-th one, and neighbouring pixels of the class see neighbouring dy.  Each class is a product of its own
+//     (pixels x channels, K = its taps x f), all classes in one launch; no multiply-add meets an inserted zero.
+//   * dw: rows are filters, columns (tap, channel), and K runs over all output pixels, which both operands keep as their
+//     slow axis: they lie in LDS as [pixel][channels] and are read with transposing reads.  The x operand is gathered
+//     row by row (a chunk of channels of pixel + tap, or zeros).  K is long (1e5) and the result small, so K is split
+//     until the chip is full; the fp32 planes are added by a second kernel, which also writes the filter's own layout.
+// Measured before (one thread or block per gradient element) and here: 64 -> 64 3x3 on 56x56 at batch 32 in fp16, NCHW,
+// dx 4988 -> 13 us (560 TFLOP/s) and dw 9467 -> 28 + 6 us (260 TFLOP/s; the x operand is read nine times from L2), with
+// 5 to 7 us for each copied tensor; 96 -> 200 3x3 / stride 2 on 35x41 at batch 8 in fp32, dx 1661 -> 31 us and dw
+// 3844 -> 22 + 5 us (47 TFLOP/s).
+// Tensors that are not channels last, or whose channel count is no multiple of a 16-byte chunk, are first copied into
+// that form in scratch (pack_kernel), and dx is copied back.
+#include "kernels/conv_backward.h"
+
+#include <algorithm>
+#include <climits>
+
+#include "kernels/conv_nhwc.h"
+#include "kernels/flex_tile.h"
+#include "runtime/hip_check.h"
+#include "runtime/scratch.h"
+
+namespace cinn_hip_kernels {
+namespace {
+
+using flex::u32x4;
+
+// ---- copies between tensor layouts ---------------------------------------------------------------------------------
+// [n][c][plane] (nchw) or [n][plane][c] -> [n][plane][cp], channels c .. cp-1 zero.  A block moves 64 pixels x 64
+// channels of one image through LDS; cp is a multiple of a 16-byte chunk.
+template <typename T, bool NCHW>
+__global__ void __launch_bounds__(256)
+pack_kernel(const T* __restrict__ in, T* __restrict__ out, int c, int plane, int cp) {
+  constexpr int E = 16 / (int)sizeof(T), CPR = 64 / E;  // chunks per 64-element row
+  __shared__ T tile[64][64 + 4 / (int)sizeof(T)];       // [pixel][channel]
+  const int p0 = blockIdx.x * 64, c0 = blockIdx.y * 64;
+  in += (int64_t)blockIdx.z * c * plane;
+  out += (int64_t)blockIdx.z * plane * cp;
+  const int rows = NCHW ? c : plane, cols = NCHW ? plane : c;  // memory is [rows][cols]
+  const int r0 = NCHW ? c0 : p0, q0 = NCHW ? p0 : c0;
+  for (int u = threadIdx.x; u < 64 * CPR; u += 256) {
+    const int r = u / CPR, q = u % CPR * E;
+    typedef T chunk_t __attribute__((ext_vector_type(E)));
+    chunk_t v = {0};
+    if (r0 + r < rows) {
+      const T* from = in + (int64_t)(r0 + r) * cols + q0 + q;
+      if (q0 + q + E <= cols) {
+        __builtin_memcpy(&v, from, 16);
+      } else {
+#pragma unroll
+        for (int e = 0; e < E; ++e)
+          if (q0 + q + e < cols) v[e] = from[e];
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) (NCHW ? tile[q + e][r] : tile[r][q + e]) = v[e];
+  }
+  __syncthreads();
+  for (int u = threadIdx.x; u < 64 * CPR; u += 256) {
+    const int p = u / CPR, q = u % CPR * E;
+    if (p0 + p >= plane || c0 + q >= cp) continue;
+    T v[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) v[e] = tile[p][q + e];
+    __builtin_memcpy(out + (int64_t)(p0 + p) * cp + c0 + q, v, 16);
+  }
+}
+
+// [n][plane][c] -> [n][c][plane], out = in + beta * out
+template <typename T>
+__global__ void __launch_bounds__(256)
+unpack_kernel(const T* __restrict__ in, T* __restrict__ out, int c, int plane, float beta) {
+  constexpr int E = 16 / (int)sizeof(T), CPR = 64 / E;
+  __shared__ T tile[64][64 + 4 / (int)sizeof(T)];  // [pixel][channel]
+  const int p0 = blockIdx.x * 64, c0 = blockIdx.y * 64;
+  in += (int64_t)blockIdx.z * c * plane;
+  out += (int64_t)blockIdx.z * plane * c;
+  for (int u = threadIdx.x; u < 64 * CPR; u += 256) {
+    const int p = u / CPR, q = u % CPR * E;
+    typedef T chunk_t __attribute__((ext_vector_type(E)));
+    chunk_t v = {0};
+    if (p0 + p < plane) {
+      const T* from = in + (int64_t)(p0 + p) * c + c0 + q;
+      if (c0 + q + E <= c) {
+        __builtin_memcpy(&v, from, 16);
+      } else {
+#pragma unroll
+        for (int e = 0; e < E; ++e)
+          if (c0 + q + e < c) v[e] = from[e];
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) tile[p][q + e] = v[e];
+  }
+  __syncthreads();
+  for (int u = threadIdx.x; u < 64 * CPR; u += 256) {
+    const int r = u / CPR, q = u % CPR * E;  // channel, first pixel
+    if (c0 + r >= c) continue;
+    T* to = out + (int64_t)(c0 + r) * plane + p0 + q;
+    typedef T chunk_t __attribute__((ext_vector_type(E)));
+    chunk_t v;
+#pragma unroll
+    for (int e = 0; e < E; ++e) v[e] = tile[q + e][r];
+    if (p0 + q + E <= plane) {
+      if (beta != 0.0f) {
+        chunk_t old;
+        __builtin_memcpy(&old, to, 16);
+#pragma unroll
+        for (int e = 0; e < E; ++e) v[e] = (T)((float)v[e] + beta * (float)old[e]);
+      }
+      __builtin_memcpy(to, &v, 16);
+    } else {
+#pragma unroll
+      for (int e = 0; e < E; ++e)
+        if (p0 + q + e < plane) to[e] = beta != 0.0f ? (T)((float)v[e] + beta * (float)to[e]) : v[e];
+    }
+  }
+}
+
+// The filter as the data gradient reads it: class slot (ry, rx), then [c][i][j][fp] with i, j counting the class's taps
+// ky = ky0 + stride i, kx likewise; f .. fp-1 are zero.  Stride 1 (one class): the forward kernel walks the taps upwards
+// in dy, so they are turned round.
+struct FilterParams {
+  int f, c, kh, kw, fp;
+  int nhwc;                    // filter [f][kh][kw][c], else [f][c][kh][kw]
+  int stride_h, stride_w, pad_h, pad_w;
+  int turn;                    // 1: turned round (stride 1)
+  int64_t slot;                // elements of a class's slot
+};
+template <typename T>
+__global__ void __launch_bounds__(256)
+filter_kernel(const T* __restrict__ w, T* __restrict__ out, FilterParams p) {
+  const int ry = blockIdx.y / p.stride_w, rx = blockIdx.y % p.stride_w;
+  const int ky0 = p.turn ? 0 : (ry + p.pad_h) % p.stride_h, kx0 = p.turn ? 0 : (rx + p.pad_w) % p.stride_w;
+  const int nky = ky0 < p.kh ? (p.kh - 1 - ky0) / p.stride_h + 1 : 0;
+  const int nkx = kx0 < p.kw ? (p.kw - 1 - kx0) / p.stride_w + 1 : 0;
+  const int64_t total = (int64_t)p.c * nky * nkx * p.fp;
+  const int64_t idx   = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (idx >= total) return;
+  const int f = (int)(idx % p.fp);
+  int rest    = (int)(idx / p.fp);
+  const int j = rest % nkx;
+  rest /= nkx;
+  const int i = rest % nky, c = rest / nky;
+  const int ky = p.turn ? p.kh - 1 - i : ky0 + p.stride_h * i;
+  const int kx = p.turn ? p.kw - 1 - j : kx0 + p.stride_w * j;
+  T v = (T)0.0f;
+  if (f < p.f)
+    v = p.nhwc ? w[(((int64_t)f * p.kh + ky) * p.kw + kx) * p.c + c] : w[(((int64_t)f * p.c + c) * p.kh + ky) * p.kw + kx];
+  out[blockIdx.y * p.slot + idx] = v;
+}
+
+// ---- data gradient at a stride -------------------------------------------------------------------------------------
+struct DataParams {
+  const void* dy;    // [n][oh][ow][fp]
+  const void* wt;    // class slots of filter_kernel
+  void* dx;          // [n][h][w][c]
+  const void* zeros;
+  int n, h, w, c, oh, ow, fp, kh, kw;
+  int stride_h, stride_w, pad_h, pad_w;
+  int64_t slot;
+  float alpha, beta;
+};
+
+// rows are the pixels of one remainder class, K = (tap i, tap j, f): a chunk is 16 bytes of dy's pixel
+// (jy + oy0 - i, jx + ox0 - j), or zeros.  Load() is called for consecutive steps.
+template <typename T, int ROWS, int THREADS>
+struct DataTile {
+  static constexpr int E = 16 / (int)sizeof(T), KS = 8 * E, CHUNKS = ROWS * 8 / THREADS;
+  const T* dy;
+  const T* zeros;
+  int oh, ow, fp, nky, nkx;
+  int base[CHUNKS], oy[CHUNKS], ox[CHUNKS];
+  int f, i, j;  // position of the thread's chunk in the reduction
+
+  __device__ __forceinline__ void Init(const DataParams& p, int row0, int rows, int hc, int wc, int oy0, int ox0, int nky_, int nkx_,
+                                       int tid) {
+    dy = static_cast<const T*>(p.dy), zeros = static_cast<const T*>(p.zeros);
+    oh = p.oh, ow = p.ow, fp = p.fp, nky = nky_, nkx = nkx_;
+#pragma unroll
+    for (int q = 0; q < CHUNKS; ++q) {
+      const int m  = min(row0 + (tid >> 3) + THREADS / 8 * q, rows - 1);
+      const int jx = m % wc, jy = m / wc % hc, n = m / (wc * hc);
+      oy[q] = jy + oy0, ox[q] = jx + ox0;
+      base[q] = ((n * oh + oy[q]) * ow + ox[q]) * fp;
+    }
+    f = (tid & 7) * E;
+    i = j = 0;
+    Wrap();
+  }
+  __device__ __forceinline__ void Wrap() {
+    while (f >= fp) {
+      f -= fp;
+      if (++j >= nkx) j = 0, ++i;
+    }
+  }
+  template <bool GUARD>
+  __device__ __forceinline__ void Load(u32x4 (&r)[CHUNKS], int, int, int) {
+    const int tap = f - (i * ow + j) * fp;
+#pragma unroll
+    for (int q = 0; q < CHUNKS; ++q) {
+      const bool ok = i < nky && (unsigned)(oy[q] - i) < (unsigned)oh && (unsigned)(ox[q] - j) < (unsigned)ow;
+      r[q] = *reinterpret_cast<const u32x4*>(ok ? dy + (base[q] + tap) : zeros);
+    }
+    f += KS;
+    Wrap();
+  }
+  __device__ __forceinline__ void Store(char* tile, const u32x4 (&r)[CHUNKS], int tid) const {
+#pragma unroll
+    for (int q = 0; q < CHUNKS; ++q)
+      *reinterpret_cast<u32x4*>(tile + flex::Tile<T, true, ROWS, THREADS>::LdsOffset(tid, q)) = r[q];
+  }
+};
+
+template <typename T, int BM, int BN, int KG>
+__global__ void __launch_bounds__(256 * KG, 2)
+conv_data_kernel(DataParams p) {
+  __shared__ __attribute__((aligned(256))) char lds[2 * (BM + BN) * 128];
+  constexpr int KS = 128 / (int)sizeof(T);
+  const int tid = threadIdx.x;
+  const int ry = blockIdx.y / p.stride_w, rx = blockIdx.y % p.stride_w;
+  const int hc = (p.h - ry + p.stride_h - 1) / p.stride_h, wc = (p.w - rx + p.stride_w - 1) / p.stride_w;
+  const int rows = hc > 0 && wc > 0 ? p.n * hc * wc : 0;
+  const int ky0 = (ry + p.pad_h) % p.stride_h, kx0 = (rx + p.pad_w) % p.stride_w;
+  const int nky = ky0 < p.kh ? (p.kh - 1 - ky0) / p.stride_h + 1 : 0;
+  const int nkx = kx0 < p.kw ? (p.kw - 1 - kx0) / p.stride_w + 1 : 0;
+  const int k   = nky * nkx * p.fp;
+  const int tiles_m = (rows + BM - 1) / BM, tiles_n = (p.c + BN - 1) / BN;
+  if ((int)blockIdx.x >= tiles_m * tiles_n) return;  // the grid is the largest class's
+  int tm, tn;
+  flex::TileOf(blockIdx.x, tiles_m, tiles_n, &tm, &tn);
+  const int m0 = tm * BM, n0 = tn * BN;
+
+  DataTile<T, BM, 256 * KG> ta;
+  flex::Tile<T, true, BN, 256 * KG> tb;
+  ta.Init(p, m0, rows, hc, wc, (ry + p.pad_h - ky0) / p.stride_h, (rx + p.pad_w - kx0) / p.stride_w, nky, nkx, tid);
+  tb.Init(static_cast<const T*>(p.wt) + blockIdx.y * p.slot, k, n0, p.c, k, tid);
+  typename flex::Mma<T, true, true, BM, BN>::acc_t acc;
+  flex::KLoop<T, true, true, BM, BN, KG>(lds, ta, tb, 0, (k + KS - 1) / KS, k / KS, k, tid, acc);
+
+  const int col0 = n0 + tid % (BN / 8) * 8;
+  const int cols = min(p.c - col0, 8);
+  T* dx = static_cast<T*>(p.dx);
+  flex::EachRowGroup<T, true, true, BM, BN, KG>(lds, acc, tid, [&](int row, int, const float (&v)[8]) {
+    const int m = m0 + row;
+    if (m >= rows || cols <= 0) return;
+    const int jx = m % wc, jy = m / wc % hc, n = m / (wc * hc);
+    T* to = dx + ((int64_t)(n * p.h + jy * p.stride_h + ry) * p.w + jx * p.stride_w + rx) * p.c + col0;
+    typedef T vec8 __attribute__((ext_vector_type(8)));
+    if (cols == 8) {
+      vec8 out, old = {0, 0, 0, 0, 0, 0, 0, 0};
+      if (p.beta != 0.0f) __builtin_memcpy(&old, to, 8 * sizeof(T));
+#pragma unroll
+      for (int e = 0; e < 8; ++e) out[e] = (T)__builtin_fmaf(p.beta, (float)old[e], p.alpha * v[e]);
+      __builtin_memcpy(to, &out, 8 * sizeof(T));
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (e < cols) to[e] = (T)__builtin_fmaf(p.beta, p.beta != 0.0f ? (float)to[e] : 0.0f, p.alpha * v[e]);
+    }
+  });
+}
+
+// ---- filter gradient -----------------------------------------------------------------------------------------------
+struct FilterGradParams {
+  const void* dy;   // [pixels][fp]
+  const void* x;    // [n][h][w][cp]
+  const void* zeros;
+  float* planes;    // [split][f][kh kw cp]
+  int f, fp, cp, h, w, oh, ow, kw, taps;
+  int stride_h, stride_w, pad_h, pad_w, dil_h, dil_w;
+  int pixels, steps, steps_per_split;
+  int tiles_m, tiles_n;
+  int adv_n, adv_oy, adv_ox;  // a K step in images, rows and columns of the output
+};
+
+// the x operand: [pixel][ROWS columns of (tap, channel)].  A thread's chunks share one column chunk, i.e. one tap;
+// their pixels advance by one K step from call to call, carried through (ox, oy, n) without a division.
+template <typename T, int ROWS, int THREADS>
+struct ImageTile {
+  typedef flex::Tile<T, false, ROWS, THREADS> Plain;
+  static constexpr int E = Plain::E, KS = Plain::KS, CHUNKS = Plain::CHUNKS;
+  const T* x;
+  const T* zeros;
+  int h, w, cp, oh, ow, stride_h, stride_w, adv_n, adv_oy, adv_ox, pixels;
+  int dy, dx, c;  // the tap's offset and the first channel
+  int image[CHUNKS], oy[CHUNKS], ox[CHUNKS];  // image: offset of the pixel's image, in pixels of x
+
+  __device__ __forceinline__ void Init(const FilterGradParams& p, int col0, int step0, int tid) {
+    x = static_cast<const T*>(p.x), zeros = static_cast<const T*>(p.zeros);
+    h = p.h, w = p.w, cp = p.cp, oh = p.oh, ow = p.ow, stride_h = p.stride_h, stride_w = p.stride_w;
+    adv_n = p.adv_n * h * w, adv_oy = p.adv_oy, adv_ox = p.adv_ox, pixels = p.pixels;
+    const int col = min(col0 + tid % Plain::CH * E, p.taps * cp - E);  // what lies beyond the last column is not stored
+    const int tap = col / cp;
+    c  = col - tap * cp;
+    dy = tap / p.kw * p.dil_h - p.pad_h;
+    dx = tap % p.kw * p.dil_w - p.pad_w;
+#pragma unroll
+    for (int i = 0; i < CHUNKS; ++i) {
+      const int pixel = step0 * KS + Plain::ChunkK(tid, i);
+      const int n     = pixel / (oh * ow), rest = pixel - n * (oh * ow);
+      oy[i] = rest / ow, ox[i] = rest - oy[i] * ow;
+      image[i] = n * h * w;
+    }
+  }
+  template <bool GUARD>
+  __device__ __forceinline__ void Load(u32x4 (&r)[CHUNKS], int step, int, int tid) {
+#pragma unroll
+    for (int i = 0; i < CHUNKS; ++i) {
+      const int iy = oy[i] * stride_h + dy, ix = ox[i] * stride_w + dx;
+      const bool ok = (unsigned)iy < (unsigned)h && (unsigned)ix < (unsigned)w && (!GUARD || step * KS + Plain::ChunkK(tid, i) < pixels);
+      r[i] = *reinterpret_cast<const u32x4*>(ok ? x + ((image[i] + iy * w + ix) * cp + c) : zeros);
+      ox[i] += adv_ox;
+      const bool row = ox[i] >= ow;
+      ox[i] -= row ? ow : 0;
+      oy[i] += adv_oy + (row ? 1 : 0);
+      const bool next = oy[i] >= oh;
+      oy[i] -= next ? oh : 0;
+      image[i] += adv_n + (next ? h * w : 0);
+    }
+  }
+  __device__ __forceinline__ void Store(char* tile, const u32x4 (&r)[CHUNKS], int tid) const {
+#pragma unroll
+    for (int i = 0; i < CHUNKS; ++i) *reinterpret_cast<u32x4*>(tile + Plain::LdsOffset(tid, i)) = r[i];
+  }
+};
+
+template <typename T, int BM, int BN, int KG>
+__global__ void __launch_bounds__(256 * KG, 2)
+conv_filter_kernel(FilterGradParams p) {
+  __shared__ __attribute__((aligned(256))) char lds[2 * (BM + BN) * 128];
+  constexpr int KS = 128 / (int)sizeof(T);
+  const int tid = threadIdx.x;
+  int tm, tn;
+  flex::TileOf(blockIdx.x, p.tiles_m, p.tiles_n, &tm, &tn);
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int s0 = blockIdx.y * p.steps_per_split, s1 = min(s0 + p.steps_per_split, p.steps);
+
+  flex::Tile<T, false, BM, 256 * KG> ta;
+  ImageTile<T, BN, 256 * KG> tb;
+  ta.Init(p.dy, p.fp, m0, p.fp, p.pixels, tid);
+  tb.Init(p, n0, s0, tid);
+  typename flex::Mma<T, false, false, BM, BN>::acc_t acc;
+  flex::KLoop<T, false, false, BM, BN, KG>(lds, ta, tb, s0, s1, p.pixels / KS, p.pixels, tid, acc);
+
+  const int columns = p.taps * p.cp;  // a multiple of a chunk, not of eight, in fp32
+  const int col0    = n0 + tid % (BN / 8) * 8;
+  float* plane      = p.planes + (int64_t)blockIdx.y * p.f * columns;
+  flex::EachRowGroup<T, false, false, BM, BN, KG>(lds, acc, tid, [&](int row, int, const float (&v)[8]) {
+    const int m = m0 + row;
+    if (m >= p.f) return;
+    float* to = plane + (int64_t)m * columns + col0;
+    if (col0 + 4 <= columns) __builtin_memcpy(to, v, 16);
+    if (col0 + 8 <= columns) __builtin_memcpy(to + 4, v + 4, 16);
+  });
+}
+
+// Adds the planes and writes dw: a block takes 64 groups of four columns, its four rows of threads every fourth plane.
+template <typename T>
+__global__ void __launch_bounds__(256)
+filter_reduce_kernel(const float* __restrict__ planes, T* __restrict__ dw, int f, int taps, int c, int cp, int splits, int nhwc,
+                     float alpha, float beta) {
+  __shared__ __attribute__((aligned(16))) float part[3][64][4];
+  const int lane = threadIdx.x & 63, row = threadIdx.x >> 6;
+  const int64_t plane = (int64_t)f * taps * cp;
+  const int64_t at    = ((int64_t)blockIdx.x * 64 + lane) * 4;
+  flex::f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (at < plane) {
+#pragma unroll 4
+    for (int s = row; s < splits; s += 4) v += *reinterpret_cast<const flex::f32x4*>(planes + s * plane + at);
+  }
+  if (row > 0) *reinterpret_cast<flex::f32x4*>(part[row - 1][lane]) = v;
+  __syncthreads();
+  if (row > 0 || at >= plane) return;
+#pragma unroll
+  for (int r = 0; r < 3; ++r) v += *reinterpret_cast<const flex::f32x4*>(part[r][lane]);
+  const int ch   = (int)(at % cp);
+  const int tap  = (int)(at / cp % taps);
+  const int64_t filter = at / cp / taps;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if (ch + e >= c) break;
+    const int64_t o = nhwc ? (filter * taps + tap) * c + ch + e : (filter * c + ch + e) * taps + tap;
+    float g = alpha * v[e];
+    if (beta != 0.0f) g += beta * (float)dw[o];
+    dw[o] = (T)g;
+  }
+}
+
+// ---- host ----------------------------------------------------------------------------------------------------------
+int ChunkElems(const cinn_type_t& t) { return 16 / (t.bits / CHAR_BIT); }
+int RoundUp(int v, int to) { return (v + to - 1) / to * to; }
+bool Aligned(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+
+bool TypeSupported(const cinn_type_t& t) {
+  return (t.code == cinn_type_float && (t.bits == 16 || t.bits == 32)) || (t.code == cinn_type_bfloat && t.bits == 16);
+}
+
+template <typename T>
+void Pack(const void* in, void* out, bool nhwc, int n, int c, int plane, int cp, hipStream_t stream) {
+  const dim3 grid((plane + 63) / 64, (cp + 63) / 64, n);
+  if (nhwc) {
+    hipLaunchKernelGGL((pack_kernel<T, false>), grid, dim3(256), 0, stream, static_cast<const T*>(in), static_cast<T*>(out), c, plane, cp);
+  } else {
+    hipLaunchKernelGGL((pack_kernel<T, true>), grid, dim3(256), 0, stream, static_cast<const T*>(in), static_cast<T*>(out), c, plane, cp);
+  }
+}
+
+template <typename T>
+void Data(const ConvBackwardArgs& a, hipStream_t stream) {
+  constexpr int E = 16 / (int)sizeof(T);
+  const int fp        = RoundUp(a.f, E);
+  const bool pack_dy  = !a.nhwc || fp != a.f || !Aligned(a.dy);
+  const bool unpack   = !a.nhwc && (a.c > 1 && a.h * a.w_in > 1);
+  const bool forward  = a.stride_h == 1 && a.stride_w == 1 && (a.kh - 1) * a.dil_h >= a.pad_h && (a.kw - 1) * a.dil_w >= a.pad_w;
+  const int classes   = forward ? 1 : a.stride_h * a.stride_w;
+  const int64_t slot  = (int64_t)RoundUp(a.c * ((a.kh + a.stride_h - 1) / a.stride_h) * ((a.kw + a.stride_w - 1) / a.stride_w) * fp, 128);
+  auto bytes = [](int64_t elems) { return ((size_t)elems * sizeof(T) + 255) & ~(size_t)255; };
+  const size_t dy_bytes = pack_dy ? bytes((int64_t)a.n * a.oh * a.ow * fp) : 0;
+  const size_t wt_bytes = bytes(classes * slot);
+  const size_t dx_bytes = unpack ? bytes((int64_t)a.n * a.h * a.w_in * a.c) : 0;
+  char* scratch = static_cast<char*>(Scratch(ScratchKind::kTranspose, dy_bytes + wt_bytes + dx_bytes, stream));
+  const void* dy = a.dy;
+  if (pack_dy) {
+    Pack<T>(a.dy, scratch, a.nhwc, a.n, a.f, a.oh * a.ow, fp, stream);
+    dy = scratch;
+  }
+  void* wt = scratch + dy_bytes;
+  void* dx = unpack ? scratch + dy_bytes + wt_bytes : a.out;
+  FilterParams fpar{a.f, a.c, a.kh, a.kw, fp, a.nhwc ? 1 : 0, forward ? 1 : a.stride_h, forward ? 1 : a.stride_w, a.pad_h, a.pad_w, forward ? 1 : 0, slot};
+  hipLaunchKernelGGL(filter_kernel<T>, dim3((unsigned)((slot + 255) / 256), classes), dim3(256), 0, stream,
+                     static_cast<const T*>(a.w), static_cast<T*>(wt), fpar);
+  const float beta = unpack ? 0.0f : a.beta;  // the copy back adds it otherwise
+  if (forward) {
+    ConvNhwcArgs c;
+    c.x = dy, c.w = wt, c.y = dx;
+    c.scale = c.shift = nullptr;
+    c.residual       = beta != 0.0f ? dx : nullptr;
+    c.alpha          = a.alpha;
+    c.residual_scale = beta;
+    c.relu = c.nchw_input = false;
+    c.n = a.n, c.h = a.oh, c.w_in = a.ow, c.c = fp;
+    c.oc = a.c, c.kh = a.kh, c.kw = a.kw, c.oh = a.h, c.ow = a.w_in;
+    c.pad_h = (a.kh - 1) * a.dil_h - a.pad_h, c.pad_w = (a.kw - 1) * a.dil_w - a.pad_w;
+    c.stride_h = c.stride_w = 1;
+    c.dil_h = a.dil_h, c.dil_w = a.dil_w;
+    c.type = a.type;
+    RunConvNhwc(c, stream);
+  } else {
+    DataParams p{dy, wt, dx, ZeroPage(), a.n, a.h, a.w_in, a.c, a.oh, a.ow, fp, a.kh, a.kw, a.stride_h, a.stride_w, a.pad_h, a.pad_w,
+                 slot, a.alpha, beta};
+    const int rows = a.n * ((a.h + a.stride_h - 1) / a.stride_h) * ((a.w_in + a.stride_w - 1) / a.stride_w);
+    auto tiles = [&](int t) { return (unsigned)(((rows + t - 1) / t) * ((a.c + t - 1) / t)); };
+    bool large = false;
+    if constexpr (sizeof(T) == 2) {
+      // two blocks of 128x128 on every CU; fewer are better off as four times as many small ones
+      if (tiles(128) * classes >= 512) {
+        hipLaunchKernelGGL((conv_data_kernel<T, 128, 128, 1>), dim3(tiles(128), classes), dim3(256), 0, stream, p);
+        large = true;
+      }
+    }
+    if (!large) hipLaunchKernelGGL((conv_data_kernel<T, 64, 64, 1>), dim3(tiles(64), classes), dim3(256), 0, stream, p);
+  }
+  if (unpack) {
+    const int plane = a.h * a.w_in;
+    hipLaunchKernelGGL((unpack_kernel<T>), dim3((plane + 63) / 64, (a.c + 63) / 64, a.n), dim3(256), 0, stream,
+                       static_cast<const T*>(dx), static_cast<T*>(a.out), a.c, plane, a.beta);
+  }
+  CINN_HIP_CALL(hipGetLastError());
+}
+
+template <typename T>
+void Filter(const ConvBackwardArgs& a, hipStream_t stream) {
+  constexpr int E = 16 / (int)sizeof(T), KS = 8 * E;
+  const int fp = RoundUp(a.f, E), cp = RoundUp(a.c, E);
+  const bool pack_dy = !a.nhwc || fp != a.f || !Aligned(a.dy);
+  const bool pack_x  = !a.nhwc || cp != a.c || !Aligned(a.x);
+  auto bytes = [](int64_t elems) { return ((size_t)elems * sizeof(T) + 255) & ~(size_t)255; };
+  const size_t dy_bytes = pack_dy ? bytes((int64_t)a.n * a.oh * a.ow * fp) : 0;
+  const size_t x_bytes  = pack_x ? bytes((int64_t)a.n * a.h * a.w_in * cp) : 0;
+  char* scratch = dy_bytes + x_bytes ? static_cast<char*>(Scratch(ScratchKind::kTranspose, dy_bytes + x_bytes, stream)) : nullptr;
+  FilterGradParams p;
+  p.dy = a.dy, p.x = a.x, p.zeros = ZeroPage();
+  if (pack_dy) {
+    Pack<T>(a.dy, scratch, a.nhwc, a.n, a.f, a.oh * a.ow, fp, stream);
+    p.dy = scratch;
+  }
+  if (pack_x) {
+    Pack<T>(a.x, scratch + dy_bytes, a.nhwc, a.n, a.c, a.h * a.w_in, cp, stream);
+    p.x = scratch + dy_bytes;
+  }
+  p.f = a.f, p.fp = fp, p.cp = cp, p.h = a.h, p.w = a.w_in, p.oh = a.oh, p.ow = a.ow, p.kw = a.kw, p.taps = a.kh * a.kw;
+  p.stride_h = a.stride_h, p.stride_w = a.stride_w, p.pad_h = a.pad_h, p.pad_w = a.pad_w, p.dil_h = a.dil_h, p.dil_w = a.dil_w;
+  p.pixels = a.n * a.oh * a.ow;
+  p.steps  = (p.pixels + KS - 1) / KS;
+  p.adv_n  = KS / (a.oh * a.ow);
+  p.adv_oy = KS / a.ow % a.oh;
+  p.adv_ox = KS % a.ow;
+  const int columns = p.taps * cp;
+  const int bm = sizeof(T) == 2 && a.f > 64 ? 128 : 64;
+  const int bn = sizeof(T) == 2 && columns > 64 ? 128 : 64;
+  p.tiles_m = (a.f + bm - 1) / bm;
+  p.tiles_n = (columns + bn - 1) / bn;
+  const int tiles = p.tiles_m * p.tiles_n;
+  // blocks for two to three rounds of the chip, at least four K steps each, at most 64 MiB of planes
+  const int64_t plane = (int64_t)a.f * columns;
+  int splits = std::max(1, (bm == 128 ? 512 : 768) / tiles);
+  splits     = std::min(splits, std::max(1, p.steps / 4));
+  splits     = (int)std::min<int64_t>(splits, std::max<int64_t>(1, ((int64_t)16 << 20) / plane));
+  p.steps_per_split = (p.steps + splits - 1) / splits;
+  splits            = (p.steps + p.steps_per_split - 1) / p.steps_per_split;
+  p.planes = static_cast<float*>(Scratch(ScratchKind::kSplitK, (size_t)splits * plane * sizeof(float), stream));
+  const dim3 grid(tiles, splits);
+  bool done = false;
+  if constexpr (sizeof(T) == 2) {
+    done = true;
+    if (bm == 128 && bn == 128) {
+      hipLaunchKernelGGL((conv_filter_kernel<T, 128, 128, 1>), grid, dim3(256), 0, stream, p);
+    } else if (bm == 128) {
+      hipLaunchKernelGGL((conv_filter_kernel<T, 128, 64, 1>), grid, dim3(256), 0, stream, p);
+    } else if (bn == 128) {
+      hipLaunchKernelGGL((conv_filter_kernel<T, 64, 128, 1>), grid, dim3(256), 0, stream, p);
+    } else {
+      done = false;
+    }
+  }
+  if (!done) hipLaunchKernelGGL((conv_filter_kernel<T, 64, 64, 1>), grid, dim3(256), 0, stream, p);
+  hipLaunchKernelGGL((filter_reduce_kernel<T>), dim3((unsigned)((plane / 4 + 63) / 64)), dim3(256), 0, stream, p.planes,
+                     static_cast<T*>(a.out), a.f, p.taps, a.c, cp, splits, a.nhwc ? 1 : 0, a.alpha, a.beta);
+  CINN_HIP_CALL(hipGetLastError());
+}
+
+// everything is addressed with 32-bit element offsets, also with the channels rounded up
+bool Fits(const ConvBackwardArgs& a) {
+  const int e = ChunkElems(a.type);
+  const int64_t cp = RoundUp(a.c, e), fp = RoundUp(a.f, e), limit = INT_MAX / 2;
+  return TypeSupported(a.type) && a.n <= 65535 && a.n * (int64_t)a.h * a.w_in * cp < limit && a.n * (int64_t)a.oh * a.ow * fp < limit &&
+         cp * a.kh * a.kw * fp < limit && cp < (1 << 20) && fp < (1 << 20);
+}
+
+}  // namespace
+
+bool TryConvBackwardData(const ConvBackwardArgs& a, hipStream_t stream) {
+  if (!Fits(a)) return false;
+  const bool forward = a.stride_h == 1 && a.stride_w == 1 && (a.kh - 1) * a.dil_h >= a.pad_h && (a.kw - 1) * a.dil_w >= a.pad_w;
+  if (!forward && (a.dil_h != 1 || a.dil_w != 1 || a.stride_h * a.stride_w > 1024)) return false;
+  if (a.type.code == cinn_type_bfloat) {
+    Data<__bf16>(a, stream);
+  } else if (a.type.bits == 16) {
+    Data<_Float16>(a, stream);
+  } else {
+    Data<float>(a, stream);
+  }
+  return true;
+}
+
+bool TryConvBackwardFilter(const ConvBackwardArgs& a, hipStream_t stream) {
+  if (!Fits(a)) return false;
+  if (a.type.code == cinn_type_bfloat) {
+    Filter<__bf16>(a, stream);
+  } else if (a.type.bits == 16) {
+    Filter<_Float16>(a, stream);
+  } else {
+    Filter<float>(a, stream);
+  }
+  return true;
+}
+
+}  // namespace cinn_hip_kernels

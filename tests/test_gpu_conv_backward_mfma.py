@@ -1,0 +1,85 @@
+"""Convolution gradients on the matrix cores (conv_backward_mfma.hip) at the edges of their tiles, K steps, chunks and
+remainder classes, in both tensor formats, against the numpy oracle.
+
+Bound: operands are exact in the type and sums are fp32 (2^-24 of the sum of magnitudes per rounding, far fewer roundings
+in a row than terms: 2^-24 sqrt(terms) + 2^-22 covers them); a 16-bit result is half an ulp off itself, and one more half
+ulp of the intermediate that alpha / beta meet where the tensor is copied back to NCHW."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from oracle import backward as ob
+from cinn_amd import _lib, runtime
+
+from test_gpu_backward import CONV_ARGTYPES, conv_dims, conv_problem, from_dev, layout, round_to, to_dev, unlayout
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # n, c, h, w, f, k, stride, pad, dilation, groups
+    (1, 1, 1, 1, 1, 1, 1, 0, 1, 1),
+    (1, 3, 5, 70, 7, 3, 1, 1, 1, 1),     # an image's channels, one odd filter count
+    (2, 64, 9, 8, 64, 3, 1, 1, 1, 1),    # whole chunks: no copies in NHWC
+    (2, 65, 7, 9, 129, 3, 1, 1, 1, 1),   # one above the tiles
+    (1, 40, 11, 13, 24, 5, 1, 2, 2, 1),  # dilation
+    (1, 16, 6, 6, 8, 1, 1, 2, 1, 1),     # more padding than the window covers: the class kernel at stride 1
+    (3, 24, 13, 10, 40, 3, 2, 1, 1, 1),  # four classes of different extents
+    (2, 8, 9, 9, 136, 1, 2, 0, 1, 1),    # three classes without a tap
+    (1, 9, 17, 16, 12, 7, 3, 3, 1, 1),
+    (1, 16, 2, 2, 16, 3, 2, 1, 1, 1),    # one output pixel
+    (40, 72, 10, 11, 200, 3, 1, 1, 1, 1),  # many K steps, split
+]
+
+
+def bound(want, scale, terms, dtype):
+    ulp = {"float32": 2.0 ** -24, "float16": 2.0 ** -11, "bfloat16": 2.0 ** -8}[dtype]
+    return (2.0 ** -24 * np.sqrt(terms) + 2.0 ** -22) * scale + 2.0 * ulp * np.abs(want) + 2.0 ** -24
+
+
+@pytest.mark.parametrize("fmt", [0, 1])
+@pytest.mark.parametrize("dtype", ["float32", "float16", "bfloat16"])
+@pytest.mark.parametrize("case", CASES)
+def test_gradients(gpu, case, dtype, fmt):
+    n, c, h, w_, f, k, s, p, d, g = case
+    x, w, dy = conv_problem(case, dtype)
+    lib = _lib.load()
+    lib.cinn_call_cudnn_conv2d_backward_data.argtypes = CONV_ARGTYPES
+    lib.cinn_call_cudnn_conv2d_backward_filter.argtypes = CONV_ARGTYPES
+    X, W, DY = (to_dev(layout(t, fmt), dtype) for t in (x, w, dy))
+    nan_x, nan_w = np.full_like(x, np.nan), np.full_like(w, np.nan)  # beta = 0 does not read what was there
+    DX, DW = to_dev(layout(nan_x, fmt), dtype), to_dev(layout(nan_w, fmt), dtype)
+    dims = conv_dims(case, x, w, dy)
+    lib.cinn_call_cudnn_conv2d_backward_data(runtime.pod_args([W, DY, DX]), 3, fmt, 1.0, 0.0, *dims, None)
+    lib.cinn_call_cudnn_conv2d_backward_filter(runtime.pod_args([X, DY, DW]), 3, fmt, 1.0, 0.0, *dims, None)
+    runtime.synchronize()
+    geometry = ((s, s), (p, p), (d, d), g)
+    want, scale = (ob.conv2d_backward_data(q, r, x.shape, *geometry) for q, r in ((w, dy), (np.abs(w), np.abs(dy))))
+    assert np.all(np.abs(unlayout(from_dev(DX, dtype), fmt) - want) <= bound(want, scale, f * k * k, dtype))
+    want, scale = (ob.conv2d_backward_filter(q, r, w.shape, *geometry) for q, r in ((x, dy), (np.abs(x), np.abs(dy))))
+    assert np.all(np.abs(unlayout(from_dev(DW, dtype), fmt) - want) <= bound(want, scale, dy.size / f, dtype))
+
+
+@pytest.mark.parametrize("fmt", [0, 1])
+@pytest.mark.parametrize("dtype", ["float32", "float16"])
+@pytest.mark.parametrize("case", [CASES[3], CASES[6]])
+def test_alpha_beta(gpu, case, dtype, fmt):
+    n, c, h, w_, f, k, s, p, d, g = case
+    x, w, dy = conv_problem(case, dtype)
+    rng = np.random.default_rng(3)
+    dx0, dw0 = (round_to(rng.standard_normal(t.shape), dtype) for t in (x, w))
+    lib = _lib.load()
+    X, W, DY, DX, DW = (to_dev(layout(t, fmt), dtype) for t in (x, w, dy, dx0, dw0))
+    dims = conv_dims(case, x, w, dy)
+    lib.cinn_call_cudnn_conv2d_backward_data.argtypes = CONV_ARGTYPES
+    lib.cinn_call_cudnn_conv2d_backward_filter.argtypes = CONV_ARGTYPES
+    lib.cinn_call_cudnn_conv2d_backward_data(runtime.pod_args([W, DY, DX]), 3, fmt, 0.5, 2.0, *dims, None)
+    lib.cinn_call_cudnn_conv2d_backward_filter(runtime.pod_args([X, DY, DW]), 3, fmt, -1.5, 0.25, *dims, None)
+    runtime.synchronize()
+    geometry = ((s, s), (p, p), (d, d), g)
+    grad, scale = (ob.conv2d_backward_data(q, r, x.shape, *geometry) for q, r in ((w, dy), (np.abs(w), np.abs(dy))))
+    err = np.abs(unlayout(from_dev(DX, dtype), fmt) - (0.5 * grad + 2.0 * dx0))
+    assert np.all(err <= bound(np.abs(0.5 * grad) + np.abs(2.0 * dx0), 0.5 * scale + 2.0 * np.abs(dx0), f * k * k, dtype))
+    grad, scale = (ob.conv2d_backward_filter(q, r, w.shape, *geometry) for q, r in ((x, dy), (np.abs(x), np.abs(dy))))
+    err = np.abs(unlayout(from_dev(DW, dtype), fmt) - (-1.5 * grad + 0.25 * dw0))
+    assert np.all(err <= bound(np.abs(1.5 * grad) + np.abs(0.25 * dw0), 1.5 * scale + 0.25 * np.abs(dw0), dy.size / f, dtype))
