@@ -1541,7 +1541,7 @@ ir::LoweredFuncRef OpLowerer::LowerLibraryCall(const Group& group) const {
     } else {
       push_ints({y[0], y[3], y[1], y[2]});
     }
-  } else if (op == "argsort" || op == "sort") {
+  } else if (op == "argsort" || op == "sort" || op == "hip_top_k") {
     // [outer][size][inner] around the sorted axis; argsort writes indices and positions, sort the values
     api            = "cinn_call_hip_argsort";
     const auto& x  = n->inputs[0]->shape;
@@ -1560,8 +1560,13 @@ ir::LoweredFuncRef OpLowerer::LowerLibraryCall(const Group& group) const {
           << op << ": " << x[axis] << " elements along the sorted axis; the GPU kernel sorts rows of at most " << longest
           << " elements of this type (one block's LDS)";
     }
-    push_ints({static_cast<int>(outer), x[axis], static_cast<int>(inner), GetAttr<bool>(n->attrs, "is_ascend", true) ? 1 : 0,
-               op == "argsort" ? 3 : 4});
+    push_ints({static_cast<int>(outer), x[axis], static_cast<int>(inner), GetAttr<bool>(n->attrs, "is_ascend", true) ? 1 : 0});
+    if (op == "hip_top_k") {
+      api = "cinn_call_hip_top_k";
+      push_ints({GetAttr<int>(n->attrs, "k", 1), GetAttr<int>(n->attrs, "outputs", 3)});
+    } else {
+      push_ints({op == "argsort" ? 3 : 4});
+    }
   } else {
     CINN_CHECK(false) << "op " << op << " has no GPU lowering";
   }

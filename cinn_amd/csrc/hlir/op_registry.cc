@@ -719,6 +719,25 @@ OpRegistry::OpRegistry() {
       return std::vector<ShapeType>{in[0]};
     };
     srt.infer_dtype = SameTypeAsFirst;
+    // the first k entries of the sorted axis: values (bit 1 of `outputs`) and int64 indices (bit 2); what FuseTopK makes
+    // of sort / argsort with a slice behind them
+    auto& top       = r->Register("hip_top_k");
+    top.pattern     = OpPatternKind::kNonFusible;
+    top.infer_shape = [check_axis](const std::vector<ShapeType>& in, const AttributeMap& a) {
+      check_axis(in, a);
+      int axis = GetAttr<int>(a, "axis", 0);
+      if (axis < 0) axis += static_cast<int>(in[0].size());
+      ShapeType out = in[0];
+      out[axis]     = GetAttr<int>(a, "k", 1);
+      return std::vector<ShapeType>(GetAttr<int>(a, "outputs", 3) == 3 ? 2 : 1, out);
+    };
+    top.infer_dtype = [](const std::vector<Type>& in, const AttributeMap& a) {
+      const int outputs = GetAttr<int>(a, "outputs", 3);
+      std::vector<Type> types;
+      if (outputs & 1) types.push_back(in[0]);
+      if (outputs & 2) types.push_back(common::Int(64));
+      return types;
+    };
   }
   {
     // pooling output size and attribute meaning as cinn/hlir/pe/nn.cc:956-1109 (PoolImpl)

@@ -264,8 +264,15 @@ void cinn_call_cudnn_softmax_forward(void* v_args, int num_args, int mode, int f
 void cinn_call_hip_argsort(void* v_args, int num_args, int outer, int size, int inner, int is_ascend, int outputs,
                            void* stream);
 
-/* Gradients of the three calls above, with the reference's argument lists.  Gather-form kernels (one thread or block
- * per gradient element, fp32 accumulation), formats 0 = NCHW / [F][C][KH][KW] and 1 = NHWC / [F][KH][KW][C]; every result
+/* The first k entries, along the sorted axis, of the order cinn_call_hip_argsort gives: outputs bit 0 = values (the
+ * input's type), bit 1 = int64 indices, each [outer][k][inner]; v_args = {x, then the requested outputs in that order}.
+ * fp16 / bf16 / fp32 / int32; at most 16384 elements along the axis.  No counterpart in the reference, whose top_k is a
+ * composition of sort, argsort, slice and cast (cinn/frontend/decomposer/top_k.cc:22-47). */
+void cinn_call_hip_top_k(void* v_args, int num_args, int outer, int size, int inner, int is_ascend, int k, int outputs,
+                         void* stream);
+
+/* Gradients of the three calls above, with the reference's argument lists.  Convolutions without groups run on the
+ * matrix cores, everything else in gather form (fp32 accumulation), formats 0 = NCHW / [F][C][KH][KW] and 1 = NHWC / [F][KH][KW][C]; every result
  * is out = alpha * gradient + beta * out.
  * cinn_call_cudnn_conv2d_backward_data (cuda_util.cc:722-843): v_args = {w, dy, dx}.
  * cinn_call_cudnn_conv2d_backward_filter (cuda_util.cc:845-967): v_args = {x, dy, dw}. */
