@@ -337,6 +337,8 @@ int cinn_amd_computation_build_and_compile(cinn_amd_builder_t b, const char* con
           opts.fuse_stem_pool = v != 0;
         } else if (k == "fuse_matmul_bias") {
           opts.fuse_matmul_bias = v != 0;
+        } else if (k == "fuse_attention") {
+          opts.fuse_attention = v != 0;
         } else if (k == "fuse_conv_chain") {
           opts.fuse_conv_chain = v != 0;
         } else if (k == "fuse_shortcut_projection") {

@@ -65,6 +65,9 @@ void InvokeArgsort(const std::vector<BakedArg>& a, void* args, int32_t n, void* 
 void InvokeTopK(const std::vector<BakedArg>& a, void* args, int32_t n, void* stream) {
   cinn_call_hip_top_k(args, n, I(a[2]), I(a[3]), I(a[4]), I(a[5]), I(a[6]), I(a[7]), stream);
 }
+void InvokeAttention(const std::vector<BakedArg>& a, void* args, int32_t n, void* stream) {
+  cinn_call_hip_attention(args, n, F(a[2]), I(a[3]), I(a[4]), I(a[5]), I(a[6]), I(a[7]), I(a[8]), I(a[9]), I(a[10]), I(a[11]), stream);
+}
 void InvokeBatchedCublas(const std::vector<BakedArg>& a, void* args, int32_t n, void* stream) {
   cinn_call_batched_cublas(args, n, I(a[2]), B(a[3]), B(a[4]), B(a[5]), F(a[6]), F(a[7]), I(a[8]), I(a[9]), I(a[10]),
                            I(a[11]), I(a[12]), I(a[13]), I(a[14]), I(a[15]), stream);
@@ -112,6 +115,8 @@ ExternApiRegistry::ExternApiRegistry() {
   Register("cinn_call_hip_argsort", InvokeArgsort, 8);
   // (kernel_args, kernel_args_num, outer, size, inner, is_ascend, k, outputs, kernel_stream)
   Register("cinn_call_hip_top_k", InvokeTopK, 9);
+  // (kernel_args, kernel_args_num, scale, batch, heads, queries, keys, appended, d, operands, layouts, parts, kernel_stream)
+  Register("cinn_call_hip_attention", InvokeAttention, 13);
   // (kernel_args, kernel_args_num, opside, trans_a, trans_b, trans_o, alpha, beta, a1..a4, b1..b4, kernel_stream)
   Register("cinn_call_batched_cublas", InvokeBatchedCublas, 17);
   Register("cinn_call_cudnn_conv2d_backward_data", InvokeConv2dBackward<&cinn_call_cudnn_conv2d_backward_data>, 25);

@@ -29,6 +29,9 @@ class CinnComputation {
     // `matmul(x, W) + bias` with a const 2-D W and a const bias in a 16-bit type: the bias is added in the product's
     // epilogue (frontend/layout_pass.h); the result differs from the two operators by one rounding
     bool fuse_matmul_bias{true};
+    // `softmax(matmul(q, k^T)) v` per head as one call that reads split heads and appended caches where they lie
+    // (frontend/attention_pass.h); scores and probabilities are not rounded to the element type on the way
+    bool fuse_attention{true};
     // two folded 1x1 convolutions in a row whose channel counts the chain kernel takes become one call that writes
     // both results (frontend/layout_pass.h); same results as the two calls
     bool fuse_conv_chain{true};

@@ -1567,6 +1567,18 @@ ir::LoweredFuncRef OpLowerer::LowerLibraryCall(const Group& group) const {
     } else {
       push_ints({op == "argsort" ? 3 : 4});
     }
+  } else if (op == "hip_attention") {
+    api = "cinn_call_hip_attention";
+    args.push_back(Expr(GetAttr<float>(n->attrs, "scale", 1.0f)));
+    for (const char* name : {"batch", "heads", "queries", "keys", "appended", "d"}) push_ints({GetAttr<int>(n->attrs, name, 0)});
+    // operand slots refer to the instruction's inputs; the call's arguments are the group's, where equal values are one
+    const int slots = GetAttr<int>(n->attrs, "operands", 0);
+    int operands    = 0;
+    for (int s = 0; s < 5; ++s) {
+      const NodeData* in = n->inputs[(slots >> (4 * s)) & 15];
+      operands |= static_cast<int>(std::find(group.inputs.begin(), group.inputs.end(), in) - group.inputs.begin()) << (4 * s);
+    }
+    push_ints({operands, GetAttr<int>(n->attrs, "layouts", 0), GetAttr<int>(n->attrs, "parts", 1)});
   } else {
     CINN_CHECK(false) << "op " << op << " has no GPU lowering";
   }

@@ -740,6 +740,15 @@ OpRegistry::OpRegistry() {
     };
   }
   {
+    // what FuseAttention makes of the two products of an attention and the softmax between them
+    auto& op       = r->Register("hip_attention");
+    op.pattern     = OpPatternKind::kNonFusible;
+    op.infer_shape = [](const std::vector<ShapeType>&, const AttributeMap& a) {
+      return std::vector<ShapeType>{GetAttr<std::vector<int>>(a, "out_shape", {})};
+    };
+    op.infer_dtype = SameTypeAsFirst;
+  }
+  {
     // pooling output size and attribute meaning as cinn/hlir/pe/nn.cc:956-1109 (PoolImpl)
     auto& op       = r->Register("pool2d");
     op.pattern     = OpPatternKind::kNonFusible;

@@ -271,6 +271,15 @@ void cinn_call_hip_argsort(void* v_args, int num_args, int outer, int size, int 
 void cinn_call_hip_top_k(void* v_args, int num_args, int outer, int size, int inner, int is_ascend, int k, int outputs,
                          void* stream);
 
+/* Attention per head: out = softmax(scale q k^T) v over `keys` rows of keys and values and `appended` rows of a second
+ * piece, d <= 128 elements a row, a multiple of 16 bytes; fp16 / bf16 / fp32, scores and sums in fp32.  The softmax
+ * subtracts the row's maximum.  Operand slots 0..5 are q, k, appended k, v, appended v, out; v_args = {inputs..., out}.
+ * operands: four bits per input slot, which input it is (several slots may share one).  layouts: four bits per slot,
+ * 0 = [batch][heads][rows][d], 1 = [batch][rows][heads][d], 2 + j = part j of [batch][rows][parts][heads][d].  No
+ * counterpart in the reference, whose attention is a composition of matmul, softmax and transposes. */
+void cinn_call_hip_attention(void* v_args, int num_args, float scale, int batch, int heads, int queries, int keys,
+                             int appended, int d, int operands, int layouts, int parts, void* stream);
+
 /* Gradients of the three calls above, with the reference's argument lists.  Convolutions without groups run on the
  * matrix cores, everything else in gather form (fp32 accumulation), formats 0 = NCHW / [F][C][KH][KW] and 1 = NHWC / [F][KH][KW][C]; every result
  * is out = alpha * gradient + beta * out.
