@@ -65,6 +65,18 @@ void InvokeArgsort(const std::vector<BakedArg>& a, void* args, int32_t n, void* 
 void InvokeTopK(const std::vector<BakedArg>& a, void* args, int32_t n, void* stream) {
   cinn_call_hip_top_k(args, n, I(a[2]), I(a[3]), I(a[4]), I(a[5]), I(a[6]), I(a[7]), stream);
 }
+void InvokeChannelStatistics(const std::vector<BakedArg>& a, void* args, int32_t n, void* stream) {
+  cinn_call_hip_channel_statistics(args, n, I(a[2]), I(a[3]), stream);
+}
+void InvokeChannelNormalize(const std::vector<BakedArg>& a, void* args, int32_t n, void* stream) {
+  cinn_call_hip_channel_normalize(args, n, I(a[2]), I(a[3]), I(a[4]), F(a[5]), I(a[6]), stream);
+}
+void InvokeChannelGradientSums(const std::vector<BakedArg>& a, void* args, int32_t n, void* stream) {
+  cinn_call_hip_channel_gradient_sums(args, n, I(a[2]), I(a[3]), I(a[4]), I(a[5]), stream);
+}
+void InvokeChannelGradient(const std::vector<BakedArg>& a, void* args, int32_t n, void* stream) {
+  cinn_call_hip_channel_gradient(args, n, I(a[2]), I(a[3]), I(a[4]), I(a[5]), F(a[6]), stream);
+}
 void InvokeAttention(const std::vector<BakedArg>& a, void* args, int32_t n, void* stream) {
   cinn_call_hip_attention(args, n, F(a[2]), I(a[3]), I(a[4]), I(a[5]), I(a[6]), I(a[7]), I(a[8]), I(a[9]), I(a[10]), I(a[11]), stream);
 }
@@ -117,6 +129,13 @@ ExternApiRegistry::ExternApiRegistry() {
   Register("cinn_call_hip_top_k", InvokeTopK, 9);
   // (kernel_args, kernel_args_num, scale, batch, heads, queries, keys, appended, d, operands, layouts, parts, kernel_stream)
   Register("cinn_call_hip_attention", InvokeAttention, 13);
+  // (kernel_args, kernel_args_num, pixels, channels, kernel_stream)
+  Register("cinn_call_hip_channel_statistics", InvokeChannelStatistics, 5);
+  // (kernel_args, kernel_args_num, pixels, channels, operands, epsilon, relu, kernel_stream)
+  Register("cinn_call_hip_channel_normalize", InvokeChannelNormalize, 8);
+  // (kernel_args, kernel_args_num, pixels, channels, operands, masked[, epsilon], kernel_stream)
+  Register("cinn_call_hip_channel_gradient_sums", InvokeChannelGradientSums, 7);
+  Register("cinn_call_hip_channel_gradient", InvokeChannelGradient, 8);
   // (kernel_args, kernel_args_num, opside, trans_a, trans_b, trans_o, alpha, beta, a1..a4, b1..b4, kernel_stream)
   Register("cinn_call_batched_cublas", InvokeBatchedCublas, 17);
   Register("cinn_call_cudnn_conv2d_backward_data", InvokeConv2dBackward<&cinn_call_cudnn_conv2d_backward_data>, 25);

@@ -51,7 +51,7 @@ std::shared_ptr<CinnComputation> CinnComputation::Compile(const common::Target& 
   if (options.fuse_conv_bn_relu && options.fuse_shortcut_projection) lowered = FuseShortcutProjection(lowered, fetch_ids);
   lowered = FuseTopK(lowered, fetch_ids);
   if (options.fuse_attention) lowered = FuseAttention(lowered, fetch_ids);
-  if (options.use_decomposer) lowered = ApplyDecomposer(lowered);
+  if (options.use_decomposer) lowered = ApplyDecomposer(lowered, fetch_ids);
   if (options.split_reductions) lowered = SplitReductions(lowered, target.get_multi_processor_count());
   comp->graph_    = std::make_shared<Graph>(lowered, fetch_ids, target);
   comp->graph_->BuildFusionGroups();

@@ -1,6 +1,8 @@
 #include "frontend/decomposer.h"
 
 #include <algorithm>
+#include <climits>
+#include <map>
 
 #include "frontend/net_builder.h"
 #include "hlir/op.h"
@@ -139,9 +141,21 @@ struct BatchNormParts {
   }
 };
 
+// Channels-last batch norms with fp32 vectors are library calls: one pass over the tensor for both sums, one that applies
+// them.
+bool ChannelCallsTake(const Variable& x, const std::string& layout, const std::vector<Variable>& vectors) {
+  if (layout != "NHWC" || !(x->type.is_float(32) || x->type.is_float(16) || x->type.is_bfloat16())) return false;
+  for (auto& v : vectors)
+    if (!v->type.is_float(32) || v->shape != std::vector<int>{x->shape[3]}) return false;
+  int64_t pixels = 1;
+  for (int i = 0; i < 3; ++i) pixels *= x->shape[i];
+  return pixels > 0 && pixels < INT_MAX && x->shape[3] > 0;
+}
+
 bool Is16Bit(const common::Type& t) { return t.is_float16() || t.is_bfloat16(); }
 
-void DecomposeBatchNormTrain(const Instruction& instr, int serial, std::vector<Instruction>* out) {
+// `relu`: the only reader of y, where it is one; returns whether it has been computed along
+bool DecomposeBatchNormTrain(const Instruction& instr, const Instruction* relu, int serial, std::vector<Instruction>* out) {
   CINN_CHECK_EQ(instr->inputs.size(), 5u) << "batch_norm_train takes x, scale, bias, moving_mean, moving_variance";
   CINN_CHECK_EQ(instr->outputs.size(), 5u);
   auto x = instr->inputs[0], scale = instr->inputs[1], bias = instr->inputs[2], moving_mean = instr->inputs[3],
@@ -151,6 +165,18 @@ void DecomposeBatchNormTrain(const Instruction& instr, int serial, std::vector<I
   auto layout    = hlir::framework::GetAttr<std::string>(instr->attrs, "data_layout", "NCHW");
   SubBuilder b(serial);
   BatchNormParts h(&b, x->shape, layout);
+  if (ChannelCallsTake(x, layout, {scale, bias, moving_mean, moving_variance})) {
+    const std::vector<Variable> stats = b.CustomInstr("hip_channel_statistics", {x}, {});
+    const Variable y = b.CustomInstr("hip_channel_normalize", {x, stats[0], stats[1], scale, bias},
+                                     {{"epsilon", epsilon}, {"relu", relu != nullptr}})[0];
+    auto ins = b.TakeInstructions({{y, relu ? (*relu)->outputs[0] : instr->outputs[0]},
+                                   {stats[0], instr->outputs[1]},
+                                   {stats[1], instr->outputs[2]},
+                                   {h.Moving(moving_mean, stats[0], momentum), instr->outputs[3]},
+                                   {h.Moving(moving_variance, stats[1], momentum), instr->outputs[4]}});
+    out->insert(out->end(), ins.begin(), ins.end());
+    return true;
+  }
   const bool narrow = Is16Bit(x->type);
   Variable xf       = narrow ? b.Cast(x, "float32") : x;
   auto mean         = h.Mean(xf);
@@ -169,9 +195,11 @@ void DecomposeBatchNormTrain(const Instruction& instr, int serial, std::vector<I
                                  {new_mean, instr->outputs[3]},
                                  {new_variance, instr->outputs[4]}});
   out->insert(out->end(), ins.begin(), ins.end());
+  return false;
 }
 
-void DecomposeBatchNormGrad(const Instruction& instr, int serial, std::vector<Instruction>* out) {
+// `mask`: the relu_grad that makes dy, when the gradient is its only reader; returns whether it has been taken along
+bool DecomposeBatchNormGrad(const Instruction& instr, const Instruction* mask, int serial, std::vector<Instruction>* out) {
   CINN_CHECK_EQ(instr->inputs.size(), 5u) << "batch_norm_grad takes dy, x, scale, save_mean, save_variance";
   CINN_CHECK_EQ(instr->outputs.size(), 3u);
   auto y_grad = instr->inputs[0], x = instr->inputs[1], scale = instr->inputs[2], save_mean = instr->inputs[3],
@@ -180,6 +208,22 @@ void DecomposeBatchNormGrad(const Instruction& instr, int serial, std::vector<In
   auto layout   = hlir::framework::GetAttr<std::string>(instr->attrs, "data_layout", "NCHW");
   SubBuilder b(serial);
   BatchNormParts h(&b, x->shape, layout);
+  if (ChannelCallsTake(x, layout, {scale, save_mean, save_variance}) && y_grad->type == x->type) {
+    // a relu's mask goes into both passes over dy
+    const bool masked = mask && (*mask)->inputs[0]->type == x->type && (*mask)->inputs[1]->type == x->type &&
+                        (*mask)->inputs[0]->shape == x->shape && (*mask)->inputs[1]->shape == x->shape;
+    const Variable dy                = masked ? (*mask)->inputs[0] : y_grad;
+    std::vector<Variable> sum_inputs = {dy, x, save_mean};
+    if (masked) sum_inputs.push_back((*mask)->inputs[1]);
+    const std::vector<Variable> sums = b.CustomInstr("hip_channel_gradient_sums", sum_inputs, {{"masked", masked}});
+    std::vector<Variable> inputs     = {dy, x, save_mean, save_variance, scale, sums[0], sums[1]};
+    if (masked) inputs.push_back((*mask)->inputs[1]);
+    const Variable x_grad = b.CustomInstr("hip_channel_gradient", inputs, {{"epsilon", epsilon}, {"masked", masked}})[0];
+    const Variable scale_grad = b.Multiply(sums[1], h.StdVarianceInv(save_variance, epsilon));
+    auto ins = b.TakeInstructions({{x_grad, instr->outputs[0]}, {scale_grad, instr->outputs[1]}, {sums[0], instr->outputs[2]}});
+    out->insert(out->end(), ins.begin(), ins.end());
+    return masked;
+  }
   const bool narrow = Is16Bit(x->type);
   Variable xf  = narrow ? b.Cast(x, "float32") : x;
   Variable dyf = Is16Bit(y_grad->type) ? b.Cast(y_grad, "float32") : y_grad;
@@ -200,6 +244,7 @@ void DecomposeBatchNormGrad(const Instruction& instr, int serial, std::vector<In
   if (narrow) x_grad = b.Cast(x_grad, common::Type2Str(x->type));
   auto ins = b.TakeInstructions({{x_grad, instr->outputs[0]}, {scale_grad, instr->outputs[1]}, {bias_grad, instr->outputs[2]}});
   out->insert(out->end(), ins.begin(), ins.end());
+  return false;
 }
 
 // relu_grad(dout, out) = select(out > 0, dout, 0) (cinn/frontend/decomposer/activation.cc:40-55)
@@ -254,10 +299,48 @@ void DecomposeElementwiseAddGrad(const Instruction& instr, int serial, std::vect
 
 }  // namespace
 
-Program ApplyDecomposer(const Program& program) {
-  std::vector<Instruction> out;
+Program ApplyDecomposer(const Program& program, const std::set<std::string>& fetch_ids) {
+  const auto& instrs = program.instructions();
+  std::map<std::string, std::vector<size_t>> users;
+  std::map<std::string, size_t> defined_at;
+  for (size_t i = 0; i < instrs.size(); ++i) {
+    for (auto& in : instrs[i]->inputs) users[in->id].push_back(i);
+    for (auto& o : instrs[i]->outputs) defined_at[o->id] = i;
+  }
+  // the instruction of type `op` that reads v, nothing else does
+  auto only_reader = [&](const Variable& v, const char* op) -> int {
+    auto it = users.find(v->id);
+    if (fetch_ids.count(v->id) || it == users.end() || it->second.size() != 1) return -1;
+    return instrs[it->second[0]]->op_type == op ? static_cast<int>(it->second[0]) : -1;
+  };
+  // relus and their gradients that a batch norm takes along
+  std::vector<bool> taken(instrs.size(), false);
+  // decided before anything is emitted: a relu_grad stands before its batch_norm_grad
+  std::map<size_t, std::vector<Instruction>> decomposed;
   int serial = 0;
-  for (auto& ins : program.instructions()) {
+  for (size_t i = 0; i < instrs.size(); ++i) {
+    const auto& ins = instrs[i];
+    if (ins->op_type == "batch_norm_train") {
+      const int relu = only_reader(ins->outputs[0], "relu");
+      if (DecomposeBatchNormTrain(ins, relu < 0 ? nullptr : &instrs[relu], serial++, &decomposed[i]) && relu >= 0) taken[relu] = true;
+    } else if (ins->op_type == "batch_norm_grad") {
+      auto def       = defined_at.find(ins->inputs[0]->id);
+      const int mask = def != defined_at.end() && instrs[def->second]->op_type == "relu_grad" &&
+                               only_reader(ins->inputs[0], "batch_norm_grad") == static_cast<int>(i)
+                           ? static_cast<int>(def->second)
+                           : -1;
+      if (DecomposeBatchNormGrad(ins, mask < 0 ? nullptr : &instrs[mask], serial++, &decomposed[i])) taken[mask] = true;
+    }
+  }
+  std::vector<Instruction> out;
+  for (size_t i = 0; i < instrs.size(); ++i) {
+    const auto& ins = instrs[i];
+    if (taken[i]) continue;
+    auto done = decomposed.find(i);
+    if (done != decomposed.end()) {
+      out.insert(out.end(), done->second.begin(), done->second.end());
+      continue;
+    }
     if (ins->op_type == "softmax") {
       DecomposeSoftmax(ins, serial++, &out);
     } else if (ins->op_type == "batch_norm") {
@@ -266,10 +349,6 @@ Program ApplyDecomposer(const Program& program) {
       DecomposeReluGrad(ins, serial++, &out);
     } else if (ins->op_type == "elementwise_add_grad") {
       DecomposeElementwiseAddGrad(ins, serial++, &out);
-    } else if (ins->op_type == "batch_norm_train") {
-      DecomposeBatchNormTrain(ins, serial++, &out);
-    } else if (ins->op_type == "batch_norm_grad") {
-      DecomposeBatchNormGrad(ins, serial++, &out);
     } else {
       out.push_back(ins);
     }

@@ -137,6 +137,40 @@ class LayoutConverter {
         nhwc_[ins->outputs[0]->id] = y;
         return;
       }
+      // a gradient follows the gradient that comes in: x and w are transposed once where the convolution itself was
+      // converted, and the call packs nothing
+      if (nchw && !forward && groups == 1 && ins->inputs[1]->shape.size() == 4 && MfmaType(x->type) && HasTwin(ins->inputs[1])) {
+        const bool data       = GetAttr<std::string>(ins->attrs, "conv_type", "") == "backward_data";
+        AttributeMap attrs    = ins->attrs;
+        attrs["data_format"]  = std::string("NHWC");
+        attrs["output_shape"] = ToNhwc(GetAttr<ShapeType>(ins->attrs, "output_shape", {}));
+        nhwc_[ins->outputs[0]->id] = emit_.Emit1("conv2d", {data ? FilterToOhwi(x) : GetNhwc(x), GetNhwc(ins->inputs[1])}, attrs);
+        return;
+      }
+    } else if (op == "batch_norm_train" || op == "batch_norm_grad") {
+      // the first output is x or its gradient; the others are vectors
+      const bool train = op == "batch_norm_train";
+      auto x           = ins->inputs[train ? 0 : 1];
+      if (GetAttr<std::string>(ins->attrs, "data_layout", "NCHW") == "NCHW" && x->shape.size() == 4 && HasTwin(x)) {
+        AttributeMap attrs   = ins->attrs;
+        attrs["data_layout"] = std::string("NHWC");
+        std::vector<Variable> inputs = ins->inputs;
+        for (int i = 0; i < (train ? 1 : 2); ++i) inputs[i] = GetNhwc(inputs[i]);
+        nhwc_[ins->outputs[0]->id] = emit_.Emit1(op, inputs, attrs);
+        for (size_t i = 1; i < ins->outputs.size(); ++i) {
+          out_.back()->outputs[i] = ins->outputs[i];
+          have_nchw_.insert(ins->outputs[i]->id);
+        }
+        return;
+      }
+    } else if (op == "pool2d_grad") {
+      const auto &x = ins->inputs[0], &y = ins->inputs[1], &dy = ins->inputs[2];
+      if (GetAttr<std::string>(ins->attrs, "data_format", "NCHW") == "NCHW" && HasTwin(x) && dy->shape == y->shape) {
+        AttributeMap attrs   = ins->attrs;
+        attrs["data_format"] = std::string("NHWC");
+        nhwc_[ins->outputs[0]->id] = emit_.Emit1("pool2d_grad", {GetNhwc(x), GetNhwc(y), GetNhwc(dy)}, attrs);
+        return;
+      }
     } else if (op == "batch_norm") {
       auto x = ins->inputs[0];
       if (GetAttr<std::string>(ins->attrs, "data_layout", "NCHW") == "NCHW" && x->shape.size() == 4 && HasTwin(x)) {
@@ -168,7 +202,7 @@ class LayoutConverter {
       }
     } else {
       const auto* def = OpRegistry::Global().Find(op);
-      if (def && def->pattern == OpPatternKind::kElementWise && ins->outputs.size() == 1 &&
+      if (def && (def->pattern == OpPatternKind::kElementWise || op == "relu_grad") && ins->outputs.size() == 1 &&
           ins->outputs[0]->shape.size() == 4 && !ins->inputs.empty()) {
         bool same_shape = true, any_twin = false;
         for (auto& in : ins->inputs) {

@@ -9,6 +9,11 @@
 // pre-run instruction when the filter is marked const).  The reference has the same kind of pass for its x86
 // NCHWc kernels (cinn/hlir/pass/alterlayout.cc).
 //
+// A training step follows: batch_norm_train, its gradient, relu_grad and pool2d_grad of a channels-last tensor and the
+// convolution gradients of a channels-last dy are channels-last too.  Written in NCHW each of the two gradient calls
+// packed dy and one unpacked its result (5.7 to 6.4 us each for 12.8 MB), and a batch norm read and wrote transposed:
+// 208 -> 139 us for the step of a 64 -> 64 3x3 layer on 32 x 56x56 in fp16, batch norm's own calls included.
+//
 // FuseConvBatchNorm: folds `conv2d -> batch_norm [-> + residual] [-> relu]` on channels-last tensors into one
 // hip_conv2d_bn_relu call whose epilogue applies y = conv * s + t with s = scale / sqrt(variance + eps),
 // t = bias - mean * s (computed by ordinary fp32 instructions, pre-run for const statistics).

@@ -1567,6 +1567,25 @@ ir::LoweredFuncRef OpLowerer::LowerLibraryCall(const Group& group) const {
     } else {
       push_ints({op == "argsort" ? 3 : 4});
     }
+  } else if (op.rfind("hip_channel_", 0) == 0) {
+    const auto& x = n->inputs[0]->shape;
+    api           = "cinn_call_" + op;
+    push_ints({x[0] * x[1] * x[2], x[3]});
+    if (op != "hip_channel_statistics") {
+      // slots refer to the instruction's inputs; the call's arguments are the group's, where equal values are one
+      uint32_t operands = 0;
+      for (size_t s = 0; s < n->inputs.size(); ++s)
+        operands |= static_cast<uint32_t>(std::find(group.inputs.begin(), group.inputs.end(), n->inputs[s]) - group.inputs.begin()) << (4 * s);
+      push_ints({static_cast<int>(operands)});
+      const float epsilon = GetAttr<float>(n->attrs, "epsilon", 1e-5f);
+      if (op == "hip_channel_normalize") {
+        args.push_back(Expr(epsilon));
+        push_ints({GetAttr<bool>(n->attrs, "relu", false) ? 1 : 0});
+      } else {
+        push_ints({GetAttr<bool>(n->attrs, "masked", false) ? 1 : 0});
+        if (op == "hip_channel_gradient") args.push_back(Expr(epsilon));
+      }
+    }
   } else if (op == "hip_attention") {
     api = "cinn_call_hip_attention";
     args.push_back(Expr(GetAttr<float>(n->attrs, "scale", 1.0f)));

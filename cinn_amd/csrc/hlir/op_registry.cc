@@ -740,6 +740,30 @@ OpRegistry::OpRegistry() {
     };
   }
   {
+    // what the decomposer makes of a channels-last training batch norm: x -> mean, variance; x, mean, variance, scale,
+    // bias -> y; dy, x, mean[, out] -> sum of dy, sum of dy * (x - mean); dy, x, mean, variance, scale, those sums[, out]
+    // -> the gradient of x.  With out, dy counts as zero where out is not positive.
+    for (const char* name : {"hip_channel_statistics", "hip_channel_gradient_sums"}) {
+      auto& op       = r->Register(name);
+      op.pattern     = OpPatternKind::kNonFusible;
+      op.num_inputs  = -1;
+      op.infer_shape = [](const std::vector<ShapeType>& in, const AttributeMap&) {
+        CINN_CHECK_EQ(in[0].size(), 4u);
+        return std::vector<ShapeType>{{in[0][3]}, {in[0][3]}};
+      };
+      op.infer_dtype = [](const std::vector<Type>&, const AttributeMap&) {
+        return std::vector<Type>{common::Float(32), common::Float(32)};
+      };
+    }
+    for (const char* name : {"hip_channel_normalize", "hip_channel_gradient"}) {
+      auto& op       = r->Register(name);
+      op.pattern     = OpPatternKind::kNonFusible;
+      op.num_inputs  = -1;
+      op.infer_shape = SameShapeAsFirst;
+      op.infer_dtype = SameTypeAsFirst;
+    }
+  }
+  {
     // what FuseAttention makes of the two products of an attention and the softmax between them
     auto& op       = r->Register("hip_attention");
     op.pattern     = OpPatternKind::kNonFusible;

@@ -280,6 +280,24 @@ void cinn_call_hip_top_k(void* v_args, int num_args, int outer, int size, int in
 void cinn_call_hip_attention(void* v_args, int num_args, float scale, int batch, int heads, int queries, int keys,
                              int appended, int d, int operands, int layouts, int parts, void* stream);
 
+/* A training batch norm of channels-last tensors [pixels][channels] (fp16 / bf16 / fp32, one type per call), the
+ * per-channel vectors in fp32.  operands: four bits per operand slot, which of the call's inputs it is; the results follow
+ * the inputs in v_args.
+ * statistics: v_args = {x, mean, variance}, the variance as E(x^2) - mean^2.
+ * normalize: slots x, mean, variance, scale, bias -> (x - mean) * rsqrt(variance + epsilon) * scale + bias, relu after it
+ * or not.
+ * gradient_sums: slots dy, x, mean[, out] -> sum of dy, sum of dy * (x - mean).
+ * gradient: slots dy, x, mean, variance, scale, the two sums[, out] -> the gradient of x.
+ * masked: dy counts as zero where out is not positive.
+ * No counterpart in the reference, whose batch norms are compositions (cinn/frontend/decomposer/batch_norm.cc:22-262). */
+void cinn_call_hip_channel_statistics(void* v_args, int num_args, int pixels, int channels, void* stream);
+void cinn_call_hip_channel_normalize(void* v_args, int num_args, int pixels, int channels, int operands, float epsilon, int relu,
+                                     void* stream);
+void cinn_call_hip_channel_gradient_sums(void* v_args, int num_args, int pixels, int channels, int operands, int masked,
+                                         void* stream);
+void cinn_call_hip_channel_gradient(void* v_args, int num_args, int pixels, int channels, int operands, int masked, float epsilon,
+                                    void* stream);
+
 /* Gradients of the three calls above, with the reference's argument lists.  Convolutions without groups run on the
  * matrix cores, everything else in gather form (fp32 accumulation), formats 0 = NCHW / [F][C][KH][KW] and 1 = NHWC / [F][KH][KW][C]; every result
  * is out = alpha * gradient + beta * out.
