@@ -15,6 +15,12 @@
 namespace cinn {
 namespace frontend {
 
+// The three projections of one input that such an attention reads, x W + b with const W and b each, as one product with
+// joined weights (joined before the first run): one launch of three times the columns, which fills the chip where one of
+// them does not, instead of three.  Queries, keys and values are then parts of its rows, which hip_attention reads where
+// they lie; whatever else reads a part gets a slice.  Runs after PretransposeConstMatmulWeights.
+Program MergeProjections(const Program& program, const std::set<std::string>& fetch_ids);
+
 Program FuseAttention(const Program& program, const std::set<std::string>& fetch_ids);
 
 }  // namespace frontend

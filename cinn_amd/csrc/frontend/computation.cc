@@ -44,6 +44,7 @@ std::shared_ptr<CinnComputation> CinnComputation::Compile(const common::Target& 
   for (auto& in : program.GetInputs()) comp->input_names_.push_back(in->id);
 
   Program lowered = PretransposeConstMatmulWeights(program);
+  if (options.fuse_attention) lowered = MergeProjections(lowered, fetch_ids);
   if (options.conv_layout_nhwc) lowered = ConvertConvLayoutToNHWC(lowered, fetch_ids);
   if (options.fuse_conv_bn_relu) lowered = FuseConvBatchNorm(lowered, fetch_ids, options.fuse_stem_pool);
   if (options.fuse_matmul_bias) lowered = FuseMatmulBias(lowered, fetch_ids);

@@ -460,6 +460,23 @@ Program FuseMatmulBias(const Program& program, const std::set<std::string>& fetc
     auto def = defined_at.find(bias->id);
     if (def != defined_at.end() && def->second > i) continue;
     if (add->outputs[0]->shape != ShapeType{m, n} || !(add->outputs[0]->type == x->type)) continue;
+    // a tensor of the result's shape that is added next: the epilogue's residual
+    Variable residual, result = add->outputs[0];
+    size_t last = add_at;
+    auto next   = users.find(result->id);
+    if (!fetch_ids.count(result->id) && next != users.end() && next->second.size() == 1) {
+      const auto& sum = instrs[next->second[0]];
+      if (sum->op_type == "elementwise_add" && sum->inputs.size() == 2 && !(sum->inputs[0] == sum->inputs[1]) && !dropped[next->second[0]]) {
+        const Variable& other = sum->inputs[0] == result ? sum->inputs[1] : sum->inputs[0];
+        auto odef             = defined_at.find(other->id);
+        const bool wide       = odef != defined_at.end() && instrs[odef->second]->op_type == "broadcast_to";
+        if (other->shape == result->shape && other->type == x->type && sum->outputs[0]->shape == result->shape && !wide) {
+          residual = other;
+          result   = sum->outputs[0];
+          last     = next->second[0];
+        }
+      }
+    }
 
     std::vector<Instruction> seq;
     Emitter e(&seq, "mmb" + std::to_string(serial++) + "_");
@@ -472,12 +489,15 @@ Program FuseMatmulBias(const Program& program, const std::set<std::string>& fetc
                           {"dilation", std::vector<int>{1, 1}}, {"groups", 1},
                           {"data_format", std::string("NHWC")}, {"relu", false},
                           {"max_pool", false}};
-    auto y4 = e.Emit1("hip_conv2d_bn_relu", {x4, w4, ones, shift}, attrs);
-    e.EmitInto(add->outputs[0], "reshape", {y4}, {{"shape", ShapeType{m, n}}});
+    std::vector<Variable> operands = {x4, w4, ones, shift};
+    if (residual.defined()) operands.push_back(e.Emit1("reshape", {residual}, {{"shape", ShapeType{m, 1, 1, n}}}));
+    auto y4 = e.Emit1("hip_conv2d_bn_relu", operands, attrs);
+    e.EmitInto(result, "reshape", {y4}, {{"shape", ShapeType{m, n}}});
     dropped[i]      = true;
     dropped[add_at] = true;
     if (bcast_at >= 0) dropped[bcast_at] = true;
-    replacement[add_at] = seq;
+    dropped[last]     = true;
+    replacement[last] = seq;
   }
   if (replacement.empty()) return program;
   std::vector<Instruction> out;
