@@ -65,6 +65,9 @@ void InvokeArgsort(const std::vector<BakedArg>& a, void* args, int32_t n, void* 
 void InvokeTopK(const std::vector<BakedArg>& a, void* args, int32_t n, void* stream) {
   cinn_call_hip_top_k(args, n, I(a[2]), I(a[3]), I(a[4]), I(a[5]), I(a[6]), I(a[7]), stream);
 }
+void InvokeMatmulBias(const std::vector<BakedArg>& a, void* args, int32_t n, void* stream) {
+  cinn_call_hip_matmul_bias(args, n, I(a[2]), I(a[3]), I(a[4]), I(a[5]), stream);
+}
 void InvokeChannelStatistics(const std::vector<BakedArg>& a, void* args, int32_t n, void* stream) {
   cinn_call_hip_channel_statistics(args, n, I(a[2]), I(a[3]), stream);
 }
@@ -129,6 +132,8 @@ ExternApiRegistry::ExternApiRegistry() {
   Register("cinn_call_hip_top_k", InvokeTopK, 9);
   // (kernel_args, kernel_args_num, scale, batch, heads, queries, keys, appended, d, operands, layouts, parts, kernel_stream)
   Register("cinn_call_hip_attention", InvokeAttention, 13);
+  // (kernel_args, kernel_args_num, trans_b, m, n, k, kernel_stream)
+  Register("cinn_call_hip_matmul_bias", InvokeMatmulBias, 7);
   // (kernel_args, kernel_args_num, pixels, channels, kernel_stream)
   Register("cinn_call_hip_channel_statistics", InvokeChannelStatistics, 5);
   // (kernel_args, kernel_args_num, pixels, channels, operands, epsilon, relu, kernel_stream)

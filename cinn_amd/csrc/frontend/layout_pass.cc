@@ -1,6 +1,7 @@
 #include "frontend/layout_pass.h"
 
 #include <algorithm>
+#include <climits>
 #include <map>
 #include <set>
 
@@ -425,12 +426,11 @@ Program FuseMatmulBias(const Program& program, const std::set<std::string>& fetc
     if (mm->op_type != "matmul" || mm->inputs.size() != 2 || mm->outputs.size() != 1) continue;
     const Variable &x = mm->inputs[0], &w = mm->inputs[1], &prod = mm->outputs[0];
     if (x->shape.size() != 2 || w->shape.size() != 2 || prod->shape.size() != 2) continue;
-    if (GetAttr<bool>(mm->attrs, "trans_a", false) || !GetAttr<bool>(mm->attrs, "trans_b", false) ||
-        GetAttr<float>(mm->attrs, "alpha", 1.0f) != 1.0f)
-      continue;
+    if (GetAttr<bool>(mm->attrs, "trans_a", false) || GetAttr<float>(mm->attrs, "alpha", 1.0f) != 1.0f) continue;
     if (!(x->type.is_float16() || x->type.is_bfloat16()) || !(w->type == x->type)) continue;
-    const int m = x->shape[0], k = x->shape[1], n = w->shape[0];
-    if (w->shape[1] != k || prod->shape != ShapeType{m, n}) continue;
+    const bool trans_b = GetAttr<bool>(mm->attrs, "trans_b", false);
+    const int m = x->shape[0], k = x->shape[1], n = w->shape[trans_b ? 0 : 1];
+    if (w->shape[trans_b ? 1 : 0] != k || prod->shape != ShapeType{m, n}) continue;
     if (fetch_ids.count(prod->id)) continue;
     auto u = users.find(prod->id);
     if (u == users.end() || u->second.size() != 1) continue;
@@ -456,10 +456,21 @@ Program FuseMatmulBias(const Program& program, const std::set<std::string>& fetc
       continue;
     }
     if (bias->shape != ShapeType{n}) continue;
-    if (!(bias->is_const || known.count(bias->id))) continue;
-    auto def = defined_at.find(bias->id);
-    if (def != defined_at.end() && def->second > i) continue;
     if (add->outputs[0]->shape != ShapeType{m, n} || !(add->outputs[0]->type == x->type)) continue;
+    auto def = defined_at.find(bias->id);
+    if (!trans_b || !(bias->is_const || known.count(bias->id)) || (def != defined_at.end() && def->second > i)) {
+      // A layer in training: operands as they are, the bias converted in every run.  That launch costs what the pass over
+      // a small result does (2 to 3 us up to 4 MB; 14.8 us at 25 MB), so only large ones are taken.
+      if (static_cast<int64_t>(m) * n < (1 << 21) || static_cast<int64_t>(m) * n >= INT_MAX || n >= (1 << 22) || k >= (1 << 22)) continue;
+      std::vector<Instruction> seq;
+      Emitter e(&seq, "mmb" + std::to_string(serial++) + "_");
+      auto shift = bias->type == common::Float(32) ? bias : e.Emit1("cast", {bias}, {{"dtype", std::string("float32")}});
+      e.EmitInto(add->outputs[0], "hip_matmul_bias", {x, w, shift}, {{"trans_b", trans_b}});
+      dropped[i] = dropped[add_at] = true;
+      if (bcast_at >= 0) dropped[bcast_at] = true;
+      replacement[add_at] = seq;
+      continue;
+    }
     // a tensor of the result's shape that is added next: the epilogue's residual
     Variable residual, result = add->outputs[0];
     size_t last = add_at;

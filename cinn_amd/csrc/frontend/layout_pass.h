@@ -38,7 +38,8 @@ Program PretransposeConstMatmulWeights(const Program& program);
 // hip_conv2d_bn_relu call on the operands seen as 1x1 images (x as [M,1,1,K], W as [N,1,1,K]) with scale 1 and the
 // bias in fp32 as shift - a classifier's bias then costs no kernel of its own.  The sum is rounded once, from the
 // fp32 accumulator plus bias, where the two operators round the product first.
-// A [M][N] tensor that is added to that sum and nothing else is added as the epilogue's residual.
+// A [M][N] tensor that is added to that sum and nothing else is added as the epilogue's residual.  Operands of a layer
+// in training (W in either order, the bias not known before the run) make a hip_matmul_bias where the result is large.
 Program FuseMatmulBias(const Program& program, const std::set<std::string>& fetch_ids);
 // Two folded 1x1, stride 1, unpadded channels-last convolutions of which the second reads the first one's result
 // (the expansion that ends a ResNet bottleneck, with its shortcut and relu, and the reduction that starts the next):

@@ -1567,6 +1567,11 @@ ir::LoweredFuncRef OpLowerer::LowerLibraryCall(const Group& group) const {
     } else {
       push_ints({op == "argsort" ? 3 : 4});
     }
+  } else if (op == "hip_matmul_bias") {
+    // the product's operands are three arguments, or two where x is multiplied by itself
+    CINN_CHECK(n->inputs[2] != n->inputs[0] && n->inputs[2] != n->inputs[1]);
+    api = "cinn_call_hip_matmul_bias";
+    push_ints({GetAttr<bool>(n->attrs, "trans_b", false) ? 1 : 0, n->outputs[0]->shape[0], n->outputs[0]->shape[1], n->inputs[0]->shape[1]});
   } else if (op.rfind("hip_channel_", 0) == 0) {
     const auto& x = n->inputs[0]->shape;
     api           = "cinn_call_" + op;

@@ -764,6 +764,16 @@ OpRegistry::OpRegistry() {
     }
   }
   {
+    // a [M][K] product with B [K][N] or, trans_b, [N][K] plus an fp32 bias [N], rounded once (FuseMatmulBias)
+    auto& op       = r->Register("hip_matmul_bias");
+    op.pattern     = OpPatternKind::kNonFusible;
+    op.num_inputs  = 3;
+    op.infer_shape = [](const std::vector<ShapeType>& in, const AttributeMap&) {
+      return std::vector<ShapeType>{{in[0][0], in[2][0]}};
+    };
+    op.infer_dtype = SameTypeAsFirst;
+  }
+  {
     // what FuseAttention makes of the two products of an attention and the softmax between them
     auto& op       = r->Register("hip_attention");
     op.pattern     = OpPatternKind::kNonFusible;

@@ -280,6 +280,10 @@ void cinn_call_hip_top_k(void* v_args, int num_args, int outer, int size, int in
 void cinn_call_hip_attention(void* v_args, int num_args, float scale, int batch, int heads, int queries, int keys,
                              int appended, int d, int operands, int layouts, int parts, void* stream);
 
+/* C [m][n] = A [m][k] op(B) + bias, one rounding; B is [k][n], or [n][k] with trans_b.  fp16 / bf16 with an fp32 bias [n];
+ * n and k below 2^22.  v_args = {A, B, bias, C}, or {A, bias, C} where B is A. */
+void cinn_call_hip_matmul_bias(void* v_args, int num_args, int trans_b, int m, int n, int k, void* stream);
+
 /* A training batch norm of channels-last tensors [pixels][channels] (fp16 / bf16 / fp32, one type per call), the
  * per-channel vectors in fp32.  operands: four bits per operand slot, which of the call's inputs it is; the results follow
  * the inputs in v_args.

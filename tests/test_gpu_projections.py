@@ -114,3 +114,21 @@ def test_residual_after_a_bias(gpu, m, k, n, dtype, first):
     # fp32 sums of k terms and one rounding
     bound = UNIT[dtype] * np.abs(want) + k * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64) + np.abs(c64) + np.abs(r64))
     assert np.all(np.abs(got - want) <= 1.01 * bound + 1e-7)
+
+
+# a layer in training: weights in either order that are no constants; results of at least 2^21 elements
+# (smaller ones keep the separate addition), k with and without whole chunks, few and many columns
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("m,k,n", [(2048, 64, 1024), (2051, 768, 1030), (16400, 72, 128), (131, 200, 16384), (262144, 8, 8), (64, 256, 32768)])
+@pytest.mark.parametrize("trans_b", [False, True])
+def test_bias_of_a_layer_in_training(gpu, m, k, n, dtype, trans_b):
+    p = _Program(dtype, m + k + n)
+    x, x64 = p.put("x", (m, k))
+    w, w64 = p.put("w", (n, k) if trans_b else (k, n), k ** -0.5)
+    c, c64 = p.put("c", (n,), 0.5)
+    (got,), names = p.run([p.b.add(p.b.matmul(x, w, False, trans_b), c)])
+    assert sum("matmul_bias" in e for e in names) == 1 and not any("add" in e for e in names), names
+    w64 = w64.T if trans_b else w64
+    want = x64 @ w64 + c64
+    bound = UNIT[dtype] * np.abs(want) + k * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64) + np.abs(c64))
+    assert np.all(np.abs(got - want) <= 1.01 * bound + 1e-7)
