@@ -415,8 +415,10 @@ void Pack(const void* in, void* out, bool nhwc, int n, int c, int plane, int cp,
   }
 }
 
+// Both are false, with nothing launched, while the stream is captured and its scratch is too small for the copies and
+// planes: the gather kernels, which need none, take such a call.
 template <typename T>
-void Data(const ConvBackwardArgs& a, hipStream_t stream) {
+bool Data(const ConvBackwardArgs& a, hipStream_t stream) {
   constexpr int E = 16 / (int)sizeof(T);
   const int fp        = RoundUp(a.f, E);
   const bool pack_dy  = !a.nhwc || fp != a.f || !Aligned(a.dy);
@@ -428,6 +430,7 @@ void Data(const ConvBackwardArgs& a, hipStream_t stream) {
   const size_t dy_bytes = pack_dy ? bytes((int64_t)a.n * a.oh * a.ow * fp) : 0;
   const size_t wt_bytes = bytes(classes * slot);
   const size_t dx_bytes = unpack ? bytes((int64_t)a.n * a.h * a.w_in * a.c) : 0;
+  if (dy_bytes + wt_bytes + dx_bytes > ScratchLimit(ScratchKind::kTranspose, stream)) return false;
   char* scratch = static_cast<char*>(Scratch(ScratchKind::kTranspose, dy_bytes + wt_bytes + dx_bytes, stream));
   const void* dy = a.dy;
   if (pack_dy) {
@@ -454,6 +457,7 @@ void Data(const ConvBackwardArgs& a, hipStream_t stream) {
     c.stride_h = c.stride_w = 1;
     c.dil_h = a.dil_h, c.dil_w = a.dil_w;
     c.type = a.type;
+    c.whole_without_scratch = true;
     RunConvNhwc(c, stream);
   } else {
     DataParams p{dy, wt, dx, ZeroPage(), a.n, a.h, a.w_in, a.c, a.oh, a.ow, fp, a.kh, a.kw, a.stride_h, a.stride_w, a.pad_h, a.pad_w,
@@ -476,10 +480,11 @@ void Data(const ConvBackwardArgs& a, hipStream_t stream) {
                        static_cast<const T*>(dx), static_cast<T*>(a.out), a.c, plane, a.beta);
   }
   CINN_HIP_CALL(hipGetLastError());
+  return true;
 }
 
 template <typename T>
-void Filter(const ConvBackwardArgs& a, hipStream_t stream) {
+bool Filter(const ConvBackwardArgs& a, hipStream_t stream) {
   constexpr int E = 16 / (int)sizeof(T), KS = 8 * E;
   const int fp = RoundUp(a.f, E), cp = RoundUp(a.c, E);
   const bool pack_dy = !a.nhwc || fp != a.f || !Aligned(a.dy);
@@ -487,17 +492,7 @@ void Filter(const ConvBackwardArgs& a, hipStream_t stream) {
   auto bytes = [](int64_t elems) { return ((size_t)elems * sizeof(T) + 255) & ~(size_t)255; };
   const size_t dy_bytes = pack_dy ? bytes((int64_t)a.n * a.oh * a.ow * fp) : 0;
   const size_t x_bytes  = pack_x ? bytes((int64_t)a.n * a.h * a.w_in * cp) : 0;
-  char* scratch = dy_bytes + x_bytes ? static_cast<char*>(Scratch(ScratchKind::kTranspose, dy_bytes + x_bytes, stream)) : nullptr;
   FilterGradParams p;
-  p.dy = a.dy, p.x = a.x, p.zeros = ZeroPage();
-  if (pack_dy) {
-    Pack<T>(a.dy, scratch, a.nhwc, a.n, a.f, a.oh * a.ow, fp, stream);
-    p.dy = scratch;
-  }
-  if (pack_x) {
-    Pack<T>(a.x, scratch + dy_bytes, a.nhwc, a.n, a.c, a.h * a.w_in, cp, stream);
-    p.x = scratch + dy_bytes;
-  }
   p.f = a.f, p.fp = fp, p.cp = cp, p.h = a.h, p.w = a.w_in, p.oh = a.oh, p.ow = a.ow, p.kw = a.kw, p.taps = a.kh * a.kw;
   p.stride_h = a.stride_h, p.stride_w = a.stride_w, p.pad_h = a.pad_h, p.pad_w = a.pad_w, p.dil_h = a.dil_h, p.dil_w = a.dil_w;
   p.pixels = a.n * a.oh * a.ow;
@@ -518,7 +513,20 @@ void Filter(const ConvBackwardArgs& a, hipStream_t stream) {
   splits     = (int)std::min<int64_t>(splits, std::max<int64_t>(1, ((int64_t)16 << 20) / plane));
   p.steps_per_split = (p.steps + splits - 1) / splits;
   splits            = (p.steps + p.steps_per_split - 1) / p.steps_per_split;
-  p.planes = static_cast<float*>(Scratch(ScratchKind::kSplitK, (size_t)splits * plane * sizeof(float), stream));
+  const size_t plane_bytes = (size_t)splits * plane * sizeof(float);
+  if (dy_bytes + x_bytes > ScratchLimit(ScratchKind::kTranspose, stream) || plane_bytes > ScratchLimit(ScratchKind::kSplitK, stream))
+    return false;
+  char* scratch = dy_bytes + x_bytes ? static_cast<char*>(Scratch(ScratchKind::kTranspose, dy_bytes + x_bytes, stream)) : nullptr;
+  p.planes = static_cast<float*>(Scratch(ScratchKind::kSplitK, plane_bytes, stream));
+  p.dy = a.dy, p.x = a.x, p.zeros = ZeroPage();
+  if (pack_dy) {
+    Pack<T>(a.dy, scratch, a.nhwc, a.n, a.f, a.oh * a.ow, fp, stream);
+    p.dy = scratch;
+  }
+  if (pack_x) {
+    Pack<T>(a.x, scratch + dy_bytes, a.nhwc, a.n, a.c, a.h * a.w_in, cp, stream);
+    p.x = scratch + dy_bytes;
+  }
   const dim3 grid(tiles, splits);
   bool done = false;
   if constexpr (sizeof(T) == 2) {
@@ -537,6 +545,7 @@ void Filter(const ConvBackwardArgs& a, hipStream_t stream) {
   hipLaunchKernelGGL((filter_reduce_kernel<T>), dim3((unsigned)((plane / 4 + 63) / 64)), dim3(256), 0, stream, p.planes,
                      static_cast<T*>(a.out), a.f, p.taps, a.c, cp, splits, a.nhwc ? 1 : 0, a.alpha, a.beta);
   CINN_HIP_CALL(hipGetLastError());
+  return true;
 }
 
 // everything is addressed with 32-bit element offsets, also with the channels rounded up
@@ -553,26 +562,16 @@ bool TryConvBackwardData(const ConvBackwardArgs& a, hipStream_t stream) {
   if (!Fits(a)) return false;
   const bool forward = a.stride_h == 1 && a.stride_w == 1 && (a.kh - 1) * a.dil_h >= a.pad_h && (a.kw - 1) * a.dil_w >= a.pad_w;
   if (!forward && (a.dil_h != 1 || a.dil_w != 1 || a.stride_h * a.stride_w > 1024)) return false;
-  if (a.type.code == cinn_type_bfloat) {
-    Data<__bf16>(a, stream);
-  } else if (a.type.bits == 16) {
-    Data<_Float16>(a, stream);
-  } else {
-    Data<float>(a, stream);
-  }
-  return true;
+  if (a.type.code == cinn_type_bfloat) return Data<__bf16>(a, stream);
+  if (a.type.bits == 16) return Data<_Float16>(a, stream);
+  return Data<float>(a, stream);
 }
 
 bool TryConvBackwardFilter(const ConvBackwardArgs& a, hipStream_t stream) {
   if (!Fits(a)) return false;
-  if (a.type.code == cinn_type_bfloat) {
-    Filter<__bf16>(a, stream);
-  } else if (a.type.bits == 16) {
-    Filter<_Float16>(a, stream);
-  } else {
-    Filter<float>(a, stream);
-  }
-  return true;
+  if (a.type.code == cinn_type_bfloat) return Filter<__bf16>(a, stream);
+  if (a.type.bits == 16) return Filter<_Float16>(a, stream);
+  return Filter<float>(a, stream);
 }
 
 }  // namespace cinn_hip_kernels

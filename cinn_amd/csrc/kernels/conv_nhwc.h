@@ -28,6 +28,8 @@ struct ConvNhwcArgs {
   int oh, ow;
   int pad_h, pad_w, stride_h, stride_w, dil_h, dil_w;
   cinn_type_t type;  // element type of x, w, y and residual
+  // a split reduction that the scratch has no room for while the stream is captured stays whole, instead of aborting
+  bool whole_without_scratch = false;
   // A second channels-last input [N][h2][w2][c2] read through a 1x1 window on the output's pixel grid, or null:
   //   y[n, oy, ox, :] = act(conv(x, w[:, :kh kw c]) + w[:, kh kw c:] x2[n, oy stride2_h, ox stride2_w, :] + ...)
   // The filter rows are then [kh][kw][c] followed by c2 more values.  Only the implicit-GEMM kernels take it

@@ -776,13 +776,18 @@ int Launch(const ConvNhwcArgs& a, const Params& p_in, hipStream_t stream, const 
     return LaunchFailed(src, err, "hipFuncSetAttribute(MaxDynamicSharedMemorySize)");
   Params p = p_in;
   PlanSplits(&p, BM, BN, sizeof(T), src.fixed_partials ? src.fixed_partials_bytes : 0);
+  const size_t room = a.whole_without_scratch ? ScratchLimit(ScratchKind::kSplitK, stream) : SIZE_MAX;
+  if (p.splits > 1 && (size_t)p.splits * p.pixels * p.oc * sizeof(float) > room) {
+    p.splits          = 1;
+    p.steps_per_split = p.tail_steps;  // all of them
+  }
   const int tiles  = ((p.pixels + BM - 1) / BM) * ((p.oc + BN - 1) / BN);
   float* workspace = nullptr;
   int blocks       = tiles;
   if constexpr (std::is_same<T, float>::value && BM == 64 && BN == 64 && !NCHW_IN) {
     if (const size_t need = PlanTailSplit(&p, BM, BN, sizeof(T)); need > 0) {
-      if (src.fixed_partials && need > src.fixed_partials_bytes) {
-        p.full_tiles = tiles, p.tail_splits = 1;  // the fixed scratch is too small: every tile stays whole
+      if ((src.fixed_partials && need > src.fixed_partials_bytes) || need > room) {
+        p.full_tiles = tiles, p.tail_splits = 1;  // the scratch is too small: every tile stays whole
       } else {
         workspace = src.fixed_partials ? src.fixed_partials : static_cast<float*>(Scratch(ScratchKind::kSplitK, need, stream));
         blocks    = p.full_tiles + (tiles - p.full_tiles) * p.tail_splits;

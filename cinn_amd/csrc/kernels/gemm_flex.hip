@@ -230,11 +230,13 @@ void Launch(const FlexGemm& g, hipStream_t stream) {
   p.scale = g.scale, p.shift = g.shift, p.residual = g.residual;
   p.alpha = g.alpha, p.residual_scale = g.residual_scale, p.relu = g.relu ? 1 : 0;
   Plan plan         = ChoosePlan(g, p.steps);
+  const int64_t plane = (int64_t)g.batch * g.m * g.n;
+  // under capture without an eager run or a reservation: K whole, which needs no scratch
+  if (plan.splits > 1 && (size_t)plan.splits * plane * sizeof(float) > ScratchLimit(ScratchKind::kSplitK, stream)) plan.splits = 1;
   p.steps_per_split = (p.steps + plan.splits - 1) / plan.splits;
   plan.splits       = (p.steps + p.steps_per_split - 1) / p.steps_per_split;
   p.tiles_m         = (g.m + plan.tile - 1) / plan.tile;
   p.tiles_n         = (g.n + plan.tile - 1) / plan.tile;
-  const int64_t plane = (int64_t)g.batch * g.m * g.n;
   p.partials = plan.splits > 1 ? static_cast<float*>(Scratch(ScratchKind::kSplitK, (size_t)plan.splits * plane * sizeof(float), stream))
                                : nullptr;
   const dim3 grid((unsigned)(p.tiles_m * p.tiles_n), g.batch, plan.splits);

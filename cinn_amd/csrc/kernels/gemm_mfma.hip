@@ -1500,6 +1500,8 @@ struct GemmProblem {
   const ConvGeom* conv{nullptr};
   // the result is a layer's activation: leave it in L2 for the next kernel
   bool keep_in_cache{false};
+  // a split that the scratch has no room for while the stream is captured stays whole, instead of aborting
+  bool whole_without_scratch{false};
 };
 
 template <typename T, bool A_KC, bool B_KC>
@@ -1603,6 +1605,10 @@ std::atomic<unsigned long long*> g_gemm_probe{nullptr};
 template <typename T, bool B_KC, int BM, int BN, int WAVES_M, int WAVES_N, bool CONV = false, int NS = 2, bool FEED = false,
           bool PAIR = false>
 void LaunchDma16(const GemmProblem& p, hipStream_t stream, int splits = 1) {
+  using cinn_hip_kernels::ScratchKind;
+  if (p.whole_without_scratch && splits > 1 &&
+      (size_t)splits * p.m * p.n * sizeof(float) > cinn_hip_kernels::ScratchLimit(ScratchKind::kSplitK, stream))
+    splits = 1;
   int64_t ldb = p.trans_b ? p.k : p.n;
   const int tiles_m = (p.m + BM - 1) / BM, tiles_n = (p.n + BN - 1) / BN;
   // XCD rectangles for tile grids large enough to have panels to share; a small grid per batch entry is numbered
@@ -2135,6 +2141,7 @@ bool TryPointwiseConvAsGemm(const ConvNhwcArgs& a, hipStream_t stream) {
   p.residual_scale = a.residual_scale;
   p.relu           = a.relu;
   p.keep_in_cache  = true;
+  p.whole_without_scratch = a.whole_without_scratch;
   const bool taken = is_bf16 ? TryDma16<__bf16>(p, stream) : TryDma16<_Float16>(p, stream);
   if (taken) CINN_HIP_CALL(hipGetLastError());
   return taken;

@@ -1,5 +1,6 @@
 #include "runtime/scratch.h"
 
+#include <cstdint>
 #include <map>
 #include <mutex>
 #include <tuple>
@@ -27,6 +28,10 @@ Arena& TheArena() {
   static Arena* arena = new Arena;  // leaked on purpose: intrinsics may run during static teardown
   return *arena;
 }
+
+constexpr int kMaxDevices = 64;
+std::mutex g_page_mu;
+void* g_pages[kMaxDevices];  // one page of zeros per device, allocated and cleared on its first use there
 
 int CurrentDevice() {
   int device = 0;
@@ -69,19 +74,29 @@ void* Scratch(ScratchKind kind, size_t bytes, hipStream_t stream) {
   return Ensure(arena, kind, bytes ? bytes : 1, stream);
 }
 
+size_t ScratchLimit(ScratchKind kind, hipStream_t stream) {
+  if (!Capturing(stream)) return SIZE_MAX;
+  const int device = CurrentDevice();
+  if (device < kMaxDevices) {
+    std::lock_guard<std::mutex> lock(g_page_mu);
+    if (!g_pages[device]) return 0;
+  }
+  Arena& arena = TheArena();
+  std::lock_guard<std::mutex> lock(arena.mu);
+  auto it = arena.live.find({device, stream, static_cast<int>(kind)});
+  return it == arena.live.end() ? 0 : it->second.capacity;
+}
+
 const void* ZeroPage() {
-  constexpr int kMaxDevices = 64;
-  static std::mutex mu;
-  static void* pages[kMaxDevices];  // one page per device, allocated and cleared on its first use there
   const int device = CurrentDevice();
   CINN_RT_CHECK(device >= 0 && device < kMaxDevices, "device %d: the library keeps a page of zeros for at most %d devices", device,
                 kMaxDevices);
-  std::lock_guard<std::mutex> lock(mu);
-  if (!pages[device]) {
-    CINN_HIP_CALL(hipMalloc(&pages[device], 256));
-    CINN_HIP_CALL(hipMemset(pages[device], 0, 256));  // synchronous with respect to the host for device memory
+  std::lock_guard<std::mutex> lock(g_page_mu);
+  if (!g_pages[device]) {
+    CINN_HIP_CALL(hipMalloc(&g_pages[device], 256));
+    CINN_HIP_CALL(hipMemset(g_pages[device], 0, 256));  // synchronous with respect to the host for device memory
   }
-  return pages[device];
+  return g_pages[device];
 }
 
 }  // namespace cinn_hip_kernels
