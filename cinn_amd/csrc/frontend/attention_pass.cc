@@ -184,9 +184,11 @@ Program FuseAttention(const Program& program, const std::set<std::string>& fetch
     auto it = defined_at.find(v->id);
     return it == defined_at.end() ? nullptr : &instrs[it->second];
   };
+  std::vector<bool> dropped(instrs.size(), false);
   auto in_place = [&](const Variable& v) {
     const Instruction* def = source(v);
-    if (!def || !SplitsHeads(*def)) return Operand{v, 0, v->shape[v->shape.size() - 2], 1};
+    // a transpose that an earlier attention's call has taken along has no operand left: that call writes v itself
+    if (!def || !SplitsHeads(*def) || dropped[defined_at[v->id]]) return Operand{v, 0, v->shape[v->shape.size() - 2], 1};
     const Variable& split  = (*def)->inputs[0];
     const Operand own{split, 1, split->shape[1], 1};
     // one part of packed projections
@@ -217,7 +219,6 @@ Program FuseAttention(const Program& program, const std::set<std::string>& fetch
   };
   auto rows = [](const Operand& o) { return o.rows; };
 
-  std::vector<bool> dropped(instrs.size(), false);
   std::map<size_t, Instruction> replacement;
   for (size_t i = 0; i < instrs.size(); ++i) {
     const auto& qk = instrs[i];
