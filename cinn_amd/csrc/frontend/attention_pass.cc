@@ -2,6 +2,7 @@
 
 #include <algorithm>
 #include <climits>
+#include <cmath>
 #include <map>
 #include <vector>
 
@@ -29,6 +30,46 @@ struct Operand {
 bool SplitsHeads(const Instruction& ins) {
   return ins->op_type == "transpose" && ins->inputs.size() == 1 && ins->inputs[0]->shape.size() == 4 &&
          GetAttr<std::vector<int>>(ins->attrs, "axis", {}) == std::vector<int>{0, 2, 1, 3};
+}
+
+// The matmul at qk, the softmax that alone reads it and the matmul that alone reads that, where hip_attention computes the
+// same: fills in the positions of the other two.
+bool IsAttention(const std::vector<Instruction>& instrs, const std::map<std::string, std::vector<size_t>>& users,
+                 const std::set<std::string>& fetch_ids, const Instruction& qk, size_t* softmax_at, size_t* pv_at) {
+  auto only_reader = [&](const Variable& v, size_t* at) {
+    auto it = users.find(v->id);
+    if (fetch_ids.count(v->id) || it == users.end() || it->second.size() != 1) return false;
+    *at = it->second[0];
+    return true;
+  };
+  if (qk->op_type != "matmul" || qk->inputs.size() != 2 || GetAttr<bool>(qk->attrs, "trans_a", false) ||
+      !GetAttr<bool>(qk->attrs, "trans_b", false))
+    return false;
+  const Variable &q = qk->inputs[0], &k = qk->inputs[1];
+  const int rank = static_cast<int>(q->shape.size());
+  if ((rank != 3 && rank != 4) || k->shape.size() != q->shape.size() || !(q->type == k->type)) return false;
+  if (!q->type.is_float(32) && !q->type.is_float(16) && !q->type.is_bfloat16()) return false;
+  // 0 times a score that overflows is no number, nor is the softmax of infinite ones: left to the operators
+  const float alpha = GetAttr<float>(qk->attrs, "alpha", 1.0f);
+  if (alpha == 0.0f || !std::isfinite(alpha)) return false;
+  if (!only_reader(qk->outputs[0], softmax_at) || instrs[*softmax_at]->op_type != "softmax") return false;
+  const auto axes = GetAttr<std::vector<int>>(instrs[*softmax_at]->attrs, "axes", {-1});
+  if (axes.size() != 1 || (axes[0] != -1 && axes[0] != rank - 1)) return false;
+  if (!only_reader(instrs[*softmax_at]->outputs[0], pv_at)) return false;
+  const auto& pv = instrs[*pv_at];
+  if (pv->op_type != "matmul" || pv->inputs.size() != 2 || !(pv->inputs[0] == instrs[*softmax_at]->outputs[0]) ||
+      GetAttr<bool>(pv->attrs, "trans_a", false) || GetAttr<bool>(pv->attrs, "trans_b", false) ||
+      GetAttr<float>(pv->attrs, "alpha", 1.0f) != 1.0f)
+    return false;
+  // the same batch entries and row length throughout
+  const Variable& v = pv->inputs[1];
+  const int d = q->shape[rank - 1], queries = q->shape[rank - 2], keys = k->shape[rank - 2];
+  if (v->shape != k->shape || !(v->type == q->type) || k->shape[rank - 1] != d || keys < 1 || queries < 1) return false;
+  if (!std::equal(q->shape.begin(), q->shape.end() - 2, k->shape.begin())) return false;
+  if (d > 128 || d % (16 / q->type.bytes()) != 0) return false;
+  const int batch = q->shape[0], heads = rank == 4 ? q->shape[1] : 1;
+  return static_cast<int64_t>(batch) * heads * queries < INT_MAX &&
+         static_cast<int64_t>(batch) * heads * d * std::max(queries, keys) < INT_MAX;
 }
 
 // x W + b with a const 2-D W stored [N][K] (its transposition may stand before it) and a const b, split into heads
@@ -95,23 +136,16 @@ Program MergeProjections(const Program& program, const std::set<std::string>& fe
   std::map<size_t, Instruction> replacement;
   int serial = 0;
   for (auto& qk : instrs) {
-    // the products FuseAttention makes one call of
-    if (qk->op_type != "matmul" || qk->inputs.size() != 2 || !GetAttr<bool>(qk->attrs, "trans_b", false) ||
-        GetAttr<bool>(qk->attrs, "trans_a", false) || qk->inputs[0]->shape.size() != 4)
-      continue;
-    const auto& type = qk->inputs[0]->type;
-    const int d      = qk->inputs[0]->shape[3];
-    if (!(type.is_float(32) || type.is_float(16) || type.is_bfloat16()) || d > 128 || d % (16 / type.bytes()) != 0) continue;
-    const Instruction* softmax = only_reader(qk->outputs[0]);
-    const Instruction* pv      = softmax && (*softmax)->op_type == "softmax" ? only_reader((*softmax)->outputs[0]) : nullptr;
-    if (!pv || (*pv)->op_type != "matmul" || (*pv)->inputs.size() != 2) continue;
+    size_t softmax_at, pv_at;
+    if (!IsAttention(instrs, users, fetch_ids, qk, &softmax_at, &pv_at) || qk->inputs[0]->shape.size() != 4) continue;
+    const Instruction& pv = instrs[pv_at];
     // what this program computes of keys and values: all of them, or what it appends to a cache
     auto computed = [&](const Variable& v) {
       const Instruction* def = source(v);
       return def && (*def)->op_type == "concat" && (*def)->inputs.size() == 2 ? (*def)->inputs[1] : v;
     };
     Projection p[3];
-    if (!projection(qk->inputs[0], &p[0]) || !projection(computed(qk->inputs[1]), &p[1]) || !projection(computed((*pv)->inputs[1]), &p[2]))
+    if (!projection(qk->inputs[0], &p[0]) || !projection(computed(qk->inputs[1]), &p[1]) || !projection(computed(pv->inputs[1]), &p[2]))
       continue;
     bool alike = p[0].add != p[1].add && p[1].add != p[2].add && p[0].add != p[2].add;
     for (auto& q : p)
@@ -222,34 +256,13 @@ Program FuseAttention(const Program& program, const std::set<std::string>& fetch
   std::map<size_t, Instruction> replacement;
   for (size_t i = 0; i < instrs.size(); ++i) {
     const auto& qk = instrs[i];
-    if (qk->op_type != "matmul" || qk->inputs.size() != 2 || GetAttr<bool>(qk->attrs, "trans_a", false) ||
-        !GetAttr<bool>(qk->attrs, "trans_b", false))
-      continue;
-    const Variable &q = qk->inputs[0], &k = qk->inputs[1];
-    const int rank = static_cast<int>(q->shape.size());
-    if ((rank != 3 && rank != 4) || k->shape.size() != q->shape.size() || !(q->type == k->type)) continue;
-    if (!q->type.is_float(32) && !q->type.is_float(16) && !q->type.is_bfloat16()) continue;
-    const int softmax_at = single_user(qk->outputs[0]);
-    if (softmax_at < 0 || instrs[softmax_at]->op_type != "softmax") continue;
-    const auto axes = GetAttr<std::vector<int>>(instrs[softmax_at]->attrs, "axes", {-1});
-    if (axes.size() != 1 || (axes[0] != -1 && axes[0] != rank - 1)) continue;
-    const int pv_at = single_user(instrs[softmax_at]->outputs[0]);
-    if (pv_at < 0) continue;
+    size_t softmax_at, pv_at;
+    if (!IsAttention(instrs, users, fetch_ids, qk, &softmax_at, &pv_at)) continue;
     const auto& pv = instrs[pv_at];
-    if (pv->op_type != "matmul" || pv->inputs.size() != 2 || !(pv->inputs[0] == instrs[softmax_at]->outputs[0]) ||
-        GetAttr<bool>(pv->attrs, "trans_a", false) || GetAttr<bool>(pv->attrs, "trans_b", false) ||
-        GetAttr<float>(pv->attrs, "alpha", 1.0f) != 1.0f)
-      continue;
-    const Variable& v = pv->inputs[1];
-    // the same batch entries and row length throughout
+    const Variable &q = qk->inputs[0], &k = qk->inputs[1], &v = pv->inputs[1];
+    const int rank = static_cast<int>(q->shape.size());
     const int d = q->shape[rank - 1], queries = q->shape[rank - 2], keys = k->shape[rank - 2];
-    if (v->shape != k->shape || !(v->type == q->type) || k->shape[rank - 1] != d || keys < 1 || queries < 1) continue;
-    if (!std::equal(q->shape.begin(), q->shape.end() - 2, k->shape.begin())) continue;
-    if (d > 128 || d % (16 / q->type.bytes()) != 0) continue;
     const int batch = q->shape[0], heads = rank == 4 ? q->shape[1] : 1;
-    if (static_cast<int64_t>(batch) * heads * queries >= INT_MAX ||
-        static_cast<int64_t>(batch) * heads * d * std::max(queries, keys) >= INT_MAX)
-      continue;
 
     auto ks = pieces(k), vs = pieces(v);
     // pieces that do not correspond: the joined tensors

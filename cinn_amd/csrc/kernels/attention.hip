@@ -59,27 +59,29 @@ __device__ __forceinline__ const char* HeadOf(const Rows& r, int b, int h) {
   return static_cast<const char*>(r.base) + (b * r.batch + h * r.head) * (int64_t)sizeof(T);
 }
 
-// exp(|scale| (s - m)); the scale's sign has gone into the query.  Full accuracy for fp32; v_exp_f32 (2^-22 or so) of one
+// exp(|scale| (s - m)); the scale's sign has gone into the query (a scale of 0 too: there the query is zero and the
+// factor 1, since 0 * -inf of a maximum not yet found or of a masked key is no number).  Full accuracy for fp32; v_exp_f32 (2^-22 or so) of one
 // fused multiply-add where the result is rounded to 16 bits anyway.  -inf for m (no finite score so far) must not make
 // -inf - -inf of scores.
 template <typename T>
 struct Exp {
   float c;
-  __device__ __forceinline__ explicit Exp(float scale) : c(fabsf(scale) * 1.4426950408889634f) {}
+  __device__ __forceinline__ explicit Exp(float scale) : c(scale == 0.0f ? 1.0f : fabsf(scale) * 1.4426950408889634f) {}
   __device__ __forceinline__ float Base(float m) const { return m == -__builtin_inff() ? 0.0f : m * c; }
   __device__ __forceinline__ float operator()(float s, float base) const { return __builtin_amdgcn_exp2f(__builtin_fmaf(s, c, -base)); }
 };
 template <>
 struct Exp<float> {
   float c;
-  __device__ __forceinline__ explicit Exp(float scale) : c(fabsf(scale)) {}
+  __device__ __forceinline__ explicit Exp(float scale) : c(scale == 0.0f ? 1.0f : fabsf(scale)) {}
   __device__ __forceinline__ float Base(float m) const { return m == -__builtin_inff() ? 0.0f : m; }
   __device__ __forceinline__ float operator()(float s, float base) const { return expf((s - base) * c); }
 };
 
-// a chunk of the query, negated where the scale is negative
+// a chunk of the query, negated where the scale is negative, zero where it is zero
 template <typename T>
 __device__ __forceinline__ u32x4 Signed(u32x4 v, float scale) {
+  if (scale == 0.0f) return u32x4{0, 0, 0, 0};
   return scale < 0.0f ? v ^ (sizeof(T) == 4 ? 0x80000000u : 0x80008000u) : v;
 }
 

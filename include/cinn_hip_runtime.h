@@ -273,7 +273,7 @@ void cinn_call_hip_top_k(void* v_args, int num_args, int outer, int size, int in
 
 /* Attention per head: out = softmax(scale q k^T) v over `keys` rows of keys and values and `appended` rows of a second
  * piece, d <= 128 elements a row, a multiple of 16 bytes; fp16 / bf16 / fp32, scores and sums in fp32.  The softmax
- * subtracts the row's maximum.  Operand slots 0..5 are q, k, appended k, v, appended v, out; v_args = {inputs..., out}.
+ * subtracts the row's maximum; with scale 0 every key counts the same.  Operand slots 0..5 are q, k, appended k, v, appended v, out; v_args = {inputs..., out}.
  * operands: four bits per input slot, which input it is (several slots may share one).  layouts: four bits per slot,
  * 0 = [batch][heads][rows][d], 1 = [batch][rows][heads][d], 2 + j = part j of [batch][rows][parts][heads][d].  No
  * counterpart in the reference, whose attention is a composition of matmul, softmax and transposes. */
