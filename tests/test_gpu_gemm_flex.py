@@ -5,9 +5,12 @@ chunk; enough tiles for the 128x128 forms; few tiles and a long K for the split 
 Bounds: the inputs are exact in the type, sums are fp32: every rounding of a sum of k products is at most 2^-24 of the
 sum of their magnitudes, and a blocked sum has far fewer of them in a row than k, so 2^-24 * sqrt(k) + 2^-22 of that
 magnitude covers it; a 16-bit result adds half an ulp of itself (2^-11 fp16, 2^-8 bf16)."""
+import ctypes
+
 import numpy as np
 import pytest
 
+from cinn_amd import _lib, runtime
 from cinn_amd.common import bfloat16_bits_to_float32, float32_to_bfloat16_bits
 
 from test_gpu_gemm import call_cublas
@@ -61,3 +64,28 @@ def test_what_lies_beyond_k_is_not_multiplied(gpu, kind, ta, tb):
     want = a[0].astype(np.float64) @ b.astype(np.float64).T
     assert np.all(np.isfinite(got[0].astype(np.float64)))
     np.testing.assert_allclose(got[0].astype(np.float64), want, rtol=2.0 ** -10, atol=2.0 ** -10)
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False)])
+@pytest.mark.parametrize("batch,m,n,k,split", [(1, 128, 128, 4096, True), (1, 256, 128, 2048, True), (3, 128, 256, 1024, True),
+                                               (1, 512, 1024, 1024, True), (1, 1024, 1024, 96, False), (2, 128, 128, 32, False)])
+def test_whole_fp32_tiles_that_leave_cus_idle_split_k(gpu, batch, m, n, k, split, ta, tb):
+    """extents that are whole 128x128 tiles: tiles of 64x64 for half the CUs or fewer and a K long enough use partial sums (the stream
+    has no scratch before), others do not"""
+    rng = np.random.default_rng(k)
+    a, af = rounded(rng, (batch, k, m) if ta else (batch, m, k), "float32")
+    b, bf = rounded(rng, (batch, n, k) if tb else (batch, k, n), "float32")
+    lib, stream = _lib.load(), runtime.Stream()
+    lib.cinn_hip_scratch_release_stream.argtypes = [ctypes.c_void_p]
+    assert lib.cinn_hip_scratch_release_stream(stream.handle) == 0
+    lib.cinn_call_cublas.argtypes = ([ctypes.c_void_p, ctypes.c_int] + [ctypes.c_bool] * 3 + [ctypes.c_float] * 2 +
+                                     [ctypes.c_int] * 8 + [ctypes.c_void_p])
+    A, B, C = (runtime.DeviceBuffer.from_numpy(t) for t in (a, b, np.zeros((batch, m, n), np.float32)))
+    lib.cinn_call_cublas(runtime.pod_args([A, B, C]), 3, ta, tb, False, 1.0, 0.0, 1, *a.shape, 1, *b.shape, stream.handle)
+    stream.synchronize()
+    capacity = ctypes.c_size_t(0)
+    assert lib.cinn_hip_scratch_info(stream.handle, ctypes.byref(capacity), None, None) == 0
+    assert (capacity.value >= 2 * batch * m * n * 4) == split
+    am, bm = (np.swapaxes(af, 1, 2) if ta else af), (np.swapaxes(bf, 1, 2) if tb else bf)
+    want, scale = am @ bm, np.abs(am) @ np.abs(bm)
+    assert np.all(np.abs(C.numpy() - want) <= (2.0 ** -24 * np.sqrt(k) + 2.0 ** -22) * scale + 2.0 ** -24 * np.abs(want))
