@@ -30,5 +30,7 @@ struct FlexGemm {
 
 // false when an extent is beyond the kernel's 32-bit tile offsets (the caller then has a slower form)
 bool TryFlexGemm(const FlexGemm& g, hipStream_t stream);
+// whether TryFlexGemm takes the product and splits its K
+bool FlexGemmSplitsK(const FlexGemm& g, hipStream_t stream);
 
 }  // namespace cinn_hip_kernels

@@ -164,6 +164,9 @@ struct Plan {
   int tile, kg, splits;
 };
 
+// the partial sums of a split
+size_t PlaneBytes(const FlexGemm& g, int splits) { return (size_t)splits * g.batch * g.m * g.n * sizeof(float); }
+
 // Block tile and K split with the smallest estimated time.  The estimate (us) adds, per CU, the K steps of the blocks
 // it gets, and what a split writes and reads back.  A block alone on its CU takes `alone` per step, blocks that share
 // one take `shared` each, at most `resident` at a time; measured on a product of 768 x 3072 x 4100 (A and B [k][rows]),
@@ -172,7 +175,7 @@ struct Plan {
 // [2] x 2336 x 3250 x 153 25 us on 128x128 tiles of one group (two blocks per CU cover each other's epilogue) against
 // 40 with two; fp32 768 x 3072 x 4100 262 us on 128x128 tiles, 205 on 64x64 and 170 with K split four ways: a step is
 // bound by the matrix pipe there, and small tiles spread evenly.
-Plan ChoosePlan(const FlexGemm& g, int steps) {
+Plan ChoosePlan(const FlexGemm& g, int steps, hipStream_t stream) {
   struct Shape {
     int tile, kg, resident;
     double alone, shared;
@@ -199,7 +202,21 @@ Plan ChoosePlan(const FlexGemm& g, int steps) {
       if (us < least) least = us, best = {t.tile, t.kg, splits};
     }
   }
+  // under capture without an eager run or a reservation: K whole, which needs no scratch
+  if (best.splits > 1 && PlaneBytes(g, best.splits) > ScratchLimit(ScratchKind::kSplitK, stream)) best.splits = 1;
   return best;
+}
+
+int Steps(const FlexGemm& g) {
+  const int ks = g.type == FlexType::kF32 ? 32 : 64;
+  return (g.k + ks - 1) / ks;
+}
+
+// a thread's chunk is a 32-bit byte offset from the tile's first element: 128 rows, or 64 k rows, of the operand
+bool Fits(const FlexGemm& g) {
+  const int64_t limit = ((int64_t)1 << 31) / (128 * (g.type == FlexType::kF32 ? 4 : 2));
+  const int64_t tiles = (int64_t)((g.m + 63) / 64) * ((g.n + 63) / 64);
+  return g.lda < limit && g.ldb < limit && tiles < INT_MAX / 8 && g.batch <= 65535;
 }
 
 template <typename T, bool A_KC, bool B_KC>
@@ -219,26 +236,22 @@ void LaunchTiles(const Plan& plan, dim3 grid, const FlexParams& p, hipStream_t s
 
 template <typename T>
 void Launch(const FlexGemm& g, hipStream_t stream) {
-  constexpr int KS = 128 / (int)sizeof(T);
   FlexParams p;
   p.a = g.a, p.b = g.b, p.c = g.c;
   p.m = g.m, p.n = g.n, p.k = g.k;
   p.lda = g.lda, p.ldb = g.ldb;
   p.stride_a = g.stride_a, p.stride_b = g.stride_b, p.stride_c = g.stride_c;
-  p.steps      = (g.k + KS - 1) / KS;
+  p.steps      = Steps(g);
   p.full_steps = std::min(FullSteps<T>(g.a_kc, g.lda, g.m, g.k), FullSteps<T>(g.b_kc, g.ldb, g.n, g.k));
   p.scale = g.scale, p.shift = g.shift, p.residual = g.residual;
   p.alpha = g.alpha, p.residual_scale = g.residual_scale, p.relu = g.relu ? 1 : 0;
-  Plan plan         = ChoosePlan(g, p.steps);
+  Plan plan         = ChoosePlan(g, p.steps, stream);
   const int64_t plane = (int64_t)g.batch * g.m * g.n;
-  // under capture without an eager run or a reservation: K whole, which needs no scratch
-  if (plan.splits > 1 && (size_t)plan.splits * plane * sizeof(float) > ScratchLimit(ScratchKind::kSplitK, stream)) plan.splits = 1;
   p.steps_per_split = (p.steps + plan.splits - 1) / plan.splits;
   plan.splits       = (p.steps + p.steps_per_split - 1) / p.steps_per_split;
   p.tiles_m         = (g.m + plan.tile - 1) / plan.tile;
   p.tiles_n         = (g.n + plan.tile - 1) / plan.tile;
-  p.partials = plan.splits > 1 ? static_cast<float*>(Scratch(ScratchKind::kSplitK, (size_t)plan.splits * plane * sizeof(float), stream))
-                               : nullptr;
+  p.partials = plan.splits > 1 ? static_cast<float*>(Scratch(ScratchKind::kSplitK, PlaneBytes(g, plan.splits), stream)) : nullptr;
   const dim3 grid((unsigned)(p.tiles_m * p.tiles_n), g.batch, plan.splits);
   if (g.a_kc && g.b_kc) LaunchTiles<T, true, true>(plan, grid, p, stream);
   if (g.a_kc && !g.b_kc) LaunchTiles<T, true, false>(plan, grid, p, stream);
@@ -258,13 +271,10 @@ void Launch(const FlexGemm& g, hipStream_t stream) {
 
 }  // namespace
 
+bool FlexGemmSplitsK(const FlexGemm& g, hipStream_t stream) { return Fits(g) && ChoosePlan(g, Steps(g), stream).splits > 1; }
+
 bool TryFlexGemm(const FlexGemm& g, hipStream_t stream) {
-  const int elem = g.type == FlexType::kF32 ? 4 : 2;
-  // a thread's chunk is a 32-bit byte offset from the tile's first element: 128 rows, or 64 k rows, of the operand
-  const int64_t limit = ((int64_t)1 << 31) / (128 * elem);
-  if (g.lda >= limit || g.ldb >= limit) return false;
-  const int64_t tiles = (int64_t)((g.m + 63) / 64) * ((g.n + 63) / 64);
-  if (tiles >= INT_MAX / 8 || g.batch > 65535) return false;
+  if (!Fits(g)) return false;
   switch (g.type) {
     case FlexType::kF16: Launch<_Float16>(g, stream); break;
     case FlexType::kBF16: Launch<__bf16>(g, stream); break;

@@ -15,7 +15,7 @@
 //     are conflict free.  Operands whose contiguous axis is not K (row-major B, transposed A) are transposed
 //     in registers (8x8 blocks of 16-bit values) on their way into LDS.  Requires M%256 == N%256 == K%64 == 0.
 //   * gemm32_mfma_kernel  - fp32 on v_mfma_f32_32x32x2f32, 128x128 tile (64x64 when that is what fills the chip),
-//     for M%128 == N%128 == K%32 == 0 and a 64x64 tile for every CU.
+//     for M%128 == N%128 == K%32 == 0, unless few tiles with a long K are better off split.
 //   * gemm_generic_kernel - any shape / transpose / type: 64x64 LDS tile, FMA units; for fp64.
 // Everything else - ragged extents, a transposed A, too few tiles to fill the chip - runs on the register-staged MFMA
 // kernel of gemm_flex.hip.
@@ -1981,13 +1981,7 @@ void RunGemm(const GemmProblem& p, hipStream_t stream) {
   // 128x128 tiles of gemm_flex.hip); with 64 such tiles, 2048^3, 75 against 26 us
   const bool fast16 = !ForceGeneric() && aligned16 && p.m % kBM == 0 && p.n % kBN == 0 && p.k % kBK == 0 &&
                       (UseRegisterStaging() || (int64_t)(p.m / kBM) * (p.n / kBN) * p.batch >= 192);
-  // The fp32 tiles walk all of K, so they take grids that give every CU a 64x64 tile; with fewer the split K of
-  // gemm_flex.hip fills the chip.  us, whole tiles | split: 128x128x4096 76 | 13, 256x256x4096 76 | 14, 512x512x512
-  // 12.6 | 11.0, 512x1024x1024 (128 tiles) 22.1 | 18.1, 768x1024x2048 (192 tiles) 40.8 | 35.7; from 256 tiles on
-  // 1024x1024x256 8.6 | 9.3, 1024x1024x1024 22.4 | 23.9, 4096x4096x1024 267 | 282.  (Some larger grids whose last round is
-  // nearly empty are better off split all the same: 1280x1024x4096 138 | 101, 768x3072x4096 207 | 172.)
   const bool whole32 = !ForceGeneric() && aligned16 && p.m % kF32Tile == 0 && p.n % kF32Tile == 0 && p.k % kF32K == 0;
-  const bool fast32  = whole32 && (int64_t)(p.m / 64) * (p.n / 64) * p.batch >= 256;
   // (a bias only exists in the epilogues of the first two: the flags do not apply to it)
   const bool bias = p.shift != nullptr;
   if ((bias || (!ForceGeneric() && !UseRegisterStaging())) && (p.type == GemmType::kBF16 || p.type == GemmType::kF16)) {
@@ -1997,7 +1991,7 @@ void RunGemm(const GemmProblem& p, hipStream_t stream) {
       return;
     }
   }
-  if (bias || (!ForceGeneric() && p.type != GemmType::kF64 && !(p.type == GemmType::kF32 ? fast32 : fast16))) {
+  if (bias || (!ForceGeneric() && p.type != GemmType::kF64)) {
     cinn_hip_kernels::FlexGemm g;
     g.type = p.type == GemmType::kF16 ? cinn_hip_kernels::FlexType::kF16
                                       : (p.type == GemmType::kBF16 ? cinn_hip_kernels::FlexType::kBF16 : cinn_hip_kernels::FlexType::kF32);
@@ -2008,7 +2002,15 @@ void RunGemm(const GemmProblem& p, hipStream_t stream) {
     g.batch = p.batch, g.stride_a = p.stride_a, g.stride_b = p.stride_b, g.stride_c = p.stride_c;
     g.alpha = p.alpha, g.shift = p.shift;
     if (p.beta != 0.0f) g.residual = p.c, g.residual_scale = p.beta;
-    if (cinn_hip_kernels::TryFlexGemm(g, stream)) return;
+    // The fp32 tiles of gemm32_mfma_kernel walk all of K.  They keep the products whose K gemm_flex.hip would not split
+    // either, where they are 5 to 15% ahead, and the grids with a 64x64 tile for every CU.  us, whole tiles | gemm_flex.hip:
+    // 128x128x128 5.2 | 6.0, 512x512x256 8.0 | 8.7, 896x1152x1024 (252 tiles) 22.5 | 24.1, all not split; split
+    // 512x512x512 12.6 | 11.0, 512x1024x1024 22.1 | 18.1, 768x1024x2048 40.8 | 36.8, 128x128x4096 76 | 13; from 256 tiles on
+    // 1024x1024x256 8.6 | 9.3, 1024x1024x1024 22.4 | 23.9, 4096x4096x1024 267 | 282.  (Some larger grids whose last round is
+    // nearly empty are better off split all the same: 1280x1024x4096 138 | 101, 768x3072x4096 207 | 172.)
+    const bool fast32 = whole32 && ((int64_t)(p.m / 64) * (p.n / 64) * p.batch >= 256 || !cinn_hip_kernels::FlexGemmSplitsK(g, stream));
+    const bool whole  = !bias && (p.type == GemmType::kF32 ? fast32 : fast16);
+    if (!whole && cinn_hip_kernels::TryFlexGemm(g, stream)) return;
     CINN_RT_CHECK(!bias, "gemm: %d x %d x %d with a bias is beyond the kernels' offsets", p.m, p.n, p.k);
   }
   switch (p.type) {
@@ -2027,7 +2029,7 @@ void RunGemm(const GemmProblem& p, hipStream_t stream) {
       }
       break;
     case GemmType::kF32:
-      if (whole32) {  // also where gemm_flex.hip has refused a small grid (its offsets)
+      if (whole32) {
         LaunchFast32(p, stream);
       } else {
         LaunchGeneric<float, float>(p, stream);
