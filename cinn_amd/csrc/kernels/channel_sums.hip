@@ -33,15 +33,23 @@ namespace {
 
 using cinn_hip_kernels::Scratch;
 using cinn_hip_kernels::ScratchKind;
+using cinn_hip_kernels::ScratchLimit;
 using cinn_hip_kernels::flex::LoadAny;
 
 struct SumsParams {
   const void *a, *x, *out;  // a: x itself, or dy
   const float* mean;
-  float* planes;  // [split][2][channels]
+  float* planes;  // [split][2][channels], or null: the sums go to first and second
+  float *first, *second;
   int64_t pixels;
-  int channels, chunk_lanes, pixels_per_split;
+  int channels, chunk_lanes, pixels_per_split, splits;
 };
+
+// mean and E(x^2) - mean^2, each step rounded as the operators round it, of the sums of x and x x
+__device__ __forceinline__ void Statistics(float count, float* s, float* t) {
+  *s = *s / count;
+  *t = __fsub_rn(*t / count, __fmul_rn(*s, *s));
+}
 
 // E elements of channels from p: a chunk, or (E = 1) one element
 template <typename T, int E>
@@ -56,65 +64,82 @@ __device__ __forceinline__ void LoadChannels(const T* p, float (&v)[E]) {
   }
 }
 
-// GRAD: sums of dy and dy (x - mean), with dy zero where MASKED and out is not positive; else of x and x x
-template <typename T, int E, bool GRAD, bool MASKED>
+// GRAD: sums of dy and dy (x - mean), with dy zero where MASKED and out is not positive; else of x and x x.
+// A block takes one split, or (DIRECT) all of them, one after the other, and writes the sums' last form itself.  (As a loop
+// that both forms run, the conv_train step of [32][56][56][64] fp16 was 1.3 us of 138 slower.)
+template <typename T, int E, bool GRAD, bool MASKED, bool DIRECT>
 __global__ void __launch_bounds__(256)
 channel_sums_kernel(SumsParams p) {
   __shared__ float meet[256 * 2 * E];
+  __shared__ float total[DIRECT ? 2 * E * 64 : 1];
   const int lanes = p.chunk_lanes, rows = 256 / lanes;
   const int tid = threadIdx.x, row = tid / lanes;
   const int ch = (blockIdx.x * lanes + tid % lanes) * E;
-  float s[E], t[E];
+  for (int split = blockIdx.y; split < (DIRECT ? p.splits : blockIdx.y + 1); ++split) {
+    float s[E], t[E];
 #pragma unroll
-  for (int e = 0; e < E; ++e) s[e] = t[e] = 0.0f;
-  if (ch < p.channels) {
-    const int64_t first = (int64_t)blockIdx.y * p.pixels_per_split;
-    const int64_t end   = min(first + p.pixels_per_split, p.pixels);
-    const T *a = static_cast<const T*>(p.a), *x = static_cast<const T*>(p.x), *o = static_cast<const T*>(p.out);
-    float mean[E];
+    for (int e = 0; e < E; ++e) s[e] = t[e] = 0.0f;
+    if (ch < p.channels) {
+      const int64_t first = (int64_t)split * p.pixels_per_split;
+      const int64_t end   = min(first + p.pixels_per_split, p.pixels);
+      const T *a = static_cast<const T*>(p.a), *x = static_cast<const T*>(p.x), *o = static_cast<const T*>(p.out);
+      float mean[E];
 #pragma unroll
-    for (int e = 0; e < E; ++e) mean[e] = GRAD ? p.mean[ch + e] : 0.0f;
-    auto add = [&](const float (&av)[E], const float (&xv)[E], const float (&ov)[E]) {
+      for (int e = 0; e < E; ++e) mean[e] = GRAD ? p.mean[ch + e] : 0.0f;
+      auto add = [&](const float (&av)[E], const float (&xv)[E], const float (&ov)[E]) {
 #pragma unroll
-      for (int e = 0; e < E; ++e) {
-        const float d = MASKED ? (ov[e] > 0.0f ? av[e] : 0.0f) : av[e];
-        s[e] += d;
-        t[e] = __builtin_fmaf(d, GRAD ? xv[e] - mean[e] : d, t[e]);
+        for (int e = 0; e < E; ++e) {
+          const float d = MASKED ? (ov[e] > 0.0f ? av[e] : 0.0f) : av[e];
+          s[e] += d;
+          t[e] = __builtin_fmaf(d, GRAD ? xv[e] - mean[e] : d, t[e]);
+        }
+      };
+      constexpr int U = GRAD ? 2 : 4;
+      int64_t q       = first + row;
+      for (; q + (U - 1) * rows < end; q += U * rows) {
+        float av[U][E], xv[U][E], ov[U][E];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int64_t at = (q + u * rows) * p.channels + ch;
+          LoadChannels<T, E>(a + at, av[u]);
+          if (GRAD) LoadChannels<T, E>(x + at, xv[u]);
+          if (MASKED) LoadChannels<T, E>(o + at, ov[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) add(av[u], xv[u], ov[u]);
       }
-    };
-    constexpr int U = GRAD ? 2 : 4;
-    int64_t q       = first + row;
-    for (; q + (U - 1) * rows < end; q += U * rows) {
-      float av[U][E], xv[U][E], ov[U][E];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int64_t at = (q + u * rows) * p.channels + ch;
-        LoadChannels<T, E>(a + at, av[u]);
-        if (GRAD) LoadChannels<T, E>(x + at, xv[u]);
-        if (MASKED) LoadChannels<T, E>(o + at, ov[u]);
+      for (; q < end; q += rows) {
+        float av[E], xv[E], ov[E];
+        const int64_t at = q * p.channels + ch;
+        LoadChannels<T, E>(a + at, av);
+        if (GRAD) LoadChannels<T, E>(x + at, xv);
+        if (MASKED) LoadChannels<T, E>(o + at, ov);
+        add(av, xv, ov);
       }
+    }
 #pragma unroll
-      for (int u = 0; u < U; ++u) add(av[u], xv[u], ov[u]);
+    for (int e = 0; e < E; ++e) meet[(2 * e) * 256 + tid] = s[e], meet[(2 * e + 1) * 256 + tid] = t[e];
+    __syncthreads();
+    // value i = 2 e + (which sum) of lane l: the sum over rows of meet[i][row * lanes + l]
+    for (int i = tid; i < 2 * E * lanes; i += 256) {
+      const int value = i / lanes, l = i % lanes;
+      float sum = 0.0f;
+      for (int r = 0; r < rows; ++r) sum += meet[value * 256 + r * lanes + l];
+      if constexpr (DIRECT) {
+        total[i] = split == 0 ? sum : total[i] + sum;
+      } else {
+        const int c = (blockIdx.x * lanes + l) * E + value / 2;
+        if (c < p.channels) p.planes[((int64_t)split * 2 + (value & 1)) * p.channels + c] = sum;
+      }
     }
-    for (; q < end; q += rows) {
-      float av[E], xv[E], ov[E];
-      const int64_t at = q * p.channels + ch;
-      LoadChannels<T, E>(a + at, av);
-      if (GRAD) LoadChannels<T, E>(x + at, xv);
-      if (MASKED) LoadChannels<T, E>(o + at, ov);
-      add(av, xv, ov);
-    }
+    if constexpr (DIRECT) __syncthreads();
   }
-#pragma unroll
-  for (int e = 0; e < E; ++e) meet[(2 * e) * 256 + tid] = s[e], meet[(2 * e + 1) * 256 + tid] = t[e];
-  __syncthreads();
-  // value i = 2 e + (which sum) of lane l: the sum over rows of meet[i][row * lanes + l]
-  for (int i = tid; i < 2 * E * lanes; i += 256) {
-    const int value = i / lanes, l = i % lanes;
-    float sum = 0.0f;
-    for (int r = 0; r < rows; ++r) sum += meet[value * 256 + r * lanes + l];
-    const int c = (blockIdx.x * lanes + l) * E + value / 2;
-    if (c < p.channels) p.planes[((int64_t)blockIdx.y * 2 + (value & 1)) * p.channels + c] = sum;
+  if constexpr (!DIRECT) return;
+  for (int i = tid; i < E * lanes; i += 256) {
+    const int c = (blockIdx.x * lanes + i % lanes) * E + i / lanes;
+    float sum = total[2 * (i / lanes) * lanes + i % lanes], other = total[(2 * (i / lanes) + 1) * lanes + i % lanes];
+    if (!GRAD) Statistics((float)p.pixels, &sum, &other);
+    if (c < p.channels) p.first[c] = sum, p.second[c] = other;
   }
 }
 
@@ -137,10 +162,7 @@ channel_planes_kernel(const float* __restrict__ planes, float* __restrict__ firs
   if (row > 0 || c >= channels) return;
 #pragma unroll
   for (int r = 1; r < 16; ++r) s += meet[0][r * 16 + lane], t += meet[1][r * 16 + lane];
-  if (statistics) {  // mean and E(x^2) - mean^2, each step rounded as the operators round it
-    s = s / count;
-    t = __fsub_rn(t / count, __fmul_rn(s, s));
-  }
+  if (statistics) Statistics(count, &s, &t);
   first[c]  = s;
   second[c] = t;
 }
@@ -252,14 +274,14 @@ void Apply(ApplyParams p, bool grad, hipStream_t stream) {
   CINN_HIP_CALL(hipGetLastError());
 }
 
-template <typename T, int E>
+template <typename T, int E, bool DIRECT>
 void LaunchSums(const SumsParams& p, dim3 grid, bool grad, hipStream_t stream) {
   if (!grad) {
-    hipLaunchKernelGGL((channel_sums_kernel<T, E, false, false>), grid, dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((channel_sums_kernel<T, E, false, false, DIRECT>), grid, dim3(256), 0, stream, p);
   } else if (p.out) {
-    hipLaunchKernelGGL((channel_sums_kernel<T, E, true, true>), grid, dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((channel_sums_kernel<T, E, true, true, DIRECT>), grid, dim3(256), 0, stream, p);
   } else {
-    hipLaunchKernelGGL((channel_sums_kernel<T, E, true, false>), grid, dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((channel_sums_kernel<T, E, true, false, DIRECT>), grid, dim3(256), 0, stream, p);
   }
 }
 
@@ -276,15 +298,25 @@ void Sums(SumsParams p, bool grad, float* first, float* second, hipStream_t stre
   int64_t splits = std::max<int64_t>(1, std::min<int64_t>(512 / column_blocks, p.pixels / (8 * rows)));
   p.pixels_per_split = (int)((p.pixels + splits - 1) / splits);
   splits             = (p.pixels + p.pixels_per_split - 1) / p.pixels_per_split;
-  p.planes = static_cast<float*>(Scratch(ScratchKind::kSplitK, (size_t)splits * 2 * p.channels * sizeof(float), stream));
-  const dim3 grid(column_blocks, (unsigned)splits);
-  if (wide) {
-    LaunchSums<T, E>(p, grid, grad, stream);
+  p.splits = (int)splits, p.first = first, p.second = second;
+  const size_t plane_bytes = (size_t)splits * 2 * p.channels * sizeof(float);
+  dim3 grid(column_blocks, (unsigned)splits);
+  if (plane_bytes > ScratchLimit(ScratchKind::kSplitK, stream)) {
+    // under capture without an eager run or a reservation: a block walks all splits of its channels, four chunks of them,
+    // and needs no planes
+    p.chunk_lanes = std::min(p.chunk_lanes, 4);
+    grid          = dim3((chunks + p.chunk_lanes - 1) / p.chunk_lanes);
   } else {
-    LaunchSums<T, 1>(p, grid, grad, stream);
+    p.planes = static_cast<float*>(Scratch(ScratchKind::kSplitK, plane_bytes, stream));
   }
-  hipLaunchKernelGGL(channel_planes_kernel, dim3((p.channels + 15) / 16), dim3(256), 0, stream, p.planes, first, second, p.channels,
-                     (int)splits, (float)p.pixels, grad ? 0 : 1);
+  if (!p.planes && wide) LaunchSums<T, E, true>(p, grid, grad, stream);
+  if (!p.planes && !wide) LaunchSums<T, 1, true>(p, grid, grad, stream);
+  if (p.planes && wide) LaunchSums<T, E, false>(p, grid, grad, stream);
+  if (p.planes && !wide) LaunchSums<T, 1, false>(p, grid, grad, stream);
+  if (p.planes) {
+    hipLaunchKernelGGL(channel_planes_kernel, dim3((p.channels + 15) / 16), dim3(256), 0, stream, p.planes, first, second, p.channels,
+                       (int)splits, (float)p.pixels, grad ? 0 : 1);
+  }
   CINN_HIP_CALL(hipGetLastError());
 }
 
@@ -338,7 +370,7 @@ extern "C" void cinn_call_hip_channel_statistics(void* v_args, int num_args, int
   CINN_RT_CHECK(num_args == 3, "channel statistics: x, mean and variance expected, got %d arguments", num_args);
   CheckExtents(pixels, channels);
   const cinn_buffer_t* x = BufferArg(v_args, 0);
-  SumsParams p{x->memory, nullptr, nullptr, nullptr, nullptr, pixels, channels, 0, 0};
+  SumsParams p{x->memory, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, pixels, channels, 0, 0, 0};
   float *mean = Vector(BufferArg(v_args, 1)), *variance = Vector(BufferArg(v_args, 2));
   ByType(x, [&](auto t) { Sums<decltype(t)>(p, false, mean, variance, static_cast<hipStream_t>(stream)); });
 }
@@ -363,7 +395,7 @@ extern "C" void cinn_call_hip_channel_gradient_sums(void* v_args, int num_args, 
   const Operands in{v_args, num_args - 2, (unsigned)operands};
   const cinn_buffer_t *dy = in(0), *x = in(1), *out = masked ? in(3) : nullptr;
   CINN_RT_CHECK(SameType(dy, x) && (!out || SameType(dy, out)), "channel gradient sums: operands of different types");
-  SumsParams p{dy->memory, x->memory, out ? out->memory : nullptr, Vector(in(2)), nullptr, pixels, channels, 0, 0};
+  SumsParams p{dy->memory, x->memory, out ? out->memory : nullptr, Vector(in(2)), nullptr, nullptr, nullptr, pixels, channels, 0, 0, 0};
   float *sum_dy = Vector(BufferArg(v_args, num_args - 2)), *sum_dyx = Vector(BufferArg(v_args, num_args - 1));
   ByType(dy, [&](auto t) { Sums<decltype(t)>(p, true, sum_dy, sum_dyx, static_cast<hipStream_t>(stream)); });
 }
