@@ -20,8 +20,8 @@ struct ConvBackwardArgs {
   cinn_type_t type;
 };
 
-// false when the shape or type is not theirs (fp64, extents beyond 32-bit offsets, dilation together with a stride),
-// or when the stream is being captured and its scratch is too small; groups are not supported
+// false when the shape or type is not theirs (fp64, extents beyond 32-bit offsets, empty ones, dilation
+// together with a stride), or when the stream is being captured and its scratch is too small; groups are not supported
 bool TryConvBackwardData(const ConvBackwardArgs& a, hipStream_t stream);
 bool TryConvBackwardFilter(const ConvBackwardArgs& a, hipStream_t stream);
 
