@@ -20,7 +20,7 @@ struct ConvBackwardArgs {
   cinn_type_t type;
 };
 
-// false when the shape or type is not theirs (fp64, extents beyond 32-bit offsets, empty ones, dilation
+// false when the shape or type is not theirs (fp64, extents beyond 32-bit offsets, empty ones, negative paddings, dilation
 // together with a stride), or when the stream is being captured and its scratch is too small; groups are not supported
 bool TryConvBackwardData(const ConvBackwardArgs& a, hipStream_t stream);
 bool TryConvBackwardFilter(const ConvBackwardArgs& a, hipStream_t stream);

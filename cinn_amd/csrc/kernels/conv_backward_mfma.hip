@@ -549,9 +549,10 @@ bool Filter(const ConvBackwardArgs& a, hipStream_t stream) {
 }
 
 // Everything is addressed with 32-bit element offsets, also with the channels rounded up.  An empty batch or output (there
-// is nothing to divide into steps then) is left to the gather kernels.
+// is nothing to divide into steps then) and a negative padding (remainder classes are counted from 0) are left to the
+// gather kernels.
 bool Fits(const ConvBackwardArgs& a) {
-  if (std::min({a.n, a.c, a.h, a.w_in, a.f, a.kh, a.kw, a.oh, a.ow}) < 1) return false;
+  if (std::min({a.n, a.c, a.h, a.w_in, a.f, a.kh, a.kw, a.oh, a.ow}) < 1 || a.pad_h < 0 || a.pad_w < 0) return false;
   const int e = ChunkElems(a.type);
   const int64_t cp = RoundUp(a.c, e), fp = RoundUp(a.f, e), limit = INT_MAX / 2;
   return TypeSupported(a.type) && a.n <= 65535 && a.n * (int64_t)a.h * a.w_in * cp < limit && a.n * (int64_t)a.oh * a.ow * fp < limit &&
