@@ -18,7 +18,7 @@
 // 5 to 7 us for each copied tensor; 96 -> 200 3x3 / stride 2 on 35x41 at batch 8 in fp32, dx 1661 -> 31 us and dw
 // 3844 -> 22 + 5 us (47 TFLOP/s).
 // Tensors that are not channels last, or whose channel count is no multiple of a 16-byte chunk, are first copied into
-// that form in scratch (pack_kernel), and dx is copied back.
+// that form in scratch (pack_kernel), and dx is copied back (with beta, after it has been copied there).
 #include "kernels/conv_backward.h"
 
 #include <algorithm>
@@ -36,7 +36,7 @@ using flex::u32x4;
 
 // ---- copies between tensor layouts ---------------------------------------------------------------------------------
 // [n][c][plane] (nchw) or [n][plane][c] -> [n][plane][cp], channels c .. cp-1 zero.  A block moves 64 pixels x 64
-// channels of one image through LDS; cp is a multiple of a 16-byte chunk.
+// channels of one image through LDS.
 template <typename T, bool NCHW>
 __global__ void __launch_bounds__(256)
 pack_kernel(const T* __restrict__ in, T* __restrict__ out, int c, int plane, int cp) {
@@ -71,14 +71,21 @@ pack_kernel(const T* __restrict__ in, T* __restrict__ out, int c, int plane, int
     T v[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) v[e] = tile[p][q + e];
-    __builtin_memcpy(out + (int64_t)(p0 + p) * cp + c0 + q, v, 16);
+    T* to = out + (int64_t)(p0 + p) * cp + c0 + q;
+    if (c0 + q + E <= cp) {
+      __builtin_memcpy(to, v, 16);
+    } else {
+#pragma unroll
+      for (int e = 0; e < E; ++e)
+        if (c0 + q + e < cp) to[e] = v[e];
+    }
   }
 }
 
-// [n][plane][c] -> [n][c][plane], out = in + beta * out
+// [n][plane][c] -> [n][c][plane]
 template <typename T>
 __global__ void __launch_bounds__(256)
-unpack_kernel(const T* __restrict__ in, T* __restrict__ out, int c, int plane, float beta) {
+unpack_kernel(const T* __restrict__ in, T* __restrict__ out, int c, int plane) {
   constexpr int E = 16 / (int)sizeof(T), CPR = 64 / E;
   __shared__ T tile[64][64 + 4 / (int)sizeof(T)];  // [pixel][channel]
   const int p0 = blockIdx.x * 64, c0 = blockIdx.y * 64;
@@ -111,17 +118,11 @@ unpack_kernel(const T* __restrict__ in, T* __restrict__ out, int c, int plane, f
 #pragma unroll
     for (int e = 0; e < E; ++e) v[e] = tile[q + e][r];
     if (p0 + q + E <= plane) {
-      if (beta != 0.0f) {
-        chunk_t old;
-        __builtin_memcpy(&old, to, 16);
-#pragma unroll
-        for (int e = 0; e < E; ++e) v[e] = (T)((float)v[e] + beta * (float)old[e]);
-      }
       __builtin_memcpy(to, &v, 16);
     } else {
 #pragma unroll
       for (int e = 0; e < E; ++e)
-        if (p0 + q + e < plane) to[e] = beta != 0.0f ? (T)((float)v[e] + beta * (float)to[e]) : v[e];
+        if (p0 + q + e < plane) to[e] = v[e];
     }
   }
 }
@@ -442,14 +443,15 @@ bool Data(const ConvBackwardArgs& a, hipStream_t stream) {
   FilterParams fpar{a.f, a.c, a.kh, a.kw, fp, a.nhwc ? 1 : 0, forward ? 1 : a.stride_h, forward ? 1 : a.stride_w, a.pad_h, a.pad_w, forward ? 1 : 0, slot};
   hipLaunchKernelGGL(filter_kernel<T>, dim3((unsigned)((slot + 255) / 256), classes), dim3(256), 0, stream,
                      static_cast<const T*>(a.w), static_cast<T*>(wt), fpar);
-  const float beta = unpack ? 0.0f : a.beta;  // the copy back adds it otherwise
+  // what the gradient is added to goes into the copy first: the sum is rounded once, in the product's epilogue
+  if (unpack && a.beta != 0.0f) Pack<T>(a.out, dx, false, a.n, a.c, a.h * a.w_in, a.c, stream);
   if (forward) {
     ConvNhwcArgs c;
     c.x = dy, c.w = wt, c.y = dx;
     c.scale = c.shift = nullptr;
-    c.residual       = beta != 0.0f ? dx : nullptr;
+    c.residual       = a.beta != 0.0f ? dx : nullptr;
     c.alpha          = a.alpha;
-    c.residual_scale = beta;
+    c.residual_scale = a.beta;
     c.relu = c.nchw_input = false;
     c.n = a.n, c.h = a.oh, c.w_in = a.ow, c.c = fp;
     c.oc = a.c, c.kh = a.kh, c.kw = a.kw, c.oh = a.h, c.ow = a.w_in;
@@ -461,7 +463,7 @@ bool Data(const ConvBackwardArgs& a, hipStream_t stream) {
     RunConvNhwc(c, stream);
   } else {
     DataParams p{dy, wt, dx, ZeroPage(), a.n, a.h, a.w_in, a.c, a.oh, a.ow, fp, a.kh, a.kw, a.stride_h, a.stride_w, a.pad_h, a.pad_w,
-                 slot, a.alpha, beta};
+                 slot, a.alpha, a.beta};
     const int rows = a.n * ((a.h + a.stride_h - 1) / a.stride_h) * ((a.w_in + a.stride_w - 1) / a.stride_w);
     auto tiles = [&](int t) { return (unsigned)(((rows + t - 1) / t) * ((a.c + t - 1) / t)); };
     bool large = false;
@@ -477,7 +479,7 @@ bool Data(const ConvBackwardArgs& a, hipStream_t stream) {
   if (unpack) {
     const int plane = a.h * a.w_in;
     hipLaunchKernelGGL((unpack_kernel<T>), dim3((plane + 63) / 64, (a.c + 63) / 64, a.n), dim3(256), 0, stream,
-                       static_cast<const T*>(dx), static_cast<T*>(a.out), a.c, plane, a.beta);
+                       static_cast<const T*>(dx), static_cast<T*>(a.out), a.c, plane);
   }
   CINN_HIP_CALL(hipGetLastError());
   return true;
