@@ -365,32 +365,87 @@ conv_filter_kernel(FilterGradParams p) {
   });
 }
 
+// One element of the filter gradient by all threads of a block, pixels outside the image left out instead of multiplied by
+// zero; every thread gets the sum.
+template <typename T>
+__device__ float FilterElement(const FilterGradParams& p, int filter, int tap, int ch, float* shared) {
+  const T *x = static_cast<const T*>(p.x), *dy = static_cast<const T*>(p.dy);
+  const int ty = tap / p.kw * p.dil_h - p.pad_h, tx = tap % p.kw * p.dil_w - p.pad_w;
+  float sum = 0.0f;
+  for (int first = 0; first < p.pixels; first += 4096) {
+    for (int q = first + threadIdx.x; q < min(first + 4096, p.pixels); q += 256) {
+      const int n = q / (p.oh * p.ow), rest = q - n * (p.oh * p.ow), oy = rest / p.ow, ox = rest - oy * p.ow;
+      const int iy = oy * p.stride_h + ty, ix = ox * p.stride_w + tx;
+      if ((unsigned)iy < (unsigned)p.h && (unsigned)ix < (unsigned)p.w)
+        sum = __builtin_fmaf((float)dy[(int64_t)q * p.fp + filter], (float)x[((int64_t)n * p.h * p.w + iy * p.w + ix) * p.cp + ch], sum);
+    }
+    if (__syncthreads_or(sum != sum)) break;  // NaN, whatever else there is
+  }
+  shared[threadIdx.x] = sum;
+  __syncthreads();
+  for (int k = 128; k > 0; k >>= 1) {
+    if ((int)threadIdx.x < k) shared[threadIdx.x] += shared[threadIdx.x + k];
+    __syncthreads();
+  }
+  sum = shared[0];
+  __syncthreads();
+  return sum;
+}
+
 // Adds the planes and writes dw: a block takes 64 groups of four columns, its four rows of threads every fourth plane.
+// Where a tap lies outside the image the product has multiplied dy by zero, which an infinite or NaN dy makes NaN although
+// the sum has no such term: NaNs of such taps are computed again, without those terms.
 template <typename T>
 __global__ void __launch_bounds__(256)
-filter_reduce_kernel(const float* __restrict__ planes, T* __restrict__ dw, int f, int taps, int c, int cp, int splits, int nhwc,
-                     float alpha, float beta) {
+filter_reduce_kernel(FilterGradParams p, T* __restrict__ dw, int c, int splits, int nhwc, float alpha, float beta) {
   __shared__ __attribute__((aligned(16))) float part[3][64][4];
+  __shared__ float shared[256];
+  __shared__ int again[64];
   const int lane = threadIdx.x & 63, row = threadIdx.x >> 6;
-  const int64_t plane = (int64_t)f * taps * cp;
+  const int64_t plane = (int64_t)p.f * p.taps * p.cp;
   const int64_t at    = ((int64_t)blockIdx.x * 64 + lane) * 4;
   flex::f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
   if (at < plane) {
 #pragma unroll 4
-    for (int s = row; s < splits; s += 4) v += *reinterpret_cast<const flex::f32x4*>(planes + s * plane + at);
+    for (int s = row; s < splits; s += 4) v += *reinterpret_cast<const flex::f32x4*>(p.planes + s * plane + at);
   }
   if (row > 0) *reinterpret_cast<flex::f32x4*>(part[row - 1][lane]) = v;
   __syncthreads();
-  if (row > 0 || at >= plane) return;
+  const int ch     = (int)(at % p.cp);
+  const int tap    = (int)(at / p.cp % p.taps);
+  const int filter = (int)(at / p.cp / p.taps);
+  bool nan = false;
+  if (row == 0 && at < plane) {
 #pragma unroll
-  for (int r = 0; r < 3; ++r) v += *reinterpret_cast<const flex::f32x4*>(part[r][lane]);
-  const int ch   = (int)(at % cp);
-  const int tap  = (int)(at / cp % taps);
-  const int64_t filter = at / cp / taps;
+    for (int r = 0; r < 3; ++r) v += *reinterpret_cast<const flex::f32x4*>(part[r][lane]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) nan = nan || (v[e] != v[e] && ch + e < c);
+  }
+  if (__syncthreads_or(nan)) {
+    if (row == 0) {
+      int mask = 0;
+      const int y0 = tap / p.kw * p.dil_h - p.pad_h, x0 = tap % p.kw * p.dil_w - p.pad_w;
+      if (nan && (y0 < 0 || x0 < 0 || y0 + (p.oh - 1) * p.stride_h >= p.h || x0 + (p.ow - 1) * p.stride_w >= p.w)) {
+        for (int e = 0; e < 4; ++e)
+          if (v[e] != v[e] && ch + e < c) mask |= 1 << e;
+      }
+      again[lane] = mask;
+    }
+    __syncthreads();
+    for (int l = 0; l < 64; ++l) {
+      const int64_t other = ((int64_t)blockIdx.x * 64 + l) * 4;
+      for (int e = 0; e < 4; ++e) {
+        if (!(again[l] >> e & 1)) continue;
+        const float sum = FilterElement<T>(p, (int)(other / p.cp / p.taps), (int)(other / p.cp % p.taps), (int)(other % p.cp) + e, shared);
+        if (row == 0 && lane == l) v[e] = sum;
+      }
+    }
+  }
+  if (row > 0 || at >= plane) return;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     if (ch + e >= c) break;
-    const int64_t o = nhwc ? (filter * taps + tap) * c + ch + e : (filter * c + ch + e) * taps + tap;
+    const int64_t o = nhwc ? ((int64_t)filter * p.taps + tap) * c + ch + e : ((int64_t)filter * c + ch + e) * p.taps + tap;
     float g = alpha * v[e];
     if (beta != 0.0f) g += beta * (float)dw[o];
     dw[o] = (T)g;
@@ -544,8 +599,8 @@ bool Filter(const ConvBackwardArgs& a, hipStream_t stream) {
     }
   }
   if (!done) hipLaunchKernelGGL((conv_filter_kernel<T, 64, 64, 1>), grid, dim3(256), 0, stream, p);
-  hipLaunchKernelGGL((filter_reduce_kernel<T>), dim3((unsigned)((plane / 4 + 63) / 64)), dim3(256), 0, stream, p.planes,
-                     static_cast<T*>(a.out), a.f, p.taps, a.c, cp, splits, a.nhwc ? 1 : 0, a.alpha, a.beta);
+  hipLaunchKernelGGL((filter_reduce_kernel<T>), dim3((unsigned)((plane / 4 + 63) / 64)), dim3(256), 0, stream, p,
+                     static_cast<T*>(a.out), a.c, splits, a.nhwc ? 1 : 0, a.alpha, a.beta);
   CINN_HIP_CALL(hipGetLastError());
   return true;
 }

@@ -1,0 +1,80 @@
+"""Infinite and NaN operands of the convolution gradients: a tap outside the image is no term of the sum, so an infinite
+filter value or output gradient does not meet a zero there, and everything else is inf or NaN exactly where the definition
+(terms left out, float64) says so."""
+import numpy as np
+import pytest
+
+from cinn_amd import _lib, runtime
+
+from test_gpu_backward import CONV_ARGTYPES, conv_dims, conv_problem, from_dev, layout, round_to, to_dev, unlayout
+from test_gpu_conv_backward_mfma import bound
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # n, c, h, w, f, k, stride, pad, dilation, groups
+    (2, 16, 9, 8, 24, 3, 1, 1, 1, 1),
+    (2, 13, 9, 8, 21, 3, 1, 1, 1, 1),    # copies in either format
+    (1, 64, 12, 12, 72, 5, 1, 4, 2, 1),  # dilation
+    (2, 24, 13, 10, 40, 3, 2, 1, 1, 1),  # remainder classes
+    (2, 8, 12, 11, 16, 1, 2, 0, 1, 1),   # classes without a tap
+    (1, 16, 6, 6, 8, 1, 1, 2, 1, 1),     # output pixels that see no pixel of the image
+    (40, 64, 14, 14, 64, 3, 1, 1, 1, 1),
+]
+
+
+def gradients(x, w, dy, s, p, d):
+    """dx and dw with the terms outside the image left out"""
+    k, (oh, ow), (h, w_) = w.shape[2], dy.shape[2:], x.shape[2:]
+    dx, dw = np.zeros(x.shape), np.zeros(w.shape)
+
+    def inside(tap, out, size):
+        o = np.arange(out)
+        i = o * s - p + tap * d
+        keep = (i >= 0) & (i < size)
+        return o[keep], i[keep]
+    for ky in range(k):
+        for kx in range(k):
+            (oy, iy), (ox, ix) = inside(ky, oh, h), inside(kx, ow, w_)
+            if len(oy) == 0 or len(ox) == 0:
+                continue
+            g = dy[:, :, oy][:, :, :, ox]
+            # term by term: a product over all filters (pixels) at once may reorder infinities, but their sum is the same
+            dx[np.ix_(range(x.shape[0]), range(x.shape[1]), iy, ix)] += np.einsum("nfyx,fc->ncyx", g, w[:, :, ky, kx])
+            dw[:, :, ky, kx] = np.einsum("ncyx,nfyx->fc", x[:, :, iy][:, :, :, ix], g)
+    return dx, dw
+
+
+def check(got, want, scale, terms, dtype):
+    got = got.astype(np.float64)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    finite = np.isfinite(want)
+    assert np.array_equal(got[~finite & ~np.isnan(want)], want[~finite & ~np.isnan(want)])
+    assert np.all(np.abs(got[finite] - want[finite]) <= bound(want[finite], scale[finite], terms, dtype))
+
+
+def run(name, fmt, alpha, beta, dims, *tensors):
+    fn = getattr(_lib.load(), name)
+    fn.argtypes = CONV_ARGTYPES
+    fn(runtime.pod_args(tensors), 3, fmt, alpha, beta, *dims, None)
+    runtime.synchronize()
+
+
+@pytest.mark.parametrize("beta", [0.0, 0.5])
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+@pytest.mark.parametrize("fmt", [0, 1])
+@pytest.mark.parametrize("dtype", ["float32", "float16", "bfloat16"])
+@pytest.mark.parametrize("case", CASES)
+def test_filter_gradient(gpu, case, dtype, fmt, value, beta):
+    n, c, h, w_, f, k, s, p, d, g = case
+    x, w, dy = conv_problem(case, dtype)
+    dy[0, 1, 0, 0] = value                    # at a corner: outside the image for some taps
+    dy[-1, 3, -1, dy.shape[3] // 2] = value   # at the lower edge
+    x[0, 2, 0, 0] = value                     # a value of the image itself is a term of every sum it is in
+    dw0 = round_to(np.random.default_rng(1).standard_normal(w.shape), dtype)
+    X, DY, DW = (to_dev(layout(t, fmt), dtype) for t in (x, dy, dw0))
+    run("cinn_call_cudnn_conv2d_backward_filter", fmt, 1.0, beta, conv_dims(case, x, w, dy), X, DY, DW)
+    with np.errstate(invalid="ignore"):
+        want = gradients(x.astype(np.float64), w, dy.astype(np.float64), s, p, d)[1] + beta * dw0
+        scale = gradients(np.abs(x).astype(np.float64), w, np.abs(dy).astype(np.float64), s, p, d)[1] + np.abs(beta * dw0)
+    check(unlayout(from_dev(DW, dtype), fmt), want, scale, dy.size / f, dtype)
