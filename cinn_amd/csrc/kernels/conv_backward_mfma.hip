@@ -9,6 +9,9 @@
 //   * dx at a larger stride: the input pixels of one remainder class (iy mod stride, ix mod stride) see the same taps,
 //     every stride-th one, and neighbouring pixels of the class see neighbouring dy.  Each class is a product of its own
 //     (pixels x channels, K = its taps x f), all classes in one launch; no multiply-add meets an inserted zero.
+//     Taps outside dy meet a zero in either form, as in the forward convolution: an infinite filter value makes NaN there.
+//     (A kernel that computes such pixels again would be one more launch, 2.8 us of the 16 that a 64 -> 64 3x3 layer on
+//     56x56 at batch 32 takes in fp16; whoever has such a filter has the NaNs from the forward pass.)
 //   * dw: rows are filters, columns (tap, channel), and K runs over all output pixels, which both operands keep as their
 //     slow axis: they lie in LDS as [pixel][channels] and are read with transposing reads.  The x operand is gathered
 //     row by row (a chunk of channels of pixel + tap, or zeros).  K is long (1e5) and the result small, so K is split

@@ -303,8 +303,9 @@ void cinn_call_hip_channel_gradient(void* v_args, int num_args, int pixels, int 
                                     void* stream);
 
 /* Gradients of the three calls above, with the reference's argument lists.  Convolutions without groups run on the
- * matrix cores, everything else in gather form (fp32 accumulation), formats 0 = NCHW / [F][C][KH][KW] and 1 = NHWC / [F][KH][KW][C]; every result
- * is out = alpha * gradient + beta * out.
+ * matrix cores, where a tap outside the image counts as a product with zero for an infinite or NaN filter value in the
+ * data gradient, as in the forward convolution; everything else in gather form (fp32 accumulation).  Formats 0 = NCHW /
+ * [F][C][KH][KW] and 1 = NHWC / [F][KH][KW][C]; every result is out = alpha * gradient + beta * out, rounded once.
  * cinn_call_cudnn_conv2d_backward_data (cuda_util.cc:722-843): v_args = {w, dy, dx}.
  * cinn_call_cudnn_conv2d_backward_filter (cuda_util.cc:845-967): v_args = {x, dy, dw}. */
 void cinn_call_cudnn_conv2d_backward_data(void* v_args, int num_args, int format, float alpha, float beta, int input_n,
