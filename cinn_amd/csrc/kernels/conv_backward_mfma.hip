@@ -130,23 +130,23 @@ unpack_kernel(const T* __restrict__ in, T* __restrict__ out, int c, int plane) {
   }
 }
 
-// The filter as the data gradient reads it: class slot (ry, rx), then [c][i][j][fp] with i, j counting the class's taps
-// ky = ky0 + stride i, kx likewise; f .. fp-1 are zero.  Stride 1 (one class): the forward kernel walks the taps upwards
-// in dy, so they are turned round.
+// The filter as the data gradient reads it: a slot for every first tap (ky0, kx0) of a class, i.e. for every class that has
+// taps at all (whatever the stride, slots do not add up to more than the filter with its extents rounded up), then
+// [c][i][j][fp] with i, j counting the class's taps ky = ky0 + stride i, kx likewise; f .. fp-1 are zero.  Stride 1 (one
+// class): the forward kernel walks the taps upwards in dy, so they are turned round.
 struct FilterParams {
   int f, c, kh, kw, fp;
   int nhwc;                    // filter [f][kh][kw][c], else [f][c][kh][kw]
-  int stride_h, stride_w, pad_h, pad_w;
+  int stride_h, stride_w;
+  int slots_w;                 // slots side by side: first taps kx0
   int turn;                    // 1: turned round (stride 1)
-  int64_t slot;                // elements of a class's slot
+  int64_t slot;                // elements of a slot
 };
 template <typename T>
 __global__ void __launch_bounds__(256)
 filter_kernel(const T* __restrict__ w, T* __restrict__ out, FilterParams p) {
-  const int ry = blockIdx.y / p.stride_w, rx = blockIdx.y % p.stride_w;
-  const int ky0 = p.turn ? 0 : (ry + p.pad_h) % p.stride_h, kx0 = p.turn ? 0 : (rx + p.pad_w) % p.stride_w;
-  const int nky = ky0 < p.kh ? (p.kh - 1 - ky0) / p.stride_h + 1 : 0;
-  const int nkx = kx0 < p.kw ? (p.kw - 1 - kx0) / p.stride_w + 1 : 0;
+  const int ky0 = blockIdx.y / p.slots_w, kx0 = blockIdx.y % p.slots_w;  // below the stride and the extent
+  const int nky = (p.kh - 1 - ky0) / p.stride_h + 1, nkx = (p.kw - 1 - kx0) / p.stride_w + 1;
   const int64_t total = (int64_t)p.c * nky * nkx * p.fp;
   const int64_t idx   = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (idx >= total) return;
@@ -171,6 +171,7 @@ struct DataParams {
   const void* zeros;
   int n, h, w, c, oh, ow, fp, kh, kw;
   int stride_h, stride_w, pad_h, pad_w;
+  int slots_w;
   int64_t slot;
   float alpha, beta;
 };
@@ -247,7 +248,7 @@ conv_data_kernel(DataParams p) {
   DataTile<T, BM, 256 * KG> ta;
   flex::Tile<T, true, BN, 256 * KG> tb;
   ta.Init(p, m0, rows, hc, wc, (ry + p.pad_h - ky0) / p.stride_h, (rx + p.pad_w - kx0) / p.stride_w, nky, nkx, tid);
-  tb.Init(static_cast<const T*>(p.wt) + blockIdx.y * p.slot, k, n0, p.c, k, tid);
+  tb.Init(static_cast<const T*>(p.wt) + (k > 0 ? (ky0 * p.slots_w + kx0) * p.slot : 0), k, n0, p.c, k, tid);
   typename flex::Mma<T, true, true, BM, BN>::acc_t acc;
   flex::KLoop<T, true, true, BM, BN, KG>(lds, ta, tb, 0, (k + KS - 1) / KS, k / KS, k, tid, acc);
 
@@ -484,10 +485,12 @@ bool Data(const ConvBackwardArgs& a, hipStream_t stream) {
   const bool unpack   = !a.nhwc && (a.c > 1 && a.h * a.w_in > 1);
   const bool forward  = a.stride_h == 1 && a.stride_w == 1 && (a.kh - 1) * a.dil_h >= a.pad_h && (a.kw - 1) * a.dil_w >= a.pad_w;
   const int classes   = forward ? 1 : a.stride_h * a.stride_w;
+  const int slots_w   = forward ? 1 : std::min(a.kw, a.stride_w);
+  const int slots     = forward ? 1 : std::min(a.kh, a.stride_h) * slots_w;  // classes that have taps
   const int64_t slot  = (int64_t)RoundUp(a.c * ((a.kh + a.stride_h - 1) / a.stride_h) * ((a.kw + a.stride_w - 1) / a.stride_w) * fp, 128);
   auto bytes = [](int64_t elems) { return ((size_t)elems * sizeof(T) + 255) & ~(size_t)255; };
   const size_t dy_bytes = pack_dy ? bytes((int64_t)a.n * a.oh * a.ow * fp) : 0;
-  const size_t wt_bytes = bytes(classes * slot);
+  const size_t wt_bytes = bytes(slots * slot);
   const size_t dx_bytes = unpack ? bytes((int64_t)a.n * a.h * a.w_in * a.c) : 0;
   if (dy_bytes + wt_bytes + dx_bytes > ScratchLimit(ScratchKind::kTranspose, stream)) return false;
   char* scratch = static_cast<char*>(Scratch(ScratchKind::kTranspose, dy_bytes + wt_bytes + dx_bytes, stream));
@@ -498,8 +501,8 @@ bool Data(const ConvBackwardArgs& a, hipStream_t stream) {
   }
   void* wt = scratch + dy_bytes;
   void* dx = unpack ? scratch + dy_bytes + wt_bytes : a.out;
-  FilterParams fpar{a.f, a.c, a.kh, a.kw, fp, a.nhwc ? 1 : 0, forward ? 1 : a.stride_h, forward ? 1 : a.stride_w, a.pad_h, a.pad_w, forward ? 1 : 0, slot};
-  hipLaunchKernelGGL(filter_kernel<T>, dim3((unsigned)((slot + 255) / 256), classes), dim3(256), 0, stream,
+  FilterParams fpar{a.f, a.c, a.kh, a.kw, fp, a.nhwc ? 1 : 0, forward ? 1 : a.stride_h, forward ? 1 : a.stride_w, slots_w, forward ? 1 : 0, slot};
+  hipLaunchKernelGGL(filter_kernel<T>, dim3((unsigned)((slot + 255) / 256), slots), dim3(256), 0, stream,
                      static_cast<const T*>(a.w), static_cast<T*>(wt), fpar);
   // what the gradient is added to goes into the copy first: the sum is rounded once, in the product's epilogue
   if (unpack && a.beta != 0.0f) Pack<T>(a.out, dx, false, a.n, a.c, a.h * a.w_in, a.c, stream);
@@ -521,7 +524,7 @@ bool Data(const ConvBackwardArgs& a, hipStream_t stream) {
     RunConvNhwc(c, stream);
   } else {
     DataParams p{dy, wt, dx, ZeroPage(), a.n, a.h, a.w_in, a.c, a.oh, a.ow, fp, a.kh, a.kw, a.stride_h, a.stride_w, a.pad_h, a.pad_w,
-                 slot, a.alpha, a.beta};
+                 slots_w, slot, a.alpha, a.beta};
     const int rows = a.n * ((a.h + a.stride_h - 1) / a.stride_h) * ((a.w_in + a.stride_w - 1) / a.stride_w);
     auto tiles = [&](int t) { return (unsigned)(((rows + t - 1) / t) * ((a.c + t - 1) / t)); };
     bool large = false;

@@ -28,6 +28,7 @@ CASES = [
     (2, 8, 9, 9, 136, 1, 2, 0, 1, 1),    # three classes without a tap
     (1, 9, 17, 16, 12, 7, 3, 3, 1, 1),
     (1, 16, 2, 2, 16, 3, 2, 1, 1, 1),    # one output pixel
+    (1, 16, 19, 22, 24, 3, 5, 1, 1, 1),  # sixteen classes without a tap among those that have one
     (40, 72, 10, 11, 200, 3, 1, 1, 1, 1),  # many K steps, split
 ]
 
@@ -85,3 +86,23 @@ def test_alpha_beta(gpu, case, dtype, fmt):
     want = -1.5 * grad + 0.25 * dw0
     err  = np.abs(unlayout(from_dev(DW, dtype), fmt) - want)
     assert np.all(err <= bound(want, 1.5 * scale + 0.25 * np.abs(dw0), dy.size / f, dtype))
+
+
+@pytest.mark.parametrize("fmt", [0, 1])
+def test_scratch_of_a_large_stride(gpu, fmt):
+    """a data gradient keeps the filter once, not once for every remainder class"""
+    case = (1, 64, 33, 30, 128, 1, 16, 0, 1, 1)
+    x, w, dy = conv_problem(case, "float16")
+    lib, stream = _lib.load(), runtime.Stream()
+    lib.cinn_call_cudnn_conv2d_backward_data.argtypes = CONV_ARGTYPES
+    lib.cinn_hip_scratch_release_stream.argtypes = [ctypes.c_void_p]
+    assert lib.cinn_hip_scratch_release_stream(stream.handle) == 0
+    W, DY, DX = (to_dev(layout(t, fmt), "float16") for t in (w, dy, np.full_like(x, np.nan)))
+    lib.cinn_call_cudnn_conv2d_backward_data(runtime.pod_args([W, DY, DX]), 3, fmt, 1.0, 0.0, *conv_dims(case, x, w, dy), stream.handle)
+    stream.synchronize()
+    capacity = ctypes.c_size_t(0)
+    assert lib.cinn_hip_scratch_info(stream.handle, None, ctypes.byref(capacity), None) == 0
+    copies = 2 * (dy.size + x.size) if fmt == 0 else 0
+    assert capacity.value <= copies + 2 * w.size + 3 * 256
+    want, scale = (ob.conv2d_backward_data(q, r, x.shape, (16, 16), (0, 0), (1, 1), 1) for q, r in ((w, dy), (np.abs(w), np.abs(dy))))
+    assert np.all(np.abs(unlayout(from_dev(DX, "float16"), fmt) - want) <= bound(want, scale, 128, "float16"))
