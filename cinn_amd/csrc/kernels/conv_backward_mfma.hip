@@ -476,7 +476,7 @@ void Pack(const void* in, void* out, bool nhwc, int n, int c, int plane, int cp,
 }
 
 // Both are false, with nothing launched, while the stream is captured and its scratch is too small for the copies and
-// planes: the gather kernels, which need none, take such a call.
+// planes, or the page of zeros does not exist yet: the gather kernels, which need none, take such a call.
 template <typename T>
 bool Data(const ConvBackwardArgs& a, hipStream_t stream) {
   constexpr int E = 16 / (int)sizeof(T);
@@ -492,7 +492,7 @@ bool Data(const ConvBackwardArgs& a, hipStream_t stream) {
   const size_t dy_bytes = pack_dy ? bytes((int64_t)a.n * a.oh * a.ow * fp) : 0;
   const size_t wt_bytes = bytes(slots * slot);
   const size_t dx_bytes = unpack ? bytes((int64_t)a.n * a.h * a.w_in * a.c) : 0;
-  if (dy_bytes + wt_bytes + dx_bytes > ScratchLimit(ScratchKind::kTranspose, stream)) return false;
+  if (!HasZeroPage(stream) || dy_bytes + wt_bytes + dx_bytes > ScratchLimit(ScratchKind::kTranspose, stream)) return false;
   char* scratch = static_cast<char*>(Scratch(ScratchKind::kTranspose, dy_bytes + wt_bytes + dx_bytes, stream));
   const void* dy = a.dy;
   if (pack_dy) {
@@ -577,7 +577,8 @@ bool Filter(const ConvBackwardArgs& a, hipStream_t stream) {
   p.steps_per_split = (p.steps + splits - 1) / splits;
   splits            = (p.steps + p.steps_per_split - 1) / p.steps_per_split;
   const size_t plane_bytes = (size_t)splits * plane * sizeof(float);
-  if (dy_bytes + x_bytes > ScratchLimit(ScratchKind::kTranspose, stream) || plane_bytes > ScratchLimit(ScratchKind::kSplitK, stream))
+  if (!HasZeroPage(stream) || dy_bytes + x_bytes > ScratchLimit(ScratchKind::kTranspose, stream) ||
+      plane_bytes > ScratchLimit(ScratchKind::kSplitK, stream))
     return false;
   char* scratch = dy_bytes + x_bytes ? static_cast<char*>(Scratch(ScratchKind::kTranspose, dy_bytes + x_bytes, stream)) : nullptr;
   p.planes = static_cast<float*>(Scratch(ScratchKind::kSplitK, plane_bytes, stream));

@@ -76,15 +76,18 @@ void* Scratch(ScratchKind kind, size_t bytes, hipStream_t stream) {
 
 size_t ScratchLimit(ScratchKind kind, hipStream_t stream) {
   if (!Capturing(stream)) return SIZE_MAX;
-  const int device = CurrentDevice();
-  if (device < kMaxDevices) {
-    std::lock_guard<std::mutex> lock(g_page_mu);
-    if (!g_pages[device]) return 0;
-  }
   Arena& arena = TheArena();
   std::lock_guard<std::mutex> lock(arena.mu);
-  auto it = arena.live.find({device, stream, static_cast<int>(kind)});
+  auto it = arena.live.find({CurrentDevice(), stream, static_cast<int>(kind)});
   return it == arena.live.end() ? 0 : it->second.capacity;
+}
+
+bool HasZeroPage(hipStream_t stream) {
+  if (!Capturing(stream)) return true;
+  const int device = CurrentDevice();
+  if (device >= kMaxDevices) return true;  // ZeroPage() says what is wrong
+  std::lock_guard<std::mutex> lock(g_page_mu);
+  return g_pages[device] != nullptr;
 }
 
 const void* ZeroPage() {

@@ -24,9 +24,12 @@ constexpr int kScratchKinds = 2;
 // that says to reserve first (one eager execution of the same calls, or cinn_hip_scratch_reserve).
 void* Scratch(ScratchKind kind, size_t bytes, hipStream_t stream);
 
-// What Scratch can give: anything, or while `stream` is being captured the current capacity (and nothing before the page
-// of zeros exists).  For calls that have a way to do with less instead of aborting.
+// What Scratch can give: anything, or while `stream` is being captured the current capacity.  For calls that have a way to
+// do with less instead of aborting.
 size_t ScratchLimit(ScratchKind kind, hipStream_t stream);
+
+// whether ZeroPage can be called: always, or while `stream` is being captured once the page exists
+bool HasZeroPage(hipStream_t stream);
 
 // 256 bytes of zeros in the current device's memory, allocated and cleared once per device (what masked-out 16-byte
 // chunks are read from)
