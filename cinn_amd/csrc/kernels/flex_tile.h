@@ -205,6 +205,12 @@ struct Mma<float, A_KC, B_KC, BM, BN> {
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
   }
+  static __device__ __forceinline__ void Add(acc_t& acc, const acc_t& more) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] += more[i][j];
+  }
   // four k of one row: chunk 2 q + (lane / 32), element e feeds MFMA (q, e) of v_mfma_f32_32x32x2_f32
   template <bool KC, int ROWS>
   static __device__ __forceinline__ f32x4 Fragment(const char* tile, int row0, int q, int lane) {
@@ -259,7 +265,9 @@ __device__ __forceinline__ void TileOf(int bid, int tiles_m, int tiles_n, int* t
 
 // The K loop over steps [s, s1): ta / tb are operand tiles with Load<guard>(registers, step, k, tid) and Store(LDS, ...);
 // steps below full_steps need no guard.  `lds` holds two stages.
-template <typename T, bool A_KC, bool B_KC, int BM, int BN, int KG, typename TA, typename TB>
+// PARTS > 0: a step's products are summed in PARTS chains of their own before they are added to acc, which then is a chain
+// of steps and not of products.
+template <typename T, bool A_KC, bool B_KC, int BM, int BN, int KG, int PARTS = 0, typename TA, typename TB>
 __device__ __forceinline__ void KLoop(char* lds, TA& ta, TB& tb, int s, int s1, int full_steps, int k_total, int tid,
                                       typename Mma<T, A_KC, B_KC, BM, BN>::acc_t& acc) {
   constexpr int STAGE   = (BM + BN) * 128;
@@ -287,6 +295,23 @@ __device__ __forceinline__ void KLoop(char* lds, TA& ta, TB& tb, int s, int s1, 
     tb.Store(stage + BM * 128, rb[slot], tid);
   };
 
+  auto multiply = [&](const char* stage) {
+    if constexpr (PARTS == 0) {
+      M::template Step<KG>(stage, stage + BM * 128, wm, wn, kg, lane, acc);
+    } else {
+      static_assert(KG == 1, "the parts of a step are its slices");
+      typename M::acc_t sum[PARTS];
+#pragma unroll
+      for (int part = 0; part < PARTS; ++part) {
+        M::Zero(sum[part]);
+        M::template Step<PARTS>(stage, stage + BM * 128, wm, wn, part, lane, sum[part]);
+      }
+#pragma unroll
+      for (int part = 1; part < PARTS; ++part) M::Add(sum[0], sum[part]);
+      M::Add(acc, sum[0]);
+    }
+  };
+
   M::Zero(acc);
 #pragma unroll
   for (int u = 0; u < PF; ++u)
@@ -301,7 +326,7 @@ __device__ __forceinline__ void KLoop(char* lds, TA& ta, TB& tb, int s, int s1, 
     for (int u = 0; u < 2; ++u) {
       char* cur = lds + (u & 1) * STAGE;
       load(s + u + PF, u % PF, true);
-      M::template Step<KG>(cur, cur + BM * 128, wm, wn, kg, lane, acc);
+      multiply(cur);
       store((u + 1) % PF, lds + ((u + 1) & 1) * STAGE);
       __syncthreads();
     }
@@ -312,7 +337,7 @@ __device__ __forceinline__ void KLoop(char* lds, TA& ta, TB& tb, int s, int s1, 
       if (s + u >= s1) break;
       char* cur = lds + (u & 1) * STAGE;
       if (s + u + PF < s1) load(s + u + PF, u % PF, s + u + PF < full_steps);
-      M::template Step<KG>(cur, cur + BM * 128, wm, wn, kg, lane, acc);
+      multiply(cur);
       if (s + u + 1 < s1) store((u + 1) % PF, lds + ((u + 1) & 1) * STAGE);
       __syncthreads();
     }

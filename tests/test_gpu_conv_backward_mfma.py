@@ -106,3 +106,22 @@ def test_scratch_of_a_large_stride(gpu, fmt):
     assert capacity.value <= copies + 2 * w.size + 3 * 256
     want, scale = (ob.conv2d_backward_data(q, r, x.shape, (16, 16), (0, 0), (1, 1), 1) for q, r in ((w, dy), (np.abs(w), np.abs(dy))))
     assert np.all(np.abs(unlayout(from_dev(DX, "float16"), fmt) - want) <= bound(want, scale, 128, "float16"))
+
+
+@pytest.mark.parametrize("case,limit", [((1, 64, 28, 28, 64, 3, 1, 1, 1, 1), 1.3e-7), ((16, 64, 28, 28, 64, 3, 1, 1, 1, 1), 1.8e-7),
+                                        ((2, 128, 14, 14, 96, 3, 1, 1, 1, 1), 1.3e-7)])
+def test_rounding_of_the_fp32_filter_gradient(gpu, case, limit):
+    """fp32 sums over 392 to 12544 pixels, relative 2-norm of the error.  A chain of n terms of random sign is off by about
+    2^-24 * 0.3 * sqrt(n): 0.7e-7 for the sixteen of a part, and as much for up to sixteen steps and planes on top of it;
+    1.3e-7 is a third above that, as one chain the sums are off by more than 2.2e-7.  12544 pixels have longer chains of
+    steps."""
+    n, c, h, w_, f, k, s, p, d, g = case
+    x, w, dy = conv_problem(case, "float32")
+    lib = _lib.load()
+    lib.cinn_call_cudnn_conv2d_backward_filter.argtypes = CONV_ARGTYPES
+    X, DY, DW = (to_dev(layout(t, 1), "float32") for t in (x, dy, w))
+    lib.cinn_call_cudnn_conv2d_backward_filter(runtime.pod_args([X, DY, DW]), 3, 1, 1.0, 0.0, *conv_dims(case, x, w, dy), None)
+    runtime.synchronize()
+    want = ob.conv2d_backward_filter(x, dy, w.shape, (s, s), (p, p), (d, d), g)
+    got = unlayout(from_dev(DW, "float32"), 1).astype(np.float64)
+    assert np.linalg.norm(got - want) <= limit * np.linalg.norm(want)
