@@ -6,7 +6,8 @@
 // memory in fp32, a reduction over runs of pixels, a reduction of those - and the gradient's mask one more pass.  Both
 // sums need the same elements, so one pass reads every tensor once and writes nothing of its size: bound by that read.
 // A thread owns 16 bytes of channels and walks pixels, four loads in flight; the rows of a block meet in LDS, the
-// blocks in a second launch of a few microseconds (an atomic counter instead would have to be cleared in every call).
+// blocks in a second launch of a few microseconds (the last block to arrive could add them instead, with a counter that it
+// sets back; that form has not been measured).
 //
 // What the sums are for is applied in a second pass (channel_apply_kernel): generated code formed square roots, divisions
 // and six per-channel loads for every element and wrote the result through a transpose.
@@ -16,8 +17,9 @@
 // 23 -> 11.6, gradient 28 -> 12.5 (51 MB at 4.1 TB/s).  [8][18][21][200] fp32: 9.1, 4.2, 8.7 and 4.6, of which a launch
 // is more than half.
 //
-// All arithmetic is fp32; a thread adds at most a few hundred terms before partial sums are added pairwise by rows,
-// blocks and planes, fewer in a chain than the generated reductions had.
+// All arithmetic is fp32, and every sum is one of short chains: a thread adds its few pixels, then rows and planes are added
+// in four chains each, what is left pairwise.  Relative error against float64, generated reductions | one chain each | here:
+// mean of [32][56][56][64] fp32 4.1e-8 | 7.3e-8 | 4.0e-8, sum of dy 1.6e-7 | 1.8e-7 | 1.1e-7.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -123,8 +125,12 @@ channel_sums_kernel(SumsParams p) {
     // value i = 2 e + (which sum) of lane l: the sum over rows of meet[i][row * lanes + l]
     for (int i = tid; i < 2 * E * lanes; i += 256) {
       const int value = i / lanes, l = i % lanes;
-      float sum = 0.0f;
-      for (int r = 0; r < rows; ++r) sum += meet[value * 256 + r * lanes + l];
+      float q[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // rows: a power of two, at least four
+      for (int r = 0; r < rows; r += 4) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) q[u] += meet[value * 256 + (r + u) * lanes + l];
+      }
+      const float sum = (q[0] + q[1]) + (q[2] + q[3]);
       if constexpr (DIRECT) {
         total[i] = split == 0 ? sum : total[i] + sum;
       } else {
@@ -149,19 +155,36 @@ channel_planes_kernel(const float* __restrict__ planes, float* __restrict__ firs
                       float count, int statistics) {
   __shared__ float meet[2][256];
   const int tid = threadIdx.x, lane = tid & 15, row = tid >> 4, c = blockIdx.x * 16 + lane;
-  float s = 0.0f, t = 0.0f;
+  float q[2][4] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
   if (c < channels) {
-#pragma unroll 8
-    for (int i = row; i < splits; i += 16) {
-      s += planes[(int64_t)(2 * i) * channels + c];
-      t += planes[(int64_t)(2 * i + 1) * channels + c];
+    int i = row;
+    // sixteen loads in flight; with twice as many the conv_train step of [32][56][56][64] fp16 takes 151 us instead of 139
+#pragma unroll 2
+    for (; i + 48 < splits; i += 64) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        q[0][u] += planes[(int64_t)(2 * (i + 16 * u)) * channels + c];
+        q[1][u] += planes[(int64_t)(2 * (i + 16 * u) + 1) * channels + c];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 3; ++u) {
+      if (i + 16 * u >= splits) continue;
+      q[0][u] += planes[(int64_t)(2 * (i + 16 * u)) * channels + c];
+      q[1][u] += planes[(int64_t)(2 * (i + 16 * u) + 1) * channels + c];
     }
   }
-  meet[0][tid] = s, meet[1][tid] = t;
+#pragma unroll
+  for (int w = 0; w < 2; ++w) meet[w][tid] = (q[w][0] + q[w][1]) + (q[w][2] + q[w][3]);
   __syncthreads();
   if (row > 0 || c >= channels) return;
 #pragma unroll
-  for (int r = 1; r < 16; ++r) s += meet[0][r * 16 + lane], t += meet[1][r * 16 + lane];
+  for (int w = 0; w < 2; ++w) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      q[w][u] = (meet[w][(4 * u) * 16 + lane] + meet[w][(4 * u + 1) * 16 + lane]) + (meet[w][(4 * u + 2) * 16 + lane] + meet[w][(4 * u + 3) * 16 + lane]);
+  }
+  float s = (q[0][0] + q[0][1]) + (q[0][2] + q[0][3]), t = (q[1][0] + q[1][1]) + (q[1][2] + q[1][3]);
   if (statistics) Statistics(count, &s, &t);
   first[c]  = s;
   second[c] = t;
