@@ -151,10 +151,13 @@ struct Stage {
   }
 };
 
-// D: d rounded up to an instance; WQ x 32 queries per block, KG groups of wavefronts that take the tiles' keys in turn
-template <typename T, int D, int WQ, int KG>
-__global__ void __launch_bounds__(64 * WQ * KG, 2)
+constexpr int kKeyGroups = 2;
+
+// D: d rounded up to an instance; WQ x 32 queries per block, groups of wavefronts that take the tiles' keys in turn
+template <typename T, int D, int WQ>
+__global__ void __launch_bounds__(64 * WQ * kKeyGroups, 2)
 attention_kernel(AttentionParams p) {
+  constexpr int KG      = kKeyGroups;
   constexpr bool F32    = sizeof(T) == 4;
   constexpr int THREADS = 64 * WQ * KG;
   constexpr int KT      = 32 * KG;                  // keys per tile
@@ -211,7 +214,7 @@ attention_kernel(AttentionParams p) {
       sv.Load((kt + 1) * KT, p.t1, total, chunks, tid);
     }
     const int left = total - kt * KT - kg * 32;  // keys of this group's 32
-    if (KG == 1 || left > 0) {
+    if (left > 0) {
       f32x16 s;
 #pragma unroll
       for (int r = 0; r < 16; ++r) s[r] = 0.0f;
@@ -286,34 +289,32 @@ attention_kernel(AttentionParams p) {
     }
   }
 
-  if constexpr (KG > 1) {
-    // the groups hold the same queries in the same registers: [register][lane] per wavefront
-    constexpr int REGS = DT * 16 + 2;
-    __syncthreads();
-    float* meet = reinterpret_cast<float*>(lds);
-    if (kg > 0) {
-      float* mine = meet + ((kg - 1) * WQ + wq) * REGS * 64 + lane;
+  // the groups hold the same queries in the same registers: [register][lane] per wavefront
+  constexpr int REGS = DT * 16 + 2;
+  __syncthreads();
+  float* meet = reinterpret_cast<float*>(lds);
+  if (kg > 0) {
+    float* mine = meet + ((kg - 1) * WQ + wq) * REGS * 64 + lane;
 #pragma unroll
-      for (int t = 0; t < DT; ++t)
+    for (int t = 0; t < DT; ++t)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) mine[(t * 16 + r) * 64] = o[t][r];
-      mine[(REGS - 2) * 64] = m;
-      mine[(REGS - 1) * 64] = l;
-    }
-    __syncthreads();
-    if (kg > 0) return;
+      for (int r = 0; r < 16; ++r) mine[(t * 16 + r) * 64] = o[t][r];
+    mine[(REGS - 2) * 64] = m;
+    mine[(REGS - 1) * 64] = l;
+  }
+  __syncthreads();
+  if (kg > 0) return;
 #pragma unroll
-    for (int g = 1; g < KG; ++g) {
-      const float* other = meet + ((g - 1) * WQ + wq) * REGS * 64 + lane;
-      const float m2 = other[(REGS - 2) * 64], top = fmaxf(m, m2), base = ex.Base(top);
-      const float keep = ex(m, base), add = ex(m2, base);
-      l = l * keep + other[(REGS - 1) * 64] * add;
+  for (int g = 1; g < KG; ++g) {
+    const float* other = meet + ((g - 1) * WQ + wq) * REGS * 64 + lane;
+    const float m2 = other[(REGS - 2) * 64], top = fmaxf(m, m2), base = ex.Base(top);
+    const float keep = ex(m, base), add = ex(m2, base);
+    l = l * keep + other[(REGS - 1) * 64] * add;
 #pragma unroll
-      for (int t = 0; t < DT; ++t)
+    for (int t = 0; t < DT; ++t)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) o[t][r] = o[t][r] * keep + other[(t * 16 + r) * 64] * add;
-      m = top;
-    }
+      for (int r = 0; r < 16; ++r) o[t][r] = o[t][r] * keep + other[(t * 16 + r) * 64] * add;
+    m = top;
   }
   if (query >= p.tq) return;
   // both halves of the wavefront hold this query; their shuffle partner has the same query and does not leave early
@@ -449,7 +450,7 @@ void LaunchRows(const AttentionParams& p, hipStream_t stream) {
 template <typename T, int D, int WQ>
 void LaunchBlocks(AttentionParams p, hipStream_t stream) {
   p.q_tiles = (p.tq + 32 * WQ - 1) / (32 * WQ);
-  hipLaunchKernelGGL((attention_kernel<T, D, WQ, 2>), dim3((unsigned)(p.bh * p.q_tiles)), dim3(128 * WQ), 0, stream, p);
+  hipLaunchKernelGGL((attention_kernel<T, D, WQ>), dim3((unsigned)(p.bh * p.q_tiles)), dim3(64 * WQ * kKeyGroups), 0, stream, p);
 }
 
 // Wavefronts of queries per block: more share a staged tile, fewer divide the work more evenly over 256 CUs.  Blocks per

@@ -226,8 +226,8 @@ struct DataTile {
   }
 };
 
-template <typename T, int BM, int BN, int KG>
-__global__ void __launch_bounds__(256 * KG, 2)
+template <typename T, int BM, int BN>
+__global__ void __launch_bounds__(256, 2)
 conv_data_kernel(DataParams p) {
   __shared__ __attribute__((aligned(256))) char lds[2 * (BM + BN) * 128];
   constexpr int KS = 128 / (int)sizeof(T);
@@ -245,17 +245,17 @@ conv_data_kernel(DataParams p) {
   flex::TileOf(blockIdx.x, tiles_m, tiles_n, &tm, &tn);
   const int m0 = tm * BM, n0 = tn * BN;
 
-  DataTile<T, BM, 256 * KG> ta;
-  flex::Tile<T, true, BN, 256 * KG> tb;
+  DataTile<T, BM, 256> ta;
+  flex::Tile<T, true, BN, 256> tb;
   ta.Init(p, m0, rows, hc, wc, (ry + p.pad_h - ky0) / p.stride_h, (rx + p.pad_w - kx0) / p.stride_w, nky, nkx, tid);
   tb.Init(static_cast<const T*>(p.wt) + (k > 0 ? (ky0 * p.slots_w + kx0) * p.slot : 0), k, n0, p.c, k, tid);
   typename flex::Mma<T, true, true, BM, BN>::acc_t acc;
-  flex::KLoop<T, true, true, BM, BN, KG>(lds, ta, tb, 0, (k + KS - 1) / KS, k / KS, k, tid, acc);
+  flex::KLoop<T, true, true, BM, BN, 1>(lds, ta, tb, 0, (k + KS - 1) / KS, k / KS, k, tid, acc);
 
   const int col0 = n0 + tid % (BN / 8) * 8;
   const int cols = min(p.c - col0, 8);
   T* dx = static_cast<T*>(p.dx);
-  flex::EachRowGroup<T, true, true, BM, BN, KG>(lds, acc, tid, [&](int row, int, const float (&v)[8]) {
+  flex::EachRowGroup<T, true, true, BM, BN, 1>(lds, acc, tid, [&](int row, int, const float (&v)[8]) {
     const int m = m0 + row;
     if (m >= rows || cols <= 0) return;
     const int jx = m % wc, jy = m / wc % hc, n = m / (wc * hc);
@@ -339,8 +339,8 @@ struct ImageTile {
   }
 };
 
-template <typename T, int BM, int BN, int KG>
-__global__ void __launch_bounds__(256 * KG, 2)
+template <typename T, int BM, int BN>
+__global__ void __launch_bounds__(256, 2)
 conv_filter_kernel(FilterGradParams p) {
   __shared__ __attribute__((aligned(256))) char lds[2 * (BM + BN) * 128];
   constexpr int KS = 128 / (int)sizeof(T);
@@ -350,8 +350,8 @@ conv_filter_kernel(FilterGradParams p) {
   const int m0 = tm * BM, n0 = tn * BN;
   const int s0 = blockIdx.y * p.steps_per_split, s1 = min(s0 + p.steps_per_split, p.steps);
 
-  flex::Tile<T, false, BM, 256 * KG> ta;
-  ImageTile<T, BN, 256 * KG> tb;
+  flex::Tile<T, false, BM, 256> ta;
+  ImageTile<T, BN, 256> tb;
   ta.Init(p.dy, p.fp, m0, p.fp, p.pixels, tid);
   tb.Init(p, n0, s0, tid);
   typename flex::Mma<T, false, false, BM, BN>::acc_t acc;
@@ -360,12 +360,12 @@ conv_filter_kernel(FilterGradParams p) {
   // chain | a step | two parts: 784 pixels 0.85e-7 | 2.25e-7 | 1.19e-7 | 1.00e-7, 12544 pixels 1.46 | 2.41 | 1.46 | 1.31,
   // 25088 pixels 1.91 | 3.26 | 1.53 | 1.38.  96 -> 200 3x3 / stride 2 on 35x35 at batch 8: 24.6 -> 25.5 us.
   constexpr int PARTS = sizeof(T) == 4 ? 2 : 0;
-  flex::KLoop<T, false, false, BM, BN, KG, PARTS>(lds, ta, tb, s0, s1, p.pixels / KS, p.pixels, tid, acc);
+  flex::KLoop<T, false, false, BM, BN, 1, PARTS>(lds, ta, tb, s0, s1, p.pixels / KS, p.pixels, tid, acc);
 
   const int columns = p.taps * p.cp;  // a multiple of a chunk, not of eight, in fp32
   const int col0    = n0 + tid % (BN / 8) * 8;
   float* plane      = p.planes + (int64_t)blockIdx.y * p.f * columns;
-  flex::EachRowGroup<T, false, false, BM, BN, KG>(lds, acc, tid, [&](int row, int, const float (&v)[8]) {
+  flex::EachRowGroup<T, false, false, BM, BN, 1>(lds, acc, tid, [&](int row, int, const float (&v)[8]) {
     const int m = m0 + row;
     if (m >= p.f) return;
     float* to = plane + (int64_t)m * columns + col0;
@@ -536,11 +536,11 @@ bool Data(const ConvBackwardArgs& a, hipStream_t stream) {
     if constexpr (sizeof(T) == 2) {
       // two blocks of 128x128 on every CU; fewer are better off as four times as many small ones
       if (tiles(128) * classes >= 512) {
-        hipLaunchKernelGGL((conv_data_kernel<T, 128, 128, 1>), dim3(tiles(128), classes), dim3(256), 0, stream, p);
+        hipLaunchKernelGGL((conv_data_kernel<T, 128, 128>), dim3(tiles(128), classes), dim3(256), 0, stream, p);
         large = true;
       }
     }
-    if (!large) hipLaunchKernelGGL((conv_data_kernel<T, 64, 64, 1>), dim3(tiles(64), classes), dim3(256), 0, stream, p);
+    if (!large) hipLaunchKernelGGL((conv_data_kernel<T, 64, 64>), dim3(tiles(64), classes), dim3(256), 0, stream, p);
   }
   if (unpack) {
     const int plane = a.h * a.w_in;
@@ -601,16 +601,16 @@ bool Filter(const ConvBackwardArgs& a, hipStream_t stream) {
   if constexpr (sizeof(T) == 2) {
     done = true;
     if (bm == 128 && bn == 128) {
-      hipLaunchKernelGGL((conv_filter_kernel<T, 128, 128, 1>), grid, dim3(256), 0, stream, p);
+      hipLaunchKernelGGL((conv_filter_kernel<T, 128, 128>), grid, dim3(256), 0, stream, p);
     } else if (bm == 128) {
-      hipLaunchKernelGGL((conv_filter_kernel<T, 128, 64, 1>), grid, dim3(256), 0, stream, p);
+      hipLaunchKernelGGL((conv_filter_kernel<T, 128, 64>), grid, dim3(256), 0, stream, p);
     } else if (bn == 128) {
-      hipLaunchKernelGGL((conv_filter_kernel<T, 64, 128, 1>), grid, dim3(256), 0, stream, p);
+      hipLaunchKernelGGL((conv_filter_kernel<T, 64, 128>), grid, dim3(256), 0, stream, p);
     } else {
       done = false;
     }
   }
-  if (!done) hipLaunchKernelGGL((conv_filter_kernel<T, 64, 64, 1>), grid, dim3(256), 0, stream, p);
+  if (!done) hipLaunchKernelGGL((conv_filter_kernel<T, 64, 64>), grid, dim3(256), 0, stream, p);
   hipLaunchKernelGGL((filter_reduce_kernel<T>), dim3((unsigned)((plane / 4 + 63) / 64)), dim3(256), 0, stream, p,
                      static_cast<T*>(a.out), a.c, splits, a.nhwc ? 1 : 0, a.alpha, a.beta);
   CINN_HIP_CALL(hipGetLastError());

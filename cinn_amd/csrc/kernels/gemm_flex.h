@@ -9,7 +9,7 @@ namespace cinn_hip_kernels {
 
 enum class FlexType : int { kF16, kBF16, kF32 };
 
-// C[m][n] = relu(acc * (scale[n] or alpha) + shift[n] + residual_scale * residual[m][n]), acc = sum_k A[m][k] B[k][n]
+// C[m][n] = acc * alpha + shift[n] + residual_scale * residual[m][n], acc = sum_k A[m][k] B[k][n]
 struct FlexGemm {
   FlexType type;
   const void* a;  // [m][k] when a_kc, else [k][m]; row pitch lda elements
@@ -20,12 +20,10 @@ struct FlexGemm {
   int64_t lda, ldb;
   int batch = 1;
   int64_t stride_a = 0, stride_b = 0, stride_c = 0;  // elements between batch entries; 0 shares the operand
-  const float* scale    = nullptr;
   const float* shift    = nullptr;
   const void* residual  = nullptr;  // of C's shape and batch stride
   float alpha           = 1.0f;
   float residual_scale  = 0.0f;
-  bool relu             = false;
 };
 
 // false when an extent is beyond the kernel's 32-bit tile offsets (the caller then has a slower form)

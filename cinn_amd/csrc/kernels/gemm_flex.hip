@@ -44,17 +44,14 @@ struct FlexParams {
   int steps;            // K steps of 128 bytes
   int steps_per_split;
   int full_steps;       // the first full_steps steps read nothing beyond K or beyond an operand's end
-  const float* scale;
   const float* shift;
   const void* residual;
   float alpha, residual_scale;
-  int relu;
 };
 
 // `residual` is 0 where there is none
-__device__ __forceinline__ float Finish(float v, float scale, float shift, float residual_scale, float residual, int relu) {
-  v = __builtin_fmaf(residual_scale, residual, __builtin_fmaf(v, scale, shift));
-  return relu ? fmaxf(v, 0.0f) : v;
+__device__ __forceinline__ float Finish(float v, float alpha, float shift, float residual_scale, float residual) {
+  return __builtin_fmaf(residual_scale, residual, __builtin_fmaf(v, alpha, shift));
 }
 
 // KG groups of four wavefronts (2 x 2 over the tile) share the block's tiles and take a K step's slices in turn; their
@@ -78,14 +75,10 @@ flex_gemm_kernel(FlexParams p) {
 
   const int col0 = n0 + tid % (BN / 8) * 8;  // the eight columns this thread finishes
   const int cols = min(p.n - col0, 8);
-  float sc[8], sh[8];
+  float sh[8];
   if (!p.partials) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int col = min(col0 + e, p.n - 1);
-      sc[e] = p.scale ? p.scale[col] : p.alpha;
-      sh[e] = p.shift ? p.shift[col] : 0.0f;
-    }
+    for (int e = 0; e < 8; ++e) sh[e] = p.shift ? p.shift[min(col0 + e, p.n - 1)] : 0.0f;
   }
   T* c              = static_cast<T*>(p.c) + blockIdx.y * p.stride_c;
   const T* residual = p.residual ? static_cast<const T*>(p.residual) + blockIdx.y * p.stride_c : nullptr;
@@ -109,13 +102,13 @@ flex_gemm_kernel(FlexParams p) {
       vec8 out, res = {0, 0, 0, 0, 0, 0, 0, 0};
       if (residual) __builtin_memcpy(&res, residual + at, 8 * sizeof(T));
 #pragma unroll
-      for (int e = 0; e < 8; ++e) out[e] = (T)Finish(v[e], sc[e], sh[e], p.residual_scale, (float)res[e], p.relu);
+      for (int e = 0; e < 8; ++e) out[e] = (T)Finish(v[e], p.alpha, sh[e], p.residual_scale, (float)res[e]);
       __builtin_memcpy(c + at, &out, 8 * sizeof(T));
     } else {
 #pragma unroll
       for (int e = 0; e < 8; ++e)
         if (e < cols)
-          c[at + e] = (T)Finish(v[e], sc[e], sh[e], p.residual_scale, residual ? (float)residual[at + e] : 0.0f, p.relu);
+          c[at + e] = (T)Finish(v[e], p.alpha, sh[e], p.residual_scale, residual ? (float)residual[at + e] : 0.0f);
     }
   });
 }
@@ -144,8 +137,7 @@ flex_reduce_kernel(FlexParams p, int splits, int64_t plane) {
   if (p.residual) __builtin_memcpy(res, static_cast<const T*>(p.residual) + at, V * sizeof(T));
 #pragma unroll
   for (int e = 0; e < V; ++e)
-    out[e] = (T)Finish(v[e], p.scale ? p.scale[col + e] : p.alpha, p.shift ? p.shift[col + e] : 0.0f, p.residual_scale,
-                       (float)res[e], p.relu);
+    out[e] = (T)Finish(v[e], p.alpha, p.shift ? p.shift[col + e] : 0.0f, p.residual_scale, (float)res[e]);
   __builtin_memcpy(static_cast<T*>(p.c) + at, out, V * sizeof(T));
 }
 
@@ -243,8 +235,8 @@ void Launch(const FlexGemm& g, hipStream_t stream) {
   p.stride_a = g.stride_a, p.stride_b = g.stride_b, p.stride_c = g.stride_c;
   p.steps      = Steps(g);
   p.full_steps = std::min(FullSteps<T>(g.a_kc, g.lda, g.m, g.k), FullSteps<T>(g.b_kc, g.ldb, g.n, g.k));
-  p.scale = g.scale, p.shift = g.shift, p.residual = g.residual;
-  p.alpha = g.alpha, p.residual_scale = g.residual_scale, p.relu = g.relu ? 1 : 0;
+  p.shift = g.shift, p.residual = g.residual;
+  p.alpha = g.alpha, p.residual_scale = g.residual_scale;
   Plan plan         = ChoosePlan(g, p.steps, stream);
   const int64_t plane = (int64_t)g.batch * g.m * g.n;
   p.steps_per_split = (p.steps + plan.splits - 1) / plan.splits;
