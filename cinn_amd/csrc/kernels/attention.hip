@@ -231,8 +231,9 @@ attention_kernel(AttentionParams p) {
 #pragma unroll
       for (int r = 1; r < 16; ++r) top = fmaxf(top, s[r]);
       top = fmaxf(m, fmaxf(top, __shfl_xor(top, 32)));
-      // What has been summed is rescaled only when a maximum has grown by more than a factor of 2^8: probabilities up to
-      // 256 lose nothing in either type, and after the first tiles few maxima do.
+      // What has been summed is rescaled only when a maximum has grown by more than a factor of 2^8 (fp32, whose exponent
+      // is natural: e^8): probabilities up to 256 (2981) lose nothing in either type, and after the first tiles few maxima
+      // grow that much.
       if (__ballot((top - m) * ex.c > 8.0f)) {
         const float keep = ex(m, ex.Base(top));
         l *= keep;
@@ -435,7 +436,10 @@ attention_row_kernel(AttentionParams p) {
 }
 
 // Queries per head up to which the row kernel is taken (every query reads all keys): a tile of the other kernel computes
-// 32 queries whatever their number.
+// 32 queries whatever their number.  us for 1 | 2 | 3 | 4 queries of d = 64 and on tiles: fp32 96 heads x 512 keys 8.6 | 11.9
+// | 18.0 | 18.6 and 29, 96 x 2048 23 | 34 | 55 | 60 and 102; fp16 12 x 512 6.2 | 6.3 | 6.4 | 6.4 and 10.3, 96 x 512 6.5 | 6.6
+// | 10.9 | 14.7 and 10.3, 96 x 2048 13 | 19 | 32 | 34 and 29.  The line is drawn by queries alone: with several heads per CU
+// tiles are ahead from two queries on (512 heads x 512 keys, fp16 16 | 28 | 38 | 49 and 15, fp32 23 | 42 | 59 | 80 and 35).
 constexpr int kRowQueries = 4;
 
 template <typename T, int LPK>
@@ -454,7 +458,10 @@ void LaunchBlocks(AttentionParams p, hipStream_t stream) {
 }
 
 // Wavefronts of queries per block: more share a staged tile, fewer divide the work more evenly over 256 CUs.  Blocks per
-// CU times a block's work, staging counted as half a wavefront.
+// CU times a block's work, staging counted as half a wavefront.  us with 1 | 2 | 4, d = 64, the choice in brackets: fp16 96
+// heads x 512 queries x 512 keys 26.7 | [17.7] | 24.1, 192 x 96 x 512 13.6 | 12.8 | [12.7], 12 x 1024 x 1024 20.2 | [17.0] |
+// 20.3; fp32 96 x 200 x 512 61 | 47 | [46], 96 x 512 x 512 92 | [71] | 90, 512 x 64 x 512 67 | [51] | 89.  Within 4% of the
+// best of the three in 24 shapes of 12 to 512 heads and 33 to 1024 queries.
 template <typename T, int D>
 void LaunchTiles(const AttentionParams& p, hipStream_t stream) {
   auto cost = [&](int wq) {

@@ -534,7 +534,11 @@ bool Data(const ConvBackwardArgs& a, hipStream_t stream) {
     auto tiles = [&](int t) { return (unsigned)(((rows + t - 1) / t) * ((a.c + t - 1) / t)); };
     bool large = false;
     if constexpr (sizeof(T) == 2) {
-      // two blocks of 128x128 on every CU; fewer are better off as four times as many small ones
+      // Two blocks of 128x128 on every CU; fewer are better off as four times as many small ones.  us on 64x64 | 128x128
+      // tiles, fp16, by the number of the latter (all classes): 84 (96 -> 200 3x3 on 35x35) 13.5 | 21.0, 208 (512 -> 512 on
+      // 14x14) 42.2 | 51.9, 392 (256 -> 256 on 28x28) 29.7 | 30.3, 784 (128 -> 128 on 56x56) 30.0 | 29.5, 1568 (256 -> 512 1x1
+      // on 56x56, three classes of four without a tap) 37.5 | 32.7, 3136 (128 -> 64 on 112x112) 71.7 | 58.1.  64 channels
+      // fill half of such a tile: 784 (64 -> 128 on 56x56) 19.4 | 27.1.
       if (tiles(128) * classes >= 512) {
         hipLaunchKernelGGL((conv_data_kernel<T, 128, 128>), dim3(tiles(128), classes), dim3(256), 0, stream, p);
         large = true;
@@ -574,7 +578,10 @@ bool Filter(const ConvBackwardArgs& a, hipStream_t stream) {
   p.tiles_m = (a.f + bm - 1) / bm;
   p.tiles_n = (columns + bn - 1) / bn;
   const int tiles = p.tiles_m * p.tiles_n;
-  // blocks for two to three rounds of the chip, at least four K steps each, at most 64 MiB of planes
+  // Blocks for two to three rounds of the chip, at least four K steps each, at most 64 MiB of planes.  us with 256 | 512 |
+  // 768 | 1024 blocks, 3x3 at batch 32: fp16, 128 rows: 128 -> 128 on 28x28 29.0 | 30.7 | 38.4 | 41.2, 256 -> 256 on 14x14
+  // 27.8 | 27.7 | 32.4 | 32.3, 512 -> 512 on 7x7 43.0 | 33.2 | 38.3 | 38.3; 64 rows: 64 -> 64 on 56x56 31.8 | 30.3 | 34.2 |
+  // 36.9; fp32: 64 -> 64 on 56x56 96 | 81 | 79 | 80, 256 -> 256 on 14x14 154 | 92 | 83 | 79.
   const int64_t plane = (int64_t)a.f * columns;
   int splits = std::max(1, (bm == 128 ? 512 : 768) / tiles);
   splits     = std::min(splits, std::max(1, p.steps / 4));
