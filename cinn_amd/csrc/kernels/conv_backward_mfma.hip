@@ -409,43 +409,39 @@ __global__ void __launch_bounds__(256)
 filter_reduce_kernel(FilterGradParams p, T* __restrict__ dw, int c, int splits, int nhwc, float alpha, float beta) {
   __shared__ __attribute__((aligned(16))) float part[3][64][4];
   __shared__ float shared[256];
-  __shared__ int again[64];
+  __shared__ int again[64], any;
   const int lane = threadIdx.x & 63, row = threadIdx.x >> 6;
-  const int64_t plane = (int64_t)p.f * p.taps * p.cp;
-  const int64_t at    = ((int64_t)blockIdx.x * 64 + lane) * 4;
+  const int plane = p.f * p.taps * p.cp, at = (blockIdx.x * 64 + lane) * 4;  // below 2^30
   flex::f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
   if (at < plane) {
 #pragma unroll 4
-    for (int s = row; s < splits; s += 4) v += *reinterpret_cast<const flex::f32x4*>(p.planes + s * plane + at);
+    for (int s = row; s < splits; s += 4) v += *reinterpret_cast<const flex::f32x4*>(p.planes + (int64_t)s * plane + at);
   }
   if (row > 0) *reinterpret_cast<flex::f32x4*>(part[row - 1][lane]) = v;
   __syncthreads();
-  const int ch     = (int)(at % p.cp);
-  const int tap    = (int)(at / p.cp % p.taps);
-  const int filter = (int)(at / p.cp / p.taps);
-  bool nan = false;
-  if (row == 0 && at < plane) {
+  const int column = at / p.cp, ch = at - column * p.cp, filter = column / p.taps, tap = column - filter * p.taps;
+  if (row == 0) {
+    int mask = 0;
+    if (at < plane) {
 #pragma unroll
-    for (int r = 0; r < 3; ++r) v += *reinterpret_cast<const flex::f32x4*>(part[r][lane]);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) nan = nan || (v[e] != v[e] && ch + e < c);
-  }
-  if (__syncthreads_or(nan)) {
-    if (row == 0) {
-      int mask = 0;
+      for (int r = 0; r < 3; ++r) v += *reinterpret_cast<const flex::f32x4*>(part[r][lane]);
       const int y0 = tap / p.kw * p.dil_h - p.pad_h, x0 = tap % p.kw * p.dil_w - p.pad_w;
-      if (nan && (y0 < 0 || x0 < 0 || y0 + (p.oh - 1) * p.stride_h >= p.h || x0 + (p.ow - 1) * p.stride_w >= p.w)) {
-        for (int e = 0; e < 4; ++e)
-          if (v[e] != v[e] && ch + e < c) mask |= 1 << e;
+      if (y0 < 0 || x0 < 0 || y0 + (p.oh - 1) * p.stride_h >= p.h || x0 + (p.ow - 1) * p.stride_w >= p.w) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) mask |= v[e] != v[e] && ch + e < c ? 1 << e : 0;
       }
-      again[lane] = mask;
     }
-    __syncthreads();
+    again[lane] = mask;
+    const bool some = __any(mask != 0);
+    if (lane == 0) any = some;
+  }
+  __syncthreads();
+  if (any) {
     for (int l = 0; l < 64; ++l) {
-      const int64_t other = ((int64_t)blockIdx.x * 64 + l) * 4;
+      const int other = (blockIdx.x * 64 + l) * 4, col = other / p.cp;
       for (int e = 0; e < 4; ++e) {
         if (!(again[l] >> e & 1)) continue;
-        const float sum = FilterElement<T>(p, (int)(other / p.cp / p.taps), (int)(other / p.cp % p.taps), (int)(other % p.cp) + e, shared);
+        const float sum = FilterElement<T>(p, col / p.taps, col % p.taps, other % p.cp + e, shared);
         if (row == 0 && lane == l) v[e] = sum;
       }
     }

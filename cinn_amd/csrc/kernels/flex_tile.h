@@ -263,10 +263,23 @@ __device__ __forceinline__ void TileOf(int bid, int tiles_m, int tiles_n, int* t
   *tn = in / rows;
 }
 
+// A K step whose products are summed in PARTS chains of their own before they are added to acc.
+template <typename M, int PARTS>
+__device__ __forceinline__ void InParts(const char* a_tile, const char* b_tile, int wm, int wn, int lane, typename M::acc_t& acc) {
+  typename M::acc_t sum[PARTS];
+#pragma unroll
+  for (int part = 0; part < PARTS; ++part) {
+    M::Zero(sum[part]);
+    M::template Step<PARTS>(a_tile, b_tile, wm, wn, part, lane, sum[part]);
+  }
+#pragma unroll
+  for (int part = 1; part < PARTS; ++part) M::Add(sum[0], sum[part]);
+  M::Add(acc, sum[0]);
+}
+
 // The K loop over steps [s, s1): ta / tb are operand tiles with Load<guard>(registers, step, k, tid) and Store(LDS, ...);
 // steps below full_steps need no guard.  `lds` holds two stages.
-// PARTS > 0: a step's products are summed in PARTS chains of their own before they are added to acc, which then is a chain
-// of steps and not of products.
+// PARTS > 0 (one K group): acc is a chain of steps and not of products.
 template <typename T, bool A_KC, bool B_KC, int BM, int BN, int KG, int PARTS = 0, typename TA, typename TB>
 __device__ __forceinline__ void KLoop(char* lds, TA& ta, TB& tb, int s, int s1, int full_steps, int k_total, int tid,
                                       typename Mma<T, A_KC, B_KC, BM, BN>::acc_t& acc) {
@@ -295,23 +308,6 @@ __device__ __forceinline__ void KLoop(char* lds, TA& ta, TB& tb, int s, int s1, 
     tb.Store(stage + BM * 128, rb[slot], tid);
   };
 
-  auto multiply = [&](const char* stage) {
-    if constexpr (PARTS == 0) {
-      M::template Step<KG>(stage, stage + BM * 128, wm, wn, kg, lane, acc);
-    } else {
-      static_assert(KG == 1, "the parts of a step are its slices");
-      typename M::acc_t sum[PARTS];
-#pragma unroll
-      for (int part = 0; part < PARTS; ++part) {
-        M::Zero(sum[part]);
-        M::template Step<PARTS>(stage, stage + BM * 128, wm, wn, part, lane, sum[part]);
-      }
-#pragma unroll
-      for (int part = 1; part < PARTS; ++part) M::Add(sum[0], sum[part]);
-      M::Add(acc, sum[0]);
-    }
-  };
-
   M::Zero(acc);
 #pragma unroll
   for (int u = 0; u < PF; ++u)
@@ -326,7 +322,11 @@ __device__ __forceinline__ void KLoop(char* lds, TA& ta, TB& tb, int s, int s1, 
     for (int u = 0; u < 2; ++u) {
       char* cur = lds + (u & 1) * STAGE;
       load(s + u + PF, u % PF, true);
-      multiply(cur);
+      if constexpr (PARTS == 0) {
+        M::template Step<KG>(cur, cur + BM * 128, wm, wn, kg, lane, acc);
+      } else {
+        InParts<M, PARTS>(cur, cur + BM * 128, wm, wn, lane, acc);
+      }
       store((u + 1) % PF, lds + ((u + 1) & 1) * STAGE);
       __syncthreads();
     }
@@ -337,7 +337,11 @@ __device__ __forceinline__ void KLoop(char* lds, TA& ta, TB& tb, int s, int s1, 
       if (s + u >= s1) break;
       char* cur = lds + (u & 1) * STAGE;
       if (s + u + PF < s1) load(s + u + PF, u % PF, s + u + PF < full_steps);
-      multiply(cur);
+      if constexpr (PARTS == 0) {
+        M::template Step<KG>(cur, cur + BM * 128, wm, wn, kg, lane, acc);
+      } else {
+        InParts<M, PARTS>(cur, cur + BM * 128, wm, wn, lane, acc);
+      }
       if (s + u + 1 < s1) store((u + 1) % PF, lds + ((u + 1) & 1) * STAGE);
       __syncthreads();
     }
