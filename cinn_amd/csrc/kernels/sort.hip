@@ -37,7 +37,9 @@ struct SortParams {
   int32_t* index;  // may be null
   int32_t* rank;   // may be null: the position of every element (count of smaller / larger elements of its row)
   void* sorted;    // may be null
+  int64_t* index64;  // may be null
   int size, inner, ti;  // ti: neighbouring columns per tile
+  int keep;             // the first `keep` slots are written (the outputs' extent along the axis); ranks are for all elements
   int tiles_per_outer;  // ceil(inner / ti)
   int descending;
 };
@@ -113,11 +115,14 @@ __global__ void __launch_bounds__(kThreads) argsort_tile_kernel(SortParams p) {
   }
   has_nan = __syncthreads_or(has_nan);
 
+  const int64_t result = (int64_t)outer * p.keep * p.inner + i0;
   auto scatter = [&](int k, int c, int slot, int position) {
-    const int64_t at = base + (int64_t)slot * p.inner + c;
-    if (p.index) p.index[at] = k;
-    if (p.sorted) static_cast<T*>(p.sorted)[at] = X[base + (int64_t)k * p.inner + c];
     if (p.rank) p.rank[base + (int64_t)k * p.inner + c] = position;
+    if (slot >= p.keep) return;
+    const int64_t at = result + (int64_t)slot * p.inner + c;
+    if (p.index) p.index[at] = k;
+    if (p.index64) p.index64[at] = k;
+    if (p.sorted) static_cast<T*>(p.sorted)[at] = X[base + (int64_t)k * p.inner + c];
   };
 
   if (!has_nan) {
@@ -465,6 +470,10 @@ __global__ void __launch_bounds__(64 * WAVES) row_select_kernel(RowParams p) {
 // Columns (inner > 1) go to the network from this size: [32, 256, 64] 106 -> 16 us, [128, 256, 512] 679 -> 529 us (a
 // column's accesses take a line each); at 64 elements the scan's whole-line tiles are ahead.
 constexpr int kColumnSort   = 256;
+// Short columns of which a good part is wanted go to the scan in top_k as well: a wavefront per column and a round per entry
+// cost more.  us for k = 1 | 5 | 16, selection against scan, fp32: [1, 16, 100000] 27 | 54 | 139 against 14 | 14 | 16, [128, 64,
+// 512] 25 | 38 | 96 against 66; [32, 100, 1000] 21 | 25 | 53 against 79.
+constexpr int kColumnScan   = 64;
 constexpr int kRowSortLimit = 16384;  // words of a row in one block's LDS (128 KiB)
 
 template <typename T>
@@ -539,6 +548,33 @@ void Launch(const SortParams& p, int blocks, size_t lds_bytes, hipStream_t strea
   }
 }
 
+// the scan: tiles of neighbouring columns
+void LaunchTiles(SortParams p, Elem elem, int outer, hipStream_t s) {
+  const size_t key_bytes = (elem == Elem::kF64 || elem == Elem::kI64) ? 8 : 4;
+  const size_t per_col   = (size_t)((p.size + 3) & ~3) * (key_bytes + 4);  // keys and, for tiles with a NaN, positions
+  CINN_RT_CHECK(per_col <= (size_t)kLdsLimit, "argsort: %d elements along the sorted axis exceed the %zu that one block's LDS holds", p.size,
+                (size_t)kLdsLimit / (key_bytes + 4));
+  // neighbouring columns per tile: whole 64-byte pieces of a row when there are that many, bounded by LDS and by the
+  // work one block should carry
+  int ti = p.inner < 16 ? p.inner : 16;
+  while (ti > 1 && (per_col * ti > (size_t)kLdsLimit / 2 || (int64_t)p.size * ti > 8192)) ti /= 2;
+  p.ti              = ti;
+  p.tiles_per_outer = (p.inner + ti - 1) / ti;
+  const int64_t blocks = (int64_t)outer * p.tiles_per_outer;
+  CINN_RT_CHECK(blocks < INT_MAX, "argsort: too many tiles");
+  const size_t lds_bytes = per_col * ti;
+  switch (elem) {
+    case Elem::kF32: Launch<float>(p, (int)blocks, lds_bytes, s); break;
+    case Elem::kF64: Launch<double>(p, (int)blocks, lds_bytes, s); break;
+    case Elem::kF16: Launch<_Float16>(p, (int)blocks, lds_bytes, s); break;
+    case Elem::kBF16: Launch<__bf16>(p, (int)blocks, lds_bytes, s); break;
+    case Elem::kI32: Launch<int32_t>(p, (int)blocks, lds_bytes, s); break;
+    case Elem::kI64: Launch<int64_t>(p, (int)blocks, lds_bytes, s); break;
+    default: break;
+  }
+  CINN_HIP_CALL(hipGetLastError());
+}
+
 }  // namespace
 
 extern "C" void cinn_call_hip_argsort(void* v_args, int num_args, int outer, int size, int inner, int is_ascend,
@@ -570,7 +606,7 @@ extern "C" void cinn_call_hip_argsort(void* v_args, int num_args, int outer, int
     CINN_RT_CHECK(b->memory != x->memory, "argsort: sorting in place is not supported");
     p.sorted = b->memory;
   }
-  p.size = size, p.inner = inner, p.descending = is_ascend ? 0 : 1;
+  p.size = p.keep = size, p.inner = inner, p.descending = is_ascend ? 0 : 1;
   auto s = static_cast<hipStream_t>(stream);
   // Rows of the trailing axis sort in a network; columns too once the scan's work outweighs its whole-line accesses.
   if (elem != Elem::kF64 && elem != Elem::kI64 && size <= kRowSortLimit && (inner == 1 || size >= kColumnSort)) {
@@ -584,29 +620,7 @@ extern "C" void cinn_call_hip_argsort(void* v_args, int num_args, int outer, int
     CINN_HIP_CALL(hipGetLastError());
     return;
   }
-  const size_t key_bytes = (elem == Elem::kF64 || elem == Elem::kI64) ? 8 : 4;
-  const size_t per_col   = (size_t)((size + 3) & ~3) * (key_bytes + 4);  // keys and, for tiles with a NaN, positions
-  CINN_RT_CHECK(per_col <= (size_t)kLdsLimit, "argsort: %d elements along the sorted axis exceed the %zu that one block's LDS holds", size,
-                (size_t)kLdsLimit / (key_bytes + 4));
-  // neighbouring columns per tile: whole 64-byte pieces of a row when there are that many, bounded by LDS and by the
-  // work one block should carry
-  int ti = inner < 16 ? inner : 16;
-  while (ti > 1 && (per_col * ti > (size_t)kLdsLimit / 2 || (int64_t)size * ti > 8192)) ti /= 2;
-  p.ti              = ti;
-  p.tiles_per_outer = (inner + ti - 1) / ti;
-  const int64_t blocks = (int64_t)outer * p.tiles_per_outer;
-  CINN_RT_CHECK(blocks < INT_MAX, "argsort: too many tiles");
-  const size_t lds_bytes = per_col * ti;
-  switch (elem) {
-    case Elem::kF32: Launch<float>(p, (int)blocks, lds_bytes, s); break;
-    case Elem::kF64: Launch<double>(p, (int)blocks, lds_bytes, s); break;
-    case Elem::kF16: Launch<_Float16>(p, (int)blocks, lds_bytes, s); break;
-    case Elem::kBF16: Launch<__bf16>(p, (int)blocks, lds_bytes, s); break;
-    case Elem::kI32: Launch<int32_t>(p, (int)blocks, lds_bytes, s); break;
-    case Elem::kI64: Launch<int64_t>(p, (int)blocks, lds_bytes, s); break;
-    default: break;
-  }
-  CINN_HIP_CALL(hipGetLastError());
+  LaunchTiles(p, elem, outer, s);
 }
 
 // The first k entries along an axis of the order cinn_call_hip_argsort gives: values (bit 1 of `outputs`) and int64
@@ -634,9 +648,17 @@ extern "C" void cinn_call_hip_top_k(void* v_args, int num_args, int outer, int s
     CINN_RT_CHECK(b->type.code == cinn_type_int && b->type.bits == 64, "top_k: the indices must be int64");
     r.index64 = reinterpret_cast<int64_t*>(b->memory);
   }
-  auto s = static_cast<hipStream_t>(stream);
+  auto s          = static_cast<hipStream_t>(stream);
+  const Elem elem = ElemOf(x);
+  if (inner > 1 && size <= kColumnScan && size <= 4 * k + 16 && elem != Elem::kF64 && elem != Elem::kI64 && elem != Elem::kUnsupported) {
+    SortParams p{};
+    p.x = r.x, p.sorted = r.sorted, p.index64 = r.index64;
+    p.size = size, p.keep = k, p.inner = inner, p.descending = is_ascend ? 0 : 1;
+    LaunchTiles(p, elem, outer, s);
+    return;
+  }
   auto run = [&](auto launch_select, auto launch_sort) { k <= kSelect ? launch_select(r, outer * inner, s) : launch_sort(r, outer * inner, s); };
-  switch (ElemOf(x)) {
+  switch (elem) {
     case Elem::kF32: run(LaunchRowSelect<float>, LaunchRowSort<float>); break;
     case Elem::kF16: run(LaunchRowSelect<_Float16>, LaunchRowSort<_Float16>); break;
     case Elem::kBF16: run(LaunchRowSelect<__bf16>, LaunchRowSort<__bf16>); break;

@@ -129,3 +129,21 @@ def test_top_k_ascending_through_the_c_abi(gpu):
     runtime.synchronize()
     index = np.argsort(x, axis=1, kind="stable")
     assert np.array_equal(I.numpy(), index[:, :4]) and np.array_equal(V.numpy(), np.sort(x, axis=1)[:, :4])
+
+
+# the scan up to 64 elements of which at least (size - 16) / 4 are wanted, the selection and the network elsewhere
+@pytest.mark.parametrize("kind", ["float32", "float16", "int32"])
+@pytest.mark.parametrize("size,inner,k", [(1, 3, 1), (16, 1000, 1), (16, 33, 16), (21, 17, 1), (20, 17, 1), (64, 5, 12), (64, 5, 11), (63, 40, 50),
+                                          (65, 9, 20), (300, 4, 5)])
+def test_top_k_of_columns(gpu, size, inner, k, kind):
+    rng = np.random.default_rng(size + inner + k)
+    x = values(rng, (3, size, inner), kind)
+    if kind != "int32":
+        x[1][rng.random((size, inner)) < 0.2] = np.nan
+    b = NetBuilder("top")
+    v = b.create_input(Int(32) if kind == "int32" else Float(16 if kind == "float16" else 32), list(x.shape), "x")
+    (got_values, got_index), comp = run(b, {v: x}, list(b.top_k(v, k, 1)))
+    assert comp.num_instructions() == 1
+    index, _, ranked = oracle.argsort(x, 1, False)
+    assert np.array_equal(got_index, index[:, :k])
+    assert np.array_equal(got_values, ranked[:, :k], equal_nan=kind != "int32")
