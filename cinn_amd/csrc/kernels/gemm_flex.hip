@@ -161,19 +161,20 @@ size_t PlaneBytes(const FlexGemm& g, int splits) { return (size_t)splits * g.bat
 
 // Block tile and K split with the smallest estimated time.  The estimate (us) adds, per CU, the K steps of the blocks
 // it gets, and what a split writes and reads back.  A block alone on its CU takes `alone` per step, blocks that share
-// one take `shared` each, at most `resident` at a time; measured on a product of 768 x 3072 x 4100 (A and B [k][rows]),
-// 2048^3, 1000^3 and 512 x 512 x 4096 with every tile and 1, 4 and 8 splits, which the estimate ranks as measured:
-// 16-bit 768 x 3072 x 4100 39 us on 128x128 tiles of two groups, 46 on 64x64 tiles, 2048^3 26 / 33, 1000^3 17 / 10;
-// [2] x 2336 x 3250 x 153 25 us on 128x128 tiles of one group (two blocks per CU cover each other's epilogue) against
-// 40 with two; fp32 768 x 3072 x 4100 262 us on 128x128 tiles, 205 on 64x64 and 170 with K split four ways: a step is
-// bound by the matrix pipe there, and small tiles spread evenly.
+// one take `shared` each, at most `resident` at a time; its start and epilogue are worth `extra` steps, which decides
+// short reductions.  Fitted to every tile at M = N = 1600, 2056, 3000, 4000 and 1000 x 3000 with K = 40 to 4000 (16 bits).
+// us on 64x64 | 128x128 | 128x128 tiles of two groups: 3000 x 3000 x 200 17.7 | 17.8 | 27.2 (with two steps' worth for every
+// tile, as the estimate once had it, the last was chosen), x 4000 134 | 137 | 119; 1600 x 1600 x 200 7.8 | 8.9 | 10.1, x 1000
+// 17.0 | 18.1 | 15.9; 4000 x 4000 x 4000 234 | 152 | 165; A^T B 768 x 3072 x 4100 46 | - | 39.  fp32 768 x 3072 x 4100 262 us on
+// 128x128 tiles, 205 on 64x64 and 170 with K split four ways: a step is bound by the matrix pipe there, and small tiles
+// spread evenly.
 Plan ChoosePlan(const FlexGemm& g, int steps, hipStream_t stream) {
   struct Shape {
     int tile, kg, resident;
-    double alone, shared;
+    double alone, shared, extra;
   };
-  static const Shape k16[] = {{64, 1, 4, 0.42, 0.21}, {128, 1, 2, 0.87, 0.55}, {128, 2, 1, 0.62, 0.62}};
-  static const Shape k32[] = {{64, 1, 4, 0.62, 0.50}};
+  static const Shape k16[] = {{64, 1, 4, 0.42, 0.245, 3.0}, {128, 1, 2, 0.87, 0.55, 4.0}, {128, 2, 1, 0.53, 0.53, 10.0}};
+  static const Shape k32[] = {{64, 1, 4, 0.62, 0.50, 2.0}};
   const bool fp32    = g.type == FlexType::kF32;
   const Shape* shape = fp32 ? k32 : k16;
   const int shapes   = fp32 ? 1 : 3;
@@ -188,8 +189,7 @@ Plan ChoosePlan(const FlexGemm& g, int steps, hipStream_t stream) {
       const int rounds    = per_cu / t.resident, rest = per_cu % t.resident;
       const double round  = std::max(t.alone, t.shared * t.resident);
       const double a_step = rounds * round + (rest ? std::max(t.alone, t.shared * rest) : 0.0);
-      // a block's start and epilogue: about two steps' worth
-      double us = a_step * ((steps + splits - 1) / splits + 2);
+      double us = a_step * ((steps + splits - 1) / splits + t.extra);
       if (splits > 1) us += 4.0 + splits * plane * 8.0 / 4e6;
       if (us < least) least = us, best = {t.tile, t.kg, splits};
     }

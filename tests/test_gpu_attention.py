@@ -1,5 +1,5 @@
 """Attention as one call (attention.hip, frontend/attention_pass.cc) at the edges of its tiles - 32 queries per wavefront,
-128 per block, 64 (fp32: 32) keys per stage, four queries for the row kernel, rows between the instantiated lengths -
+32 to 128 per block, 64 keys per stage, four queries for the row kernel, rows between the instantiated lengths -
 against float64, and in every layout the pass reads in place against the calls it replaces.
 
 Bounds: a score is an fp32 sum of d products (2^-24 sqrt(d) + 2^-22 of the products' magnitudes); the relative error of a

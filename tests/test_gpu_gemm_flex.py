@@ -19,9 +19,10 @@ pytestmark = pytest.mark.gpu
 
 SHAPES = [
     (1, 1, 1, 1), (1, 1, 7, 3), (1, 3, 1, 65), (1, 63, 65, 64), (1, 65, 63, 129), (1, 129, 127, 127), (5, 1, 215, 48),
-    (3, 48, 1, 215), (1, 17, 300, 172), (2, 1500, 1300, 33),  # two K steps on 128x128 tiles of one group
-    (1, 1290, 1540, 700),  # 128x128 tiles of two groups
-    (1, 70, 90, 3001),     # K split
+    (3, 48, 1, 215), (1, 17, 300, 172), (2, 1500, 1300, 33), (1, 1290, 1540, 700),  # many 64x64 tiles
+    (1, 2050, 2000, 200),   # 16 bits: 128x128 tiles of one group
+    (1, 1290, 1540, 1410),  # 16 bits: 128x128 tiles of two groups
+    (1, 70, 90, 3001),      # K split
 ]
 
 
@@ -71,7 +72,7 @@ def test_what_lies_beyond_k_is_not_multiplied(gpu, kind, ta, tb):
                                                (1, 512, 1024, 1024, True), (1, 1024, 1024, 96, False), (2, 128, 128, 32, False),
                                                (1, 896, 1152, 1024, False)])
 def test_whole_fp32_tiles_that_leave_cus_idle_split_k(gpu, batch, m, n, k, split, ta, tb):
-    """extents that are whole 128x128 tiles: tiles of 64x64 for half the CUs or fewer and a K long enough use partial sums (the stream
+    """extents that are whole 128x128 tiles: a K that is worth splitting over the CUs left idle uses partial sums (the stream
     has no scratch before), others do not"""
     rng = np.random.default_rng(k)
     a, af = rounded(rng, (batch, k, m) if ta else (batch, m, k), "float32")
