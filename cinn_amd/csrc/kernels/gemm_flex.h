@@ -26,9 +26,14 @@ struct FlexGemm {
   float residual_scale  = 0.0f;
 };
 
+// block tile, groups of wavefronts and K split, and the estimate (microseconds) they were chosen by
+struct FlexPlan {
+  int tile, kg, splits;
+  double us;
+};
+
 // false when an extent is beyond the kernel's 32-bit tile offsets (the caller then has a slower form)
-bool TryFlexGemm(const FlexGemm& g, hipStream_t stream);
-// whether TryFlexGemm takes the product and splits its K
-bool FlexGemmSplitsK(const FlexGemm& g, hipStream_t stream);
+bool PlanFlexGemm(const FlexGemm& g, hipStream_t stream, FlexPlan* plan);
+void RunFlexGemm(const FlexGemm& g, FlexPlan plan, hipStream_t stream);
 
 }  // namespace cinn_hip_kernels

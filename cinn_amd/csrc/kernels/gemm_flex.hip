@@ -2,9 +2,8 @@
 //
 //   C[m][n] = epilogue( sum_k A[m][k] B[k][n] ),  A stored [m][k] or [k][m], B stored [n][k] or [k][n]
 //
-// The direct-to-LDS kernels of gemm_mfma.hip need whole, aligned 16-byte chunks and a K-contiguous A.  Everything else
-// comes here: transposed A (the weight gradient of a linear layer), extents that are no multiple of anything, many
-// small batch entries.  What it does instead:
+// The direct-to-LDS kernels of gemm_mfma.hip need whole, aligned 16-byte chunks and enough tiles.  Everything else comes
+// here: extents that are no multiple of anything, few tiles, many small batch entries.  What it does instead:
 //   * an operand keeps its own order on the way into LDS: a K-contiguous one as [row][128 bytes of k], the other as
 //     [k][rows].  Fragments of the latter are read with ds_read_b64_tr_b16 (16-bit) or as single floats, so nothing is
 //     transposed in registers or in memory beforehand;
@@ -14,7 +13,7 @@
 //   * rows beyond M / N repeat the last one; what they produce is not stored;
 //   * grids too small for the chip split K over blockIdx.z, and a second kernel adds the fp32 planes.
 // Measured before (transposing copies in front of a convolution kernel, one launch per batch entry, or scalar FMAs
-// where K was no multiple of a chunk) and here, us: fp16 A^T B 768 x 3072 x 4100 871 -> 39 (495 TFLOP/s), [64] x 1 x 215
+// where K was no multiple of a chunk) and here, us: fp16 A^T B 768 x 3072 x 4100 871 -> 39 (direct-to-LDS 28.5), [64] x 1 x 215
 // x 48 262 -> 4.0, 1000^3 15.3 -> 10.4; bf16 [2] x 2336 x 3250 x 153 120 -> 25, 512 x 512 x 4096 26 -> 14; fp32 1000^3
 // 36 -> 24 (84 TFLOP/s), A^T B 768 x 3072 x 4100 218 -> 171 (113 TFLOP/s).  A step of a 64x64 tile is bound by the trip of its chunks to LDS
 // (0.42 us for a block alone), of a 128x128 tile by the register staging around its MFMAs (0.6 us for 0.2 of MFMA).
@@ -152,10 +151,6 @@ int FullSteps(bool kc, int64_t ld, int rows, int k) {
   return room < 0 ? 0 : (int)((std::min<int64_t>(room / ld, k - 1) + 1) / KS);
 }
 
-struct Plan {
-  int tile, kg, splits;
-};
-
 // the partial sums of a split
 size_t PlaneBytes(const FlexGemm& g, int splits) { return (size_t)splits * g.batch * g.m * g.n * sizeof(float); }
 
@@ -168,7 +163,7 @@ size_t PlaneBytes(const FlexGemm& g, int splits) { return (size_t)splits * g.bat
 // 17.0 | 18.1 | 15.9; 4000 x 4000 x 4000 234 | 152 | 165; A^T B 768 x 3072 x 4100 46 | - | 39.  fp32 768 x 3072 x 4100 262 us on
 // 128x128 tiles, 205 on 64x64 and 170 with K split four ways: a step is bound by the matrix pipe there, and small tiles
 // spread evenly.
-Plan ChoosePlan(const FlexGemm& g, int steps, hipStream_t stream) {
+FlexPlan ChoosePlan(const FlexGemm& g, int steps, hipStream_t stream) {
   struct Shape {
     int tile, kg, resident;
     double alone, shared, extra;
@@ -179,8 +174,7 @@ Plan ChoosePlan(const FlexGemm& g, int steps, hipStream_t stream) {
   const Shape* shape = fp32 ? k32 : k16;
   const int shapes   = fp32 ? 1 : 3;
   const double plane = (double)g.batch * g.m * g.n;
-  Plan best{64, 1, 1};
-  double least = 1e30;
+  FlexPlan best{64, 1, 1, 1e30};
   for (int i = 0; i < shapes; ++i) {
     const Shape& t = shape[i];
     const double tiles = (double)((g.m + t.tile - 1) / t.tile) * ((g.n + t.tile - 1) / t.tile) * g.batch;
@@ -191,7 +185,7 @@ Plan ChoosePlan(const FlexGemm& g, int steps, hipStream_t stream) {
       const double a_step = rounds * round + (rest ? std::max(t.alone, t.shared * rest) : 0.0);
       double us = a_step * ((steps + splits - 1) / splits + t.extra);
       if (splits > 1) us += 4.0 + splits * plane * 8.0 / 4e6;
-      if (us < least) least = us, best = {t.tile, t.kg, splits};
+      if (us < best.us) best = {t.tile, t.kg, splits, us};
     }
   }
   // under capture without an eager run or a reservation: K whole, which needs no scratch
@@ -212,7 +206,7 @@ bool Fits(const FlexGemm& g) {
 }
 
 template <typename T, bool A_KC, bool B_KC>
-void LaunchTiles(const Plan& plan, dim3 grid, const FlexParams& p, hipStream_t stream) {
+void LaunchTiles(const FlexPlan& plan, dim3 grid, const FlexParams& p, hipStream_t stream) {
   if (plan.tile == 64) {
     hipLaunchKernelGGL((flex_gemm_kernel<T, A_KC, B_KC, 64, 64, 1>), grid, dim3(256), 0, stream, p);
     return;
@@ -227,7 +221,7 @@ void LaunchTiles(const Plan& plan, dim3 grid, const FlexParams& p, hipStream_t s
 }
 
 template <typename T>
-void Launch(const FlexGemm& g, hipStream_t stream) {
+void Launch(const FlexGemm& g, FlexPlan plan, hipStream_t stream) {
   FlexParams p;
   p.a = g.a, p.b = g.b, p.c = g.c;
   p.m = g.m, p.n = g.n, p.k = g.k;
@@ -237,7 +231,6 @@ void Launch(const FlexGemm& g, hipStream_t stream) {
   p.full_steps = std::min(FullSteps<T>(g.a_kc, g.lda, g.m, g.k), FullSteps<T>(g.b_kc, g.ldb, g.n, g.k));
   p.shift = g.shift, p.residual = g.residual;
   p.alpha = g.alpha, p.residual_scale = g.residual_scale;
-  Plan plan         = ChoosePlan(g, p.steps, stream);
   const int64_t plane = (int64_t)g.batch * g.m * g.n;
   p.steps_per_split = (p.steps + plan.splits - 1) / plan.splits;
   plan.splits       = (p.steps + p.steps_per_split - 1) / p.steps_per_split;
@@ -263,16 +256,18 @@ void Launch(const FlexGemm& g, hipStream_t stream) {
 
 }  // namespace
 
-bool FlexGemmSplitsK(const FlexGemm& g, hipStream_t stream) { return Fits(g) && ChoosePlan(g, Steps(g), stream).splits > 1; }
-
-bool TryFlexGemm(const FlexGemm& g, hipStream_t stream) {
+bool PlanFlexGemm(const FlexGemm& g, hipStream_t stream, FlexPlan* plan) {
   if (!Fits(g)) return false;
-  switch (g.type) {
-    case FlexType::kF16: Launch<_Float16>(g, stream); break;
-    case FlexType::kBF16: Launch<__bf16>(g, stream); break;
-    case FlexType::kF32: Launch<float>(g, stream); break;
-  }
+  *plan = ChoosePlan(g, Steps(g), stream);
   return true;
+}
+
+void RunFlexGemm(const FlexGemm& g, FlexPlan plan, hipStream_t stream) {
+  switch (g.type) {
+    case FlexType::kF16: Launch<_Float16>(g, plan, stream); break;
+    case FlexType::kBF16: Launch<__bf16>(g, plan, stream); break;
+    case FlexType::kF32: Launch<float>(g, plan, stream); break;
+  }
 }
 
 }  // namespace cinn_hip_kernels

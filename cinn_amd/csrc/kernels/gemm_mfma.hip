@@ -3,25 +3,21 @@
 //   C[M,N] = alpha * op(A)[M,K] * op(B)[K,N] + beta * C          (row-major, optional batch)
 //
 // Kernels:
-//   * gemm16_dma_kernel   - bf16 / fp16 with A stored [M][K] (the common case) and K % 64 == 0, on
+//   * gemm16_dma_kernel   - bf16 / fp16 in whole 16-byte chunks and (mostly) K % 64 == 0, on
 //     v_mfma_f32_16x16x32: 256x256x64 tile, 512 threads, direct global -> LDS loads of whole 128-byte lines into two
-//     stages, transposing LDS reads for row-major B; also as 128x128 tiles (two or four stages) and 256x64 tiles, and
-//     with the A operand gathered from a channels-last image (implicit-GEMM convolution); see the comment at the kernel.
-//   * gemm16_mfma_kernel  - bf16 / fp16 inputs, transposed A with a chip full of 256x256 tiles, fp32 accumulation on v_mfma_f32_32x32x16_{bf16,f16}.
-//     256x256 block tile, 64-deep K step, 256 threads = 4 wavefronts in a 2x2 grid, each wavefront owning a
-//     128x128 tile (16 MFMA accumulator tiles = 256 accumulator registers).  Both operand tiles live in LDS
-//     as [row][k] with k contiguous, 128 bytes per row, double buffered (2 x 64 KiB of the 160 KiB per CU);
-//     16-byte chunks are XOR-swizzled so that the ds_read_b128 of MFMA fragments and the transposing stores
-//     are conflict free.  Operands whose contiguous axis is not K (row-major B, transposed A) are transposed
-//     in registers (8x8 blocks of 16-bit values) on their way into LDS.  Requires M%256 == N%256 == K%64 == 0.
+//     stages, transposing LDS reads for row-major B and transposed A; also as 128x128 tiles (two or four stages) and 256x64
+//     tiles, and with the A operand gathered from a channels-last image (implicit-GEMM convolution); see the comment at the
+//     kernel.
 //   * gemm32_mfma_kernel  - fp32 on v_mfma_f32_32x32x2f32, 128x128 tile (64x64 when that is what fills the chip),
 //     for M%128 == N%128 == K%32 == 0, unless few tiles with a long K are better off split.
 //   * gemm_generic_kernel - any shape / transpose / type: 64x64 LDS tile, FMA units; for fp64.
-// Everything else - ragged extents, a transposed A, too few tiles to fill the chip - runs on the register-staged MFMA
+// Everything else - ragged extents, too few tiles to fill the chip - runs on the register-staged MFMA
 // kernel of gemm_flex.hip.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <type_traits>
 
 #include <climits>
@@ -48,9 +44,6 @@ struct Half16;
 template <>
 struct Half16<__bf16> {
   typedef bf16x8 vec8;
-  static __device__ __forceinline__ f32x16 mfma(vec8 a, vec8 b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-  }
   static __device__ __forceinline__ f32x4 mfma16(vec8 a, vec8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
   }
@@ -58,9 +51,6 @@ struct Half16<__bf16> {
 template <>
 struct Half16<_Float16> {
   typedef f16x8 vec8;
-  static __device__ __forceinline__ f32x16 mfma(vec8 a, vec8 b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-  }
   static __device__ __forceinline__ f32x4 mfma16(vec8 a, vec8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
   }
@@ -75,168 +65,8 @@ __device__ __forceinline__ uint32_t PackPair(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, pair_t));
 }
 
-constexpr int kBM      = 256;
-constexpr int kBN      = 256;
-constexpr int kBK      = 64;
-constexpr int kThreads = 256;
-// one operand tile: 256 rows x 64 halves = 256 x 128 bytes
-constexpr int kTileBytes  = kBM * kBK * 2;
-constexpr int kStageBytes = 2 * kTileBytes;  // A tile + B tile
-
-// byte offset of 16-byte chunk `chunk` (0..7) of row `row` inside an operand tile
-__device__ __forceinline__ int TileOffset(int row, int chunk) {
-  int key = (row ^ (row >> 3)) & 7;
-  return row * 128 + ((chunk ^ key) << 4);
-}
-
-// 8x8 transpose of 16-bit values held as 8 rows of 4 dwords: out[c] = column c of in
-__device__ __forceinline__ void Transpose8x8(const u32x4 (&in)[8], u32x4 (&out)[8]) {
-#pragma unroll
-  for (int c = 0; c < 8; ++c) {
-    const int d  = c >> 1;  // dword that holds column c
-    const bool hi = c & 1;  // upper half of that dword
-#pragma unroll
-    for (int rp = 0; rp < 4; ++rp) {
-      unsigned a = in[2 * rp][d];
-      unsigned b = in[2 * rp + 1][d];
-      // low half from row 2rp, high half from row 2rp+1
-      out[c][rp] = hi ? __builtin_amdgcn_perm(b, a, 0x07060302u) : __builtin_amdgcn_perm(b, a, 0x05040100u);
-    }
-  }
-}
-
-// Global -> register staging of one 256-row operand tile, two access patterns.
-// K_CONTIG: the operand is [rows][K] in memory (K contiguous): thread t copies chunk (t & 7) of rows
-//           (t >> 3) + 32 i.  Otherwise the operand is [K][rows] (rows contiguous): thread t owns the 8x8
-//           block at k-block (t >> 5), row-block (t & 31) and transposes it.
-template <bool K_CONTIG>
-struct TileLoader {
-  u32x4 regs[8];
-  __device__ __forceinline__ void Load(const uint16_t* __restrict__ base, int64_t ld, int row0, int k0, int tid) {
-    if (K_CONTIG) {
-      const uint16_t* p = base + (int64_t)(row0 + (tid >> 3)) * ld + k0 + (tid & 7) * 8;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) regs[i] = *reinterpret_cast<const u32x4*>(p + (int64_t)(32 * i) * ld);
-    } else {
-      const uint16_t* p = base + (int64_t)(k0 + (tid >> 5) * 8) * ld + row0 + (tid & 31) * 8;
-#pragma unroll
-      for (int r = 0; r < 8; ++r) regs[r] = *reinterpret_cast<const u32x4*>(p + (int64_t)r * ld);
-    }
-  }
-  __device__ __forceinline__ void Store(char* tile, int tid) {
-    if (K_CONTIG) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-        *reinterpret_cast<u32x4*>(tile + TileOffset((tid >> 3) + 32 * i, tid & 7)) = regs[i];
-    } else {
-      u32x4 t[8];
-      Transpose8x8(regs, t);
-#pragma unroll
-      for (int c = 0; c < 8; ++c) *reinterpret_cast<u32x4*>(tile + TileOffset((tid & 31) * 8 + c, tid >> 5)) = t[c];
-    }
-  }
-};
-
-// A_KC: A is stored [M][K] (not transposed).  B_KC: B is stored [N][K] (transposed).
-template <typename T, bool A_KC, bool B_KC>
-__global__ void __launch_bounds__(kThreads)
-gemm16_mfma_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B, uint16_t* __restrict__ C, int M, int N,
-                   int K, int64_t lda, int64_t ldb, int64_t ldc, float alpha, float beta, int64_t stride_a,
-                   int64_t stride_b, int64_t stride_c) {
-  extern __shared__ __attribute__((aligned(16))) char lds[];
-  typedef typename Half16<T>::vec8 vec8;
-
-  const int tid  = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int wm   = wave >> 1;  // wavefront row in the 2x2 grid
-  const int wn   = wave & 1;
-
-  // XCD-aware tile order: consecutive workgroup ids go to different XCDs (8 of them, each with its own L2), so
-  // give every XCD a contiguous band of tiles that share A row panels
-  const int tiles_n = N / kBN;
-  const int tiles   = (M / kBM) * tiles_n;
-  int bid           = blockIdx.x;
-  if ((tiles & 7) == 0) bid = (bid & 7) * (tiles >> 3) + (bid >> 3);
-  const int m0 = (bid / tiles_n) * kBM;
-  const int n0 = (bid % tiles_n) * kBN;
-
-  A += (int64_t)blockIdx.y * stride_a;
-  B += (int64_t)blockIdx.y * stride_b;
-  C += (int64_t)blockIdx.y * stride_c;
-
-  f32x16 acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-
-  TileLoader<A_KC> la;
-  TileLoader<B_KC> lb;
-  const int kt_count = K / kBK;
-
-  la.Load(A, lda, m0, 0, tid);
-  lb.Load(B, ldb, n0, 0, tid);
-  la.Store(lds, tid);
-  lb.Store(lds + kTileBytes, tid);
-  __syncthreads();
-
-  const int frag_row = lane & 31;
-  const int frag_kg  = lane >> 5;
-
-  for (int kt = 0; kt < kt_count; ++kt) {
-    char* cur = lds + (kt & 1) * kStageBytes;
-    char* nxt = lds + ((kt + 1) & 1) * kStageBytes;
-    const bool more = kt + 1 < kt_count;
-    if (more) {
-      la.Load(A, lda, m0, (kt + 1) * kBK, tid);
-      lb.Load(B, ldb, n0, (kt + 1) * kBK, tid);
-    }
-    const char* a_tile = cur;
-    const char* b_tile = cur + kTileBytes;
-#pragma unroll
-    for (int kk = 0; kk < kBK / 16; ++kk) {
-      vec8 af[4], bf[4];
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        af[t] = *reinterpret_cast<const vec8*>(a_tile + TileOffset(wm * 128 + t * 32 + frag_row, kk * 2 + frag_kg));
-        bf[t] = *reinterpret_cast<const vec8*>(b_tile + TileOffset(wn * 128 + t * 32 + frag_row, kk * 2 + frag_kg));
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = Half16<T>::mfma(af[i], bf[j], acc[i][j]);
-    }
-    if (more) {
-      la.Store(nxt, tid);
-      lb.Store(nxt + kTileBytes, tid);
-    }
-    __syncthreads();
-  }
-
-  // epilogue: accumulator element r of lane l sits at row 8*(r/4) + 4*(l/32) + r%4, column l%32 of its tile
-  T* Ct = reinterpret_cast<T*>(C);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int col = n0 + wn * 128 + j * 32 + (lane & 31);
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int row = m0 + wm * 128 + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        T* dst  = Ct + (int64_t)row * ldc + col;
-        float v = alpha * acc[i][j][r];
-        if (beta != 0.0f) v += beta * (float)*dst;
-        *dst = (T)v;
-      }
-    }
-  }
-}
-
 // ---------------------------------------------------------------------------------------------------
-// bf16 / fp16 with A stored [M][K]: direct global -> LDS loads (global_load_lds_dwordx4), 8 wavefronts.
+// bf16 / fp16: direct global -> LDS loads (global_load_lds_dwordx4), 8 wavefronts.
 // 256x256 block tile, K step 64, 512 threads in a 2 (M) x 4 (N) wavefront grid, each wavefront a 128x64 tile = 8 x 4
 // accumulators of v_mfma_f32_16x16x32 (measured on sustained MFMA-only loops with random operands: 2.14 PFLOP/s
 // with 16x16x32 against 1.92 with 32x32x16 - the chip is power limited and the narrow shape moves less accumulator
@@ -268,7 +98,7 @@ gemm16_mfma_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ 
 // In core clocks a K step takes about 2330 clocks for 2048 of MFMA at 4096^3 (the rest: the slower wavefront of each
 // SIMD waiting for its loads and the barrier, about 190 clocks, and issue gaps); what the kernel delivers beyond that
 // is set by the clock the chip sustains under this load (1.7-1.9 GHz measured against the 2.4 GHz of the quoted peak).
-// Requires M % BM == N % BN == K % 64 == 0.
+// M and N need not be multiples of the tile; K % 64 == 0 except where both operands are stored with K outermost.
 // ---------------------------------------------------------------------------------------------------
 constexpr int kDmaThreads = 512;
 typedef short s16x4 __attribute__((ext_vector_type(4)));
@@ -301,7 +131,6 @@ __device__ __forceinline__ void AsyncCopy16Slot(const void* base_uniform, unsign
 }
 
 constexpr int kD64BK   = 64;
-constexpr int kD64Tile = kBM * kD64BK * 2;  // one operand tile of a stage: 32 KiB
 
 // epilogue operands of gemm16_dma_kernel: v = acc * (scale[col] or alpha) + shift[col] + residual_scale * R, relu
 struct DmaEpilogue {
@@ -360,8 +189,10 @@ struct ConvGeom {
 // implicit GEMM, K = 4608) a K step took 1102 clocks for 512 of MFMA with the loads issued by the computing
 // wavefronts and 531 without any loads.
 // PAIR (with CONV): the convolution has a second input (ConvGeom::x2) whose channels continue the K loop.
+// A_KC = false: A is stored [K][M] and kept as [k][m] in LDS, like a row-major B, read with the same transposing reads.
+// With both operands stored that way K may be anything: the k-rows beyond it are fetched from `geom.zero_page`.
 template <typename T, bool B_KC, int BM, int BN, int WAVES_M, int WAVES_N, bool CONV = false, int NS = 2, bool FEED = false,
-          bool PAIR = false>
+          bool PAIR = false, bool A_KC = true>
 __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N * (FEED ? 2 : 1))
 gemm16_dma_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B, uint16_t* C, int M, int N, int K,
                   int64_t lda, int64_t ldb, int64_t ldc, DmaEpilogue epi, int64_t stride_a, int64_t stride_b,
@@ -384,6 +215,8 @@ gemm16_dma_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B
   // (registers are what the 256x256 tile has none left of)
   constexpr int STASH = PAIR ? THREADS * LPA * 8 : 0;
   static_assert(!PAIR || CONV, "a second input belongs to a convolution");
+  static_assert(A_KC || !CONV, "a convolution gathers rows of K");
+  constexpr bool K_TAIL = FEED && !A_KC && !B_KC;  // K need not be whole steps
   static_assert(NS >= 2 && NS * STAGE + STASH <= 160 * 1024, "the stages do not fit LDS");
   __shared__ __attribute__((aligned(1024))) char lds[NS * STAGE + STASH];
   const unsigned lds_addr =
@@ -432,7 +265,9 @@ gemm16_dma_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B
   // this block's K steps: all of them, or the split's share
   const int kt0 = epi.partials ? (int)blockIdx.z * epi.steps_per_split : 0;
   const int64_t b_step = (B_KC ? kD64BK : (int64_t)kD64BK * ldb) * 2;  // bytes per K step
-  const char* const a_base = reinterpret_cast<const char*>(A + (int64_t)m0 * lda) - kBias + (int64_t)kt0 * (kD64BK * 2);
+  const int64_t a_step = (A_KC ? kD64BK : (int64_t)kD64BK * lda) * 2;
+  const char* const a_base =
+      reinterpret_cast<const char*>(A + (A_KC ? (int64_t)m0 * lda : (int64_t)m0)) - kBias + (int64_t)kt0 * a_step;
   const char* const b_base =
       reinterpret_cast<const char*>(B + (B_KC ? (int64_t)n0 * ldb : (int64_t)n0)) - kBias + kt0 * b_step;
   const int a_last = M - 1 - m0;  // last valid row of this tile (>= 0)
@@ -467,7 +302,7 @@ gemm16_dma_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B
         stash[(2 * t) * THREADS]     = pixel < M ? (iy2 & 0xffff) | (ix2 << 16) : 0x8000;
         stash[(2 * t + 1) * THREADS] = ((unsigned)((n * geom.h2 + iy2) * geom.w2 + ix2) * (unsigned)geom.c2 + (((lane & 7) ^ key) << 3)) * 2u;
       }
-    } else {
+    } else if (A_KC) {
       const int row_c = row < a_last ? row : a_last;
       a_off[t] = (unsigned)(((int64_t)row_c * lda + (((lane & 7) ^ key) << 3)) * 2 + kBias - 1024 * (t & 3));
     }
@@ -502,6 +337,27 @@ gemm16_dma_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B
       }
     }
   };
+  // chunk of a [k][ROWS halves] tile that load q of the tile brings to this lane: k-row and byte offset from k-row 0
+  // (WIDTH % 8 == 0: the last whole chunk of this tile's columns stands in for those beyond)
+  auto k_row_of = [&](int q, int rows) -> int { return q * (512 / rows) + lane / (rows / 8); };
+  auto k_row_offset = [&](int q, int rows, int64_t ld, int last) -> unsigned {
+    const int krow    = k_row_of(q, rows);
+    const int chunk   = (lane % (rows / 8)) ^ (2 * (krow & 3)) ^ (8 * ((krow >> 4) & 1));
+    const int last_c  = (last + 1) / 8 - 1;
+    const int chunk_c = chunk < last_c ? chunk : last_c;
+    return (unsigned)(((int64_t)krow * ld + (chunk_c << 3)) * 2);
+  };
+  // A_KC = false on the 256x256 tile: the loads of a wavefront cover 16 consecutive k-rows of an operand, two each, so the
+  // swizzle of load t is that of load t % 2 and the rest of its offset is uniform: two registers for each operand instead
+  // of one for each load, which did not fit (31 spilled, 4096^3 at 352 us instead of 105).
+  constexpr bool TIGHT = !A_KC && TM == 8;
+  constexpr int SAME   = TIGHT ? 2 : LPA;
+  static_assert(!TIGHT || (BM == 256 && BN == 256 && LPA == 8 && LPB == 8), "16 k-rows for each wavefront");
+  if (!A_KC) {
+#pragma unroll
+    for (int t = 0; t < SAME; ++t)
+      a_off[t] = k_row_offset(lwave * LPA + t, BM, lda, a_last) + (unsigned)(TIGHT ? kBias : kBias - 1024 * (t & 3));
+  }
 #pragma unroll
   for (int t = 0; t < LPB; ++t) {
     const int q = lwave * LPB + t;
@@ -511,14 +367,27 @@ gemm16_dma_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B
       const int row_c = row < b_last ? row : b_last;
       b_off[t]      = (unsigned)(((int64_t)row_c * ldb + (((lane & 7) ^ key) << 3)) * 2 + kBias - 1024 * (t & 3));
     } else {
-      constexpr int CH = BN / 8;  // 16-byte chunks per k-row
-      const int krow   = q * (64 / CH) + lane / CH;
-      const int chunk  = (lane % CH) ^ (2 * (krow & 3)) ^ (8 * ((krow >> 4) & 1));
-      const int last_c = (b_last + 1) / 8 - 1;  // N % 8 == 0: the last whole chunk of this tile's columns
-      const int chunk_c = chunk < last_c ? chunk : last_c;
-      b_off[t]         = (unsigned)(((int64_t)krow * ldb + (chunk_c << 3)) * 2 + kBias - 1024 * (t & 3));
+      b_off[t] = k_row_offset(q, BN, ldb, b_last) + (unsigned)(TIGHT ? kBias : kBias - 1024 * (t & 3));
     }
   }
+  // the step that reaches beyond K, counted like issue_one's kt (-1: none)
+  const int tail_kt = K_TAIL && K % kD64BK != 0 ? K / kD64BK - kt0 : -1;
+  const int tail_k  = K % kD64BK;  // its k-rows
+  // load t (load q of the tile) of a k-row operand whose step begins at `base`
+  auto issue_k_rows = [&](const char* base, const unsigned* off, int64_t ld, char* tile, int q, int t, int rows, int kt) {
+    if (K_TAIL && kt == tail_kt) {
+      const char* from = base + (off[t] + 1024 * (t & 3));
+      if (k_row_of(q, rows) >= tail_k) from = static_cast<const char*>(geom.zero_page);
+      AsyncCopy16To(from, lds_addr + (unsigned)(tile - lds) + q * 1024);
+      return;
+    }
+    SetLdsBase(lds_addr + (unsigned)(tile - lds) + (q - (t & 3)) * 1024);
+    if (TIGHT) {
+      AsyncCopy16Slot(base + (t / 2) * 8 * ld - 1024 * (t & 3), off[t % 2], t & 3);
+    } else {
+      AsyncCopy16Slot(base, off[t], t & 3);
+    }
+  };
   // load t of step kt: first the LPA loads of the A tile, then the LPB loads of the B tile
   auto issue_one = [&](char* a_tile, char* b_tile, int kt, int t) {
     if (t < LPA) {
@@ -532,10 +401,14 @@ gemm16_dma_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B
         const char* from = inside ? src + (a_off[t] + tap_off)
                                   : static_cast<const char*>(geom.zero_page) + ((lane & 7) << 4);
         AsyncCopy16To(from, lds_addr + (unsigned)(a_tile - lds) + (lwave * LPA + t) * 1024);
+      } else if (!A_KC) {
+        issue_k_rows(a_base + kt * a_step, a_off, lda, a_tile, lwave * LPA + t, t, BM, kt);
       } else {
         SetLdsBase(lds_addr + (unsigned)(a_tile - lds) + (lwave * LPA + (t & ~3)) * 1024);
         AsyncCopy16Slot(a_base + (int64_t)kt * (kD64BK * 2), a_off[t], t & 3);
       }
+    } else if (!A_KC && !B_KC) {
+      issue_k_rows(b_base + kt * b_step, b_off, ldb, b_tile, lwave * LPB + t - LPA, t - LPA, BN, kt);
     } else {
       SetLdsBase(lds_addr + (unsigned)(b_tile - lds) + (lwave * LPB + ((t - LPA) & ~3)) * 1024);
       AsyncCopy16Slot(b_base + kt * b_step, b_off[t - LPA], (t - LPA) & 3);
@@ -564,26 +437,39 @@ gemm16_dma_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B
   int frag_off[2];
 #pragma unroll
   for (int kk = 0; kk < 2; ++kk) frag_off[kk] = frag_row * 128 + (((kk * 4 + frag_kg) ^ frag_key) << 4);
+  // a transposing read hands lane i of a group of 16 four consecutive k of column i: the group addresses a block of
+  // 4 k-rows x 16 columns, every lane four columns of one k-row
+  // Tile i of a wavefront lies 32 i bytes on; the bits of i are free in the chunk number of tile 0, so that is an
+  // exclusive or on top of the swizzle.  `at` is the lane's offset in tile 0 of slice 0: one register for each operand, which
+  // the 256x256 tile with a transposed A makes opaque at every read (the addresses of all its tiles would not fit).
+  auto k_rows_at = [&](int column, int rows) -> int {
+    const int k = 8 * frag_kg + ((lane & 15) >> 2);
+    const int n = column + 4 * (lane & 3);
+    return k * (rows * 2) + (((n >> 3) ^ (2 * (k & 3)) ^ (8 * ((k >> 4) & 1))) << 4) + (n & 7) * 2;
+  };
+  int a_at = A_KC ? 0 : k_rows_at(wm * TM * 16, BM), b_at = B_KC ? 0 : k_rows_at(wn * TN * 16, BN);
+  auto read_k_rows = [&](const char* tile, int at, int kk, int i, int rows) -> vec8 {
+    s16x4 part[2];
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+      part[r] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          (s16x4 __attribute__((address_space(3)))*)(tile + (at ^ (32 * i)) + (kk * 32 + 4 * r) * (rows * 2)));
+    s16x8 both = __builtin_shufflevector(part[0], part[1], 0, 1, 2, 3, 4, 5, 6, 7);
+    return __builtin_bit_cast(vec8, both);
+  };
   auto read_a = [&](const char* a_tile, int kk, int i) -> vec8 {
+    if (!A_KC) {
+      if (TIGHT) asm volatile("" : "+v"(a_at));
+      return read_k_rows(a_tile, a_at, kk, i, BM);
+    }
     return *reinterpret_cast<const vec8*>(a_tile + frag_off[kk] + (wm * TM + i) * 2048);
   };
   auto read_b = [&](const char* b_tile, int kk, int j) -> vec8 {
-    if (B_KC) {
-      return *reinterpret_cast<const vec8*>(b_tile + frag_off[kk] + (wn * TN + j) * 2048);
-    } else {
-      // a transposing read hands lane i of a group of 16 four consecutive k of column i: the group addresses a block
-      // of 4 k-rows x 16 columns, every lane four columns of one k-row
-      s16x4 part[2];
-#pragma unroll
-      for (int r = 0; r < 2; ++r) {
-        const int k   = kk * 32 + 8 * frag_kg + 4 * r + ((lane & 15) >> 2);
-        const int n   = wn * (TN * 16) + j * 16 + 4 * (lane & 3);
-        const int off = k * (BN * 2) + (((n >> 3) ^ (2 * (k & 3)) ^ (8 * ((k >> 4) & 1))) << 4) + (n & 7) * 2;
-        part[r] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(b_tile + off));
-      }
-      s16x8 both = __builtin_shufflevector(part[0], part[1], 0, 1, 2, 3, 4, 5, 6, 7);
-      return __builtin_bit_cast(vec8, both);
+    if (!B_KC) {
+      if (TIGHT) asm volatile("" : "+v"(b_at));
+      return read_k_rows(b_tile, b_at, kk, j, BN);
     }
+    return *reinterpret_cast<const vec8*>(b_tile + frag_off[kk] + (wn * TN + j) * 2048);
   };
 #define CINN_SB __builtin_amdgcn_sched_barrier(0)
   // A K step is ROWS = 2 TM rows of TN MFMAs: row r multiplies the A fragment of tile r % TM, slice r / TM (32 deep),
@@ -611,7 +497,7 @@ gemm16_dma_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B
   vec8 ring[4];
   vec8 bf[2][TN];
 
-  const int nk_all = K / kD64BK;
+  const int nk_all = K_TAIL ? (K + kD64BK - 1) / kD64BK : K / kD64BK;
   const int nk     = epi.partials ? (nk_all - kt0 < epi.steps_per_split ? nk_all - kt0 : epi.steps_per_split) : nk_all;
   constexpr int L = LPA + LPB;  // loads of a loader wavefront per stage
   // vmcnt(n): at most n of the wavefront's loads still in flight; they complete in the order they were issued
@@ -1504,23 +1390,6 @@ struct GemmProblem {
   bool whole_without_scratch{false};
 };
 
-template <typename T, bool A_KC, bool B_KC>
-void LaunchFast16(const GemmProblem& p, hipStream_t stream) {
-  auto kernel = gemm16_mfma_kernel<T, A_KC, B_KC>;
-  static const bool configured = [&] {  // once per instantiation, thread-safe
-    CINN_HIP_CALL(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      2 * kStageBytes));
-    return true;
-  }();
-  (void)configured;
-  int64_t lda = p.trans_a ? p.m : p.k;
-  int64_t ldb = p.trans_b ? p.k : p.n;
-  dim3 grid((p.m / kBM) * (p.n / kBN), p.batch, 1);
-  hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 2 * kStageBytes, stream, static_cast<const uint16_t*>(p.a),
-                     static_cast<const uint16_t*>(p.b), static_cast<uint16_t*>(p.c), p.m, p.n, p.k, lda, ldb,
-                     (int64_t)p.n, p.alpha, p.beta, p.stride_a, p.stride_b, p.stride_c);
-}
-
 // Sum of the fp32 partial tiles of a split reduction, then the epilogue of gemm16_dma_kernel: 8 columns per thread
 // (N % 8 == 0), the same fused multiply-adds and the single rounding to T.
 template <typename T>
@@ -1603,7 +1472,7 @@ void XcdRectanglesPadded(int tiles_m, int tiles_n, int* xcd_cols, int* sub_rows,
 std::atomic<unsigned long long*> g_gemm_probe{nullptr};
 
 template <typename T, bool B_KC, int BM, int BN, int WAVES_M, int WAVES_N, bool CONV = false, int NS = 2, bool FEED = false,
-          bool PAIR = false>
+          bool PAIR = false, bool A_KC = true>
 void LaunchDma16(const GemmProblem& p, hipStream_t stream, int splits = 1) {
   using cinn_hip_kernels::ScratchKind;
   if (p.whole_without_scratch && splits > 1 &&
@@ -1623,7 +1492,7 @@ void LaunchDma16(const GemmProblem& p, hipStream_t stream, int splits = 1) {
   if (splits > 1) {
     CINN_RT_CHECK(p.batch == 1 && p.beta == 0.0f, "a split reduction takes one unbatched product without a beta term");
     epi.partials        = static_cast<float*>(cinn_hip_kernels::Scratch(cinn_hip_kernels::ScratchKind::kSplitK, (size_t)splits * p.m * p.n * sizeof(float), stream));
-    epi.steps_per_split = (p.k / kD64BK + splits - 1) / splits;
+    epi.steps_per_split = ((p.k + kD64BK - 1) / kD64BK + splits - 1) / splits;
   }
   epi.scale          = p.scale;
   epi.shift          = p.shift;
@@ -1635,11 +1504,12 @@ void LaunchDma16(const GemmProblem& p, hipStream_t stream, int splits = 1) {
   epi.streaming = !p.keep_in_cache && (int64_t)p.batch * p.m * p.n * 2 >= (16 << 20);
   ConvGeom geom{};
   if (CONV) geom = *p.conv;
-  hipLaunchKernelGGL((gemm16_dma_kernel<T, B_KC, BM, BN, WAVES_M, WAVES_N, CONV, NS, FEED, PAIR>), grid,
+  if (!A_KC && !B_KC && p.k % kD64BK != 0) geom.zero_page = cinn_hip_kernels::ZeroPage();
+  hipLaunchKernelGGL((gemm16_dma_kernel<T, B_KC, BM, BN, WAVES_M, WAVES_N, CONV, NS, FEED, PAIR, A_KC>), grid,
                      dim3(64 * WAVES_M * WAVES_N * (FEED ? 2 : 1)), 0,
                      stream, static_cast<const uint16_t*>(p.a), static_cast<const uint16_t*>(p.b),
-                     static_cast<uint16_t*>(p.c), p.m, p.n, p.k, (int64_t)p.k, ldb, (int64_t)p.n, epi, p.stride_a,
-                     p.stride_b, p.stride_c, xcd_cols, sub_rows, sub_cols, geom);
+                     static_cast<uint16_t*>(p.c), p.m, p.n, p.k, (int64_t)(A_KC ? p.k : p.m), ldb, (int64_t)p.n, epi,
+                     p.stride_a, p.stride_b, p.stride_c, xcd_cols, sub_rows, sub_cols, geom);
   if (splits > 1) {
     const int64_t total8 = (int64_t)p.m * p.n / 8;
     hipLaunchKernelGGL((gemm16_split_reduce_kernel<T>), dim3((unsigned)((total8 + 255) / 256)), dim3(256), 0, stream,
@@ -1755,6 +1625,66 @@ bool TrySkinny(const GemmProblem& p, hipStream_t stream) {
 bool FeedWavefronts() {
   static const bool on = !(getenv("FLAGS_cinn_hip_gemm_feed") && atoi(getenv("FLAGS_cinn_hip_gemm_feed")) == 0);
   return on;
+}
+
+cinn_hip_kernels::FlexGemm FlexOf(const GemmProblem& p) {
+  using cinn_hip_kernels::FlexType;
+  cinn_hip_kernels::FlexGemm g;
+  g.type = p.type == GemmType::kF16 ? FlexType::kF16 : (p.type == GemmType::kBF16 ? FlexType::kBF16 : FlexType::kF32);
+  g.a = p.a, g.b = p.b, g.c = p.c;
+  g.m = p.m, g.n = p.n, g.k = p.k;
+  g.a_kc = !p.trans_a, g.b_kc = p.trans_b;
+  g.lda = p.trans_a ? p.m : p.k, g.ldb = p.trans_b ? p.k : p.n;
+  g.batch = p.batch, g.stride_a = p.stride_a, g.stride_b = p.stride_b, g.stride_c = p.stride_c;
+  g.alpha = p.alpha, g.shift = p.shift;
+  if (p.beta != 0.0f) g.residual = p.c, g.residual_scale = p.beta;
+  return g;
+}
+
+// A stored [K][M] in whole, aligned 16-byte chunks (the weight gradient of a linear layer): 256x256 tiles, or 128x128 tiles
+// with feeding wavefronts, where these are faster than what gemm_flex.hip would run.  The former, and a B stored [N][K],
+// take K in whole steps.
+// The estimates (us): a round of blocks costs its start and epilogue (the rounds after the first a cold start), and for
+// every K step what the tile's operands take to reach LDS, which grows with the CUs that pull (and with them the clock
+// falls); the blocks of a small batch entry are spread over all XCDs and share nothing in L2.  fp16, gemm_flex.hip | 128x128 | 256x256:
+// A^T B 768x3072x4100 39.3 | 28.5 | -, 2048^3 25.4 | 21.2 | 40.6, 1024x4096x8200 80 | 66 | -, 4096x1024x512 12.3 | 9.9 | 15.7,
+// 3000x3000x1024 41.7 | 38.9 | 26.1, 4096x3072x768 36.1 | 32.8 | 23.6, 4096^3 153 | 140 | 104.5 (a register-staged kernel of
+// 256x256 tiles took 149); not taken 1024^3 8.0 | 12.1 | 23, 768x768x4100 18.6 | 27.1 | -, 512x512x16384 31 | 89 | -.
+// With one start for every round [5] x 4096x4096x40 went from 59 to 80 and [5] x 1760x2288x72 from 22.5 to 30.4.
+// B stored [N][K]: 4096^3 148 | 129 | 101, 2048^3 25 | 21 | 39, 4096x1024x512 11.9 | 8.8 | 15.3.
+// `flex_us`: the estimate for gemm_flex.hip
+template <typename T>
+bool TryDmaTransposedA(const GemmProblem& p, double flex_us, hipStream_t stream) {
+  const bool whole_k = p.k % kD64BK == 0;
+  if (p.m % 8 != 0 || p.n % 8 != 0 || (p.trans_b && !whole_k)) return false;
+  if (reinterpret_cast<uintptr_t>(p.a) % 16 != 0 || reinterpret_cast<uintptr_t>(p.b) % 16 != 0 ||
+      reinterpret_cast<uintptr_t>(p.c) % 16 != 0 || reinterpret_cast<uintptr_t>(p.residual) % 16 != 0 ||
+      p.stride_a % 8 != 0 || p.stride_b % 8 != 0 || p.stride_c % 8 != 0)
+    return false;
+  // lanes address a tile with 32-bit byte offsets: 64 k-rows of M or N, 256 rows of K
+  if (p.k >= (1 << 22) || p.n >= (1 << 24) || p.m >= (1 << 24)) return false;
+  if (!whole_k && !cinn_hip_kernels::HasZeroPage(stream)) return false;
+  const double steps = (p.k + kD64BK - 1) / kD64BK;
+  auto estimate = [&](int tile, double start, double step, double crowd) {
+    const double entry = (double)((p.m + tile - 1) / tile) * ((p.n + tile - 1) / tile), tiles = entry * p.batch;
+    const double spread = p.batch > 1 && entry < 64 ? 1.6 : 1.0;
+    const double rounds = std::ceil(tiles / 256);
+    return 3.5 + start + (rounds - 1.0) * (start + 2.0) + rounds * steps * spread * (step + crowd * std::min(1.0, tiles / 256));
+  };
+  const double us128 = estimate(128, 2.0, 0.32, 0.17), us256 = whole_k ? estimate(256, 4.5, 0.85, 0.65) : 1e30;
+  if (std::min(us128, us256) >= flex_us) return false;
+  if (p.trans_b) {
+    if (us256 < us128) {
+      LaunchDma16<T, true, 256, 256, 2, 4, false, 2, false, false, false>(p, stream);
+    } else {
+      LaunchDma16<T, true, 128, 128, 2, 2, false, 4, true, false, false>(p, stream);
+    }
+  } else if (us256 < us128) {
+    LaunchDma16<T, false, 256, 256, 2, 4, false, 2, false, false, false>(p, stream);
+  } else {
+    LaunchDma16<T, false, 128, 128, 2, 2, false, 4, true, false, false>(p, stream);
+  }
+  return true;
 }
 
 // A stored [M][K], K % 64 == 0, N % 8 == 0 (whole 16-byte chunks per row of C and of a row-major B): 256x256 tiles
@@ -1909,21 +1839,6 @@ bool TryDma16(const GemmProblem& p, hipStream_t stream) {
   return false;
 }
 
-bool UseRegisterStaging() {
-  static const bool on = getenv("FLAGS_cinn_hip_gemm_register_staging") && atoi(getenv("FLAGS_cinn_hip_gemm_register_staging")) != 0;
-  return on;
-}
-
-// 256x256 tiles with register staging: every operand layout (used for A stored [K][M])
-template <typename T>
-void DispatchFast16(const GemmProblem& p, hipStream_t stream) {
-  bool a_kc = !p.trans_a, b_kc = p.trans_b;
-  if (a_kc && b_kc) LaunchFast16<T, true, true>(p, stream);
-  if (a_kc && !b_kc) LaunchFast16<T, true, false>(p, stream);
-  if (!a_kc && b_kc) LaunchFast16<T, false, true>(p, stream);
-  if (!a_kc && !b_kc) LaunchFast16<T, false, false>(p, stream);
-}
-
 template <typename T, typename ACC>
 void LaunchGeneric(const GemmProblem& p, hipStream_t stream) {
   int64_t lda = p.trans_a ? p.m : p.k;
@@ -1977,57 +1892,46 @@ void RunGemm(const GemmProblem& p, hipStream_t stream) {
   CINN_RT_CHECK(p.batch <= 65535, "gemm: batch %d exceeds the grid limit", p.batch);
   const bool aligned16 = reinterpret_cast<uintptr_t>(p.a) % 16 == 0 && reinterpret_cast<uintptr_t>(p.b) % 16 == 0 &&
                          p.stride_a % 8 == 0 && p.stride_b % 8 == 0;
-  // 256x256 tiles with register staging take a transposed A that fills the chip with them: 4096^3 164 us (171 on the
-  // 128x128 tiles of gemm_flex.hip); with 64 such tiles, 2048^3, 75 against 26 us
-  const bool fast16 = !ForceGeneric() && aligned16 && p.m % kBM == 0 && p.n % kBN == 0 && p.k % kBK == 0 &&
-                      (UseRegisterStaging() || (int64_t)(p.m / kBM) * (p.n / kBN) * p.batch >= 192);
   const bool whole32 = !ForceGeneric() && aligned16 && p.m % kF32Tile == 0 && p.n % kF32Tile == 0 && p.k % kF32K == 0;
   // (a bias only exists in the epilogues of the first two: the flags do not apply to it)
   const bool bias = p.shift != nullptr;
-  if ((bias || (!ForceGeneric() && !UseRegisterStaging())) && (p.type == GemmType::kBF16 || p.type == GemmType::kF16)) {
-    const bool taken = p.type == GemmType::kBF16 ? TryDma16<__bf16>(p, stream) : TryDma16<_Float16>(p, stream);
+  const bool flexible             = bias || (!ForceGeneric() && p.type != GemmType::kF64);
+  const cinn_hip_kernels::FlexGemm g = FlexOf(p);
+  cinn_hip_kernels::FlexPlan plan{0, 0, 0, 1e30};
+  bool planned = false;  // gemm_flex.hip takes the product, like `plan`
+  if (flexible && (p.type == GemmType::kBF16 || p.type == GemmType::kF16)) {
+    const bool bf16 = p.type == GemmType::kBF16;
+    bool taken      = false;
+    if (p.trans_a) {
+      planned = cinn_hip_kernels::PlanFlexGemm(g, stream, &plan);
+      taken   = bf16 ? TryDmaTransposedA<__bf16>(p, plan.us, stream) : TryDmaTransposedA<_Float16>(p, plan.us, stream);
+    } else {
+      taken = bf16 ? TryDma16<__bf16>(p, stream) : TryDma16<_Float16>(p, stream);
+    }
     if (taken) {
       CINN_HIP_CALL(hipGetLastError());
       return;
     }
   }
-  if (bias || (!ForceGeneric() && p.type != GemmType::kF64)) {
-    cinn_hip_kernels::FlexGemm g;
-    g.type = p.type == GemmType::kF16 ? cinn_hip_kernels::FlexType::kF16
-                                      : (p.type == GemmType::kBF16 ? cinn_hip_kernels::FlexType::kBF16 : cinn_hip_kernels::FlexType::kF32);
-    g.a = p.a, g.b = p.b, g.c = p.c;
-    g.m = p.m, g.n = p.n, g.k = p.k;
-    g.a_kc = !p.trans_a, g.b_kc = p.trans_b;
-    g.lda = p.trans_a ? p.m : p.k, g.ldb = p.trans_b ? p.k : p.n;
-    g.batch = p.batch, g.stride_a = p.stride_a, g.stride_b = p.stride_b, g.stride_c = p.stride_c;
-    g.alpha = p.alpha, g.shift = p.shift;
-    if (p.beta != 0.0f) g.residual = p.c, g.residual_scale = p.beta;
+  if (flexible) {
+    if (!planned) planned = cinn_hip_kernels::PlanFlexGemm(g, stream, &plan);
     // The fp32 tiles of gemm32_mfma_kernel walk all of K.  They keep the products whose K gemm_flex.hip would not split
     // either, where they are 5 to 15% ahead, and the grids with a 64x64 tile for every CU.  us, whole tiles | gemm_flex.hip:
     // 128x128x128 5.2 | 6.0, 512x512x256 8.0 | 8.7, 896x1152x1024 (252 tiles) 22.5 | 24.1, all not split; split
     // 512x512x512 12.6 | 11.0, 512x1024x1024 22.1 | 18.1, 768x1024x2048 40.8 | 36.8, 128x128x4096 76 | 13; from 256 tiles on
     // 1024x1024x256 8.6 | 9.3, 1024x1024x1024 22.4 | 23.9, 4096x4096x1024 267 | 282.  (Some larger grids whose last round is
     // nearly empty are better off split all the same: 1280x1024x4096 138 | 101, 768x3072x4096 207 | 172.)
-    const bool fast32 = whole32 && ((int64_t)(p.m / 64) * (p.n / 64) * p.batch >= 256 || !cinn_hip_kernels::FlexGemmSplitsK(g, stream));
-    const bool whole  = !bias && (p.type == GemmType::kF32 ? fast32 : fast16);
-    if (!whole && cinn_hip_kernels::TryFlexGemm(g, stream)) return;
+    const bool fast32 = whole32 && ((int64_t)(p.m / 64) * (p.n / 64) * p.batch >= 256 || plan.splits <= 1);
+    const bool whole  = !bias && p.type == GemmType::kF32 && fast32;
+    if (!whole && planned) {
+      cinn_hip_kernels::RunFlexGemm(g, plan, stream);
+      return;
+    }
     CINN_RT_CHECK(!bias, "gemm: %d x %d x %d with a bias is beyond the kernels' offsets", p.m, p.n, p.k);
   }
   switch (p.type) {
-    case GemmType::kBF16:
-      if (fast16) {
-        DispatchFast16<__bf16>(p, stream);
-      } else {
-        LaunchGeneric<__bf16, float>(p, stream);
-      }
-      break;
-    case GemmType::kF16:
-      if (fast16) {
-        DispatchFast16<_Float16>(p, stream);
-      } else {
-        LaunchGeneric<_Float16, float>(p, stream);
-      }
-      break;
+    case GemmType::kBF16: LaunchGeneric<__bf16, float>(p, stream); break;
+    case GemmType::kF16: LaunchGeneric<_Float16, float>(p, stream); break;
     case GemmType::kF32:
       if (whole32) {
         LaunchFast32(p, stream);
@@ -2075,7 +1979,7 @@ bool TryPointwiseConvAsGemm(const ConvNhwcArgs& a, hipStream_t stream) {
   const bool enabled = mode != 0;
   // a second input has no other implementation: the measurement flags do not apply to it
   const bool pair = a.x2 != nullptr;
-  if (!pair && (!enabled || ForceGeneric() || UseRegisterStaging())) return false;
+  if (!pair && (!enabled || ForceGeneric())) return false;
   const bool is_f16  = a.type.code == cinn_type_float && a.type.bits == 16;
   const bool is_bf16 = a.type.code == cinn_type_bfloat && a.type.bits == 16;
   if (!is_f16 && !is_bf16) return false;
