@@ -68,6 +68,9 @@ void InvokeTopK(const std::vector<BakedArg>& a, void* args, int32_t n, void* str
 void InvokeMatmulBias(const std::vector<BakedArg>& a, void* args, int32_t n, void* stream) {
   cinn_call_hip_matmul_bias(args, n, I(a[2]), I(a[3]), I(a[4]), I(a[5]), stream);
 }
+void InvokeMatmulRows(const std::vector<BakedArg>& a, void* args, int32_t n, void* stream) {
+  cinn_call_hip_matmul_rows(args, n, I(a[2]), I(a[3]), I(a[4]), I(a[5]), I(a[6]), F(a[7]), I(a[8]), stream);
+}
 void InvokeChannelStatistics(const std::vector<BakedArg>& a, void* args, int32_t n, void* stream) {
   cinn_call_hip_channel_statistics(args, n, I(a[2]), I(a[3]), stream);
 }
@@ -134,6 +137,8 @@ ExternApiRegistry::ExternApiRegistry() {
   Register("cinn_call_hip_attention", InvokeAttention, 13);
   // (kernel_args, kernel_args_num, trans_b, m, n, k, kernel_stream)
   Register("cinn_call_hip_matmul_bias", InvokeMatmulBias, 7);
+  // (kernel_args, kernel_args_num, m, n, k, operands, outputs, epsilon, gelu, kernel_stream)
+  Register("cinn_call_hip_matmul_rows", InvokeMatmulRows, 10);
   // (kernel_args, kernel_args_num, pixels, channels, kernel_stream)
   Register("cinn_call_hip_channel_statistics", InvokeChannelStatistics, 5);
   // (kernel_args, kernel_args_num, pixels, channels, operands, epsilon, relu, kernel_stream)

@@ -4,6 +4,7 @@
 #include "frontend/decomposer.h"
 #include "frontend/layout_pass.h"
 #include "frontend/reduce_split_pass.h"
+#include "frontend/row_product_pass.h"
 #include "frontend/top_k_pass.h"
 
 namespace cinn {
@@ -51,6 +52,7 @@ std::shared_ptr<CinnComputation> CinnComputation::Compile(const common::Target& 
   if (options.fuse_conv_bn_relu && options.fuse_conv_chain) lowered = FuseConvChain(lowered, fetch_ids);
   if (options.fuse_conv_bn_relu && options.fuse_shortcut_projection) lowered = FuseShortcutProjection(lowered, fetch_ids);
   lowered = FuseTopK(lowered, fetch_ids);
+  if (options.fuse_matmul_bias) lowered = FuseRowProducts(lowered, fetch_ids);
   if (options.fuse_attention) lowered = FuseAttention(lowered, fetch_ids);
   if (options.use_decomposer) lowered = ApplyDecomposer(lowered, fetch_ids);
   if (options.split_reductions) lowered = SplitReductions(lowered, target.get_multi_processor_count());

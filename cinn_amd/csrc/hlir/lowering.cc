@@ -1572,6 +1572,20 @@ ir::LoweredFuncRef OpLowerer::LowerLibraryCall(const Group& group) const {
     CINN_CHECK(n->inputs[2] != n->inputs[0] && n->inputs[2] != n->inputs[1]);
     api = "cinn_call_hip_matmul_bias";
     push_ints({GetAttr<bool>(n->attrs, "trans_b", false) ? 1 : 0, n->outputs[0]->shape[0], n->outputs[0]->shape[1], n->inputs[0]->shape[1]});
+  } else if (op == "hip_matmul_rows") {
+    // slots x, W, scale, shift, residual, gamma, beta: which of the call's arguments (equal values are one), 15 = none
+    api             = "cinn_call_hip_matmul_rows";
+    const bool residual = GetAttr<bool>(n->attrs, "residual", false), norm = GetAttr<bool>(n->attrs, "norm", false);
+    int operands        = 0;
+    size_t next         = 0;
+    for (int slot = 0; slot < 7; ++slot) {
+      const bool present = slot < 4 || (slot == 4 ? residual : norm);
+      const int at       = present ? static_cast<int>(std::find(group.inputs.begin(), group.inputs.end(), n->inputs[next++]) - group.inputs.begin()) : 15;
+      operands |= at << (4 * slot);
+    }
+    push_ints({n->inputs[0]->shape[0], n->inputs[1]->shape[0], n->inputs[0]->shape[1], operands, static_cast<int>(n->outputs.size())});
+    args.push_back(Expr(GetAttr<float>(n->attrs, "epsilon", 0.0f)));
+    push_ints({GetAttr<bool>(n->attrs, "gelu", false) ? 1 : 0});
   } else if (op.rfind("hip_channel_", 0) == 0) {
     const auto& x = n->inputs[0]->shape;
     api           = "cinn_call_" + op;

@@ -774,6 +774,17 @@ OpRegistry::OpRegistry() {
     op.infer_dtype = SameTypeAsFirst;
   }
   {
+    // x [m][k], W [n][k], scale, shift [, residual] [, gamma, beta]: what FuseRowProducts makes of a layer of few rows
+    auto& op       = r->Register("hip_matmul_rows");
+    op.pattern     = OpPatternKind::kNonFusible;
+    op.num_inputs  = -1;
+    op.num_outputs = -1;
+    op.infer_shape = [](const std::vector<ShapeType>& in, const AttributeMap&) {
+      return std::vector<ShapeType>{{in[0][0], in[1][0]}};
+    };
+    op.infer_dtype = SameTypeAsFirst;
+  }
+  {
     // what FuseAttention makes of the two products of an attention and the softmax between them
     auto& op       = r->Register("hip_attention");
     op.pattern     = OpPatternKind::kNonFusible;

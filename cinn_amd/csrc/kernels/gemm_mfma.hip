@@ -28,6 +28,7 @@
 #include "cinn_hip_runtime.h"
 #include "kernels/conv_nhwc.h"
 #include "kernels/gemm_flex.h"
+#include "kernels/gemm_rows.h"
 #include "runtime/hip_check.h"
 
 namespace {
@@ -1043,90 +1044,6 @@ gemm16_shortk_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict_
 }
 
 // ---------------------------------------------------------------------------------------------------
-// Few rows (M <= 64: a classifier at inference batch sizes, a decoding step): C[M][N] = A[M][K] . B[N][K]^T is bound by
-// one pass over B.  The tiled kernels give such a product M-tiles that are mostly padding and a handful of blocks; here
-// a block owns 16 output columns of MT row tiles (rows from 16 MT blockIdx.y: the launcher gives every row tile a block
-// of its own) and its eight wavefronts split K.  A lane's share of a 16x16x32 fragment is 8
-// consecutive k of one row - 16 contiguous bytes in both operands - so fragments come straight from global memory, no
-// LDS on the way: every wavefront keeps U k-blocks of loads in flight (two register sets), B is read exactly once
-// from memory, A (at most 64 rows) comes out of L2.  The eight partial tiles meet in LDS; wavefront t finishes row
-// tile t (scale / shift, residual, relu - the epilogue of gemm16_dma_kernel - then 2-byte stores: the result is small).
-template <typename T, int MT>
-__global__ void __launch_bounds__(512)
-gemm16_skinny_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B, uint16_t* __restrict__ C, int M, int N,
-                     int K, DmaEpilogue epi) {
-  typedef typename Half16<T>::vec8 vec8;
-  constexpr int NWAVES = 8;
-  constexpr int U      = 4;  // k-blocks per register set
-  __shared__ __attribute__((aligned(16))) float s_part[NWAVES][MT][64][4];
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int n0   = blockIdx.x * 16;
-  const int m0   = blockIdx.y * (MT * 16);  // first of this block's rows
-  const int fr   = lane & 15;               // row of the fragment this lane reads (a row of A, a column of C for B)
-  const int fk   = (lane >> 4) * 8;  // its 8 elements of a 32-deep k block
-  const int kw   = K / NWAVES;       // this wavefront's share of K, a multiple of 32
-  const int nkb  = kw / 32;
-  const int bcol = min(n0 + fr, N - 1);
-  const uint16_t* bp = B + (int64_t)bcol * K + wave * kw + fk;
-  const uint16_t* ap[MT];
-#pragma unroll
-  for (int t = 0; t < MT; ++t) ap[t] = A + (int64_t)min(m0 + t * 16 + fr, M - 1) * K + wave * kw + fk;
-  f32x4 acc[MT];
-#pragma unroll
-  for (int t = 0; t < MT; ++t) acc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  vec8 bf[2][U], af[2][U][MT];
-  auto request = [&](int set, int kb0) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int kb = min(kb0 + u, nkb - 1);  // beyond the share: the last block again, not multiplied
-      bf[set][u]   = *reinterpret_cast<const vec8*>(bp + kb * 32);
-#pragma unroll
-      for (int t = 0; t < MT; ++t) af[set][u][t] = *reinterpret_cast<const vec8*>(ap[t] + kb * 32);
-    }
-  };
-  auto multiply = [&](int set, int kb0) {
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (kb0 + u < nkb) {
-#pragma unroll
-        for (int t = 0; t < MT; ++t) acc[t] = Half16<T>::mfma16(af[set][u][t], bf[set][u], acc[t]);
-      }
-  };
-  request(0, 0);
-  for (int kb0 = 0; kb0 < nkb; kb0 += 2 * U) {
-    if (kb0 + U < nkb) request(1, kb0 + U);
-    multiply(0, kb0);
-    if (kb0 + 2 * U < nkb) request(0, kb0 + 2 * U);
-    multiply(1, kb0 + U);
-  }
-#pragma unroll
-  for (int t = 0; t < MT; ++t) *reinterpret_cast<f32x4*>(&s_part[wave][t][lane][0]) = acc[t];
-  __syncthreads();
-  if (wave >= MT) return;
-  // wavefront t: row tile t.  Lane = (column n0 + lane % 16, rows 16 t + 4 (lane / 16) .. + 3)
-  f32x4 sum = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-  for (int w = 0; w < NWAVES; ++w) sum += *reinterpret_cast<const f32x4*>(&s_part[w][wave][lane][0]);
-  const int col = n0 + fr;
-  if (col >= N) return;
-  const float sc = epi.scale ? epi.scale[col] : epi.alpha;
-  const float sh = epi.shift ? epi.shift[col] : 0.0f;
-  T* Ct          = reinterpret_cast<T*>(C);
-  const T* Rt    = reinterpret_cast<const T*>(epi.residual);
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int row = m0 + wave * 16 + 4 * (lane >> 4) + r;
-    if (row >= M) continue;
-    float v = __builtin_fmaf(sum[r], sc, sh);
-    if (Rt) v = __builtin_fmaf(epi.residual_scale, (float)Rt[(int64_t)row * N + col], v);
-    asm volatile("" : "+v"(v));  // one rounding to T, see gemm16_dma_kernel's epilogue
-    if (epi.relu) v = v > 0.0f ? v : 0.0f;
-    Ct[(int64_t)row * N + col] = (T)v;
-  }
-}
-
-// ---------------------------------------------------------------------------------------------------
 // fp32 on v_mfma_f32_32x32x2f32: 128x128 (or 64x64) tile, K step KS = 32 or 64, 4 wavefronts each a quarter of the tile.
 // LDS holds A as [k][m] and B as [k][n] (row stride TILE + 4 floats) so that a fragment read is one conflict-free
 // ds_read_b32 per lane; the K step is deep enough (16 MFMAs of 64 clocks per accumulator) to cover the latency of
@@ -1580,44 +1497,21 @@ bool TryShortK(const GemmProblem& p, hipStream_t stream) {
   return true;
 }
 
-// gemm16_skinny_kernel: at most 64 rows, A [M][K] and B stored [N][K] (a const weight after the program pass has
-// transposed it), one unbatched product, K a multiple of 256 (eight wavefronts of 32-deep blocks).
-// FLAGS_cinn_hip_gemm_skinny=0 switches it off.
-template <typename T>
+// gemm_rows.hip: at most 64 rows, A [M][K] and B stored [N][K] (a const weight after the program pass has transposed it),
+// one unbatched product.  FLAGS_cinn_hip_gemm_skinny=0 switches it off.
 bool TrySkinny(const GemmProblem& p, hipStream_t stream) {
   static const bool enabled = !(getenv("FLAGS_cinn_hip_gemm_skinny") && atoi(getenv("FLAGS_cinn_hip_gemm_skinny")) == 0);
   if (!enabled || p.conv || p.trans_a || !p.trans_b || p.batch != 1) return false;
-  if (p.m > 64 || p.k % 256 != 0 || (int64_t)p.n * p.k >= INT_MAX) return false;
-  if (reinterpret_cast<uintptr_t>(p.a) % 16 != 0 || reinterpret_cast<uintptr_t>(p.b) % 16 != 0) return false;
-  DmaEpilogue epi;
-  epi.partials        = nullptr;
-  epi.steps_per_split = 0;
-  epi.scale           = p.scale;
-  epi.shift           = p.shift;
-  epi.alpha           = p.alpha;
-  epi.relu            = p.relu ? 1 : 0;
-  epi.residual        = p.residual ? p.residual : (p.beta != 0.0f ? p.c : nullptr);
-  epi.residual_scale  = p.residual ? p.residual_scale : p.beta;
-  epi.streaming       = 0;
-  int mt = (p.m + 15) / 16;
-  dim3 grid((unsigned)((p.n + 15) / 16));
-  // Fewer column blocks than CUs: one block per 16 rows as well.  A block's traffic is its 16 columns of B plus the
-  // rows of A it multiplies, and with all of A (128 KB at 32 x 2048, against 64 KB of B) the few CUs at work are bound
-  // by what one CU can pull in; row blocks read B again, out of L2.  ResNet-50's classifier, 32 x 2048 -> 1000: 126
-  // blocks instead of 63, 2.2 us less.  With the chip full, the row tiles stay in one block's registers (B read once).
-  // FLAGS_cinn_hip_gemm_skinny_rows: 0 never splits the rows, 2 always.
-  static const int rows_flag = getenv("FLAGS_cinn_hip_gemm_skinny_rows") ? atoi(getenv("FLAGS_cinn_hip_gemm_skinny_rows")) : 1;
-  if (rows_flag == 2 || (rows_flag == 1 && grid.x < 256)) grid.y = mt, mt = 1;
-#define CINN_SKINNY(MT)                                                                                        \
-  hipLaunchKernelGGL((gemm16_skinny_kernel<T, MT>), grid, dim3(512), 0, stream, static_cast<const uint16_t*>(p.a), \
-                     static_cast<const uint16_t*>(p.b), static_cast<uint16_t*>(p.c), p.m, p.n, p.k, epi)
-  switch (mt) {
-    case 1: CINN_SKINNY(1); break;
-    case 2: CINN_SKINNY(2); break;
-    case 3: CINN_SKINNY(3); break;
-    default: CINN_SKINNY(4); break;
-  }
-#undef CINN_SKINNY
+  cinn_hip_kernels::RowProduct r{};
+  r.bf16 = p.type == GemmType::kBF16;
+  r.a = p.a, r.b = p.b, r.c[0] = p.c;
+  r.width = p.n;
+  r.m = p.m, r.n = p.n, r.k = p.k;
+  r.scale = p.scale, r.shift = p.shift, r.alpha = p.alpha, r.relu = p.relu;
+  r.residual       = p.residual ? p.residual : (p.beta != 0.0f ? p.c : nullptr);
+  r.residual_scale = p.residual ? p.residual_scale : p.beta;
+  if (!cinn_hip_kernels::RowProductSupported(r)) return false;
+  cinn_hip_kernels::RunRowProduct(r, stream);
   return true;
 }
 
@@ -1692,7 +1586,7 @@ bool TryDmaTransposedA(const GemmProblem& p, double flex_us, hipStream_t stream)
 // tile (the last tile row / column computes some rows / columns that are not stored); false when neither applies
 template <typename T>
 bool TryDma16(const GemmProblem& p, hipStream_t stream) {
-  if (TrySkinny<T>(p, stream)) return true;
+  if (TrySkinny(p, stream)) return true;
   if (p.trans_a || p.k % 64 != 0 || p.n % 8 != 0) return false;
   if (TryShortK<T>(p, stream)) return true;
   // every access moves 16 bytes
@@ -2004,8 +1898,8 @@ bool TryPointwiseConvAsGemm(const ConvNhwcArgs& a, hipStream_t stream) {
     // few tiles but a long reduction: the single-wavefront 64x64 tiles of the GEMM kernel (see TryDma16)
     const bool long_k = forced_tile == 64 || (forced_tile == 0 && a.oc % 64 == 0 &&
                                               (a.c >= 2048 || (a.c >= 1024 && ((pixels + 127) / 128) * ((a.oc + 127) / 128) < 128)));
-    // at most 64 pixels (a matmul with few rows written as a 1x1 layer, its bias as the shift): gemm16_skinny_kernel
-    const bool few_rows = forced_tile == 0 && pixels <= 64 && a.c % 256 == 0;
+    // at most 64 pixels (a matmul with few rows written as a 1x1 layer, its bias as the shift): gemm_rows.hip
+    const bool few_rows = forced_tile == 0 && pixels <= 64 && a.c % 32 == 0;
     if (mode != 2 && !shortk && !long_k && !few_rows &&
         (a.c < 128 || (!narrow && ((pixels + 127) / 128) * ((a.oc + 127) / 128) < 192)))
       return false;

@@ -1,0 +1,37 @@
+// Internal interface of the kernel for products of few rows (gemm_rows.hip).
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+namespace cinn_hip_kernels {
+
+// C [m][n] = act( norm(A) [m][k] . B^T * scale + shift + residual_scale * residual ), B stored [n][k], fp16 or bf16 (all
+// matrices), m <= 64, k % 32 == 0.
+struct RowProduct {
+  bool bf16;
+  const void* a;
+  const void* b;
+  void* c[3];          // n / width tensors [m][width], which take as many columns each
+  int width;
+  int m, n, k;
+  const float* scale;  // per column, or null: alpha
+  const float* shift;  // per column, or null
+  float alpha;
+  const void* residual;  // [m][n], or null; one result tensor then
+  float residual_scale;
+  bool relu, gelu;
+  // layer norm of A's rows before the product: (x - mean) / sqrt(variance + epsilon) * gamma + beta, rounded to the type;
+  // gamma and beta [k] of the matrices' type, null: none
+  const void* gamma;
+  const void* beta;
+  float epsilon;
+};
+
+constexpr int kRowProductMaxNormK = 1280;
+
+// false where the kernel does not take the extents or alignments
+bool RowProductSupported(const RowProduct& p);
+void RunRowProduct(const RowProduct& p, hipStream_t stream);
+
+}  // namespace cinn_hip_kernels

@@ -1,0 +1,278 @@
+// Products of few rows for gfx950 (M <= 64: a classifier at inference batch sizes, a decoding step), fp16 / bf16:
+//   C [M][N] = act( norm(A) [M][K] . B [N][K]^T * scale + shift + residual )
+//
+// Bound by one pass over B.  The tiled kernels give such a product M-tiles that are mostly padding and a handful of blocks;
+// here a block owns 16 output columns of MT row tiles (rows from 16 MT blockIdx.y: the launcher gives every row tile a block
+// of its own where that still leaves CUs) and its eight wavefronts split K in 32-deep blocks.  A lane's share
+// of a 16x16x32 fragment is 8 consecutive k of one row - 16 contiguous bytes in both operands - so fragments come straight
+// from global memory, no LDS on the way: every wavefront keeps 2 U k-blocks of loads in flight, B is read exactly once from
+// memory, A (at most 64 rows) comes out of L2.  The partial tiles meet in LDS; wavefront t finishes row tile t (2-byte
+// stores: the result is small).
+//
+// At these sizes a launch costs as much as the product (an empty kernel 3.3 us from launch to launch, 8 x 768 -> 768 5 us),
+// so what surrounds the product in a decoding step is part of it:
+//   * NORM: the layer norm of A's rows.  Every block has the rows' elements in registers anyway; sums of x and x x over a
+//     lane's k, its row's other lanes and wavefronts (through LDS) give mean and variance, and the fragments are normalised
+//     where they are.  One block barrier more;
+//   * gelu, on the fp32 sum;
+//   * several result tensors side by side (query, key and value of a token), each a contiguous matrix of its own.
+// A block of one new token per sequence (8 sequences, hidden 768, 12 heads, 511 cached, fp16): nine launches in 46.0 us
+// before, five in 35.9 here.  K need only be whole k-blocks: 8 x 960 -> 960, which ran on 64x64 tiles, 7.0 -> 4.2 us.
+#include "kernels/gemm_rows.h"
+
+#include <climits>
+#include <cstdlib>
+#include <type_traits>
+
+#include "cinn_hip_runtime.h"
+#include "runtime/hip_check.h"
+
+namespace cinn_hip_kernels {
+namespace {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+
+template <typename T>
+struct Half16;
+template <>
+struct Half16<__bf16> {
+  typedef bf16x8 vec8;
+  static __device__ __forceinline__ f32x4 mfma(vec8 a, vec8 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+  }
+};
+template <>
+struct Half16<_Float16> {
+  typedef f16x8 vec8;
+  static __device__ __forceinline__ f32x4 mfma(vec8 a, vec8 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+  }
+};
+
+constexpr int NW = 8;  // wavefronts of a block
+// k-blocks of a wavefront that a normalised row keeps in registers
+constexpr int kNormBlocks = kRowProductMaxNormK / 32 / NW;
+
+template <typename T, int MT, bool NORM, bool GELU>
+__global__ void __launch_bounds__(64 * NW)
+gemm_rows_kernel(RowProduct p) {
+  typedef typename Half16<T>::vec8 vec8;
+  static_assert(!NORM || MT == 1, "rows are normalised by blocks of one row tile");
+  __shared__ __attribute__((aligned(16))) float s_part[NW][MT][64][4];
+  __shared__ float s_sum[NORM ? NW : 1][16][2];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n0   = blockIdx.x * 16;
+  const int m0   = blockIdx.y * (MT * 16);  // first of this block's rows
+  const int fr   = lane & 15;               // row of the fragment this lane reads (a row of A, a column of C for B)
+  const int fk   = (lane >> 4) * 8;         // its 8 elements of a 32-deep k block
+  // this wavefront's k-blocks: `mine` consecutive ones (neighbours share 128-byte lines), none when K is short
+  const int blocks = p.k / 32, share = (blocks + NW - 1) / NW;
+  const int first = min(wave * share, blocks - 1);
+  const int mine  = min(share, blocks - wave * share);
+  const T* bp     = static_cast<const T*>(p.b) + (int64_t)min(n0 + fr, p.n - 1) * p.k + first * 32 + fk;
+  const T* ap[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) ap[t] = static_cast<const T*>(p.a) + (int64_t)min(m0 + t * 16 + fr, p.m - 1) * p.k + first * 32 + fk;
+  // offset of block `i`; beyond the share the last one again (not multiplied)
+  auto k_of = [&](int i) { return max(min(i, mine - 1), 0) * 32; };
+  f32x4 acc[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) acc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  if constexpr (NORM) {
+    vec8 af[kNormBlocks], bf[kNormBlocks], g[kNormBlocks], be[kNormBlocks];
+#pragma unroll
+    for (int i = 0; i < kNormBlocks; ++i) af[i] = *reinterpret_cast<const vec8*>(ap[0] + k_of(i));
+#pragma unroll
+    for (int i = 0; i < kNormBlocks; ++i) {
+      bf[i] = *reinterpret_cast<const vec8*>(bp + k_of(i));
+      g[i]  = *reinterpret_cast<const vec8*>(static_cast<const T*>(p.gamma) + first * 32 + fk + k_of(i));
+      be[i] = *reinterpret_cast<const vec8*>(static_cast<const T*>(p.beta) + first * 32 + fk + k_of(i));
+    }
+    float s = 0.0f, q = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kNormBlocks; ++i)
+      if (i < mine) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float x = (float)af[i][e];
+          s += x;
+          q = __builtin_fmaf(x, x, q);
+        }
+      }
+    s += __shfl_xor(s, 16), q += __shfl_xor(q, 16);
+    s += __shfl_xor(s, 32), q += __shfl_xor(q, 32);
+    if (lane < 16) s_sum[wave][lane][0] = s, s_sum[wave][lane][1] = q;
+    __syncthreads();
+    s = q = 0.0f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) s += s_sum[w][fr][0], q += s_sum[w][fr][1];
+    const float mean = s / (float)p.k;
+    const float var  = fmaxf(q / (float)p.k - mean * mean, 0.0f);
+    const float inv  = 1.0f / sqrtf(var + p.epsilon);
+#pragma unroll
+    for (int i = 0; i < kNormBlocks; ++i)
+      if (i < mine) {
+        vec8 x;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = (T)__builtin_fmaf(((float)af[i][e] - mean) * inv, (float)g[i][e], (float)be[i][e]);
+        acc[0] = Half16<T>::mfma(x, bf[i], acc[0]);
+      }
+  } else {
+    constexpr int U = 4;  // k-blocks per register set
+    vec8 bf[2][U], af[2][U][MT];
+    auto request = [&](int set, int i0) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int k = k_of(i0 + u);
+        bf[set][u]  = *reinterpret_cast<const vec8*>(bp + k);
+#pragma unroll
+        for (int t = 0; t < MT; ++t) af[set][u][t] = *reinterpret_cast<const vec8*>(ap[t] + k);
+      }
+    };
+    auto multiply = [&](int set, int i0) {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (i0 + u < mine) {
+#pragma unroll
+          for (int t = 0; t < MT; ++t) acc[t] = Half16<T>::mfma(af[set][u][t], bf[set][u], acc[t]);
+        }
+    };
+    request(0, 0);
+    for (int i = 0; i < mine; i += 2 * U) {
+      if (i + U < mine) request(1, i + U);
+      multiply(0, i);
+      if (i + 2 * U < mine) request(0, i + 2 * U);
+      multiply(1, i + U);
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < MT; ++t) *reinterpret_cast<f32x4*>(&s_part[wave][t][lane][0]) = acc[t];
+  __syncthreads();
+  if (wave >= MT) return;
+  // wavefront t: row tile t.  Lane = (column n0 + lane % 16, rows 16 t + 4 (lane / 16) .. + 3)
+  f32x4 sum = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int w = 0; w < NW; ++w) sum += *reinterpret_cast<const f32x4*>(&s_part[w][wave][lane][0]);
+  const int col = n0 + fr;
+  if (col >= p.n) return;
+  const float sc  = p.scale ? p.scale[col] : p.alpha;
+  const float sh  = p.shift ? p.shift[col] : 0.0f;
+  const int width = p.width;  // of a result tensor
+  const int part  = (col >= width) + (col >= 2 * width);
+  T* to           = static_cast<T*>(part == 0 ? p.c[0] : part == 1 ? p.c[1] : p.c[2]) + (col - part * width);
+  const T* res    = static_cast<const T*>(p.residual);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int row = m0 + wave * 16 + 4 * (lane >> 4) + r;
+    if (row >= p.m) continue;
+    float v = __builtin_fmaf(sum[r], sc, sh);
+    if (res) v = __builtin_fmaf(p.residual_scale, (float)res[(int64_t)row * p.n + col], v);
+    asm volatile("" : "+v"(v));  // fp32 first, then one rounding to T: the same for every row
+    if (p.relu) v = v > 0.0f ? v : 0.0f;
+    if constexpr (GELU) v = v * __builtin_fmaf(0.5f, erff(v * 0.70710678f), 0.5f);
+    to[(int64_t)row * width] = (T)v;
+  }
+}
+
+template <typename T>
+void Launch(const RowProduct& p, hipStream_t stream) {
+  int mt = (p.m + 15) / 16;
+  dim3 grid((unsigned)((p.n + 15) / 16));
+  // Fewer column blocks than CUs: one block per 16 rows as well.  A block's traffic is its 16 columns of B plus the
+  // rows of A it multiplies, and with all of A (128 KB at 32 x 2048, against 64 KB of B) the few CUs at work are bound
+  // by what one CU can pull in; row blocks read B again, out of L2.  ResNet-50's classifier, 32 x 2048 -> 1000: 126
+  // blocks instead of 63, 2.2 us less.  With the chip full, the row tiles stay in one block's registers (B read once).
+  // FLAGS_cinn_hip_gemm_skinny_rows: 0 never splits the rows, 2 always.
+  static const int rows_flag = getenv("FLAGS_cinn_hip_gemm_skinny_rows") ? atoi(getenv("FLAGS_cinn_hip_gemm_skinny_rows")) : 1;
+  if (p.gamma || p.gelu || rows_flag == 2 || (rows_flag == 1 && grid.x < 256)) grid.y = mt, mt = 1;
+#define CINN_ROWS(MT, NORM, GELU) hipLaunchKernelGGL((gemm_rows_kernel<T, MT, NORM, GELU>), grid, dim3(64 * NW), 0, stream, p)
+  // (8 x 768 x 3072 takes 6.7 us; 8.3 with sixteen wavefronts, 8.2 with all twelve k-blocks of a wavefront requested at once)
+  if (p.gamma && p.gelu) {
+    CINN_ROWS(1, true, true);
+  } else if (p.gamma) {
+    CINN_ROWS(1, true, false);
+  } else if (p.gelu) {
+    CINN_ROWS(1, false, true);
+  } else {
+    switch (mt) {
+      case 1: CINN_ROWS(1, false, false); break;
+      case 2: CINN_ROWS(2, false, false); break;
+      case 3: CINN_ROWS(3, false, false); break;
+      default: CINN_ROWS(4, false, false); break;
+    }
+  }
+#undef CINN_ROWS
+  CINN_HIP_CALL(hipGetLastError());
+}
+
+bool Aligned(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+
+}  // namespace
+
+bool RowProductSupported(const RowProduct& p) {
+  if (p.m < 1 || p.m > 64 || p.n < 1 || p.k < 32 || p.k % 32 != 0 || (int64_t)p.n * p.k >= INT_MAX) return false;
+  if (p.width < 1 || p.n % p.width != 0 || p.n / p.width > 3 || (p.n > p.width && p.residual)) return false;
+  if (p.gamma && (!p.beta || p.k > kRowProductMaxNormK || !Aligned(p.gamma) || !Aligned(p.beta))) return false;
+  return Aligned(p.a) && Aligned(p.b);
+}
+
+void RunRowProduct(const RowProduct& p, hipStream_t stream) {
+  if (p.bf16) {
+    Launch<__bf16>(p, stream);
+  } else {
+    Launch<_Float16>(p, stream);
+  }
+}
+
+}  // namespace cinn_hip_kernels
+
+extern "C" void cinn_call_hip_matmul_rows(void* v_args, int num_args, int m, int n, int k, int operands, int outputs, float epsilon,
+                                          int gelu, void* stream) {
+  CINN_HIP_CLEAR_STALE_ERROR();
+  using namespace cinn_hip_kernels;
+  CINN_RT_CHECK(outputs >= 1 && outputs <= 3 && num_args > outputs, "cinn_call_hip_matmul_rows: %d of %d arguments are results", outputs, num_args);
+  auto* args  = static_cast<cinn_pod_value_t*>(v_args);
+  auto buffer = [&](int index) {
+    CINN_RT_CHECK(args[index].type_code_ == CINN_POD_BUFFER_P, "cinn_call_hip_matmul_rows: argument %d is not a buffer", index);
+    auto* b = static_cast<cinn_buffer_t*>(args[index].value_.v_handle);
+    CINN_RT_CHECK(b && b->memory, "cinn_call_hip_matmul_rows: argument %d has no device memory", index);
+    return b;
+  };
+  auto operand = [&](int slot) -> cinn_buffer_t* {
+    const int at = (int)(((unsigned)operands >> (4 * slot)) & 15);
+    if (at == 15) return nullptr;
+    CINN_RT_CHECK(at < num_args - outputs, "cinn_call_hip_matmul_rows: operand %d is argument %d of %d inputs", slot, at, num_args - outputs);
+    return buffer(at);
+  };
+  cinn_buffer_t* in[7];
+  for (int s = 0; s < 7; ++s) in[s] = operand(s);
+  CINN_RT_CHECK(in[0] && in[1] && !in[5] == !in[6], "cinn_call_hip_matmul_rows: x and W, and gamma and beta or neither, expected");
+  const cinn_type_t type = in[0]->type;
+  RowProduct p{};
+  p.bf16 = type.code == cinn_type_bfloat;
+  CINN_RT_CHECK(type.bits == 16 && (p.bf16 || type.code == cinn_type_float), "cinn_call_hip_matmul_rows: fp16 or bf16 operands expected");
+  for (int s : {1, 4, 5, 6})
+    CINN_RT_CHECK(!in[s] || (in[s]->type.code == type.code && in[s]->type.bits == 16), "cinn_call_hip_matmul_rows: operand %d differs in type", s);
+  for (int s : {2, 3})
+    CINN_RT_CHECK(!in[s] || (in[s]->type.code == cinn_type_float && in[s]->type.bits == 32), "cinn_call_hip_matmul_rows: scale and shift are fp32");
+  auto memory = [&](int slot) -> void* { return in[slot] ? in[slot]->memory : nullptr; };
+  p.a = memory(0), p.b = memory(1);
+  p.scale = static_cast<const float*>(memory(2)), p.shift = static_cast<const float*>(memory(3));
+  p.alpha    = 1.0f;
+  p.residual = memory(4), p.residual_scale = 1.0f;
+  p.gamma = memory(5), p.beta = memory(6), p.epsilon = epsilon;
+  p.gelu = gelu != 0;
+  p.m = m, p.n = n, p.k = k;
+  CINN_RT_CHECK(n > 0 && n % outputs == 0, "cinn_call_hip_matmul_rows: %d columns for %d results", n, outputs);
+  p.width = n / outputs;
+  for (int i = 0; i < outputs; ++i) {
+    cinn_buffer_t* out = buffer(num_args - outputs + i);
+    CINN_RT_CHECK(out->type.code == type.code && out->type.bits == 16, "cinn_call_hip_matmul_rows: result %d differs in type", i);
+    p.c[i] = out->memory;
+  }
+  CINN_RT_CHECK(RowProductSupported(p), "cinn_call_hip_matmul_rows: %d x %d x %d is not taken", m, n, k);
+  RunRowProduct(p, static_cast<hipStream_t>(stream));
+}

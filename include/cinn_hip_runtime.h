@@ -284,6 +284,14 @@ void cinn_call_hip_attention(void* v_args, int num_args, float scale, int batch,
  * n and k below 2^22.  v_args = {A, B, bias, C}, or {A, bias, C} where B is A. */
 void cinn_call_hip_matmul_bias(void* v_args, int num_args, int trans_b, int m, int n, int k, void* stream);
 
+/* A linear layer of at most 64 rows with what surrounds it: act(norm(x) [m][k] W^T * scale + shift + residual), W [n][k], fp16 or
+ * bf16 with fp32 scale and shift [n]; k a multiple of 32.  norm: layer norm of the rows with gamma and beta [k] of x's type
+ * (k at most 1280); act: gelu on the fp32 sum, or nothing.  outputs 2 or 3 (without a residual): the columns go to that many
+ * tensors [m][n / outputs], side by side.  operands: four bits for each of the slots x, W, scale, shift, residual, gamma,
+ * beta, which input it is, 15 for none; v_args = {inputs..., outputs...}. */
+void cinn_call_hip_matmul_rows(void* v_args, int num_args, int m, int n, int k, int operands, int outputs, float epsilon, int gelu,
+                               void* stream);
+
 /* A training batch norm of channels-last tensors [pixels][channels] (fp16 / bf16 / fp32, one type per call), the
  * per-channel vectors in fp32.  operands: four bits per operand slot, which of the call's inputs it is; the results follow
  * the inputs in v_args.
