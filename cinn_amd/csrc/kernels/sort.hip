@@ -417,51 +417,128 @@ __device__ __forceinline__ u64 WaveMin(u64 v) {
   return Word(low, WaveMin32(key == low ? (uint32_t)v : 0xffffffffu));
 }
 
-// The first `keep` (at most kSelect) elements of a row, taken one by one: a lane keeps E words and their least one, a
-// wavefront takes the least of those, its owner looks for its next one.  A row of more than 1024 elements has several
-// wavefronts, each takes the first `keep` of its part, and the first wavefront takes the first of all from those.
-// 2048 rows of 1000 fp32 values: the first five in 10 us (two full sorts, two slices and a cast: 464 us), each further
-// one 0.55 us; the first 16 in 16 us, where sorting all takes 21 - hence the limit.
-constexpr int kSelect = 16;
-template <typename T, int E, int WAVES>
+// The first `keep` (at most 64) of a wavefront's words, E per lane, written to first[0 .. keep - 1] in order.  The keep-th
+// least of the lanes' least keys bounds the keys that can be among them, and few others lie below it: for the first five of
+// 1000 random values seven words are left on average, for the first fifty about ninety.  These are gathered, C per lane, and
+// each counts the ones before it.  Of the words at the bound itself the first `keep`
+// suffice (looked at for C > 1 only).  Should more than 64 C words be
+// left - a lane has many of a row's first elements - they are taken one by one, the owner of each looking for its next one.
+// candidates: 64 C words of LDS of this wavefront's own, as first is.  w[e] of a lane is ahead of w[e] of the lanes behind it
+// and of all w[e + 1] where the keys are equal.
+template <int E, int C>
+__device__ __forceinline__ void SelectFirst(u64 (&w)[E], int keep, u64* candidates, u64* first) {
+  const int lane = threadIdx.x & 63;
+  uint32_t rest  = (uint32_t)(w[0] >> 32), limit = 0;
+#pragma unroll
+  for (int e = 1; e < E; ++e) rest = min(rest, (uint32_t)(w[e] >> 32));
+#pragma unroll 1
+  for (int s = 0; s < keep; ++s) {
+    limit = WaveMin32(rest);
+    if (lane == __builtin_ctzll(__ballot(rest == limit))) rest = 0xffffffffu;
+  }
+  const u64 before = ((u64)1 << lane) - 1;
+  int count = 0, equals = 0;
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const uint32_t key = (uint32_t)(w[e] >> 32);
+    u64 mask           = __ballot(C > 1 ? key < limit : key <= limit);
+    if constexpr (C > 1) {
+      const u64 equal = __ballot(key == limit);
+      if (equal != 0 && equals < keep) {
+        mask |= __ballot(key == limit && equals + __popcll(equal & before) < keep);
+        equals += __popcll(equal);
+      }
+    }
+    if (mask == 0) continue;
+    const int at = count + __popcll(mask & before);
+    if ((mask >> lane & 1) && at < 64 * C) candidates[at] = w[e];
+    count += __popcll(mask);
+  }
+  if (count <= 64 * C) {
+    // the wavefront's own words: its LDS accesses keep their order, the compiler must not change it
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    u64 mine[C];
+    int slot[C];
+#pragma unroll
+    for (int u = 0; u < C; ++u) mine[u] = lane + 64 * u < count ? candidates[lane + 64 * u] : ~0ull, slot[u] = 0;
+#pragma unroll
+    for (int v = 0; v < C; ++v) {
+#pragma unroll 1
+      for (int c = 0; c < min(count - 64 * v, 64); ++c) {
+        const u64 other =
+            Word((uint32_t)__builtin_amdgcn_readlane((int)(mine[v] >> 32), c), (uint32_t)__builtin_amdgcn_readlane((int)mine[v], c));
+#pragma unroll
+        for (int u = 0; u < C; ++u) slot[u] += other < mine[u] ? 1 : 0;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < C; ++u)
+      if (lane + 64 * u < count && slot[u] < keep) first[slot[u]] = mine[u];
+  } else {
+    u64 least = w[0];
+#pragma unroll
+    for (int e = 1; e < E; ++e) least = w[e] < least ? w[e] : least;
+#pragma unroll 1
+    for (int s = 0; s < keep; ++s) {
+      const u64 got = WaveMin(least);
+      if (lane == s) first[s] = got;
+      if (least == got) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) w[e] = w[e] == got ? ~0ull : w[e];
+        least = w[0];
+#pragma unroll
+        for (int e = 1; e < E; ++e) least = w[e] < least ? w[e] : least;
+      }
+    }
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// The first `keep` (at most kSelect) elements of a row.  A row of more than 1024 elements has several wavefronts; each selects
+// the first `keep` of its part.  Of up to sixteen (C = 1) the first wavefront selects again, of more each looks up how many of
+// the other parts' are before it.
+// Bound by the launch and the read of the row for few elements (2048 rows of 1000 fp32 values, k = 1: 5.6 us), by the wave
+// reductions that find the bound for many.  Taking the elements one by one - a 64-bit look at all of the owner's words for
+// each - against this: k = 5 7.8 -> 6.3 us, k = 10 10.5 -> 7.0, k = 16 13.8 -> 7.9; 64 rows of 8000 fp16, k = 10 18.0 -> 8.7;
+// 600 rows of 3000, k = 5 9.2 -> 6.5.
+constexpr int kSelect = 64;  // what a wavefront can select
+template <typename T, int E, int WAVES, int C>
 __global__ void __launch_bounds__(64 * WAVES) row_select_kernel(RowParams p) {
-  __shared__ u64 part[WAVES > 1 ? WAVES * kSelect : 1];
+  __shared__ u64 candidates[WAVES * 64 * C];
+  __shared__ u64 part[WAVES][kSelect], first[WAVES > 1 && C == 1 ? 16 : 1];
   __shared__ uint32_t shared[16];
-  const int t = threadIdx.x, lane = t & 63;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int64_t base = (int64_t)(blockIdx.x / p.inner) * p.size * p.inner + blockIdx.x % p.inner;
   u64 w[E];
   LoadWords<T, E, 64 * WAVES>(p, base, t, 64 * WAVES, p.size, shared, w);
-  u64 mine = 0;  // lane s keeps the word of slot s
-  auto take = [&](auto& words) {
-    constexpr int COUNT = sizeof(words) / sizeof(u64);
-    u64 least = words[0];
+  SelectFirst<E, C>(w, p.keep, candidates + wave * 64 * C, part[wave]);
+  if (WAVES > 1) __syncthreads();
+  if constexpr (WAVES > 1 && C == 1) {
+    if (wave > 0) return;
+    u64 all[WAVES / 4];
 #pragma unroll
-    for (int e = 1; e < COUNT; ++e) least = words[e] < least ? words[e] : least;
-#pragma unroll 1
-    for (int s = 0; s < p.keep; ++s) {
-      const u64 got = WaveMin(least);
-      if (lane == s) mine = got;
-      if (least == got) {
-#pragma unroll
-        for (int e = 0; e < COUNT; ++e) words[e] = words[e] == got ? ~0ull : words[e];
-        least = words[0];
-#pragma unroll
-        for (int e = 1; e < COUNT; ++e) least = words[e] < least ? words[e] : least;
-      }
-    }
-  };
-  take(w);
-  if constexpr (WAVES > 1) {
-    if (lane < p.keep) part[(t >> 6) * kSelect + lane] = mine;
-    __syncthreads();
-    if (t >= 64) return;
-    u64 all[WAVES * kSelect / 64];
-#pragma unroll
-    for (int e = 0; e < WAVES * kSelect / 64; ++e) all[e] = (lane % kSelect) < p.keep ? part[e * 64 + lane] : ~0ull;
-    take(all);
+    for (int e = 0; e < WAVES / 4; ++e) all[e] = (lane & 15) < p.keep ? part[e * 4 + (lane >> 4)][lane & 15] : ~0ull;
+    SelectFirst<WAVES / 4, 1>(all, p.keep, candidates, first);
   }
   if (lane >= p.keep) return;
-  const int64_t at = (int64_t)(blockIdx.x / p.inner) * p.keep * p.inner + blockIdx.x % p.inner + (int64_t)lane * p.inner;
+  const u64 mine = WAVES > 1 && C == 1 ? first[lane] : part[wave][lane];
+  int slot       = lane;
+  if constexpr (WAVES > 1 && C > 1) {
+#pragma unroll 1
+    for (int other = 0; other < WAVES; ++other) {
+      if (other == wave) continue;
+      int low = 0;  // words of the other part before this one: its list is in order
+#pragma unroll
+      for (int step = kSelect / 2; step > 0; step /= 2)
+        if (low + step <= p.keep && part[other][low + step - 1] < mine) low += step;
+      if (low < p.keep && part[other][low] < mine) ++low;
+      slot += low;
+    }
+    if (slot >= p.keep) return;
+  }
+  const int64_t at = (int64_t)(blockIdx.x / p.inner) * p.keep * p.inner + blockIdx.x % p.inner + (int64_t)slot * p.inner;
   const uint32_t i = (uint32_t)mine;
   if (p.index64) p.index64[at] = (int64_t)i;
   if (p.sorted) static_cast<T*>(p.sorted)[at] = static_cast<const T*>(p.x)[base + (int64_t)i * p.inner];
@@ -494,7 +571,18 @@ void LaunchRowSort(const RowParams& p, int rows, hipStream_t stream) {
 }
 template <typename T>
 void LaunchRowSelect(const RowParams& p, int rows, hipStream_t stream) {
-#define CINN_ROW_SELECT(E, WAVES) hipLaunchKernelGGL((row_select_kernel<T, E, WAVES>), dim3(rows), dim3(64 * WAVES), 0, stream, p)
+  // words per lane for what is left of a selection: 16 of 64 lanes' least ones bound about 20 words of 1000, 32 about 45 and
+  // 50 about 90, with a spread that takes the last over 128 in a few rows of a hundred
+#define CINN_ROW_SELECT_C(E, WAVES, C) \
+  hipLaunchKernelGGL((row_select_kernel<T, E, WAVES, C>), dim3(rows), dim3(64 * WAVES), 0, stream, p)
+#define CINN_ROW_SELECT(E, WAVES)      \
+  if (p.keep <= 16) {                  \
+    CINN_ROW_SELECT_C(E, WAVES, 1);    \
+  } else if (p.keep <= 32) {           \
+    CINN_ROW_SELECT_C(E, WAVES, 2);    \
+  } else {                             \
+    CINN_ROW_SELECT_C(E, WAVES, 4);    \
+  }
   if (p.size <= 256) {
     CINN_ROW_SELECT(4, 1);
   } else if (p.size <= 1024) {
@@ -505,7 +593,14 @@ void LaunchRowSelect(const RowParams& p, int rows, hipStream_t stream) {
     CINN_ROW_SELECT(16, 16);
   }
 #undef CINN_ROW_SELECT
+#undef CINN_ROW_SELECT_C
 }
+
+// Up to which k the selection is ahead of the network.  us, network | selection, fp32: 2048 rows of 1000, k = 17 21.1 | 9.2,
+// k = 32 21.1 | 12.0, k = 50 21.2 | 18.9; 600 rows of 1500, k = 50 41.2 | 20.1, k = 64 41.2 | 59 (with as many elements as
+// lanes the bound is the largest of the lanes' least words, and most rows are taken one by one); 64 rows of 8000 fp16, k = 50
+// 77.9 | 28.4.  The network of 256 words on one wavefront is short: 4000 rows of 250, k = 17 9.5, k = 50 9.7 | 17.0.
+int SelectLimit(int size) { return size <= 256 ? 16 : 50; }
 
 enum class Elem { kF32, kF64, kF16, kBF16, kI32, kI64, kUnsupported };
 
@@ -657,7 +752,7 @@ extern "C" void cinn_call_hip_top_k(void* v_args, int num_args, int outer, int s
     LaunchTiles(p, elem, outer, s);
     return;
   }
-  auto run = [&](auto launch_select, auto launch_sort) { k <= kSelect ? launch_select(r, outer * inner, s) : launch_sort(r, outer * inner, s); };
+  auto run = [&](auto launch_select, auto launch_sort) { k <= SelectLimit(size) ? launch_select(r, outer * inner, s) : launch_sort(r, outer * inner, s); };
   switch (elem) {
     case Elem::kF32: run(LaunchRowSelect<float>, LaunchRowSort<float>); break;
     case Elem::kF16: run(LaunchRowSelect<_Float16>, LaunchRowSort<_Float16>); break;

@@ -101,6 +101,24 @@ def test_top_k(gpu, size, kind, k):
     assert np.array_equal(got_values, ranked[:, :k], equal_nan=kind != "int32")
 
 
+@pytest.mark.parametrize("equal", [1, 59, 60, 61, 300])
+@pytest.mark.parametrize("k", [1, 16, 17, 50, 64])
+@pytest.mark.parametrize("size", [64, 65, 1000, 1025, 4097])
+def test_top_k_of_distinct_scores_and_equal_ones(gpu, size, k, equal):
+    """the words up to the bound are ranked against each other, more than 64 or 128 of them are taken one by one: distinct
+    scores, scores of which the k-th largest is shared, and a row whose largest ones a few lanes hold"""
+    rng = np.random.default_rng(size + k)
+    x = rng.permuted(np.tile(np.arange(size, dtype=np.float32) - size // 2, (5, 1)), axis=1)
+    x[4, rng.permutation(size)] = np.where(np.arange(size) % 64 < 3, size, 0) + x[4]
+    for row in x[2:]:
+        row[np.argsort(-row, kind="stable")[k - 1:k - 1 + equal]] = size
+    b = NetBuilder("top")
+    v = b.create_input(Float(32), list(x.shape), "x")
+    (values, where), _ = run(b, {v: x}, list(b.top_k(v, k, 1)))
+    index = np.argsort(-x, axis=1, kind="stable")[:, :k]
+    assert np.array_equal(where, index) and np.array_equal(values, np.take_along_axis(x, index, 1))
+
+
 def test_top_k_of_one_output_or_shared_results(gpu):
     """only the values or only the indices are wanted; a full sort that something else reads stays"""
     rng = np.random.default_rng(1)
