@@ -14,11 +14,12 @@
 //     56x56 at batch 32 takes in fp16; whoever has such a filter has the NaNs from the forward pass.)
 //   * dw: rows are filters, columns (tap, channel), and K runs over all output pixels, which both operands keep as their
 //     slow axis: they lie in LDS as [pixel][channels] and are read with transposing reads.  The x operand is gathered
-//     row by row (a chunk of channels of pixel + tap, or zeros).  K is long (1e5) and the result small, so K is split
-//     until the chip is full; the fp32 planes are added by a second kernel, which also writes the filter's own layout.
+//     row by row (a chunk of channels of pixel + tap, or zeros); at a stride of one the taps of a filter row share what is
+//     read (conv_filter_taps_kernel).  K is long (1e5) and the result small, so K is split until the chip is full; the
+//     fp32 planes are added by a second kernel, which also writes the filter's own layout.
 // Measured before (one thread or block per gradient element) and here: 64 -> 64 3x3 on 56x56 at batch 32 in fp16, NCHW,
-// dx 4988 -> 13 us (560 TFLOP/s) and dw 9467 -> 28 + 6 us (260 TFLOP/s; the x operand is read nine times from L2), with
-// 5 to 7 us for each copied tensor; 96 -> 200 3x3 / stride 2 on 35x41 at batch 8 in fp32, dx 1661 -> 31 us and dw
+// dx 4988 -> 13 us (560 TFLOP/s) and dw 9467 -> 28 + 6 us (with the x operand read nine times from L2), 19 + 5 us by
+// neighbouring taps, with 5 to 7 us for each copied tensor; 96 -> 200 3x3 / stride 2 on 35x41 at batch 8 in fp32, dx 1661 -> 31 us and dw
 // 3844 -> 22 + 5 us (47 TFLOP/s).
 // Tensors that are not channels last, or whose channel count is no multiple of a 16-byte chunk, are first copied into
 // that form in scratch (pack_kernel), and dx is copied back (with beta, after it has been copied there).
@@ -286,6 +287,7 @@ struct FilterGradParams {
   int pixels, steps, steps_per_split;
   int tiles_m, tiles_n;
   int adv_n, adv_oy, adv_ox;  // a K step in images, rows and columns of the output
+  int spill;  // 1: taps meet zeros of dy inside the image too (conv_filter_taps_kernel)
 };
 
 // the x operand: [pixel][ROWS columns of (tap, channel)].  A thread's chunks share one column chunk, i.e. one tap;
@@ -374,6 +376,190 @@ conv_filter_kernel(FilterGradParams p) {
   });
 }
 
+// ---- filter gradient, neighbouring taps of a row ----------------------------------------------------------------------
+// At a stride of one the taps kx, kx + 1 and kx + 2 of a filter row multiply the same dy by the same pixels of x, one apart.
+// conv_filter_kernel reads x once for each of them; here a block's columns are 64 channels x three such taps, and one tile of x
+// serves all three: of the four k a transposing read brings, three reads hold the eight of every tap (tap kx starts kx later).
+//
+// K runs over positions: the pixels of an output row and kTaps - 1 more behind it, where dy is taken as zero, so that the
+// pixel a tap reads is the position's own plus the tap, in the same row.  A K step is 64 positions of which the last
+// kTaps - 1 only lend their pixels to the ones before them (dy zero once more); the next step begins with them.
+// Positions, image rows and addresses advance without a division; what is outside comes back as zero from the buffer loads'
+// range check.  Zeros of dy meet pixels of the image, so NaNs are computed again for every tap (filter_reduce_kernel).
+//
+// Eight wavefronts: two halves of each K step, added in LDS at the end (half the planes of two blocks), each 2 x 2 over filters
+// and channels.
+// 64 -> 64 3x3 on 56x56 at batch 32, fp16: 27.2 -> 18.9 us (392 TFLOP/s) and the reduction of the planes 6.1 -> 4.7; 82 MB
+// come out of L2 instead of 188, and 21 steps per block (of one per CU) take about half of the time, the rest is the launch,
+// the first operands and 12 MB of planes.
+constexpr int kTaps = 3, kFresh = 64 - (kTaps - 1);  // positions of a K step that are its own
+
+struct TapsParams {
+  FilterGradParams g;
+  int tiles_c, groups, tiles;  // tiles: m fastest, then channels, groups of taps, rows of the filter
+  int splits, lanes_log2;      // splits: a multiple of 1 << lanes_log2
+  int period, rows;            // positions of an output row; output rows of all images
+  int adv_at, adv_row;         // a K step in positions and rows
+  int adv_oy, adv_n;           // adv_row in output rows and images
+};
+
+template <typename T>
+__global__ void __launch_bounds__(512, 1)
+conv_filter_taps_kernel(TapsParams p) {
+  constexpr int BM = 64, BN = 64;                                                // filters, channels
+  constexpr int A_BYTES = BM * 128, B_ROWS = 68, STAGE = A_BYTES + B_ROWS * 128;  // reads reach four rows beyond the step
+  constexpr int COLS = kTaps * BN, SLD = COLS + 4;
+  constexpr int TM = 2, TN = 2, PF = 4;
+  typedef flex::Tile<T, false, 64, 512> Tile;  // a chunk of either operand per thread and step
+  typedef flex::Mma<T, false, false, BM, BN> M;
+  typedef typename M::vec8 vec8;
+  static_assert(64 * SLD * 4 >= 2 * STAGE, "the staging tile of the results covers the stages");
+  __shared__ __attribute__((aligned(256))) char lds[64 * SLD * 4];
+  const FilterGradParams& g = p.g;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kg = wave >> 2, wm = (wave >> 1) & 1, wn = wave & 1;
+
+  // every split's tiles on one XCD (blocks go to the 8 of them in turn), one after the other: they read the same pixels
+  const int order = blockIdx.x >> p.lanes_log2;
+  const int split = (order / p.tiles << p.lanes_log2) + (blockIdx.x & ((1 << p.lanes_log2) - 1));
+  int tile        = order % p.tiles;
+  const int m0    = tile % g.tiles_m * BM;
+  tile /= g.tiles_m;
+  const int c0 = tile % p.tiles_c * BN;
+  tile /= p.tiles_c;
+  const int kx0 = tile % p.groups * kTaps, ky = tile / p.groups;
+  const int s0 = split * g.steps_per_split, s1 = min(s0 + g.steps_per_split, g.steps);
+
+  const __amdgpu_buffer_rsrc_t dy_rsrc =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(g.dy), 0, g.pixels * g.fp * (int)sizeof(T), 0x00020000);
+  const __amdgpu_buffer_rsrc_t x_rsrc =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(g.x), 0, p.rows / g.oh * g.h * g.w * g.cp * (int)sizeof(T), 0x00020000);
+  constexpr unsigned kOutside = 0x80000000u;
+
+  // The thread's chunk of either operand: its position in the output row, the row of all images and of its image, offsets of
+  // the row's first pixel.  Channels beyond the last chunk repeat it (and are not stored).
+  const int k   = Tile::ChunkK(tid, 0);
+  const int t   = s0 * kFresh + k;
+  int row = t / p.period, at = t - row * p.period;
+  const int image0 = row / g.oh, iy_first = ky * g.dil_h - g.pad_h, iy_end = g.oh * g.stride_h + iy_first, shift = kx0 - g.pad_w;
+  int iy = (row - image0 * g.oh) * g.stride_h + iy_first;
+  const unsigned a_line = (unsigned)(g.ow * g.fp), b_line = (unsigned)(g.w * g.cp);
+  unsigned a_row = (unsigned)row * a_line, b_row = ((unsigned)(image0 * g.h) + (unsigned)iy) * b_line;
+  const unsigned a_col = (unsigned)min(m0 + tid % Tile::CH * 8, g.fp - 8), b_col = (unsigned)min(c0 + tid % Tile::CH * 8, g.cp - 8);
+  const unsigned a_step = (unsigned)p.adv_row * a_line, b_step = (unsigned)(p.adv_n * g.h + p.adv_oy * g.stride_h) * b_line;
+  const unsigned b_next = (unsigned)g.stride_h * b_line, b_image = (unsigned)(g.h - g.oh * g.stride_h) * b_line;
+
+  u32x4 ra[PF], rb[PF];
+  auto load = [&](int slot) {
+    const int ix    = at + shift;
+    const bool a_ok = k < kFresh && at < g.ow && row < p.rows;
+    const bool b_ok = (unsigned)iy < (unsigned)g.h && (unsigned)ix < (unsigned)g.w && row < p.rows;
+    ra[slot] = __builtin_amdgcn_raw_buffer_load_b128(
+        dy_rsrc, a_ok ? (a_row + (unsigned)__mul24(at, g.fp) + a_col) * (unsigned)sizeof(T) : kOutside, 0, 0);
+    rb[slot] = __builtin_amdgcn_raw_buffer_load_b128(
+        x_rsrc, b_ok ? (b_row + (unsigned)__mul24(ix, g.cp) + b_col) * (unsigned)sizeof(T) : kOutside, 0, 0);
+    at += p.adv_at;
+    const bool next = at >= p.period;
+    at -= next ? p.period : 0;
+    row += p.adv_row + (next ? 1 : 0);
+    a_row += a_step + (next ? a_line : 0);
+    iy += p.adv_oy * g.stride_h + (next ? g.stride_h : 0);
+    b_row += b_step + (next ? b_next : 0);
+    const bool image = iy >= iy_end;
+    iy -= image ? g.oh * g.stride_h : 0;
+    b_row += image ? b_image : 0;
+  };
+  auto store = [&](int slot, char* stage) {
+    *reinterpret_cast<u32x4*>(stage + Tile::LdsOffset(tid, 0))           = ra[slot];
+    *reinterpret_cast<u32x4*>(stage + A_BYTES + Tile::LdsOffset(tid, 0)) = rb[slot];
+  };
+
+  flex::f32x4 acc[TM][kTaps][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int q = 0; q < kTaps; ++q)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][q][j] = flex::f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  const int group = ((lane >> 4) & 1) * 2 + (lane >> 5);  // the eight k of this lane, as Mma::Fragment takes them
+  auto multiply = [&](const char* stage) {
+    vec8 a[TM];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) a[i] = M::template Fragment<false, BM>(stage, wm * (BM / 2) + i * 16, kg, lane);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      flex::s16x4 part[3];
+#pragma unroll
+      for (int r = 0; r < 3; ++r) {
+        const int k = kg * 32 + 8 * group + 4 * r + ((lane & 15) >> 2), n = wn * 32 + j * 16 + 4 * (lane & 3);
+        const char* at = stage + A_BYTES + Tile::RowOffset(k, n >> 3) + (n & 7) * 2;
+        part[r] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((flex::s16x4 __attribute__((address_space(3)))*)at);
+      }
+      const flex::s16x8 low  = __builtin_shufflevector(part[0], part[1], 0, 1, 2, 3, 4, 5, 6, 7);
+      const flex::s16x8 high = __builtin_shufflevector(part[2], part[2], 0, 1, 2, 3, 0, 1, 2, 3);
+      const vec8 b[kTaps]    = {__builtin_bit_cast(vec8, low), __builtin_bit_cast(vec8, __builtin_shufflevector(low, high, 1, 2, 3, 4, 5, 6, 7, 8)),
+                                __builtin_bit_cast(vec8, __builtin_shufflevector(low, high, 2, 3, 4, 5, 6, 7, 8, 9))};
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int q = 0; q < kTaps; ++q) acc[i][q][j] = flex::Half16<T>::mfma(a[i], b[q], acc[i][q][j]);
+    }
+  };
+
+  // the rows behind a step's tile of x, which meet dy's zeros: zero as well, once
+  if (tid < 2 * (B_ROWS - 64) * 8) {
+    const int i = tid & 31;
+    *reinterpret_cast<u32x4*>(lds + (tid >> 5) * STAGE + A_BYTES + Tile::RowOffset(64 + (i >> 3), i & 7)) = u32x4{0, 0, 0, 0};
+  }
+#pragma unroll
+  for (int u = 0; u < PF; ++u) load(u);
+  store(0, lds);
+  __syncthreads();
+  // a ring of PF steps in registers (flex::KLoop's); steps behind the last one are requested too: they are outside, or
+  // pixels of the next split, and are not multiplied
+  for (int s = s0; s < s1; s += PF) {
+#pragma unroll
+    for (int u = 0; u < PF; ++u) {
+      if (s + u >= s1) break;
+      load(u);
+      multiply(lds + (u & 1) * STAGE);
+      store((u + 1) % PF, lds + ((u + 1) & 1) * STAGE);
+      __syncthreads();
+    }
+  }
+
+  // the tile through LDS, the two halves of K added there
+  float* st    = reinterpret_cast<float*>(lds);
+  float* plane = g.planes + (int64_t)split * g.f * g.taps * g.cp;
+#pragma unroll
+  for (int half = 0; half < 2; ++half) {
+    if (kg == half) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int q = 0; q < kTaps; ++q)
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              float* to = st + (wm * 32 + i * 16 + 4 * (lane >> 4) + r) * SLD + q * BN + wn * 32 + j * 16 + (lane & 15);
+              *to       = half == 0 ? acc[i][q][j][r] : *to + acc[i][q][j][r];
+            }
+    }
+    __syncthreads();
+  }
+#pragma unroll 1
+  for (int i = tid; i < BM * COLS / 8; i += 512) {
+    const int f = i / (COLS / 8), col = i % (COLS / 8), q = col / (BN / 8), c = c0 + col % (BN / 8) * 8;
+    if (m0 + f >= g.f || kx0 + q >= g.kw || c >= g.cp) continue;
+    const float* from = &st[f * SLD + col * 8];
+    float* to         = plane + ((int64_t)(m0 + f) * g.taps + ky * g.kw + kx0 + q) * g.cp + c;
+    *reinterpret_cast<flex::f32x4*>(to)     = *reinterpret_cast<const flex::f32x4*>(from);
+    *reinterpret_cast<flex::f32x4*>(to + 4) = *reinterpret_cast<const flex::f32x4*>(from + 4);
+  }
+}
+
 // One element of the filter gradient by all threads of a block, pixels outside the image left out instead of multiplied by
 // zero; every thread gets the sum.
 template <typename T>
@@ -426,7 +612,7 @@ filter_reduce_kernel(FilterGradParams p, T* __restrict__ dw, int c, int splits, 
 #pragma unroll
       for (int r = 0; r < 3; ++r) v += *reinterpret_cast<const flex::f32x4*>(part[r][lane]);
       const int y0 = tap / p.kw * p.dil_h - p.pad_h, x0 = tap % p.kw * p.dil_w - p.pad_w;
-      if (y0 < 0 || x0 < 0 || y0 + (p.oh - 1) * p.stride_h >= p.h || x0 + (p.ow - 1) * p.stride_w >= p.w) {
+      if (p.spill || y0 < 0 || x0 < 0 || y0 + (p.oh - 1) * p.stride_h >= p.h || x0 + (p.ow - 1) * p.stride_w >= p.w) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) mask |= v[e] != v[e] && ch + e < c ? 1 << e : 0;
       }
@@ -551,6 +737,38 @@ bool Data(const ConvBackwardArgs& a, hipStream_t stream) {
   return true;
 }
 
+// Whether a filter gradient goes to conv_filter_taps_kernel, and its launch.  `tile_bytes`: what conv_filter_kernel's tiles
+// would take out of L2.  Both are bound by that, so the taps together take layers where they take a fifth less: conv_train
+// step, us, conv_filter_kernel | here, by the ratio of these bytes, fp16, 3x3 unless noted: 0.44 (64 -> 64 on 56x56, batch 32)
+// 133.3 | 120.1, 0.56 (64 -> 64 5x5 on 41x35, batch 8) 80.5 | 78.9, 0.61 (7x7, batch 4) 83.5 | 82.5, 0.71 (32 -> 32 on 60x60,
+// batch 8) 61.2 | 59.3, 0.74 (128 -> 128 on 28x28, batch 32) 94.5 | 89.8, 0.79 (256 -> 256 on 14x14) 87.0 | 85.6; 0.88 (512 ->
+// 512 on 7x7: two positions of nine are behind the row) 112.7 | 118.6, 0.93 (96 -> 200 on 41x35, batch 8) 93.6 | 94.0, 1.06
+// (16 -> 32 on 60x60) 57.6 | 57.7.
+template <typename T>
+bool PlanTaps(const ConvBackwardArgs& a, const FilterGradParams& p, int64_t plane, int64_t tile_bytes, TapsParams* t) {
+  if (sizeof(T) != 2 || a.stride_w != 1 || a.dil_w != 1 || a.kw < kTaps) return false;
+  t->g         = p;
+  t->g.tiles_m = (a.f + 63) / 64;
+  t->tiles_c   = (p.cp + 63) / 64;
+  t->groups    = (a.kw + kTaps - 1) / kTaps;
+  t->period    = a.ow + kTaps - 1;
+  t->rows      = a.n * a.oh;
+  t->g.steps   = (int)(((int64_t)t->rows * t->period + kFresh - 1) / kFresh);
+  const int64_t tiles = (int64_t)t->g.tiles_m * t->tiles_c * t->groups * a.kh;
+  if (tiles * t->g.steps * (64 + 64) * 128 * 5 > tile_bytes * 4) return false;
+  t->tiles  = (int)tiles;
+  t->adv_at = kFresh % t->period, t->adv_row = kFresh / t->period;
+  t->adv_oy = t->adv_row % a.oh, t->adv_n = t->adv_row / a.oh;
+  // One block per CU, at least four K steps each, at most 64 MiB of planes.  Two blocks per CU write and read twice the
+  // planes: the steps above 127.0, 84.4, 88.8, 65.7, 103.2 and 98.4 us.  (128 filters per block: 128 -> 128 91.9, 256 -> 256 89.1.)
+  int splits = std::max(1, std::min(256 / t->tiles, t->g.steps / 4));
+  splits     = (int)std::min<int64_t>(splits, std::max<int64_t>(1, ((int64_t)16 << 20) / plane));
+  t->lanes_log2 = splits >= 8 ? 3 : splits >= 4 ? 2 : splits >= 2 ? 1 : 0;
+  t->splits     = splits >> t->lanes_log2 << t->lanes_log2;
+  t->g.steps_per_split = (t->g.steps + t->splits - 1) / t->splits;
+  return true;
+}
+
 template <typename T>
 bool Filter(const ConvBackwardArgs& a, hipStream_t stream) {
   constexpr int E = 16 / (int)sizeof(T), KS = 8 * E;
@@ -584,6 +802,10 @@ bool Filter(const ConvBackwardArgs& a, hipStream_t stream) {
   splits     = (int)std::min<int64_t>(splits, std::max<int64_t>(1, ((int64_t)16 << 20) / plane));
   p.steps_per_split = (p.steps + splits - 1) / splits;
   splits            = (p.steps + p.steps_per_split - 1) / p.steps_per_split;
+  TapsParams t;
+  const bool taps = PlanTaps<T>(a, p, plane, (int64_t)tiles * p.steps * (bm + bn) * 128, &t);
+  if (taps) splits = t.splits;
+  p.spill = taps ? 1 : 0;
   const size_t plane_bytes = (size_t)splits * plane * sizeof(float);
   if (!HasZeroPage(stream) || dy_bytes + x_bytes > ScratchLimit(ScratchKind::kTranspose, stream) ||
       plane_bytes > ScratchLimit(ScratchKind::kSplitK, stream))
@@ -603,7 +825,10 @@ bool Filter(const ConvBackwardArgs& a, hipStream_t stream) {
   bool done = false;
   if constexpr (sizeof(T) == 2) {
     done = true;
-    if (bm == 128 && bn == 128) {
+    if (taps) {
+      t.g.dy = p.dy, t.g.x = p.x, t.g.planes = p.planes;
+      hipLaunchKernelGGL((conv_filter_taps_kernel<T>), dim3((unsigned)(t.tiles * t.splits)), dim3(512), 0, stream, t);
+    } else if (bm == 128 && bn == 128) {
       hipLaunchKernelGGL((conv_filter_kernel<T, 128, 128>), grid, dim3(256), 0, stream, p);
     } else if (bm == 128) {
       hipLaunchKernelGGL((conv_filter_kernel<T, 128, 64>), grid, dim3(256), 0, stream, p);
