@@ -427,7 +427,8 @@ Program FuseMatmulBias(const Program& program, const std::set<std::string>& fetc
     const Variable &x = mm->inputs[0], &w = mm->inputs[1], &prod = mm->outputs[0];
     if (x->shape.size() != 2 || w->shape.size() != 2 || prod->shape.size() != 2) continue;
     if (GetAttr<bool>(mm->attrs, "trans_a", false) || GetAttr<float>(mm->attrs, "alpha", 1.0f) != 1.0f) continue;
-    if (!(x->type.is_float16() || x->type.is_bfloat16()) || !(w->type == x->type)) continue;
+    const bool single = x->type == common::Float(32);
+    if (!(x->type.is_float16() || x->type.is_bfloat16() || single) || !(w->type == x->type)) continue;
     const bool trans_b = GetAttr<bool>(mm->attrs, "trans_b", false);
     const int m = x->shape[0], k = x->shape[1], n = w->shape[trans_b ? 0 : 1];
     if (w->shape[trans_b ? 1 : 0] != k || prod->shape != ShapeType{m, n}) continue;
@@ -458,13 +459,22 @@ Program FuseMatmulBias(const Program& program, const std::set<std::string>& fetc
     if (bias->shape != ShapeType{n}) continue;
     if (add->outputs[0]->shape != ShapeType{m, n} || !(add->outputs[0]->type == x->type)) continue;
     auto def = defined_at.find(bias->id);
-    if (!trans_b || !(bias->is_const || known.count(bias->id)) || (def != defined_at.end() && def->second > i)) {
-      // A layer in training: operands as they are, the bias converted in every run.  That launch costs what the pass over
-      // a small result does (2 to 3 us up to 4 MB; 14.8 us at 25 MB), so only large ones are taken.
-      if (static_cast<int64_t>(m) * n < (1 << 21) || static_cast<int64_t>(m) * n >= INT_MAX || n >= (1 << 22) || k >= (1 << 22)) continue;
+    if (single || !trans_b || !(bias->is_const || known.count(bias->id)) || (def != defined_at.end() && def->second > i)) {
+      // A layer in training: operands and bias as they are.
+      if (static_cast<int64_t>(m) * n >= INT_MAX || n >= (1 << 22) || k >= (1 << 22)) continue;
+      if (!(bias->type == x->type || bias->type == common::Float(32))) continue;
+      // In single precision the products with whole tiles have a kernel without a bias that is up to 6% ahead, and what
+      // reads the sum in the program is mostly a generated kernel that adds it on its way: only sums that are results.
+      if (single && users.count(add->outputs[0]->id)) continue;
       std::vector<Instruction> seq;
       Emitter e(&seq, "mmb" + std::to_string(serial++) + "_");
-      auto shift = bias->type == common::Float(32) ? bias : e.Emit1("cast", {bias}, {{"dtype", std::string("float32")}});
+      // A W stored [N][K] has the direct-to-LDS kernels' instances of the convolutions, which take an fp32 bias: converted in
+      // every run, a launch of 2 to 5 us that a small result's addition costs as well.
+      Variable shift = bias;
+      if (trans_b && !(bias->type == common::Float(32))) {
+        if (static_cast<int64_t>(m) * n < (1 << 21)) continue;
+        shift = e.Emit1("cast", {bias}, {{"dtype", std::string("float32")}});
+      }
       e.EmitInto(add->outputs[0], "hip_matmul_bias", {x, w, shift}, {{"trans_b", trans_b}});
       dropped[i] = dropped[add_at] = true;
       if (bcast_at >= 0) dropped[bcast_at] = true;

@@ -764,7 +764,7 @@ OpRegistry::OpRegistry() {
     }
   }
   {
-    // a [M][K] product with B [K][N] or, trans_b, [N][K] plus an fp32 bias [N], rounded once (FuseMatmulBias)
+    // a [M][K] product with B [K][N] or, trans_b, [N][K] plus a bias [N] of their type or fp32, rounded once (FuseMatmulBias)
     auto& op       = r->Register("hip_matmul_bias");
     op.pattern     = OpPatternKind::kNonFusible;
     op.num_inputs  = 3;

@@ -21,6 +21,7 @@ struct FlexGemm {
   int batch = 1;
   int64_t stride_a = 0, stride_b = 0, stride_c = 0;  // elements between batch entries; 0 shares the operand
   const float* shift    = nullptr;
+  const void* shift16   = nullptr;  // the shift in the matrices' 16-bit type
   const void* residual  = nullptr;  // of C's shape and batch stride
   float alpha           = 1.0f;
   float residual_scale  = 0.0f;

@@ -280,8 +280,8 @@ void cinn_call_hip_top_k(void* v_args, int num_args, int outer, int size, int in
 void cinn_call_hip_attention(void* v_args, int num_args, float scale, int batch, int heads, int queries, int keys,
                              int appended, int d, int operands, int layouts, int parts, void* stream);
 
-/* C [m][n] = A [m][k] op(B) + bias, one rounding; B is [k][n], or [n][k] with trans_b.  fp16 / bf16 with an fp32 bias [n];
- * n and k below 2^22.  v_args = {A, B, bias, C}, or {A, bias, C} where B is A. */
+/* C [m][n] = A [m][k] op(B) + bias, one rounding; B is [k][n], or [n][k] with trans_b.  fp16 / bf16 / fp32 with a bias [n]
+ * of the same type or fp32; n and k below 2^22.  v_args = {A, B, bias, C}, or {A, bias, C} where B is A. */
 void cinn_call_hip_matmul_bias(void* v_args, int num_args, int trans_b, int m, int n, int k, void* stream);
 
 /* A linear layer of at most 64 rows with what surrounds it: act(norm(x) [m][k] W^T * scale + shift + residual), W [n][k], fp16 or

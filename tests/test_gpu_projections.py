@@ -6,6 +6,8 @@ import pytest
 from cinn_amd.common import BFloat16, DefaultAMDGPUTarget, Float, bfloat16_bits_to_float32, float32_to_bfloat16_bits
 from cinn_amd.frontend import Computation, NetBuilder
 
+from helpers import run
+
 pytestmark = pytest.mark.gpu
 
 UNIT = {"float32": 2.0 ** -24, "float16": 2.0 ** -11, "bfloat16": 2.0 ** -8}
@@ -116,8 +118,7 @@ def test_residual_after_a_bias(gpu, m, k, n, dtype, first):
     assert np.all(np.abs(got - want) <= 1.01 * bound + 1e-7)
 
 
-# a layer in training: weights in either order that are no constants; results of at least 2^21 elements
-# (smaller ones keep the separate addition), k with and without whole chunks, few and many columns
+# a layer in training: weights in either order that are no constants; k with and without whole chunks, few and many columns
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
 @pytest.mark.parametrize("m,k,n", [(2048, 64, 1024), (2051, 768, 1030), (16400, 72, 128), (131, 200, 16384), (262144, 8, 8), (64, 256, 32768)])
 @pytest.mark.parametrize("trans_b", [False, True])
@@ -132,3 +133,43 @@ def test_bias_of_a_layer_in_training(gpu, m, k, n, dtype, trans_b):
     want = x64 @ w64 + c64
     bound = UNIT[dtype] * np.abs(want) + k * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64) + np.abs(c64))
     assert np.all(np.abs(got - want) <= 1.01 * bound + 1e-7)
+
+
+# the same with small results and ragged extents, in fp32 too, where K is split and where it is not; the bias has the
+# operands' type or fp32
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16", "float32"])
+@pytest.mark.parametrize("m,k,n", [(1, 1, 1), (5, 40, 9), (33, 64, 8), (64, 128, 40), (200, 90, 147), (130, 4100, 136), (256, 512, 512)])
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("wide_bias", [False, True])
+def test_bias_of_a_small_layer_in_training(gpu, m, k, n, dtype, trans_b, wide_bias):
+    import ctypes
+    from cinn_amd import _lib, runtime
+    from test_gpu_backward import from_dev, round_to, to_dev
+    rng = np.random.default_rng(m + k + n)
+    x, w = round_to(rng.standard_normal((m, k)), dtype), round_to(rng.standard_normal((n, k) if trans_b else (k, n)) * k ** -0.5, dtype)
+    c = round_to(rng.standard_normal(n), "float32" if wide_bias else dtype)
+    X, W, C, Y = to_dev(x, dtype), to_dev(w, dtype), to_dev(c, "float32" if wide_bias else dtype), to_dev(np.full((m, n), np.nan), dtype)
+    fn = _lib.load().cinn_call_hip_matmul_bias
+    fn.argtypes, fn.restype = [ctypes.c_void_p] + [ctypes.c_int] * 5 + [ctypes.c_void_p], None
+    fn(runtime.pod_args([X, W, C, Y]), 4, int(trans_b), m, n, k, None)
+    runtime.synchronize()
+    x64, w64 = x.astype(np.float64), (w.T if trans_b else w).astype(np.float64)
+    want  = x64 @ w64 + c
+    bound = UNIT[dtype] * np.abs(want) + k * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64) + np.abs(c))
+    assert np.all(np.abs(from_dev(Y, dtype) - want) <= 1.01 * bound + 1e-7)
+
+
+@pytest.mark.parametrize("read_again", [False, True])
+def test_bias_of_an_fp32_layer(gpu, read_again):
+    """a sum that is a result only comes out of the product; one that is read in the program stays an addition"""
+    rng = np.random.default_rng(1)
+    b = NetBuilder("fc")
+    x, w, c = (b.create_input(Float(32), s, e) for e, s in (("x", [70, 90]), ("w", [90, 50]), ("c", [50])))
+    y = b.add(b.matmul(x, w), c)
+    out = b.relu(y) if read_again else y
+    data = {v: rng.standard_normal(v.shape()).astype(np.float32) for v in (x, w, c)}
+    (got,), comp = run(b, data, [out])
+    names = [comp.instruction_info(i)[0] for i in range(comp.num_instructions())]
+    assert any("matmul_bias" in e for e in names) == (not read_again) and len(names) == 1 + read_again
+    want = data[x].astype(np.float64) @ data[w] + data[c]
+    np.testing.assert_allclose(got, np.maximum(want, 0) if read_again else want, rtol=1e-4, atol=1e-4)
