@@ -39,7 +39,7 @@ Program PretransposeConstMatmulWeights(const Program& program);
 // bias in fp32 as shift - a classifier's bias then costs no kernel of its own.  The sum is rounded once, from the
 // fp32 accumulator plus bias, where the two operators round the product first.
 // A [M][N] tensor that is added to that sum and nothing else is added as the epilogue's residual.  Operands of a layer
-// in training (W in either order, the bias not known before the run) make a hip_matmul_bias where the result is large.
+// in training (W in either order, the bias not known before the run) make a hip_matmul_bias.
 Program FuseMatmulBias(const Program& program, const std::set<std::string>& fetch_ids);
 // Two folded 1x1, stride 1, unpadded channels-last convolutions of which the second reads the first one's result
 // (the expansion that ends a ResNet bottleneck, with its shortcut and relu, and the reduction that starts the next):

@@ -133,6 +133,10 @@ __device__ __forceinline__ void AsyncCopy16Slot(const void* base_uniform, unsign
 
 constexpr int kD64BK   = 64;
 
+// The bias of a layer in training is read as it is stored.  A value of `relu` says so: one more argument, and a branch in the
+// instances with a B stored [N][K] as well, was 3 to 7 us of ResNet-50's 775 at batch 32.
+constexpr int kNarrowShift = 2;
+
 // epilogue operands of gemm16_dma_kernel: v = acc * (scale[col] or alpha) + shift[col] + residual_scale * R, relu
 struct DmaEpilogue {
   const float* scale;     // per output column, or null: alpha
@@ -140,7 +144,7 @@ struct DmaEpilogue {
   const void* residual;   // [M][N] like C (may be C itself: the beta term of a GEMM), or null
   float alpha;
   float residual_scale;
-  int relu;
+  int relu;               // 1: relu; kNarrowShift: none, and shift has the matrices' type (row-major B, no residual)
   int streaming;          // store the result with non-temporal stores (large outputs nobody re-reads from L2)
   // Split reduction: blockIdx.z = s takes the K steps [s * steps_per_split, (s + 1) * steps_per_split) and writes its
   // raw fp32 sums to partials[s][M][N]; the epilogue is applied by gemm16_split_reduce_kernel.  Null: no split.
@@ -150,7 +154,6 @@ struct DmaEpilogue {
   // probe + 8 * (linear block index) - the constant 100 MHz clock and the core clock counter at block start, after the
   // first operands have landed, after the K loop and after the last store was issued.  Null in normal use.
   unsigned long long* probe = nullptr;
-  const void* shift16;    // the shift in the matrices' type, or null (row-major B only: a layer in training)
 };
 
 // `first_wave` must be wavefront-uniform (a scalar branch: a lane-dependent one ahead of the direct-to-LDS loads makes
@@ -708,6 +711,8 @@ gemm16_dma_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B
   const T* Rt = reinterpret_cast<const T*>(epi.residual);
   if (Rt) Rt += (int64_t)blockIdx.y * stride_c;
   float sc[TN][4], sh[TN][4];
+  const bool narrow  = !B_KC && epi.relu == kNarrowShift;
+  const float* shift = narrow ? nullptr : epi.shift;
 #pragma unroll
   for (int j = 0; j < TN; ++j)
 #pragma unroll
@@ -715,17 +720,16 @@ gemm16_dma_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B
       int col  = n0 + wn * (TN * 16) + j * 16 + 4 * (lane >> 4) + r;
       col      = col < N ? col : N - 1;
       sc[j][r] = epi.scale ? epi.scale[col] : epi.alpha;
-      sh[j][r] = epi.shift ? epi.shift[col] : 0.0f;
+      sh[j][r] = shift ? shift[col] : 0.0f;
     }
-  // (as a choice for every column, in the instances that ResNet-50's layers use, it cost 7 us of 780 at batch 32)
   if constexpr (!B_KC) {
-    if (epi.shift16) {
+    if (narrow) {
 #pragma unroll
       for (int j = 0; j < TN; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int col = n0 + wn * (TN * 16) + j * 16 + 4 * (lane >> 4) + r;
-          sh[j][r]      = (float)reinterpret_cast<const T*>(epi.shift16)[col < N ? col : N - 1];
+          sh[j][r]      = (float)reinterpret_cast<const T*>(epi.shift)[col < N ? col : N - 1];
         }
     }
   }
@@ -761,7 +765,7 @@ gemm16_dma_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B
           }
       };
       if (!feeder) {
-        if (epi.relu) {
+        if (B_KC ? epi.relu != 0 : epi.relu == 1) {
           stage_pass(std::true_type{});
         } else {
           stage_pass(std::false_type{});
@@ -910,8 +914,11 @@ gemm16_shortk_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict_
   if (RES) Rt += (int64_t)blockIdx.y * stride_c;
   for (int i = tid; i < NW; i += 256) {
     s_scale[i] = epi.scale ? epi.scale[n0 + i] : epi.alpha;
-    s_shift[i] = epi.shift ? epi.shift[n0 + i] : 0.0f;
-    if (!B_KC && epi.shift16) s_shift[i] = (float)reinterpret_cast<const T*>(epi.shift16)[n0 + i];
+    if (!B_KC && epi.relu == kNarrowShift) {
+      s_shift[i] = (float)reinterpret_cast<const T*>(epi.shift)[n0 + i];
+    } else {
+      s_shift[i] = epi.shift ? epi.shift[n0 + i] : 0.0f;
+    }
   }
   const int frow = lane & 15;        // row of the fragment this lane reads
   const int fk   = (lane >> 4) * 8;  // its 8 elements of a 32-deep k block
@@ -1427,10 +1434,9 @@ void LaunchDma16(const GemmProblem& p, hipStream_t stream, int splits = 1) {
     epi.steps_per_split = ((p.k + kD64BK - 1) / kD64BK + splits - 1) / splits;
   }
   epi.scale          = p.scale;
-  epi.shift          = p.shift;
-  epi.shift16        = p.shift16;
+  epi.shift          = p.shift16 ? static_cast<const float*>(p.shift16) : p.shift;
   epi.alpha          = p.alpha;
-  epi.relu           = p.relu ? 1 : 0;
+  epi.relu           = p.shift16 ? kNarrowShift : (p.relu ? 1 : 0);
   epi.residual       = p.residual ? p.residual : (p.beta != 0.0f ? p.c : nullptr);
   epi.residual_scale = p.residual ? p.residual_scale : p.beta;
   // plain GEMMs whose result exceeds half of the L2 capacity (8 x 4 MiB) stream it out
@@ -1462,10 +1468,9 @@ void LaunchShortK(const GemmProblem& p, hipStream_t stream) {
   slots     = (slots + 7) / 8 * 8;
   DmaEpilogue epi;
   epi.scale          = p.scale;
-  epi.shift          = p.shift;
-  epi.shift16        = p.shift16;
+  epi.shift          = p.shift16 ? static_cast<const float*>(p.shift16) : p.shift;
   epi.alpha          = p.alpha;
-  epi.relu           = p.relu ? 1 : 0;
+  epi.relu           = p.shift16 ? kNarrowShift : (p.relu ? 1 : 0);
   epi.residual       = p.residual ? p.residual : (p.beta != 0.0f ? p.c : nullptr);
   epi.residual_scale = p.residual ? p.residual_scale : p.beta;
   epi.streaming      = !p.keep_in_cache && (int64_t)p.batch * p.m * p.n * 2 >= (16 << 20);
@@ -1477,7 +1482,7 @@ void LaunchShortK(const GemmProblem& p, hipStream_t stream) {
                      p.stride_c, ny)
 #define CINN_SHORTK(RES, B_KC)      \
   do {                              \
-    if (epi.relu) {                 \
+    if (epi.relu == 1) {            \
       CINN_SHORTK_R(RES, B_KC, true);  \
     } else {                        \
       CINN_SHORTK_R(RES, B_KC, false); \
@@ -1603,7 +1608,7 @@ bool TryDmaTransposedA(const GemmProblem& p, double flex_us, hipStream_t stream)
 // tile (the last tile row / column computes some rows / columns that are not stored); false when neither applies
 template <typename T>
 bool TryDma16(const GemmProblem& p, hipStream_t stream) {
-  if (p.shift16 && p.trans_b) return false;
+  if (p.shift16 && (p.trans_b || p.relu || p.residual || p.beta != 0.0f)) return false;
   if (TrySkinny(p, stream)) return true;
   if (p.trans_a || p.k % 64 != 0 || p.n % 8 != 0) return false;
   if (TryShortK<T>(p, stream)) return true;
