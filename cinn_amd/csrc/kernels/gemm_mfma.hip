@@ -1603,6 +1603,25 @@ bool TryDmaTransposedA(const GemmProblem& p, double flex_us, hipStream_t stream)
   return true;
 }
 
+// Into how many parts the K of a product on 64x64 tiles is split (at most one block per CU).  A block takes 4.9 us and 0.227
+// for every K step, the reduction 1.3 and 0.45 for every MB of partial sums.  us, whole | in two | in four, fp16: 96 x 768 x
+// 3072 15.7 | 12.6 | 9.8, 200 x 768 x 3072 15.8 | 12.8 | 10.7, 96 x 1280 x 5120 23.2 | 16.0 | 12.1, 96 x 384 x 1536 10.0 | 9.3
+// | 8.6; not 200 x 1280 x 1280 9.3 | 10.2, 800 x 384 x 1536 10.1 | 10.8; with more blocks than CUs 800 x 768 x 3072 16.0 | 16.4 | 20.0, 413 x 1280 x 5120 23.2 | 21.3 | 24.4.
+int Splits64(const GemmProblem& p, hipStream_t stream) {
+  const int64_t tiles = (int64_t)((p.m + 63) / 64) * ((p.n + 63) / 64);
+  const int steps     = p.k / kD64BK;
+  const double plane  = (double)p.m * p.n * 4e-6;  // MB
+  int best            = 1;
+  double best_us      = 4.9 + 0.227 * steps - 0.8;  // what the estimate may be wrong by
+  for (int s = 2; s <= 8 && tiles * s <= 256 && steps / s >= 4 && p.beta == 0.0f; ++s) {
+    const double us = 4.9 + 0.227 * ((steps + s - 1) / s) + 1.3 + 0.45 * plane * s;
+    if (us < best_us) best = s, best_us = us;
+  }
+  // under capture without an eager run or a reservation: K whole, which needs no scratch
+  if (best > 1 && (size_t)best * p.m * p.n * sizeof(float) > cinn_hip_kernels::ScratchLimit(cinn_hip_kernels::ScratchKind::kSplitK, stream)) best = 1;
+  return best;
+}
+
 // A stored [M][K], K % 64 == 0, N % 8 == 0 (whole 16-byte chunks per row of C and of a row-major B): 256x256 tiles
 // when they fill the chip, else 128x128 tiles when there are enough of those; M and N need not be multiples of the
 // tile (the last tile row / column computes some rows / columns that are not stored); false when neither applies
@@ -1649,9 +1668,10 @@ bool TryDma16(const GemmProblem& p, hipStream_t stream) {
   // 64x64 tiles of the convolution kernel with split K and its reduce kernel.  (3x3 layers measured slower here.)
   // From K = 1024 with up to 127 such tiles as well (1024 -> 256 1x1 on 14x14 at batch 32, 98 tiles: 9.8 against 12.7 us
   // on the register-staged 64x64 tiles and 10.5 us on 128x128 tiles with four stages).
+  // Fewer of them than half of the CUs: K split as far as the estimate says.
   const bool few_tiles_long_k = (tiles128 < 96 && p.k >= 2048) || (tiles128 < 128 && p.k >= 1024);
   if (p.trans_b && !p.conv && ((forced == 0 && FeedWavefronts() && few_tiles_long_k && p.batch == 1) || forced == 64)) {
-    LaunchDma16<T, true, 64, 64, 1, 1, false, 4, true>(p, stream);
+    LaunchDma16<T, true, 64, 64, 1, 1, false, 4, true>(p, stream, forced == 64 ? 1 : Splits64(p, stream));
     return true;
   }
   if (p.conv && p.conv->x2 != nullptr) {
@@ -1717,7 +1737,12 @@ bool TryDma16(const GemmProblem& p, hipStream_t stream) {
   // two K steps or fewer: a block is all start-up and epilogue, and two co-resident blocks of 128x128 overlap them
   // (128 -> 512 1x1 on 28x28 with its residual at batch 32: 20.4 against 21.3 us)
   const bool short_k = p.k <= 128 && tiles128 >= 128;
-  if (tiles256 >= 192 && forced != 128 && !wasteful256 && !(short_k && forced == 0)) {
+  // More 128x128 tiles than two blocks per CU hold take a second round, which one round of 256x256 tiles is ahead of.  us,
+  // 128x128 | 256x256, fp16: 8192 x 1280 x 1280 (640 tiles | 160) 38.1 | 30.9, 8192 x 1280 x 5120 125 | 90, 2300 x 3840 x 1280
+  // (540 | 135) 37.2 | 29.6, 4096 x 2304 x 768 (576 | 144) 25.2 | 21.7; within one round 1500 x 5120 x 1280 (480 | 120) 24.3 |
+  // 28.6, 2300 x 3072 x 768 (432 | 108) 17.3 | 20.6.
+  const bool one_round256 = tiles128 > 512 && tiles256 <= 256 && forced == 0 && p.batch == 1;
+  if (((tiles256 >= 192 && !wasteful256) || one_round256) && forced != 128 && !(short_k && forced == 0)) {
     if (p.trans_b) {
       LaunchDma16<T, true, 256, 256, 2, 4>(p, stream);
     } else {
@@ -1725,7 +1750,13 @@ bool TryDma16(const GemmProblem& p, hipStream_t stream) {
     }
     return true;
   }
-  if ((tiles128 >= 128 && forced != 256) || (forced == 128 && tiles128 > 0)) {
+  // (fewer than 128 of them in one round that takes 64x64 tiles more than one block per CU.  us, 64x64 tiles of gemm_flex.hip
+  // or of the convolution kernel | here, fp16: 413 x 3840 x 1280 (120 tiles of 128x128) 13.0 | 11.5, 1500 x 1280 x 1280 (120)
+  // 13.3 | 11.4, 800 x 1280 x 1280 (70) 12.1 | 10.7, 4096 x 384 x 1536 (96) 14.1 | 12.0, 413 x 3072 x 768 (96) 9.7 | 8.7, 200 x
+  // 5120 x 1280 (80) 12.1 | 10.8; 4096 x 384 x 384 (96) 7.0 | 7.4, 800 x 1280 x 5120 (70), split by the former, 27.4 | 32.4)
+  const int64_t tiles64 = (int64_t)((p.m + 63) / 64) * ((p.n + 63) / 64) * p.batch;
+  const bool one_round128 = tiles64 > 256 && tiles128 <= 256 && p.k >= 768 && (tiles128 >= 96 || p.k <= 3072) && p.batch == 1;
+  if (((tiles128 >= 128 || one_round128) && forced != 256) || (forced == 128 && tiles128 > 0)) {
     if (stages == 4 && FeedWavefronts()) {
       if (p.trans_b) {
         LaunchDma16<T, true, 128, 128, 2, 2, false, 4, true>(p, stream);
@@ -1921,10 +1952,13 @@ bool TryPointwiseConvAsGemm(const ConvNhwcArgs& a, hipStream_t stream) {
     // few tiles but a long reduction: the single-wavefront 64x64 tiles of the GEMM kernel (see TryDma16)
     const bool long_k = forced_tile == 64 || (forced_tile == 0 && a.oc % 64 == 0 &&
                                               (a.c >= 2048 || (a.c >= 1024 && ((pixels + 127) / 128) * ((a.oc + 127) / 128) < 128)));
+    // more 64x64 tiles than CUs and 128x128 tiles for one block on most of them, K long enough (see TryDma16; 800 x 3072 x 768
+    // 13.2 | 9.6 us, 413 x 5120 x 1280 20.8 | 11.9, 2300 x 1280 x 1280 18.9 | 12.7)
+    const int64_t tiles64 = ((pixels + 63) / 64) * ((a.oc + 63) / 64), tiles128 = ((pixels + 127) / 128) * ((a.oc + 127) / 128);
+    const bool one_round128 = forced_tile == 0 && a.c % 64 == 0 && tiles64 > 256 && tiles128 < 192 && (a.c >= 768 || (a.c >= 384 && tiles128 >= 128));
     // at most 64 pixels (a matmul with few rows written as a 1x1 layer, its bias as the shift): gemm_rows.hip
     const bool few_rows = forced_tile == 0 && pixels <= 64 && a.c % 32 == 0;
-    if (mode != 2 && !shortk && !long_k && !few_rows &&
-        (a.c < 128 || (!narrow && ((pixels + 127) / 128) * ((a.oc + 127) / 128) < 192)))
+    if (mode != 2 && !shortk && !long_k && !few_rows && !one_round128 && (a.c < 128 || (!narrow && tiles128 < 192)))
       return false;
     p.k = a.c;
   } else {
