@@ -263,6 +263,7 @@ LoweringOptions LoweringOptions::FromEnv() {
   LoweringOptions o;
   o.max_cached_elems_per_thread = EnvInt("FLAGS_cinn_hip_reduce_cached_elems", o.max_cached_elems_per_thread);
   o.wave_row_elems_per_lane     = EnvInt("FLAGS_cinn_hip_reduce_wave_elems", o.wave_row_elems_per_lane);
+  o.block_row_reductions        = EnvInt("FLAGS_cinn_hip_reduce_block_reductions", o.block_row_reductions);
   o.block_row_elems_per_thread  = EnvInt("FLAGS_cinn_hip_reduce_block_elems", o.block_row_elems_per_thread);
   o.nontemporal_store_bytes     = static_cast<int64_t>(EnvInt("FLAGS_cinn_hip_nontemporal_store_mb", 8)) << 20;
   o.nontemporal_load_bytes      = static_cast<int64_t>(EnvInt("FLAGS_cinn_hip_nontemporal_load_mb", 0)) << 20;
@@ -1039,22 +1040,27 @@ ir::LoweredFuncRef OpLowerer::LowerRowReduce(const Group& group, bool merged_mem
   CINN_CHECK_EQ(wave, 64) << "the row-reduce template is written for 64-lane wavefronts";
   int64_t per_lane       = (plan.cols + wave - 1) / wave;
   const int64_t row_vecs = (plan.cols + plan.vec - 1) / plan.vec;
+  int reductions         = 0;
+  for (auto* n : group.nodes) reductions += n->op->pattern == OpPatternKind::kReduction ? 1 : 0;
+  const bool few_rows = plan.rows <= target_.get_multi_processor_count(), whole_vec = plan.vec * min_bytes >= 16;
+  const bool shared_row = options_.block_row_reductions > 0 && reductions >= options_.block_row_reductions &&
+                          per_lane > 32 && (min_bytes >= 4 || few_rows);
   if (options_.sub_wave_rows && row_vecs <= wave / 2) {
     // short rows: a team of the fewest lanes that hold the row with one vector each, 64 / team rows per wavefront
     int team = 1;
     while (team < row_vecs) team *= 2;
     plan.team           = team;
     plan.rows_per_block = 256 / team;
-  } else if (per_lane <= options_.wave_row_elems_per_lane) {
+  } else if (per_lane <= options_.wave_row_elems_per_lane && !shared_row) {
     plan.team           = wave;
     plan.rows_per_block = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(options_.rows_per_block, plan.rows)));
   } else {
     // whole block per row: the smallest power-of-two block (up to 1024 threads) that keeps the row
     // within the register budget
-    int team = 128;
-    while (team < target_.max_num_threads() && (plan.cols + team - 1) / team > options_.block_row_elems_per_thread) {
-      team *= 2;
-    }
+    int team          = 128;
+    const int largest = shared_row ? 512 : target_.max_num_threads();
+    const int elems   = shared_row && (few_rows || !whole_vec) ? 8 : options_.block_row_elems_per_thread;
+    while (team < largest && (plan.cols + team - 1) / team > elems) team *= 2;
     plan.team           = team;
     plan.rows_per_block = 1;
   }
