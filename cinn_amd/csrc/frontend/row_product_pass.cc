@@ -192,6 +192,12 @@ class RowProductFuser {
     if (conv->inputs.size() < 4 || conv->inputs.size() > 5 || conv->outputs.size() != 1 || GetAttr<bool>(conv->attrs, "relu", false) ||
         GetAttr<bool>(conv->attrs, "max_pool", false) || GetAttr<std::string>(conv->attrs, "data_format", "") != "NHWC")
       return;
+    // a 1x1 filter may still look beside the one pixel (padding, and a stride that leaves one output)
+    if (GetAttr<std::vector<int>>(conv->attrs, "stride", {1, 1}) != std::vector<int>{1, 1} ||
+        GetAttr<std::vector<int>>(conv->attrs, "padding", {0, 0}) != std::vector<int>{0, 0} ||
+        GetAttr<std::vector<int>>(conv->attrs, "dilation", {1, 1}) != std::vector<int>{1, 1} ||
+        GetAttr<int>(conv->attrs, "groups", 1) != 1 || GetAttr<std::string>(conv->attrs, "input_layout", "NHWC") != "NHWC")
+      return;
     // the layer's operands seen as 1x1 images
     auto matrix = [&](const Variable& image) -> const Variable* {
       const Instruction* def = Source(image, "reshape");

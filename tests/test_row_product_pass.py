@@ -1,0 +1,55 @@
+"""Which layers FuseRowProducts takes: names of the calls of compiled programs (no GPU needed), and values."""
+import numpy as np
+import pytest
+
+from cinn_amd.common import Float
+from cinn_amd.frontend import NetBuilder
+
+from helpers import compile_only, run
+
+M, K, N = 8, 64, 32
+
+
+def names(comp):
+    return [comp.instruction_info(i)[0] for i in range(comp.num_instructions())]
+
+
+def pointwise_layer(geometry, pixels=1):
+    """a folded 1x1 convolution and batch norm on images of one pixel, seen as a matrix before and behind it, and gelu"""
+    b, rng, data = NetBuilder("pointwise"), np.random.default_rng(3), {}
+
+    def put(name, shape, low=-1.0, const=True):
+        data[name] = rng.uniform(low, 1.0, shape).astype(np.float16)
+        v = b.create_input(Float(16), list(shape), name)
+        v.set_const(const)
+        return v
+
+    x, w = put("x", (M, K), const=False), put("w", (N, K))
+    z = b.conv2d(b.reshape(x, [M, 1, 1, K]), b.reshape(w, [N, 1, 1, K]), data_format="NHWC", **geometry)
+    norm = b.batchnorm(z, put("g", (N,)), put("b", (N,)), put("m", (N,)), put("v", (N,), 0.5), data_layout="NHWC")[0]
+    return b, b.gelu(b.reshape(norm, [M, N])), data
+
+
+GEOMETRIES = [dict(), dict(strides=[3, 3], paddings=[1, 1])]  # the latter's one output pixel sees padding alone
+
+
+@pytest.mark.parametrize("geometry", GEOMETRIES)
+def test_pointwise_layer_is_a_product_only_where_it_sees_its_pixel(geometry):
+    b, y, _ = pointwise_layer(geometry)
+    assert any("matmul_rows" in e for e in names(compile_only(b, [y]))) == (geometry == {})
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("geometry", GEOMETRIES)
+def test_pointwise_layer_values(gpu, geometry):
+    from scipy.special import erf
+    b, y, data = pointwise_layer(geometry)
+    (got,), _ = run(b, data, [y])
+    d = {e: v.astype(np.float64) for e, v in data.items()}
+    product = d["x"] @ d["w"].T if geometry == {} else np.zeros((M, N))
+    scale = d["g"] / np.sqrt(d["v"] + 1e-5)
+    want = product * scale + d["b"] - d["m"] * scale
+    want = want * 0.5 * (1 + erf(want / np.sqrt(2)))
+    # 64 terms in fp32, results rounded to fp16 once behind the product and once behind gelu (|gelu'| < 1.13)
+    size = np.abs(product * scale) + np.abs(d["b"]) + np.abs(d["m"] * scale)
+    assert np.all(np.abs(got - want) <= 2.2 * 2.0 ** -11 * size + 2.0 ** -24)
