@@ -747,6 +747,8 @@ bool Data(const ConvBackwardArgs& a, hipStream_t stream) {
 template <typename T>
 bool PlanTaps(const ConvBackwardArgs& a, const FilterGradParams& p, int64_t plane, int64_t tile_bytes, TapsParams* t) {
   if (sizeof(T) != 2 || a.stride_w != 1 || a.dil_w != 1 || a.kw < kTaps) return false;
+  // positions in a row are multiplied as signed 24-bit numbers (__mul24); channels are below 2^20
+  if (std::max(a.ow, a.w_in) > (1 << 23)) return false;
   t->g         = p;
   t->g.tiles_m = (a.f + 63) / 64;
   t->tiles_c   = (p.cp + 63) / 64;

@@ -43,3 +43,25 @@ def test_filter_gradient(gpu, case, dtype, fmt):
     runtime.synchronize()
     want, scale = (ob.conv2d_backward_filter(q, r, w.shape, (s, s), (p, p), (d, d), g) for q, r in ((x, dy), (np.abs(x), np.abs(dy))))
     assert np.all(np.abs(unlayout(from_dev(DW, dtype), fmt) - want) <= bound(want, scale, dy.size / f, dtype))
+
+
+def test_row_longer_than_24_bits(gpu):
+    """one row of more than 2^23 pixels (fp16, channels last, 1x3): its last pixels and a few of its first, the others zero"""
+    n, c, w_ = 1, 24, (1 << 23) + 9
+    rng = np.random.default_rng(0)
+    x, dy = (np.zeros((w_, c), np.float16) for _ in range(2))
+    at = np.r_[0:8, w_ - 24:w_]
+    for t in (x, dy):
+        t[at] = rng.standard_normal((len(at), c))
+    dims = (n, c, 1, w_, c, c, 1, 3, 0, 1, 1, 1, 1, 1, 1, n, c, 1, w_)
+    lib = _lib.load()
+    lib.cinn_call_cudnn_conv2d_backward_filter.argtypes = CONV_ARGTYPES
+    X, DY = (to_dev(t.reshape(n, 1, w_, c), "float16") for t in (x, dy))
+    DW = to_dev(np.full((c, 1, 3, c), np.nan, np.float16), "float16")
+    lib.cinn_call_cudnn_conv2d_backward_filter(runtime.pod_args([X, DY, DW]), 3, 1, 1.0, 0.0, *dims, None)
+    runtime.synchronize()
+    got = from_dev(DW, "float16")
+    for tap in range(3):
+        rows = at[(at + tap - 1 >= 0) & (at + tap - 1 < w_)]
+        a, b = dy[rows].astype(np.float64), x[rows + tap - 1].astype(np.float64)
+        assert np.all(np.abs(got[:, 0, tap] - a.T @ b) <= bound(a.T @ b, np.abs(a).T @ np.abs(b), len(at), "float16"))
