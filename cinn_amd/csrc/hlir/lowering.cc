@@ -1043,8 +1043,9 @@ ir::LoweredFuncRef OpLowerer::LowerRowReduce(const Group& group, bool merged_mem
   int reductions         = 0;
   for (auto* n : group.nodes) reductions += n->op->pattern == OpPatternKind::kReduction ? 1 : 0;
   const bool few_rows = plan.rows <= target_.get_multi_processor_count(), whole_vec = plan.vec * min_bytes >= 16;
+  // (longer rows have a block in any case, of as many threads as keep them in registers)
   const bool shared_row = options_.block_row_reductions > 0 && reductions >= options_.block_row_reductions &&
-                          per_lane > 32 && (min_bytes >= 4 || few_rows);
+                          per_lane > 32 && per_lane <= options_.wave_row_elems_per_lane && (min_bytes >= 4 || few_rows);
   if (options_.sub_wave_rows && row_vecs <= wave / 2) {
     // short rows: a team of the fewest lanes that hold the row with one vector each, 64 / team rows per wavefront
     int team = 1;
@@ -1057,10 +1058,9 @@ ir::LoweredFuncRef OpLowerer::LowerRowReduce(const Group& group, bool merged_mem
   } else {
     // whole block per row: the smallest power-of-two block (up to 1024 threads) that keeps the row
     // within the register budget
-    int team          = 128;
-    const int largest = shared_row ? 512 : target_.max_num_threads();
-    const int elems   = shared_row && (few_rows || !whole_vec) ? 8 : options_.block_row_elems_per_thread;
-    while (team < largest && (plan.cols + team - 1) / team > elems) team *= 2;
+    int team        = 128;
+    const int elems = shared_row && (few_rows || !whole_vec) ? 8 : options_.block_row_elems_per_thread;
+    while (team < target_.max_num_threads() && (plan.cols + team - 1) / team > elems) team *= 2;
     plan.team           = team;
     plan.rows_per_block = 1;
   }

@@ -35,7 +35,9 @@ struct LoweringOptions {
   // layer norm, sum and argmax of one tensor, us, a wavefront | a block per row, fp32: 4096 x 4096 33.9 | 32.2, 4000 x 2600
   // 30.4 | 22.4, 4000 x 2601 44.6 | 27.6, 1170 x 3545 18.3 | 14.2, 300 x 3000 9.1 | 6.4, 60 x 3904 10.6 | 5.0; fp16 250 x 2050
   // 12.9 | 7.2, 100 x 4000 9.9 | 7.3, but 4000 x 2600 16.2 | 19.4.  Shorter rows: 5000 x 1538 29.4 | 19.5, but 9000 x 1161 25.8 |
-  // 29.5, 5000 x 2047 28.1 | 29.4.  0: as the limits above say.
+  // 29.5, 5000 x 2047 28.1 | 29.4.  Rows that have a block by the limits above keep it: softmax, sum and argmax, blocks of 512 |
+  // 1024 threads, 64 x 32769 21.3 | 9.6, 512 x 32769 40.5 | 23.9, 1 x 50257 40.0 | 10.2, 512 x 50257 81 | 52 (registers hold 64
+  // elements per thread).  0: as the limits above say.
   int block_row_reductions{3};
   // outputs of at least this many bytes are written with non-temporal stores (0 disables): a large
   // streamed output would otherwise evict the input rows still to be read from the last-level cache
