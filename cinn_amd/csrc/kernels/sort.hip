@@ -596,11 +596,22 @@ void LaunchRowSelect(const RowParams& p, int rows, hipStream_t stream) {
 #undef CINN_ROW_SELECT_C
 }
 
-// Up to which k the selection is ahead of the network.  us, network | selection, fp32: 2048 rows of 1000, k = 17 21.1 | 9.2,
-// k = 32 21.1 | 12.0, k = 50 21.2 | 18.9; 600 rows of 1500, k = 50 41.2 | 20.1, k = 64 41.2 | 59 (with as many elements as
-// lanes the bound is the largest of the lanes' least words, and most rows are taken one by one); 64 rows of 8000 fp16, k = 50
-// 77.9 | 28.4.  The network of 256 words on one wavefront is short: 4000 rows of 250, k = 17 9.5, k = 50 9.7 | 17.0.
-int SelectLimit(int size) { return size <= 256 ? 16 : 50; }
+// Up to which k the selection is ahead of the network.  The network's time is the blocks per CU (four wavefronts for 257 to
+// 1024 words, sixteen above), the selection's the chain of one wavefront, which grows with k and with the words up to the bound.
+// us, network | selection, fp32: up to 256 rows of 400, k = 24 8.9 | 7.4, k = 32 8.9 | 8.9, k = 50 8.9 | 14; of 1000, k = 20 9.1 | 8.3, k =
+// 24 9.1 | 8.9, k = 50 9.1 | 16.4; 600 rows of 1000, k = 32 11.7 | 10.7; 1024 of 400, k = 40 13.8 | 12.1, k = 50 13.2 | 15.2; 1500 of 400, k = 50
+// 17.8 | 16.1; 2048 of 1000, k = 50 22.6 | 18.3.  (Where many scores are equal, rounded to halves, the selection takes a seventh more:
+// 256 rows of 1000, k = 24 9.1 | 10.2, 1500, k = 50 18.4 | 20.8.)  64 rows of 1500, k = 50 18.4 | 16.1, of 4000 18.9 | 18.6 (with equal
+// ones 18.9 | 19.9); 64 rows of 8000 fp16, k = 50 77.9 | 28.4; k = 64 of 600 rows of 1500 41.2 | 59 (with as many elements as lanes the
+// bound is the largest of the lanes' least words, and most rows are taken one by one).  The network of 256 words on one wavefront
+// is short: 4000 rows of 250, k = 17 9.5, k = 50 9.7 | 17.0.
+int SelectLimit(int size, int rows) {
+  if (size <= 256) return 16;
+  const int per_cu = (rows + 255) / 256;  // the network's blocks
+  if (size > 1024 || per_cu >= 8) return 50;
+  static const int kWide[8] = {0, 20, 24, 32, 32, 40, 40, 40}, kNarrow[8] = {0, 24, 32, 32, 40, 40, 50, 50};
+  return size <= 768 ? kNarrow[per_cu] : kWide[per_cu];
+}
 
 enum class Elem { kF32, kF64, kF16, kBF16, kI32, kI64, kUnsupported };
 
@@ -752,7 +763,7 @@ extern "C" void cinn_call_hip_top_k(void* v_args, int num_args, int outer, int s
     LaunchTiles(p, elem, outer, s);
     return;
   }
-  auto run = [&](auto launch_select, auto launch_sort) { k <= SelectLimit(size) ? launch_select(r, outer * inner, s) : launch_sort(r, outer * inner, s); };
+  auto run = [&](auto launch_select, auto launch_sort) { k <= SelectLimit(size, outer * inner) ? launch_select(r, outer * inner, s) : launch_sort(r, outer * inner, s); };
   switch (elem) {
     case Elem::kF32: run(LaunchRowSelect<float>, LaunchRowSort<float>); break;
     case Elem::kF16: run(LaunchRowSelect<_Float16>, LaunchRowSort<_Float16>); break;

@@ -119,6 +119,23 @@ def test_top_k_of_distinct_scores_and_equal_ones(gpu, size, k, equal):
     assert np.array_equal(where, index) and np.array_equal(values, np.take_along_axis(x, index, 1))
 
 
+# rows of up to 1024 elements go to the selection or to the network by their number, for k from 21 to 50
+@pytest.mark.parametrize("equal", ["distinct", "few values", "one value"])
+@pytest.mark.parametrize("rows,k", [(256, 20), (256, 24), (257, 25), (512, 32), (513, 33), (1024, 40), (1281, 41), (1792, 50), (1793, 50), (1793, 51), (600, 1)])
+@pytest.mark.parametrize("size", [257, 1000])
+def test_top_k_of_many_rows(gpu, size, rows, k, equal):
+    rng = np.random.default_rng(size + rows + k)
+    if equal == "distinct":
+        x = rng.permuted(np.tile(np.arange(size, dtype=np.float32), (rows, 1)), axis=1)
+    else:
+        x = rng.integers(0, 9 if equal == "few values" else 1, (rows, size)).astype(np.float32)
+    b = NetBuilder("top")
+    v = b.create_input(Float(32), list(x.shape), "x")
+    (values, where), _ = run(b, {v: x}, list(b.top_k(v, k, 1)))
+    index = np.argsort(-x, axis=1, kind="stable")[:, :k]
+    assert np.array_equal(where, index) and np.array_equal(values, np.take_along_axis(x, index, 1))
+
+
 def test_top_k_of_one_output_or_shared_results(gpu):
     """only the values or only the indices are wanted; a full sort that something else reads stays"""
     rng = np.random.default_rng(1)
