@@ -221,8 +221,11 @@ class RowProductFuser {
     size_t last              = static_cast<size_t>(back);
 
     Norm norm;
-    const bool normalised = k <= cinn_hip_kernels::kRowProductMaxNormK && OnlyReader(x4) >= 0 && MatchNorm(x, &norm);
-    if (normalised) {
+    const int reader = OnlyReader(y);
+    cinn_hip_kernels::RowFusion fuse{k <= cinn_hip_kernels::kRowProductMaxNormK && OnlyReader(x4) >= 0 && MatchNorm(x, &norm),
+                                     reader >= 0 && instrs_[reader]->op_type == "gelu" && !dropped_[reader]};
+    fuse = cinn_hip_kernels::ChooseRowFusion(m, n, k, fuse);
+    if (fuse.norm) {
       call->inputs[0] = norm.x;
       call->inputs.push_back(norm.gamma);
       call->inputs.push_back(norm.beta);
@@ -230,17 +233,15 @@ class RowProductFuser {
     }
     for (size_t j : {size_t(0), size_t(1), size_t(4)})  // the views as images
       if (j < conv->inputs.size() && OnlyReader(conv->inputs[j]) >= 0) drop.push_back(defined_at_.at(conv->inputs[j]->id));
-    const int reader = OnlyReader(y);
-    const bool gelu  = reader >= 0 && instrs_[reader]->op_type == "gelu" && !dropped_[reader];
     std::vector<size_t> columns;
-    if (gelu) {
+    if (fuse.gelu) {
       y    = instrs_[reader]->outputs[0];
       last = static_cast<size_t>(reader);
       drop.push_back(last);
     } else if (!residual) {
       columns = Columns(y);
     }
-    if (!normalised && !gelu && columns.empty() && !plain) return;
+    if (!fuse.norm && !fuse.gelu && !((plain || !columns.empty()) && cinn_hip_kernels::RowProductPays(m, n, k, !columns.empty()))) return;
     if (columns.empty()) {
       call->outputs = {y};
     } else {
@@ -251,7 +252,7 @@ class RowProductFuser {
         drop.push_back(c);
       }
     }
-    call->attrs = {{"residual", residual != nullptr}, {"norm", normalised}, {"gelu", gelu}, {"epsilon", normalised ? norm.epsilon : 0.0f}};
+    call->attrs = {{"residual", residual != nullptr}, {"norm", fuse.norm}, {"gelu", fuse.gelu}, {"epsilon", fuse.norm ? norm.epsilon : 0.0f}};
     for (size_t d : drop) dropped_[d] = true;
     replacement_.emplace(last, call);
     for (auto& o : call->outputs) TransposesToReshapes(o);

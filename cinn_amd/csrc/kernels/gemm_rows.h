@@ -32,6 +32,14 @@ constexpr int kRowProductMaxNormK = 1280;
 
 // false where the kernel does not take the extents or alignments
 bool RowProductSupported(const RowProduct& p);
+// whether the kernel is ahead of the tiled ones for a product that it takes; `saves_launch`: several results, which would
+// be copied out of one
+bool RowProductPays(int m, int n, int k, bool saves_launch);
+// which of a layer norm before the product and a gelu behind it (those that there are) are faster inside
+struct RowFusion {
+  bool norm, gelu;
+};
+RowFusion ChooseRowFusion(int m, int n, int k, RowFusion there);
 void RunRowProduct(const RowProduct& p, hipStream_t stream);
 
 }  // namespace cinn_hip_kernels

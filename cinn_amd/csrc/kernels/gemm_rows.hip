@@ -5,8 +5,8 @@
 // here a block owns 16 output columns of MT row tiles (rows from 16 MT blockIdx.y: the launcher gives every row tile a block
 // of its own where that still leaves CUs) and its eight wavefronts split K in 32-deep blocks.  A lane's share
 // of a 16x16x32 fragment is 8 consecutive k of one row - 16 contiguous bytes in both operands - so fragments come straight
-// from global memory, no LDS on the way: every wavefront keeps 2 U k-blocks of loads in flight, B is read exactly once from
-// memory, A (at most 64 rows) comes out of L2.  The partial tiles meet in LDS; wavefront t finishes row tile t (2-byte
+// from global memory, no LDS on the way: every wavefront keeps 2 U k-blocks of loads in flight, B is read from memory once (by
+// a block of all rows, or by one per row tile of which the others find it in L2), A (at most 64 rows) comes out of L2.  The partial tiles meet in LDS; wavefront t finishes row tile t (2-byte
 // stores: the result is small).
 //
 // At these sizes a launch costs as much as the product (an empty kernel 3.3 us from launch to launch, 8 x 768 -> 768 5 us),
@@ -217,6 +217,40 @@ bool RowProductSupported(const RowProduct& p) {
   if (p.width < 1 || p.n % p.width != 0 || p.n / p.width > 3 || (p.n > p.width && p.residual)) return false;
   if (p.gamma && (!p.beta || p.k > kRowProductMaxNormK || !Aligned(p.gamma) || !Aligned(p.beta))) return false;
   return Aligned(p.a) && Aligned(p.b);
+}
+
+// Every wavefront waits for its own rows of B: with one block per CU (16 columns each; 16 rows, or all of them from 256 blocks of
+// columns on) that hides the launch, further ones take about as long again, where the tiled kernels need a few hundred tiles for
+// the same result.  us, tiled | here, fp16, at most as many blocks as CUs: 16 x 192 -> 4096 3.9 | 3.8, 64 x 960 -> 1000 7.3 | 4.3, two row
+// tiles in each 32 x 192 -> 4096 4.0 | 4.6, 32 x 384 -> 4096 4.7 | 4.6; two on a CU: 1 x 384 -> 8192 4.7 | 3.7, 16 x 384 -> 8192 4.8 | 5.2, 16 x 960 ->
+// 8192 7.1 | 6.1, 48 x 960 -> 4096 (three row tiles) 7.3 | 6.3; three: 1 x 1984 -> 12288 12.4 | 11.5, 48 x 960 -> 3072 7.3 | 9.0, 32 x 960 -> 8192
+// 7.2 | 8.0; more: 64 x 192 -> 8192 4.3 | 10.7.  Where K is no multiple of 64 the tiled kernel is the register-staged one: 1 x 1120 -> 16384 10.4 |
+// 8.2, 32 x 224 -> 3072 4.9 | 4.2, 64 x 224 -> 4096 5.2 | 4.8, 32 x 544 -> 8192 6.6 | 4.9, but 32 x 2080 -> 8192 13.0 | 13.5, 48 x 224 -> 3072 5.1 | 6.1.
+// K in whole shares of all wavefronts has always come here.
+bool RowProductPays(int m, int n, int k, bool saves_launch) {
+  if (k % 256 == 0) return true;
+  const int columns = (n + 15) / 16, tiles = (m + 15) / 16;
+  const double load = columns < 256 ? (columns * tiles + 255) / 256 : (columns + 255) / 256 * (0.5 + 0.5 * tiles);
+  if (saves_launch && load <= 3.0) return true;
+  if (k % 64 != 0) return load <= (m <= 4 ? 4.0 : 2.5) || (load <= 3.0 && (k <= 128 || k > 256) && k < 1536);
+  if (m <= 4) return load <= (k < 512 ? 2.0 : 3.0);
+  return load <= (k < 256 ? 1.0 : k < 512 ? 1.5 : 2.0);
+}
+
+// Blocks of one row tile each: B is read for every one of them, and each normalises its rows again, so that the second and third
+// round of blocks cost what a kernel of their own does - unless the product alone would be blocks of one row tile as well.  us,
+// separate | inside, fp16, norm: one round 32 x 320 -> 2048 6.7 | 5.7, 64 x 960 -> 1024 10.0 | 6.1; two 32 x 384 -> 4096 7.0 | 8.5, 16 x 960 -> 8192
+// 9.8 | 9.0; three 48 x 960 -> 4096 10.0 | 12.3, 48 x 1280 -> 4096 13.0 | 12.6; more 48 x 384 -> 6272 7.3 | 18.6, 64 x 1280 -> 4096 14.9 | 16.1; the
+// same blocks alone 64 x 768 -> 3072 12.7 | 12.1, 48 x 512 -> 3072 10.8 | 11.8.  gelu: two rounds 16 x 384 -> 8192 7.6 | 5.6, three 64 x 192 -> 3072
+// 7.1 | 8.5, four 64 x 960 -> 4096 10.3 | 10.6, 64 x 960 -> 8192 10.8 | 20.6; the same blocks alone 64 x 768 -> 3072 12.6 | 10.3.  Both: one round
+// 64 x 320 -> 1024 9.9 | 6.2, two 16 x 128 -> 8192 8.3 | 8.9, 48 x 192 -> 2048 9.2 | 8.9, three 64 x 320 -> 3072 10.0 | 12.6, six 64 x 1280 -> 6144 28.1 |
+// 24.9, eight 64 x 1280 -> 8192 28.9 | 32.6, four 64 x 768 -> 4096 13.0 | 16.9; the same blocks alone 64 x 768 -> 3072 15.5 | 13.1.
+RowFusion ChooseRowFusion(int m, int n, int k, RowFusion there) {
+  const int rounds = ((n + 15) / 16 * ((m + 15) / 16) + 255) / 256;
+  const bool same  = k % 256 == 0 && n <= 4080;  // the blocks of the product alone
+  if (there.norm && there.gelu && (same || rounds <= 1 || (rounds <= 2 && k >= 192) || (rounds <= 6 && k >= 1152))) return there;
+  if (there.gelu && (same || rounds <= 2)) return {false, true};
+  return {there.norm && (rounds <= 1 || (same && k >= 768) || (rounds <= 2 && k >= 896) || (rounds <= 3 && k >= 1152)), false};
 }
 
 void RunRowProduct(const RowProduct& p, hipStream_t stream) {

@@ -53,3 +53,34 @@ def test_pointwise_layer_values(gpu, geometry):
     # 64 terms in fp32, results rounded to fp16 once behind the product and once behind gelu (|gelu'| < 1.13)
     size = np.abs(product * scale) + np.abs(d["b"]) + np.abs(d["m"] * scale)
     assert np.all(np.abs(got - want) <= 2.2 * 2.0 ** -11 * size + 2.0 ** -24)
+
+
+def linear_layer(m, k, n, norm, gelu):
+    b = NetBuilder("linear")
+
+    def put(name, shape, const=True):
+        v = b.create_input(Float(16), list(shape), name)
+        v.set_const(const)
+        return v
+
+    x = put("x", (m, k), False)
+    if norm:
+        x = b.paddle_layer_norm(x, put("g", (k,)), put("s", (k,)))[0]
+    y = b.add(b.matmul(x, put("w", (k, n))), put("c", (n,)))
+    return b, b.gelu(y) if gelu else y
+
+
+# one round of blocks (16 columns x 16 rows) takes everything along, several only what is faster inside
+@pytest.mark.parametrize("m,k,n,norm,gelu,calls", [
+    (8, 768, 3072, True, True, 1), (16, 384, 4096, True, False, 1), (64, 320, 1024, True, True, 1),
+    (48, 384, 6272, True, False, 2),   # the norm is a kernel of its own
+    (64, 768, 8192, True, True, 3),    # and gelu
+    (16, 128, 8192, True, True, 2),    # gelu inside
+    (16, 960, 8192, True, False, 1),
+    (48, 1280, 4096, True, True, 1),
+    (64, 960, 8192, False, True, 2),
+])
+def test_what_a_product_of_few_rows_takes_along(m, k, n, norm, gelu, calls):
+    b, y = linear_layer(m, k, n, norm, gelu)
+    got = names(compile_only(b, [y]))
+    assert len(got) == calls, got
