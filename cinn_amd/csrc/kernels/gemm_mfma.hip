@@ -1524,6 +1524,7 @@ bool TryShortK(const GemmProblem& p, hipStream_t stream) {
 bool TrySkinny(const GemmProblem& p, hipStream_t stream) {
   static const bool enabled = !(getenv("FLAGS_cinn_hip_gemm_skinny") && atoi(getenv("FLAGS_cinn_hip_gemm_skinny")) == 0);
   if (!enabled || p.conv || p.trans_a || !p.trans_b || p.batch != 1) return false;
+  if (reinterpret_cast<uintptr_t>(p.a) % 16 != 0 || reinterpret_cast<uintptr_t>(p.b) % 16 != 0) return false;
   cinn_hip_kernels::RowProduct r{};
   r.bf16 = p.type == GemmType::kBF16;
   r.a = p.a, r.b = p.b, r.c[0] = p.c;

@@ -30,7 +30,7 @@ struct RowProduct {
 
 constexpr int kRowProductMaxNormK = 1280;
 
-// false where the kernel does not take the extents or alignments
+// false where the kernel does not take the extents; operands lie at any address of their type
 bool RowProductSupported(const RowProduct& p);
 // whether the kernel is ahead of the tiled ones for a product that it takes; `saves_launch`: several results, which would
 // be copied out of one

@@ -39,6 +39,7 @@ struct Half16;
 template <>
 struct Half16<__bf16> {
   typedef bf16x8 vec8;
+  typedef bf16x8 loaded __attribute__((aligned(2)));  // 16 bytes at any element's address: the same load instruction
   static __device__ __forceinline__ f32x4 mfma(vec8 a, vec8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
   }
@@ -46,6 +47,7 @@ struct Half16<__bf16> {
 template <>
 struct Half16<_Float16> {
   typedef f16x8 vec8;
+  typedef f16x8 loaded __attribute__((aligned(2)));
   static __device__ __forceinline__ f32x4 mfma(vec8 a, vec8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
   }
@@ -59,6 +61,7 @@ template <typename T, int MT, bool NORM, bool GELU>
 __global__ void __launch_bounds__(64 * NW)
 gemm_rows_kernel(RowProduct p) {
   typedef typename Half16<T>::vec8 vec8;
+  typedef typename Half16<T>::loaded loaded;
   static_assert(!NORM || MT == 1, "rows are normalised by blocks of one row tile");
   __shared__ __attribute__((aligned(16))) float s_part[NW][MT][64][4];
   __shared__ float s_sum[NORM ? NW : 1][16][2];
@@ -84,12 +87,12 @@ gemm_rows_kernel(RowProduct p) {
   if constexpr (NORM) {
     vec8 af[kNormBlocks], bf[kNormBlocks], g[kNormBlocks], be[kNormBlocks];
 #pragma unroll
-    for (int i = 0; i < kNormBlocks; ++i) af[i] = *reinterpret_cast<const vec8*>(ap[0] + k_of(i));
+    for (int i = 0; i < kNormBlocks; ++i) af[i] = *reinterpret_cast<const loaded*>(ap[0] + k_of(i));
 #pragma unroll
     for (int i = 0; i < kNormBlocks; ++i) {
-      bf[i] = *reinterpret_cast<const vec8*>(bp + k_of(i));
-      g[i]  = *reinterpret_cast<const vec8*>(static_cast<const T*>(p.gamma) + first * 32 + fk + k_of(i));
-      be[i] = *reinterpret_cast<const vec8*>(static_cast<const T*>(p.beta) + first * 32 + fk + k_of(i));
+      bf[i] = *reinterpret_cast<const loaded*>(bp + k_of(i));
+      g[i]  = *reinterpret_cast<const loaded*>(static_cast<const T*>(p.gamma) + first * 32 + fk + k_of(i));
+      be[i] = *reinterpret_cast<const loaded*>(static_cast<const T*>(p.beta) + first * 32 + fk + k_of(i));
     }
     float s = 0.0f, q = 0.0f;
 #pragma unroll
@@ -127,9 +130,9 @@ gemm_rows_kernel(RowProduct p) {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int k = k_of(i0 + u);
-        bf[set][u]  = *reinterpret_cast<const vec8*>(bp + k);
+        bf[set][u]  = *reinterpret_cast<const loaded*>(bp + k);
 #pragma unroll
-        for (int t = 0; t < MT; ++t) af[set][u][t] = *reinterpret_cast<const vec8*>(ap[t] + k);
+        for (int t = 0; t < MT; ++t) af[set][u][t] = *reinterpret_cast<const loaded*>(ap[t] + k);
       }
     };
     auto multiply = [&](int set, int i0) {
@@ -208,15 +211,12 @@ void Launch(const RowProduct& p, hipStream_t stream) {
   CINN_HIP_CALL(hipGetLastError());
 }
 
-bool Aligned(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
-
 }  // namespace
 
 bool RowProductSupported(const RowProduct& p) {
   if (p.m < 1 || p.m > 64 || p.n < 1 || p.k < 32 || p.k % 32 != 0 || (int64_t)p.n * p.k >= INT_MAX) return false;
   if (p.width < 1 || p.n % p.width != 0 || p.n / p.width > 3 || (p.n > p.width && p.residual)) return false;
-  if (p.gamma && (!p.beta || p.k > kRowProductMaxNormK || !Aligned(p.gamma) || !Aligned(p.beta))) return false;
-  return Aligned(p.a) && Aligned(p.b);
+  return !p.gamma || (p.beta && p.k <= kRowProductMaxNormK);
 }
 
 // Every wavefront waits for its own rows of B: with one block per CU (16 columns each; 16 rows, or all of them from 256 blocks of

@@ -288,7 +288,7 @@ void cinn_call_hip_matmul_bias(void* v_args, int num_args, int trans_b, int m, i
  * bf16 with fp32 scale and shift [n]; k a multiple of 32.  norm: layer norm of the rows with gamma and beta [k] of x's type
  * (k at most 1280); act: gelu on the fp32 sum, or nothing.  outputs 2 or 3 (without a residual): the columns go to that many
  * tensors [m][n / outputs], side by side.  operands: four bits for each of the slots x, W, scale, shift, residual, gamma,
- * beta, which input it is, 15 for none; v_args = {inputs..., outputs...}. */
+ * beta, which input it is, 15 for none; v_args = {inputs..., outputs...}, at any address of their type. */
 void cinn_call_hip_matmul_rows(void* v_args, int num_args, int m, int n, int k, int operands, int outputs, float epsilon, int gelu,
                                void* stream);
 

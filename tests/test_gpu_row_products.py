@@ -4,11 +4,14 @@ than wavefronts, of uneven shares and the longest that is normalised; columns th
 
 Bounds: norm in fp32, rounded once to the type (u = 2^-11 or 2^-8 of a value), a product of k terms with fp32 sums and one
 rounding of the result.  |gelu'| < 1.13."""
+import ctypes
 import math
 
 import numpy as np
 import pytest
 from scipy.special import erf
+
+from cinn_amd import _lib, runtime
 
 from test_gpu_projections import UNIT, _Program
 
@@ -97,3 +100,36 @@ def test_block_of_one_token(gpu, n, t, past, heads, d, fetched, dtype):
     # every intermediate is rounded a handful of times; errors of independent roundings add up in squares
     for g, w in zip(got, [x64 + y64] + want):
         assert np.linalg.norm(g - w) <= 4 * u * np.linalg.norm(w)
+
+
+@pytest.mark.parametrize("norm", [False, True])
+@pytest.mark.parametrize("offset", [0, 2, 8, 14])
+def test_operands_at_any_address(gpu, offset, norm):
+    """the call takes what the 1x1 convolution it stands for takes: operands that start anywhere in an allocation"""
+    m, k, n, rng, u = 9, 96, 40, np.random.default_rng(offset), UNIT["float16"]
+    data = [rng.standard_normal(s).astype(np.float16) for s in ((m, k), (n, k), (k,), (k,))]
+
+    def view(a):
+        room = runtime.DeviceBuffer((a.size + 8,), "float16")
+        room.copy_from(np.r_[np.zeros(offset // 2, np.float16), a.ravel(), np.zeros(8 - offset // 2, np.float16)])
+        room.buffer.memory = room.ptr.value + offset
+        return room
+
+    x, w, g, s = (view(a) for a in data)
+    scale, shift = (runtime.DeviceBuffer.from_numpy(a.astype(np.float32)) for a in (np.ones(n), np.arange(n)))
+    out = view(np.zeros((m, n), np.float16))
+    inputs = [x, w, scale, shift] + ([g, s] if norm else [])
+    operands = 0x3210 | 15 << 16 | (5 << 24 | 4 << 20 if norm else 255 << 20)
+    fn = _lib.load().cinn_call_hip_matmul_rows
+    fn.restype, fn.argtypes = None, [ctypes.c_void_p] + [ctypes.c_int] * 6 + [ctypes.c_float, ctypes.c_int, ctypes.c_void_p]
+    fn(runtime.pod_args(inputs + [out]), len(inputs) + 1, m, n, k, operands, 1, 1e-5, 0, None)
+    runtime.synchronize()
+    got = out.numpy()[offset // 2:][:m * n].reshape(m, n).astype(np.float64)
+    x64, w64, g64, s64 = (a.astype(np.float64) for a in data)
+    if norm:
+        x64 = norm64(x64, g64, s64)
+    want = x64 @ w64.T + np.arange(n)
+    bound = k * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64).T) + u * np.abs(want) + 2.0 ** -24 * n
+    if norm:
+        bound += (u + 2.0 ** -18) * (np.abs(x64) + np.abs(s64)) @ np.abs(w64).T
+    assert np.all(np.abs(got - want) <= 1.01 * bound + 1e-7)
