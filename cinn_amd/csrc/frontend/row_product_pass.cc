@@ -2,6 +2,7 @@
 
 #include <algorithm>
 #include <climits>
+#include <cstdlib>
 #include <map>
 #include <vector>
 
@@ -270,7 +271,12 @@ class RowProductFuser {
 
 }  // namespace
 
-Program FuseRowProducts(const Program& program, const std::set<std::string>& fetch_ids) { return RowProductFuser(program, fetch_ids).Run(); }
+Program FuseRowProducts(const Program& program, const std::set<std::string>& fetch_ids) {
+  // the switch of the kernel that runs what is made here
+  const char* skinny = getenv("FLAGS_cinn_hip_gemm_skinny");
+  if (skinny && atoi(skinny) == 0) return program;
+  return RowProductFuser(program, fetch_ids).Run();
+}
 
 }  // namespace frontend
 }  // namespace cinn

@@ -84,3 +84,10 @@ def test_what_a_product_of_few_rows_takes_along(m, k, n, norm, gelu, calls):
     b, y = linear_layer(m, k, n, norm, gelu)
     got = names(compile_only(b, [y]))
     assert len(got) == calls, got
+
+
+@pytest.mark.parametrize("flag,taken", [("0", False), ("1", True)])
+def test_switch_of_the_kernel(monkeypatch, flag, taken):
+    monkeypatch.setenv("FLAGS_cinn_hip_gemm_skinny", flag)
+    b, y = linear_layer(8, 256, 512, True, True)
+    assert any("matmul_rows" in e for e in names(compile_only(b, [y]))) == taken
