@@ -737,15 +737,29 @@ bool Data(const ConvBackwardArgs& a, hipStream_t stream) {
   return true;
 }
 
-// Whether a filter gradient goes to conv_filter_taps_kernel, and its launch.  `tile_bytes`: what conv_filter_kernel's tiles
-// would take out of L2.  Both are bound by that, so the taps together take layers where they take a fifth less: conv_train
-// step, us, conv_filter_kernel | here, by the ratio of these bytes, fp16, 3x3 unless noted: 0.44 (64 -> 64 on 56x56, batch 32)
-// 133.3 | 120.1, 0.56 (64 -> 64 5x5 on 41x35, batch 8) 80.5 | 78.9, 0.61 (7x7, batch 4) 83.5 | 82.5, 0.71 (32 -> 32 on 60x60,
-// batch 8) 61.2 | 59.3, 0.74 (128 -> 128 on 28x28, batch 32) 94.5 | 89.8, 0.79 (256 -> 256 on 14x14) 87.0 | 85.6; 0.88 (512 ->
-// 512 on 7x7: two positions of nine are behind the row) 112.7 | 118.6, 0.93 (96 -> 200 on 41x35, batch 8) 93.6 | 94.0, 1.06
-// (16 -> 32 on 60x60) 57.6 | 57.7.
+// Estimates of a filter gradient's two kernels in 16 bits, us: the start, the K steps of a block, the planes.  Fitted to 420 layers,
+// channels last, 3x3 to 7x7, 8 to 512 channels and filters (error 4 to 7% of the time on average).  A step of conv_filter_kernel's takes longer
+// the more blocks a CU has (at most three of 64 rows, two of 128), one of conv_filter_taps_kernel's, of one block per CU, as
+// long as it takes.
+double FilterMicroseconds(int rows, int64_t blocks, int steps, double plane_mb) {
+  const int full = rows == 64 ? 3 : 2, per_cu = (int)std::min<int64_t>((blocks + 255) / 256, full);
+  const double step64[3] = {0.66, 1.0, 1.54}, step128[2] = {0.88, 1.2};
+  const double rounds = (double)((blocks + 256 * full - 1) / (256 * full));
+  return (rows == 64 ? 6.3 + 0.64 * plane_mb : 7.1 + 0.5 * plane_mb) + rounds * steps * (rows == 64 ? step64 : step128)[per_cu - 1];
+}
+double TapsMicroseconds(int64_t blocks, int steps, double plane_mb) {
+  return 7.2 + 0.81 * plane_mb + (double)((blocks + 255) / 256) * steps * 0.51;
+}
+
+// Whether a filter gradient goes to conv_filter_taps_kernel, and its launch: where it needs a fifth less out of L2 than
+// conv_filter_kernel's tiles (`p`, `bm` rows each, `splits` of K; `tile_bytes`) and is estimated to be faster.
+// Measured, us with the reduction of the planes, conv_filter_kernel | here, fp16, 3x3 unless noted: 64 -> 64 on 56x56, batch 32, 33.3 | 23.6,
+// 296 -> 24 on 11x88, batch 32, 30.0 | 24.0, 96 -> 40 on 56x60, batch 25, 36.5 | 30.0, 184 -> 56 7x7 on 53x21, batch 7, 35.5 | 31.7; not taken: short
+// ones, 80 -> 8 on 24x31, 8.6 | 10.4, and those whose tiles leave a part of the CUs without a block, 504 -> 136 on 42x18, batch 20, 61.5 |
+// 80.0 (144 blocks), 424 -> 48 5x5 on 58x37, batch 15, 103 | 149 (140), 392 -> 8 7x7 on 74x96, batch 6, 214 | 353 (147).  Of 167 layers that read a
+// fifth less, 60 are taken: 10% faster on average, the worst 6% slower.
 template <typename T>
-bool PlanTaps(const ConvBackwardArgs& a, const FilterGradParams& p, int64_t plane, int64_t tile_bytes, TapsParams* t) {
+bool PlanTaps(const ConvBackwardArgs& a, const FilterGradParams& p, int bm, int old_splits, int64_t plane, int64_t tile_bytes, TapsParams* t) {
   if (sizeof(T) != 2 || a.stride_w != 1 || a.dil_w != 1 || a.kw < kTaps) return false;
   // positions in a row are multiplied as signed 24-bit numbers (__mul24); channels are below 2^20
   if (std::max(a.ow, a.w_in) > (1 << 23)) return false;
@@ -768,7 +782,9 @@ bool PlanTaps(const ConvBackwardArgs& a, const FilterGradParams& p, int64_t plan
   t->lanes_log2 = splits >= 8 ? 3 : splits >= 4 ? 2 : splits >= 2 ? 1 : 0;
   t->splits     = splits >> t->lanes_log2 << t->lanes_log2;
   t->g.steps_per_split = (t->g.steps + t->splits - 1) / t->splits;
-  return true;
+  const double mb = (double)plane * sizeof(float) * 1e-6;
+  return TapsMicroseconds(tiles * t->splits, t->g.steps_per_split, t->splits * mb) <
+         FilterMicroseconds(bm, (int64_t)p.tiles_m * p.tiles_n * old_splits, p.steps_per_split, old_splits * mb);
 }
 
 template <typename T>
@@ -805,7 +821,7 @@ bool Filter(const ConvBackwardArgs& a, hipStream_t stream) {
   p.steps_per_split = (p.steps + splits - 1) / splits;
   splits            = (p.steps + p.steps_per_split - 1) / p.steps_per_split;
   TapsParams t;
-  const bool taps = PlanTaps<T>(a, p, plane, (int64_t)tiles * p.steps * (bm + bn) * 128, &t);
+  const bool taps = PlanTaps<T>(a, p, bm, splits, plane, (int64_t)tiles * p.steps * (bm + bn) * 128, &t);
   if (taps) splits = t.splits;
   p.spill = taps ? 1 : 0;
   const size_t plane_bytes = (size_t)splits * plane * sizeof(float);
