@@ -763,6 +763,16 @@ bool PlanTaps(const ConvBackwardArgs& a, const FilterGradParams& p, int bm, int 
   if (sizeof(T) != 2 || a.stride_w != 1 || a.dil_w != 1 || a.kw < kTaps) return false;
   // positions in a row are multiplied as signed 24-bit numbers (__mul24); channels are below 2^20
   if (std::max(a.ow, a.w_in) > (1 << 23)) return false;
+  // Only filters of which at most one tap stays inside the image for all pixels: an infinite or NaN x meets zeros of dy here, so
+  // NaNs of every tap are computed again, a block per element, where the other kernel leaves those of such taps as they are.  A step
+  // whose dy overflowed has nothing else: 64 -> 64 3x3 on 56x56, batch 32, channels last, without padding, us, that kernel | here, finite dy 32.8 | 23.8,
+  // all NaN 32.6 | 1845 (padded 1802 | 1837).
+  auto inside = [](int taps, int dil, int stride, int pad, int out, int size) {
+    int count = 0;
+    for (int k = 0; k < taps; ++k) count += k * dil >= pad && k * dil - pad + (out - 1) * stride < size ? 1 : 0;
+    return (int64_t)count;
+  };
+  if (inside(a.kh, a.dil_h, a.stride_h, a.pad_h, a.oh, a.h) * inside(a.kw, a.dil_w, a.stride_w, a.pad_w, a.ow, a.w_in) > 1) return false;
   t->g         = p;
   t->g.tiles_m = (a.f + 63) / 64;
   t->tiles_c   = (p.cp + 63) / 64;

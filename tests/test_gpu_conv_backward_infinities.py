@@ -109,3 +109,41 @@ def test_data_gradient(gpu, case, filter_too, dtype, fmt, value, beta):
         assert np.all(np.isin(np.nonzero(np.isnan(got) & ~np.isnan(want) & ~inner)[1], [2, 4]))  # the channels of those values
         got[~inner] = want[~inner]
     check(got, want, scale, f * k * k, dtype)
+
+
+# Neighbouring taps share what is read (fp16 / bf16, stride 1): positions behind an output row and the last two of every K step have
+# a zero in place of dy, and x of a pixel inside the image.  Here a step is a row: its last two positions read the next row's first pixels,
+# for the centre tap too, which reaches no padding.
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+@pytest.mark.parametrize("fmt", [0, 1])
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+def test_filter_gradient_of_a_pixel_that_meets_no_dy(gpu, dtype, fmt, value):
+    case = (8, 64, 4, 60, 8, 3, 1, 1, 1, 1)
+    n, c, h, w_, f, k, s, p, d, g = case
+    x, w, dy = conv_problem(case, dtype)
+    dy[np.abs(dy) < 0.01] = 0.01  # nothing that an infinity would turn to NaN
+    dy = round_to(dy, dtype)
+    x[1, 5, 2, 0] = x[3, 9, 1, 1] = x[4, 11, 0, w_ - 1] = value
+    X, DY, DW = (to_dev(layout(t, fmt), dtype) for t in (x, dy, np.zeros_like(w)))
+    run("cinn_call_cudnn_conv2d_backward_filter", fmt, 1.0, 0.0, conv_dims(case, x, w, dy), X, DY, DW)
+    with np.errstate(invalid="ignore"):
+        want = gradients(x.astype(np.float64), w, dy.astype(np.float64), s, p, d)[1]
+        scale = gradients(np.abs(x).astype(np.float64), w, np.abs(dy).astype(np.float64), s, p, d)[1]
+    if np.isinf(value):
+        assert not np.isnan(want).any() and np.isinf(want[:, 5, 1, 1]).all()
+    check(unlayout(from_dev(DW, dtype), fmt), want, scale, dy.size / f, dtype)
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+def test_filter_gradient_without_padding(gpu, dtype):
+    """an infinity of x where no padding is: inf or NaN exactly where it is a term"""
+    case = (32, 64, 12, 90, 24, 3, 1, 0, 1, 1)
+    n, c, h, w_, f, k, s, p, d, g = case
+    x, w, dy = conv_problem(case, dtype)
+    x[2, 7, 5, w_ - 1] = x[1, 3, 0, 0] = np.inf
+    X, DY, DW = (to_dev(layout(t, 1), dtype) for t in (x, dy, np.zeros_like(w)))
+    run("cinn_call_cudnn_conv2d_backward_filter", 1, 1.0, 0.0, conv_dims(case, x, w, dy), X, DY, DW)
+    with np.errstate(invalid="ignore"):
+        want = gradients(x.astype(np.float64), w, dy.astype(np.float64), s, p, d)[1]
+        scale = gradients(np.abs(x).astype(np.float64), w, np.abs(dy).astype(np.float64), s, p, d)[1]
+    check(unlayout(from_dev(DW, dtype), 1), want, scale, dy.size / f, dtype)
