@@ -156,7 +156,7 @@ def test_16bit_direct_to_lds_kernel(gpu, kind, tb, alpha, beta, batch, m, n, k):
                                    (40, 4112, 256),    # 257 column blocks: the three row tiles stay in one block
                                    (64, 4096, 512)])   # 256 column blocks, four row tiles per block
 def test_16bit_products_with_few_rows(gpu, kind, alpha, beta, m, n, k):
-    """gemm16_skinny_kernel: at most 64 rows, B stored [N][K], K a multiple of 256 - one block per 16 columns (and, below 256
+    """gemm_rows_kernel: at most 64 rows, B stored [N][K], K a multiple of 256 here - one block per 16 columns (and, below 256
     such blocks, per 16 rows), K split over its wavefronts, fragments straight from global memory.  Same bar as the tiled kernels: fp32 accumulation and
     epilogue, one rounding to the 16-bit type."""
     rng = np.random.default_rng(m * 7 + n + k)

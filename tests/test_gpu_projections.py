@@ -135,6 +135,13 @@ def test_bias_of_a_layer_in_training(gpu, m, k, n, dtype, trans_b):
     assert np.all(np.abs(got - want) <= 1.01 * bound + 1e-7)
 
 
+# the kernels for one step of K and for 256x256 tiles, which read the 16-bit bias themselves
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("m,k,n", [(16384, 64, 128), (16400, 64, 256), (4096, 192, 3072), (4090, 192, 3080)])
+def test_narrow_bias_in_every_epilogue(gpu, m, k, n, dtype):
+    test_bias_of_a_layer_in_training(gpu, m, k, n, dtype, False)
+
+
 # the same with small results and ragged extents, in fp32 too, where K is split and where it is not; the bias has the
 # operands' type or fp32
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16", "float32"])

@@ -91,3 +91,46 @@ def test_switch_of_the_kernel(monkeypatch, flag, taken):
     monkeypatch.setenv("FLAGS_cinn_hip_gemm_skinny", flag)
     b, y = linear_layer(8, 256, 512, True, True)
     assert any("matmul_rows" in e for e in names(compile_only(b, [y]))) == taken
+
+
+def norm_and_layers(fetch, readers=1, epsilon=1e-5):
+    """a layer norm, `readers` linear layers of its result; `fetch`: which of its other results the program returns"""
+    b, rng, data = NetBuilder("norm"), np.random.default_rng(5), {}
+
+    def put(name, shape, const=True):
+        data[name] = (rng.standard_normal(shape) + (1.0 if name == "g" else 0.0)).astype(np.float16)
+        v = b.create_input(Float(16), list(shape), name)
+        v.set_const(const)
+        return v
+
+    outs = b.paddle_layer_norm(put("x", (M, K), False), put("g", (K,)), put("s", (K,)), epsilon)
+    results = [b.add(b.matmul(outs[0], put("w%d" % i, (K, N))), put("c%d" % i, (N,))) for i in range(readers)]
+    return b, results + [outs[i] for i in fetch], data
+
+
+# what keeps the norm a kernel of its own: its mean, variance or result is wanted, or two products that are not joined read it
+@pytest.mark.parametrize("fetch,readers,inside", [([], 1, True), ([1], 1, False), ([2], 1, False), ([0], 1, False), ([], 2, False)])
+def test_norms_that_are_read_by_others(fetch, readers, inside):
+    b, outs, _ = norm_and_layers(fetch, readers)
+    got = names(compile_only(b, outs))
+    assert (len(got) == 1 and "matmul_rows" in got[0]) == inside, got
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fetch,readers,epsilon", [([], 1, 0.3), ([1], 1, 1e-5), ([2], 1, 1e-5), ([0], 1, 0.3), ([], 2, 1e-5), ([0, 1, 2], 2, 1e-5)])
+def test_norm_values(gpu, fetch, readers, epsilon):
+    b, outs, data = norm_and_layers(fetch, readers, epsilon)
+    got, _ = run(b, data, outs)
+    d = {e: v.astype(np.float64) for e, v in data.items()}
+    mean, var = d["x"].mean(1), d["x"].var(1)
+    norm = (d["x"] - mean[:, None]) / np.sqrt(var[:, None] + epsilon) * d["g"] + d["s"]
+    u = 2.0 ** -11
+    # the normalised value is rounded once (its fp32 variance loses 2^-18 or so), the sum once
+    slack = (u + 2.0 ** -18) * (np.abs(norm) + np.abs(d["s"]))
+    for i in range(readers):
+        want = norm @ d["w%d" % i] + d["c%d" % i]
+        assert np.all(np.abs(got[i] - want) <= 1.01 * (slack @ np.abs(d["w%d" % i]) + 2 * u * np.abs(want)) + 1e-4)
+    wants = (norm, mean, var)
+    for g, i in zip(got[readers:], fetch):
+        size = (np.abs(norm) + np.abs(d["s"]), np.abs(d["x"]).mean(1), 1.0 + var)[i]
+        assert np.all(np.abs(g.reshape(wants[i].shape) - wants[i]) <= 2 * u * size + 1e-6)
