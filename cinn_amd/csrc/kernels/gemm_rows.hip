@@ -226,13 +226,15 @@ bool RowProductSupported(const RowProduct& p) {
 // 8192 7.1 | 6.1, 48 x 960 -> 4096 (three row tiles) 7.3 | 6.3; three: 1 x 1984 -> 12288 12.4 | 11.5, 48 x 960 -> 3072 7.3 | 9.0, 32 x 960 -> 8192
 // 7.2 | 8.0; more: 64 x 192 -> 8192 4.3 | 10.7.  Where K is no multiple of 64 the tiled kernel is the register-staged one: 1 x 1120 -> 16384 10.4 |
 // 8.2, 32 x 224 -> 3072 4.9 | 4.2, 64 x 224 -> 4096 5.2 | 4.8, 32 x 544 -> 8192 6.6 | 4.9, but 32 x 2080 -> 8192 13.0 | 13.5, 48 x 224 -> 3072 5.1 | 6.1.
-// K in whole shares of all wavefronts has always come here.
+// It and the one for ragged rows of C split a long K over more blocks than there are columns: 64 x 6112 -> 64 9.1 | 9.7, 24 x 7968 -> 200 9.1 |
+// 11.7 (but 1 x 6112 -> 1000 8.7 | 7.0), 64 x 5024 -> 2048 11.7 | 14.9, 24 x 3968 -> 25 7.2 | 8.7.  K in whole shares of all wavefronts has always come here.
 bool RowProductPays(int m, int n, int k, bool saves_launch) {
   if (k % 256 == 0) return true;
   const int columns = (n + 15) / 16, tiles = (m + 15) / 16;
   const double load = columns < 256 ? (columns * tiles + 255) / 256 : (columns + 255) / 256 * (0.5 + 0.5 * tiles);
   if (saves_launch && load <= 3.0) return true;
-  if (k % 64 != 0) return load <= (m <= 4 ? 4.0 : 2.5) || (load <= 3.0 && (k <= 128 || k > 256) && k < 1536);
+  if (k % 64 != 0) return load <= 1.0 ? k < (m <= 4 ? 8192 : 5632) : (load <= (m <= 4 ? 4.0 : 2.5) && k < 3584) || (load <= 3.0 && (k <= 128 || k > 256) && k < 1536);
+  if (n % 8 != 0 && k > (m <= 4 ? 4096 : 2560)) return false;
   if (m <= 4) return load <= (k < 512 ? 2.0 : 3.0);
   return load <= (k < 256 ? 1.0 : k < 512 ? 1.5 : 2.0);
 }
