@@ -242,7 +242,7 @@ class RowProductFuser {
     } else if (!residual) {
       columns = Columns(y);
     }
-    if (!fuse.norm && !fuse.gelu && !((plain || !columns.empty()) && cinn_hip_kernels::RowProductPays(m, n, k, !columns.empty()))) return;
+    if (!fuse.norm && !fuse.gelu && !((plain || !columns.empty()) && cinn_hip_kernels::RowProductPays(m, n, k, !columns.empty(), false))) return;
     if (columns.empty()) {
       call->outputs = {y};
     } else {

@@ -33,8 +33,8 @@ constexpr int kRowProductMaxNormK = 1280;
 // false where the kernel does not take the extents; operands lie at any address of their type
 bool RowProductSupported(const RowProduct& p);
 // whether the kernel is ahead of the tiled ones for a product that it takes; `saves_launch`: several results, which would
-// be copied out of one
-bool RowProductPays(int m, int n, int k, bool saves_launch);
+// be copied out of one; `splits`: without a scale, which gemm_flex.hip would take and split its K
+bool RowProductPays(int m, int n, int k, bool saves_launch, bool splits);
 // which of a layer norm before the product and a gelu behind it (those that there are) are faster inside
 struct RowFusion {
   bool norm, gelu;

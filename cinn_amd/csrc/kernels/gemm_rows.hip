@@ -225,16 +225,18 @@ bool RowProductSupported(const RowProduct& p) {
 // tiles in each 32 x 192 -> 4096 4.0 | 4.6, 32 x 384 -> 4096 4.7 | 4.6; two on a CU: 1 x 384 -> 8192 4.7 | 3.7, 16 x 384 -> 8192 4.8 | 5.2, 16 x 960 ->
 // 8192 7.1 | 6.1, 48 x 960 -> 4096 (three row tiles) 7.3 | 6.3; three: 1 x 1984 -> 12288 12.4 | 11.5, 48 x 960 -> 3072 7.3 | 9.0, 32 x 960 -> 8192
 // 7.2 | 8.0; more: 64 x 192 -> 8192 4.3 | 10.7.  Where K is no multiple of 64 the tiled kernel is the register-staged one: 1 x 1120 -> 16384 10.4 |
-// 8.2, 32 x 224 -> 3072 4.9 | 4.2, 64 x 224 -> 4096 5.2 | 4.8, 32 x 544 -> 8192 6.6 | 4.9, but 32 x 2080 -> 8192 13.0 | 13.5, 48 x 224 -> 3072 5.1 | 6.1.
-// It and the one for ragged rows of C split a long K over more blocks than there are columns: 64 x 6112 -> 64 9.1 | 9.7, 24 x 7968 -> 200 9.1 |
-// 11.7 (but 1 x 6112 -> 1000 8.7 | 7.0), 64 x 5024 -> 2048 11.7 | 14.9, 24 x 3968 -> 25 7.2 | 8.7.  K in whole shares of all wavefronts has always come here.
-bool RowProductPays(int m, int n, int k, bool saves_launch) {
+// 8.2, 32 x 224 -> 3072 4.9 | 4.2, 64 x 224 -> 4096 5.2 | 4.8, 32 x 544 -> 8192 6.6 | 4.9, but 32 x 2080 -> 8192 13.0 | 13.5, 48 x 224 -> 3072 5.1 | 6.1, 64 x 6112 -> 4096 17.8 | 24.
+// K in whole shares of all wavefronts has always come here.
+// That kernel splits a long K over more blocks than there are columns, where it can take the product (a plain one: `splits`): 64 x 6112 -> 64
+// 9.1 | 9.7, 24 x 7968 -> 200 9.1 | 11.7 (but 1 x 6112 -> 1000 8.7 | 7.0), 64 x 5024 -> 2048 11.7 | 14.9, 24 x 3968 -> 25 7.2 | 8.7; a layer with its scale
+// and shift has a convolution's tiles instead, 8 x 6112 -> 4096 with gelu 18.7 | 10.0.
+bool RowProductPays(int m, int n, int k, bool saves_launch, bool splits) {
   if (k % 256 == 0) return true;
   const int columns = (n + 15) / 16, tiles = (m + 15) / 16;
   const double load = columns < 256 ? (columns * tiles + 255) / 256 : (columns + 255) / 256 * (0.5 + 0.5 * tiles);
+  if (splits && (k % 64 != 0 ? k >= (load > 1.0 ? 3584 : m <= 4 ? 8192 : 5632) : n % 8 != 0 && k > (m <= 4 ? 4096 : 2560))) return false;
   if (saves_launch && load <= 3.0) return true;
-  if (k % 64 != 0) return load <= 1.0 ? k < (m <= 4 ? 8192 : 5632) : (load <= (m <= 4 ? 4.0 : 2.5) && k < 3584) || (load <= 3.0 && (k <= 128 || k > 256) && k < 1536);
-  if (n % 8 != 0 && k > (m <= 4 ? 4096 : 2560)) return false;
+  if (k % 64 != 0) return load <= (m <= 4 ? 4.0 : k < 3072 ? 2.5 : 2.0) || (load <= 3.0 && (k <= 128 || k > 256) && k < 1536);
   if (m <= 4) return load <= (k < 512 ? 2.0 : 3.0);
   return load <= (k < 256 ? 1.0 : k < 512 ? 1.5 : 2.0);
 }
@@ -243,16 +245,18 @@ bool RowProductPays(int m, int n, int k, bool saves_launch) {
 // round of blocks cost what a kernel of their own does - unless the product alone would be blocks of one row tile as well.  us,
 // separate | inside, fp16, norm: one round 32 x 320 -> 2048 6.7 | 5.7, 64 x 960 -> 1024 10.0 | 6.1; two 32 x 384 -> 4096 7.0 | 8.5, 16 x 960 -> 8192
 // 9.8 | 9.0; three 48 x 960 -> 4096 10.0 | 12.3, 48 x 1280 -> 4096 13.0 | 12.6; more 48 x 384 -> 6272 7.3 | 18.6, 64 x 1280 -> 4096 14.9 | 16.1; the
-// same blocks alone 64 x 768 -> 3072 12.7 | 12.1, 48 x 512 -> 3072 10.8 | 11.8.  gelu: two rounds 16 x 384 -> 8192 7.6 | 5.6, three 64 x 192 -> 3072
-// 7.1 | 8.5, four 64 x 960 -> 4096 10.3 | 10.6, 64 x 960 -> 8192 10.8 | 20.6; the same blocks alone 64 x 768 -> 3072 12.6 | 10.3.  Both: one round
+// same blocks alone 64 x 768 -> 3072 12.7 | 12.1, 48 x 512 -> 3072 10.8 | 11.8, in a
+// block of a transformer (48 tokens of 512, three results) all of it 41.0 | 38.5.  gelu: two rounds 16 x 384 -> 8192 7.6 | 5.6, three 64 x 192 -> 3072
+// 7.1 | 8.5, four 64 x 960 -> 4096 10.3 | 10.6, 64 x 960 -> 8192 10.8 | 20.6; the same blocks alone 64 x 768 -> 3072 12.6 | 10.3, 1 x
+// 2048 -> 16384 17.1 | 14.0, but 32 x 8192 -> 4096 (alone one round of two row tiles) 26.8 | 31.5.  Both: one round
 // 64 x 320 -> 1024 9.9 | 6.2, two 16 x 128 -> 8192 8.3 | 8.9, 48 x 192 -> 2048 9.2 | 8.9, three 64 x 320 -> 3072 10.0 | 12.6, six 64 x 1280 -> 6144 28.1 |
 // 24.9, eight 64 x 1280 -> 8192 28.9 | 32.6, four 64 x 768 -> 4096 13.0 | 16.9; the same blocks alone 64 x 768 -> 3072 15.5 | 13.1.
 RowFusion ChooseRowFusion(int m, int n, int k, RowFusion there) {
   const int rounds = ((n + 15) / 16 * ((m + 15) / 16) + 255) / 256;
   const bool same  = k % 256 == 0 && n <= 4080;  // the blocks of the product alone
   if (there.norm && there.gelu && (same || rounds <= 1 || (rounds <= 2 && k >= 192) || (rounds <= 6 && k >= 1152))) return there;
-  if (there.gelu && (same || rounds <= 2)) return {false, true};
-  return {there.norm && (rounds <= 1 || (same && k >= 768) || (rounds <= 2 && k >= 896) || (rounds <= 3 && k >= 1152)), false};
+  if (there.gelu && ((rounds <= 2 && k < 3072) || ((n <= 4080 || m <= 16) && RowProductPays(m, n, k, false, false)))) return {false, true};
+  return {there.norm && (rounds <= 1 || (same && k >= (rounds <= 2 ? 512 : 768)) || (rounds <= 2 && k >= 896) || (rounds <= 3 && k >= 1152)), false};
 }
 
 void RunRowProduct(const RowProduct& p, hipStream_t stream) {
