@@ -15,7 +15,8 @@ namespace frontend {
 //   * the gelu that alone reads it, on the fp32 sum,
 //   * one result tensor for each of two or three slices that divide its columns.  Transposes behind them that only move an
 //     axis of one become reshapes, which are no kernel.
-// Layers with none of these keep their call in a program without any.
+// Each where the kernel is faster with it than without (gemm_rows.hip).  Layers with none of these keep their call in a program
+// without any.  FLAGS_cinn_hip_gemm_skinny=0 leaves the program as it is.
 Program FuseRowProducts(const Program& program, const std::set<std::string>& fetch_ids);
 
 }  // namespace frontend

@@ -28,6 +28,8 @@ struct RowProduct {
   float epsilon;
 };
 
+// longest row that is normalised: a lane holds 16 bytes of x, W, gamma and beta for each of its wavefront's five blocks of K (114
+// registers; above 128 a CU holds one block)
 constexpr int kRowProductMaxNormK = 1280;
 
 // false where the kernel does not take the extents; operands lie at any address of their type

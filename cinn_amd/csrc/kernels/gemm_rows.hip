@@ -225,7 +225,8 @@ bool RowProductSupported(const RowProduct& p) {
 // tiles in each 32 x 192 -> 4096 4.0 | 4.6, 32 x 384 -> 4096 4.7 | 4.6; two on a CU: 1 x 384 -> 8192 4.7 | 3.7, 16 x 384 -> 8192 4.8 | 5.2, 16 x 960 ->
 // 8192 7.1 | 6.1, 48 x 960 -> 4096 (three row tiles) 7.3 | 6.3; three: 1 x 1984 -> 12288 12.4 | 11.5, 48 x 960 -> 3072 7.3 | 9.0, 32 x 960 -> 8192
 // 7.2 | 8.0; more: 64 x 192 -> 8192 4.3 | 10.7.  Where K is no multiple of 64 the tiled kernel is the register-staged one: 1 x 1120 -> 16384 10.4 |
-// 8.2, 32 x 224 -> 3072 4.9 | 4.2, 64 x 224 -> 4096 5.2 | 4.8, 32 x 544 -> 8192 6.6 | 4.9, but 32 x 2080 -> 8192 13.0 | 13.5, 48 x 224 -> 3072 5.1 | 6.1, 64 x 6112 -> 4096 17.8 | 24.
+// 8.2, 32 x 224 -> 3072 4.9 | 4.2, 64 x 224 -> 4096 5.2 | 4.8, 32 x 544 -> 8192 6.6 | 4.9, but 32 x 2080 -> 8192 13.0 | 13.5, 48 x 224 -> 3072 5.1 | 6.1, 64 x 6112 -> 4096 and gelu 20.4 |
+// 26.5.
 // K in whole shares of all wavefronts has always come here.
 // That kernel splits a long K over more blocks than there are columns, where it can take the product (a plain one: `splits`): 64 x 6112 -> 64
 // 9.1 | 9.7, 24 x 7968 -> 200 9.1 | 11.7 (but 1 x 6112 -> 1000 8.7 | 7.0), 64 x 5024 -> 2048 11.7 | 14.9, 24 x 3968 -> 25 7.2 | 8.7; a layer with its scale
