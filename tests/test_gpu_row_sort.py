@@ -106,7 +106,8 @@ def test_top_k(gpu, size, kind, k):
 @pytest.mark.parametrize("size", [64, 65, 1000, 1025, 4097])
 def test_top_k_of_distinct_scores_and_equal_ones(gpu, size, k, equal):
     """the words up to the bound are ranked against each other, more than 64 or 128 of them are taken one by one: distinct
-    scores, scores of which the k-th largest is shared, and a row whose largest ones a few lanes hold"""
+    scores, scores of which the k-th largest is shared, and a row whose largest ones a few lanes hold.  (For k of 50 and up to 1024
+    elements these few rows are sorted by the network; test_top_k_of_many_rows has the selection.)"""
     rng = np.random.default_rng(size + k)
     x = rng.permuted(np.tile(np.arange(size, dtype=np.float32) - size // 2, (5, 1)), axis=1)
     x[4, rng.permutation(size)] = np.where(np.arange(size) % 64 < 3, size, 0) + x[4]
