@@ -420,33 +420,28 @@ __device__ __forceinline__ u64 WaveMin(u64 v) {
 // The first `keep` (at most 64) of a wavefront's words, E per lane, written to first[0 .. keep - 1] in order.  The keep-th
 // least of the lanes' least keys bounds the keys that can be among them, and few others lie below it: for the first five of
 // 1000 random values seven words are left on average, for the first fifty about ninety.  These are gathered, C per lane, and
-// each counts the ones before it.  Of the words at the bound itself the first `keep` suffice, where w[e] of a lane is ahead of
-// w[e] of the lanes behind it and of all w[e + 1] for equal keys (IN_ORDER); for C = 1 they are told apart only if many lanes
-// hold the bound.  (2048 rows of 1000 equal values, k = 5, with all of them gathered and then taken one by one: 9.5 us, so 6.2; told
-// apart in every row, distinct values take 6.8 us instead of 6.3.)  Should more than 64 C words be left - a lane has many of a
-// row's first elements - they are taken one by one, the owner of each looking for its next one.
-// candidates: 64 C words of LDS of this wavefront's own, as first is.
-template <int E, int C, bool IN_ORDER>
+// each counts the ones before it.  Of the words at the bound itself the first `keep`
+// suffice (looked at for C > 1 only).  Should more than 64 C words be
+// left - a lane has many of a row's first elements - they are taken one by one, the owner of each looking for its next one.
+// candidates: 64 C words of LDS of this wavefront's own, as first is.  w[e] of a lane is ahead of w[e] of the lanes behind it
+// and of all w[e + 1] where the keys are equal.
+template <int E, int C>
 __device__ __forceinline__ void SelectFirst(u64 (&w)[E], int keep, u64* candidates, u64* first) {
   const int lane = threadIdx.x & 63;
-  uint32_t least = (uint32_t)(w[0] >> 32), limit = 0;
+  uint32_t rest  = (uint32_t)(w[0] >> 32), limit = 0;
 #pragma unroll
-  for (int e = 1; e < E; ++e) least = min(least, (uint32_t)(w[e] >> 32));
-  uint32_t rest = least;
+  for (int e = 1; e < E; ++e) rest = min(rest, (uint32_t)(w[e] >> 32));
 #pragma unroll 1
   for (int s = 0; s < keep; ++s) {
     limit = WaveMin32(rest);
     if (lane == __builtin_ctzll(__ballot(rest == limit))) rest = 0xffffffffu;
   }
   const u64 before = ((u64)1 << lane) - 1;
-  // C = 1: the words at the bound are among the others, or behind them up to `keep`
-  const bool apart     = C == 1 && IN_ORDER && (__popcll(__ballot(least == limit)) > 8 || limit == 0xffffffffu);
-  const uint32_t below = apart ? limit : limit + 1;
   int count = 0, equals = 0;
 #pragma unroll
   for (int e = 0; e < E; ++e) {
     const uint32_t key = (uint32_t)(w[e] >> 32);
-    u64 mask           = __ballot(C > 1 ? key < limit : IN_ORDER ? key < below : key <= limit);
+    u64 mask           = __ballot(C > 1 ? key < limit : key <= limit);
     if constexpr (C > 1) {
       const u64 equal = __ballot(key == limit);
       if (equal != 0 && equals < keep) {
@@ -458,17 +453,6 @@ __device__ __forceinline__ void SelectFirst(u64 (&w)[E], int keep, u64* candidat
     const int at = count + __popcll(mask & before);
     if ((mask >> lane & 1) && at < 64 * C) candidates[at] = w[e];
     count += __popcll(mask);
-  }
-  if (apart) {
-    const int enough = count + keep;
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-      if (count >= enough) continue;
-      const u64 equal = __ballot((uint32_t)(w[e] >> 32) == limit);
-      const int at    = count + __popcll(equal & before);
-      if ((equal >> lane & 1) && at < min(enough, 64 * C)) candidates[at] = w[e];
-      count = min(count + __popcll(equal), enough);
-    }
   }
   if (count <= 64 * C) {
     // the wavefront's own words: its LDS accesses keep their order, the compiler must not change it
@@ -492,19 +476,19 @@ __device__ __forceinline__ void SelectFirst(u64 (&w)[E], int keep, u64* candidat
     for (int u = 0; u < C; ++u)
       if (lane + 64 * u < count && slot[u] < keep) first[slot[u]] = mine[u];
   } else {
-    u64 word = w[0];
+    u64 least = w[0];
 #pragma unroll
-    for (int e = 1; e < E; ++e) word = w[e] < word ? w[e] : word;
+    for (int e = 1; e < E; ++e) least = w[e] < least ? w[e] : least;
 #pragma unroll 1
     for (int s = 0; s < keep; ++s) {
-      const u64 got = WaveMin(word);
+      const u64 got = WaveMin(least);
       if (lane == s) first[s] = got;
-      if (word == got) {
+      if (least == got) {
 #pragma unroll
         for (int e = 0; e < E; ++e) w[e] = w[e] == got ? ~0ull : w[e];
-        word = w[0];
+        least = w[0];
 #pragma unroll
-        for (int e = 1; e < E; ++e) word = w[e] < word ? w[e] : word;
+        for (int e = 1; e < E; ++e) least = w[e] < least ? w[e] : least;
       }
     }
   }
@@ -529,14 +513,14 @@ __global__ void __launch_bounds__(64 * WAVES) row_select_kernel(RowParams p) {
   const int64_t base = (int64_t)(blockIdx.x / p.inner) * p.size * p.inner + blockIdx.x % p.inner;
   u64 w[E];
   LoadWords<T, E, 64 * WAVES>(p, base, t, 64 * WAVES, p.size, shared, w);
-  SelectFirst<E, C, true>(w, p.keep, candidates + wave * 64 * C, part[wave]);
+  SelectFirst<E, C>(w, p.keep, candidates + wave * 64 * C, part[wave]);
   if (WAVES > 1) __syncthreads();
   if constexpr (WAVES > 1 && C == 1) {
     if (wave > 0) return;
     u64 all[WAVES / 4];
 #pragma unroll
     for (int e = 0; e < WAVES / 4; ++e) all[e] = (lane & 15) < p.keep ? part[e * 4 + (lane >> 4)][lane & 15] : ~0ull;
-    SelectFirst<WAVES / 4, 1, false>(all, p.keep, candidates, first);
+    SelectFirst<WAVES / 4, 1>(all, p.keep, candidates, first);
   }
   if (lane >= p.keep) return;
   const u64 mine = WAVES > 1 && C == 1 ? first[lane] : part[wave][lane];
