@@ -51,6 +51,9 @@ bool TryPointwiseConvAsGemm(const ConvNhwcArgs& a, hipStream_t stream);
 // rows fit LDS (conv_patch_mfma.hip): the input patch of a band of output rows stays resident in LDS, only the filter
 // streams; same epilogue.  false when the shape does not qualify.
 bool TryConvPatch(const ConvNhwcArgs& a, hipStream_t stream);
+// few pixels (conv_few_mfma.hip): whole K steps of 128 bytes in every tap, same epilogue; one launch of
+// small tiles whose wavefronts share K.  false when the shape does not qualify or the tiled kernels are faster.
+bool TryConvFew(const ConvNhwcArgs& a, hipStream_t stream);
 // Two 1x1, stride 1, unpadded convolutions in a row on channels-last 16-bit tensors, seen as matrix products over the
 // m = N * H * W pixels: e = act1(x w1^T * scale1 + shift1 + residual) [m][n1], y = act2(e w2^T * scale2 + shift2)
 // [m][n2], with x [m][k1], w1 [n1][k1], w2 [n2][n1]; both e and y are written (conv_chain_mfma.hip).

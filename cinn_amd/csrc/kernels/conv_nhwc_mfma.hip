@@ -957,6 +957,7 @@ void RunConvNhwc(const ConvNhwcArgs& a, hipStream_t stream) {
     RunConvStem(a, stream);
     return;
   }
+  if (TryConvFew(a, stream)) return;
   if (TryConvPatch(a, stream)) return;
   if (TryPointwiseConvAsGemm(a, stream)) return;
   const Params p = MakeParams(a);
