@@ -2,12 +2,13 @@
 //   C [M][N] = act( norm(A) [M][K] . B [N][K]^T * scale + shift + residual )
 //
 // Bound by one pass over B.  The tiled kernels give such a product M-tiles that are mostly padding and a handful of blocks;
-// here a block owns 16 output columns of MT row tiles (rows from 16 MT blockIdx.y: the launcher gives every row tile a block
-// of its own where that still leaves CUs) and its eight wavefronts split K in 32-deep blocks.  A lane's share
-// of a 16x16x32 fragment is 8 consecutive k of one row - 16 contiguous bytes in both operands - so fragments come straight
-// from global memory, no LDS on the way: every wavefront keeps 2 U k-blocks of loads in flight, B is read from memory once (by
-// a block of all rows, or by one per row tile of which the others find it in L2), A (at most 64 rows) comes out of L2.  The partial tiles meet in LDS; wavefront t finishes row tile t (2-byte
-// stores: the result is small).
+// here small tiles give most CUs a block and its wavefronts split K.
+//   * gemm_rows_ring_kernel: whole K steps of 64 in aligned rows, operands through rings in LDS in whole lines (few_tile.h: a CU
+//     pulls in three times as much that way);
+//   * gemm_rows_kernel: any other K of 32-deep blocks, operands at any address of their type.  A block owns 16 output columns of
+//     MT row tiles, its eight wavefronts split K, fragments come straight from global memory, 2 U k-blocks of loads in flight.
+// us, the latter | the former, fp16: 8 x 768 -> 768 4.1 | 3.3, 8 x 3072 -> 768 7.2 | 4.7, 64 x 1280 -> 5120 24.7 | 6.4, 16 x 4096 -> 4096 with gelu 10.4 |
+// 6.1; norm inside 8 x 768 -> 3072 5.4 | 4.1, with gelu 6.0 | 4.6.
 //
 // At these sizes a launch costs as much as the product (an empty kernel 3.3 us from launch to launch, 8 x 768 -> 768 5 us),
 // so what surrounds the product in a decoding step is part of it:
@@ -17,14 +18,16 @@
 //   * gelu, on the fp32 sum;
 //   * several result tensors side by side (query, key and value of a token), each a contiguous matrix of its own.
 // A block of one new token per sequence (8 sequences, hidden 768, 12 heads, 511 cached, fp16): nine launches in 46.0 us
-// before, five in 35.9 here.  K need only be whole k-blocks: 8 x 960 -> 960, which ran on 64x64 tiles, 7.0 -> 4.2 us.
+// before, five in 28.8 here (35.9 with fragments straight from memory).
 #include "kernels/gemm_rows.h"
 
+#include <algorithm>
 #include <climits>
 #include <cstdlib>
 #include <type_traits>
 
 #include "cinn_hip_runtime.h"
+#include "kernels/few_tile.h"
 #include "runtime/hip_check.h"
 
 namespace cinn_hip_kernels {
@@ -180,8 +183,228 @@ gemm_rows_kernel(RowProduct p) {
   }
 }
 
+// ---- whole, aligned K steps of 64: operands through rings in LDS (few_tile.h) ------------------------------------------
+using few::u32x4;
+
+// NORM: K steps of a wavefront that hold its share of a normalised row (0: no norm).  A's are requested at once and have LDS of
+// their own; the rows' sums of x and x x run while B's are on their way, then fragments are normalised between LDS and the
+// product.  B is requested at once too where a block has a CU to itself (TN = 1: 8 x 768 -> 3072 4.1 us, two steps at a time
+// 4.5), two steps at a time where rounds of blocks want its LDS (1 x 1280 -> 9984 9.7 | 7.8).
+template <typename T, int TM, int TN, int WAVES, int NORM>
+__global__ void __launch_bounds__(64 * WAVES)
+gemm_rows_ring_kernel(RowProduct p, int tiles_m, int tiles_n) {
+  constexpr int SLOTS = NORM && TN == 1 ? std::max(NORM, 2) : 2;
+  typedef few::Ring<T, TM, TN, SLOTS, NORM == 0> Ring;
+  typedef typename Half16<T>::vec8 vec8;
+  typedef T vec4 __attribute__((ext_vector_type(4)));
+  static_assert(!NORM || TM == 1, "rows are normalised by blocks of one row tile");
+  __shared__ __attribute__((aligned(1024))) char lds[WAVES * Ring::BYTES];
+  __shared__ __attribute__((aligned(1024))) char rows[NORM ? WAVES * NORM * Ring::FRAG : 16];
+  __shared__ float s_sum[NORM ? WAVES : 1][16][2];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  Ring ring(lds, wave, lane);
+  int tm, tn;
+  few::TileOf(blockIdx.x, tiles_m, tiles_n, false, &tm, &tn);
+  const int m0 = tm * (16 * TM), n0 = tn * (16 * TN);
+  const int row_bytes = p.k * 2, steps = p.k / 64;
+  unsigned a_off[2 * TM], b_off[2 * TN];  // of the lane's chunks; rows beyond the last repeat it
+#pragma unroll
+  for (int i = 0; i < 2 * TM; ++i)
+    a_off[i] = (unsigned)min(m0 + 8 * i + (lane >> 3), p.m - 1) * (unsigned)row_bytes + (few::ChunkAt(lane & 7, 8 * (i & 1) + (lane >> 3)) << 4);
+#pragma unroll
+  for (int j = 0; j < 2 * TN; ++j)
+    b_off[j] = (unsigned)min(n0 + 8 * j + (lane >> 3), p.n - 1) * (unsigned)row_bytes + (few::ChunkAt(lane & 7, 8 * (j & 1) + (lane >> 3)) << 4);
+  // what the epilogue reads, see below
+  constexpr int FINISH = (TM * TN + WAVES - 1) / WAVES;
+  f32x4 sc[FINISH], sh[FINISH];
+  vec4 res[FINISH];
+#pragma unroll
+  for (int f = 0; f < FINISH; ++f) {
+    const int frag = wave + f * WAVES, row = m0 + 16 * (frag / TN) + (lane & 15), col = n0 + 16 * (frag % TN) + (lane >> 4) * 4;
+    const bool mine = frag < TM * TN && row < p.m && col < p.n;
+    sc[f]  = f32x4{p.alpha, p.alpha, p.alpha, p.alpha};
+    sh[f]  = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    res[f] = vec4{(T)0.0f, (T)0.0f, (T)0.0f, (T)0.0f};
+    if (mine && p.scale) sc[f] = *reinterpret_cast<const f32x4*>(p.scale + col);
+    if (mine && p.shift) sh[f] = *reinterpret_cast<const f32x4*>(p.shift + col);
+    if (mine && p.residual) res[f] = *reinterpret_cast<const vec4*>(static_cast<const T*>(p.residual) + (int64_t)row * p.n + col);
+  }
+  const int s0 = steps * wave / WAVES, mine = steps * (wave + 1) / WAVES - s0;
+  const char* a = static_cast<const char*>(p.a) + (int64_t)s0 * few::kStepBytes;
+  const char* b = static_cast<const char*>(p.b) + (int64_t)s0 * few::kStepBytes;
+  if constexpr (NORM == 0) {
+    ring.Run(mine, [&](int slot) {
+#pragma unroll
+      for (int j = 0; j < 2 * TN; ++j) few::CopyAt(ring.W(slot, j), b, b_off[j]);
+#pragma unroll
+      for (int i = 0; i < 2 * TM; ++i) few::CopyAt(ring.X(slot, i), a, a_off[i]);
+      a += few::kStepBytes, b += few::kStepBytes;
+    });
+  } else {
+    vec8 g[NORM][2], be[NORM][2];
+#pragma unroll
+    for (int d = 0; d < NORM; ++d)
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        const int k  = (s0 + max(min(d, mine - 1), 0)) * 64 + half * 32 + (lane >> 4) * 8;
+        g[d][half]  = *reinterpret_cast<const vec8*>(static_cast<const T*>(p.gamma) + k);
+        be[d][half] = *reinterpret_cast<const vec8*>(static_cast<const T*>(p.beta) + k);
+      }
+    const char* my_rows     = rows + wave * NORM * Ring::FRAG;
+    const unsigned rows_at = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) char*)my_rows);
+#pragma unroll
+    for (int d = 0; d < NORM; ++d)
+      if (d < mine) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) few::CopyAt(rows_at + d * Ring::FRAG + i * (Ring::FRAG / 2), a + d * few::kStepBytes, a_off[i]);
+      }
+    auto request = [&](int d) {
+#pragma unroll
+      for (int j = 0; j < 2 * TN; ++j) few::CopyAt(ring.W(d % SLOTS, j), b + d * few::kStepBytes, b_off[j]);
+    };
+#pragma unroll
+    for (int d = 0; d < NORM && d < SLOTS; ++d)
+      if (d < mine) request(d);
+    switch (min(mine, SLOTS)) {  // A is there, B may be on its way
+      case 0: break;
+      case 1: few::WaitLoads<2 * TN>(); break;
+      case 2: few::WaitLoads<4 * TN>(); break;
+      case 3: few::WaitLoads<6 * TN>(); break;
+      case 4: few::WaitLoads<8 * TN>(); break;
+      default: few::WaitLoads<10 * TN>(); break;
+    }
+    float s = 0.0f, q = 0.0f;
+    vec8 x[NORM][2];
+#pragma unroll
+    for (int d = 0; d < NORM; ++d)
+      if (d < mine) {
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+          x[d][half] = *reinterpret_cast<const vec8*>(my_rows + d * Ring::FRAG + ring.offset[half]);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float v = (float)x[d][half][e];
+            s += v;
+            q = __builtin_fmaf(v, v, q);
+          }
+        }
+      }
+    s += __shfl_xor(s, 16), q += __shfl_xor(q, 16);
+    s += __shfl_xor(s, 32), q += __shfl_xor(q, 32);
+    if (lane < 16) s_sum[wave][lane][0] = s, s_sum[wave][lane][1] = q;
+    __syncthreads();
+    s = q = 0.0f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) s += s_sum[w][lane & 15][0], q += s_sum[w][lane & 15][1];
+    const float mean = s / (float)p.k;
+    const float var  = fmaxf(q / (float)p.k - mean * mean, 0.0f);
+    const float inv  = 1.0f / sqrtf(var + p.epsilon);
+#pragma unroll
+    for (int d = 0; d < NORM; ++d)
+      if (d < mine) {
+        if (SLOTS >= NORM) {
+          if (d == 0) few::WaitLoads<0>();
+        } else if (d + 1 < mine) {
+          few::WaitLoads<2 * TN>();
+        } else {
+          few::WaitLoads<0>();
+        }
+        ring.Read(d % SLOTS);
+        if (d + SLOTS < NORM && d + SLOTS < mine) {
+          few::WaitLdsReads();  // the slot is free
+          request(d + SLOTS);
+        }
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+          vec8 y;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) y[e] = (T)__builtin_fmaf(((float)x[d][half][e] - mean) * inv, (float)g[d][half][e], (float)be[d][half][e]);
+#pragma unroll
+          for (int j = 0; j < TN; ++j) ring.acc[0][j] = few::Multiply<T>(ring.ws[j][half], __builtin_bit_cast(u32x4, y), ring.acc[0][j]);
+        }
+      }
+  }
+  ring.template Meet<WAVES>(lds, wave, lane, [&](int f, int i, int j, f32x4 sum) {
+    const int row = m0 + 16 * i + (lane & 15), col = n0 + 16 * j + (lane >> 4) * 4;
+    if (row >= p.m || col >= p.n) return;
+    const int part = (col >= p.width) + (col >= 2 * p.width);
+    T* to          = static_cast<T*>(part == 0 ? p.c[0] : part == 1 ? p.c[1] : p.c[2]) + (int64_t)row * p.width + (col - part * p.width);
+    vec4 out;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float v = __builtin_fmaf(sum[e], sc[f][e], sh[f][e]);
+      if (p.residual) v = __builtin_fmaf(p.residual_scale, (float)res[f][e], v);
+      asm volatile("" : "+v"(v));  // fp32 first, then one rounding to T: the same for every row
+      if (p.relu) v = v > 0.0f ? v : 0.0f;
+      if (p.gelu) v = v * __builtin_fmaf(0.5f, erff(v * 0.70710678f), 0.5f);
+      out[e] = (T)v;
+    }
+    *reinterpret_cast<vec4*>(to) = out;
+  });
+}
+
+template <typename T, int TM, int TN, int WAVES, int NORM>
+void LaunchRing(const RowProduct& p, hipStream_t stream) {
+  const int tiles_m = (p.m + 16 * TM - 1) / (16 * TM), tiles_n = (p.n + 16 * TN - 1) / (16 * TN);
+  hipLaunchKernelGGL((gemm_rows_ring_kernel<T, TM, TN, WAVES, NORM>), dim3((unsigned)(tiles_m * tiles_n)), dim3(64 * WAVES), 0, stream, p, tiles_m,
+                     tiles_n);
+}
+
+template <typename T, int TN>
+void LaunchNorm(const RowProduct& p, hipStream_t stream) {
+  switch ((p.k / 64 + 3) / 4) {
+    case 1: LaunchRing<T, 1, TN, 4, 1>(p, stream); break;
+    case 2: LaunchRing<T, 1, TN, 4, 2>(p, stream); break;
+    case 3: LaunchRing<T, 1, TN, 4, 3>(p, stream); break;
+    case 4: LaunchRing<T, 1, TN, 4, 4>(p, stream); break;
+    default: LaunchRing<T, 1, TN, 4, 5>(p, stream); break;
+  }
+}
+
+// whole K steps in aligned rows, results in aligned groups of four columns
+bool RingTakes(const RowProduct& p) {
+  uintptr_t wide = 0, four = 0;
+  for (const void* q : {p.a, p.b, static_cast<const void*>(p.scale), static_cast<const void*>(p.shift), p.gamma, p.beta}) wide |= reinterpret_cast<uintptr_t>(q);
+  for (const void* q : {p.residual, static_cast<const void*>(p.c[0]), static_cast<const void*>(p.c[1]), static_cast<const void*>(p.c[2])}) four |= reinterpret_cast<uintptr_t>(q);
+  return p.k % 64 == 0 && p.n % 4 == 0 && p.width % 4 == 0 && wide % 16 == 0 && four % 8 == 0 && (int64_t)p.m * p.k < (1 << 30) && (int64_t)p.n * p.k < (1 << 30);
+}
+
+template <typename T>
+bool TryRing(const RowProduct& p, hipStream_t stream) {
+  if (!RingTakes(p)) return false;
+  if (p.gamma) {
+    // With a block for every CU twice the columns in each: 1 x 384 -> 6272 4.4 | 3.8, 32 x 768 -> 3072 5.5 | 4.5, 16 x 1280 -> 5120 8.8 |
+    // 5.7 (its rings leave room for one block on a CU); 256 blocks 16 x 1024 -> 4096 4.7 | 5.0
+    if ((p.m + 15) / 16 * ((p.n + 15) / 16) > 256) {
+      LaunchNorm<T, 2>(p, stream);
+    } else {
+      LaunchNorm<T, 1>(p, stream);
+    }
+    return true;
+  }
+  struct Tile {
+    int tm, tn, nw;
+    void (*launch)(const RowProduct&, hipStream_t);
+  };
+  static const Tile tiles[] = {{1, 1, 8, LaunchRing<T, 1, 1, 8, 0>}, {1, 1, 4, LaunchRing<T, 1, 1, 4, 0>}, {1, 2, 4, LaunchRing<T, 1, 2, 4, 0>},
+                               {2, 2, 4, LaunchRing<T, 2, 2, 4, 0>}, {2, 4, 4, LaunchRing<T, 2, 4, 4, 0>}, {4, 4, 4, LaunchRing<T, 4, 4, 4, 0>}};
+  const Tile* best = nullptr;
+  double best_us   = 0.0;
+  for (const Tile& t : tiles) {
+    const double us = few::Estimate(p.m, p.n, p.k / 64, false, t.tm, t.tn, t.nw);
+    if (!best || us < best_us) best = &t, best_us = us;
+  }
+  best->launch(p, stream);
+  return true;
+}
+
 template <typename T>
 void Launch(const RowProduct& p, hipStream_t stream) {
+  if (TryRing<T>(p, stream)) {
+    CINN_HIP_CALL(hipGetLastError());
+    return;
+  }
   int mt = (p.m + 15) / 16;
   dim3 grid((unsigned)((p.n + 15) / 16));
   // Fewer column blocks than CUs: one block per 16 rows as well.  A block's traffic is its 16 columns of B plus the
@@ -219,7 +442,7 @@ bool RowProductSupported(const RowProduct& p) {
   return !p.gamma || (p.beta && p.k <= kRowProductMaxNormK);
 }
 
-// Every wavefront waits for its own rows of B: with one block per CU (16 columns each; 16 rows, or all of them from 256 blocks of
+// For gemm_rows_kernel: every wavefront waits for its own rows of B: with one block per CU (16 columns each; 16 rows, or all of them from 256 blocks of
 // columns on) that hides the launch, further ones take about as long again, where the tiled kernels need a few hundred tiles for
 // the same result.  us, tiled | here, fp16, at most as many blocks as CUs: 16 x 192 -> 4096 3.9 | 3.8, 64 x 960 -> 1000 7.3 | 4.3, two row
 // tiles in each 32 x 192 -> 4096 4.0 | 4.6, 32 x 384 -> 4096 4.7 | 4.6; two on a CU: 1 x 384 -> 8192 4.7 | 3.7, 16 x 384 -> 8192 4.8 | 5.2, 16 x 960 ->
@@ -232,6 +455,12 @@ bool RowProductSupported(const RowProduct& p) {
 // 9.1 | 9.7, 24 x 7968 -> 200 9.1 | 11.7 (but 1 x 6112 -> 1000 8.7 | 7.0), 64 x 5024 -> 2048 11.7 | 14.9, 24 x 3968 -> 25 7.2 | 8.7; a layer with its scale
 // and shift has a convolution's tiles instead, 8 x 6112 -> 4096 with gelu 18.7 | 10.0.
 bool RowProductPays(int m, int n, int k, bool saves_launch, bool splits) {
+  if (k % 64 == 0 && n % 4 == 0) {
+    // More than two row tiles of many columns: the tiled kernels' larger tiles pull in less, until K is long enough to be shared.  us,
+    // tiled | here, fp16: 64 x 64 -> 12288 3.7 | 5.3, 64 x 512 -> 12288 5.8 | 6.4, 64 x 512 -> 32768 8.7 | 12.8, 64 x 1024 -> 32768 14.5 | 18.8, 32 x 192 ->
+    // 32768 5.8 | 6.6; 64 x 128 -> 8192 3.9 | 3.9, 64 x 2048 -> 16384 15.0 | 15.2, 32 x 320 -> 32768 6.8 | 6.9, 16 x 1024 -> 8192 7.9 | 3.4.
+    return saves_launch || n <= 8192 || m <= 16 || (m <= 32 && (n <= 16384 || k >= 320)) || k >= (n <= 16384 ? 1024 : 2048);
+  }
   if (k % 256 == 0) return true;
   const int columns = (n + 15) / 16, tiles = (m + 15) / 16;
   const double load = columns < 256 ? (columns * tiles + 255) / 256 : (columns + 255) / 256 * (0.5 + 0.5 * tiles);
@@ -242,7 +471,7 @@ bool RowProductPays(int m, int n, int k, bool saves_launch, bool splits) {
   return load <= (k < 256 ? 1.0 : k < 512 ? 1.5 : 2.0);
 }
 
-// Blocks of one row tile each: B is read for every one of them, and each normalises its rows again, so that the second and third
+// For gemm_rows_kernel, blocks of one row tile each: B is read for every one of them, and each normalises its rows again, so that the second and third
 // round of blocks cost what a kernel of their own does - unless the product alone would be blocks of one row tile as well.  us,
 // separate | inside, fp16, norm: one round 32 x 320 -> 2048 6.7 | 5.7, 64 x 960 -> 1024 10.0 | 6.1; two 32 x 384 -> 4096 7.0 | 8.5, 16 x 960 -> 8192
 // 9.8 | 9.0; three 48 x 960 -> 4096 10.0 | 12.3, 48 x 1280 -> 4096 13.0 | 12.6; more 48 x 384 -> 6272 7.3 | 18.6, 64 x 1280 -> 4096 14.9 | 16.1; the
@@ -253,6 +482,16 @@ bool RowProductPays(int m, int n, int k, bool saves_launch, bool splits) {
 // 64 x 320 -> 1024 9.9 | 6.2, two 16 x 128 -> 8192 8.3 | 8.9, 48 x 192 -> 2048 9.2 | 8.9, three 64 x 320 -> 3072 10.0 | 12.6, six 64 x 1280 -> 6144 28.1 |
 // 24.9, eight 64 x 1280 -> 8192 28.9 | 32.6, four 64 x 768 -> 4096 13.0 | 16.9; the same blocks alone 64 x 768 -> 3072 15.5 | 13.1.
 RowFusion ChooseRowFusion(int m, int n, int k, RowFusion there) {
+  if (k % 64 == 0 && n % 4 == 0) {
+    // gemm_rows_ring_kernel, blocks of 16 or of 32 columns.  us, outside | inside, norm: 1 x 128 -> 4096 5.3 | 3.1, 16 x 1280 -> 5120 6.6 | 5.8,
+    // 32 x 1024 -> 4096 (256 blocks of 32) 5.9 | 5.3, 32 x 512 -> 8192 (512) 5.7 | 5.1, 64 x 768 -> 3072 (384) 6.4 | 6.1; 64 x 384 -> 6272 (784)
+    // 6.3 | 6.9, 8 x 1280 -> 9984 (312) 7.5 | 7.8, 64 x 1024 -> 4096 (512) 6.4 | 7.0, 48 x 1280 -> 5120 (480) 8.1 | 8.2.  gelu: 1 x 768 -> 3072 5.8 |
+    // 3.5, 64 x 512 -> 16384 9.4 | 8.3.  What lies beyond these lines stays as such layers have always been compiled: norm outside at 16 x
+    // 128 -> 8192, inside at 48 x 1280 -> 4096, gelu outside from 64 x 768 -> 8192 on (with K = 2048 10.8 | 9.2).
+    const int tiles = (m + 15) / 16, narrow = tiles * ((n + 15) / 16), wide = tiles * ((n + 31) / 32);
+    const bool norm = narrow <= 256 || ((k >= 192 || n < 8192) && (wide <= 256 || (wide <= 512 && (k < 1024 || (k > 1024 && tiles >= 3)))));
+    return {there.norm && norm, there.gelu && (narrow < 2048 || k < 768)};
+  }
   const int rounds = ((n + 15) / 16 * ((m + 15) / 16) + 255) / 256;
   const bool same  = k % 256 == 0 && n <= 4080;  // the blocks of the product alone
   if (there.norm && there.gelu && (same || rounds <= 1 || (rounds <= 2 && k >= 192) || (rounds <= 6 && k >= 1152))) return there;
