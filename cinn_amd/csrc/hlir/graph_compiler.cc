@@ -10,6 +10,7 @@
 
 #include "hlir/accuracy_checker.h"
 #include "hlir/memory_plan.h"
+#include "kernels/product_group.h"
 #include "optim/optimize.h"
 
 namespace cinn {
@@ -339,7 +340,7 @@ const std::vector<int>& Program::GraphLanes() {
 void Program::RunLanes(void* stream) {
   PlanLanes();
   if (!any_side_) {
-    for (auto& ins : instrs_) ins->Run(stream);
+    RunInOrder(stream);
     return;
   }
   auto main_s = static_cast<hipStream_t>(stream);
@@ -371,9 +372,26 @@ void Program::RunPreRunInstructions(void* stream) {
   prerun_done_ = true;
 }
 
+void Program::RunInOrder(void* stream) {
+  const size_t n = instrs_.size();
+  // a look at an instruction's results, or a range around it, is about that instruction's own launches
+  const bool apart = Flags().blocking() || Flags().range_push;
+  for (size_t i = 0; i < n;) {
+    size_t end = i + 1;
+    while (!apart && instrs_[i]->product && end < n && instrs_[end]->product) ++end;
+    if (end == i + 1) {
+      instrs_[i++]->Run(stream);
+      continue;
+    }
+    cinn_hip_kernels::ProductGroup products;
+    for (; i < end; ++i) instrs_[i]->Run(stream);
+    products.Run();
+  }
+}
+
 void Program::Execute(void* stream) {
   if (!prerun_done_) RunPreRunInstructions(stream);
-  for (auto& ins : instrs_) ins->Run(stream);
+  RunInOrder(stream);
   if (!stream) CINN_HIP_STATUS(cinn_hip_device_synchronize());
 }
 
@@ -507,6 +525,10 @@ std::unique_ptr<Program> GraphCompiler::Build(const CompileOptions& options) {
     CINN_CHECK(fn) << "compiled function " << u.func_name << " not found";
     instr->SetLoweredFunc(fn);
     instr->pre_run = u.pre_run;
+    if (u.members.size() == 1 && u.members[0]->nodes.size() == 1 && target_.arch == common::Target::Arch::AMDGPU) {
+      const std::string& op = u.members[0]->nodes[0]->op_type();
+      instr->product        = op == "matmul" || op == "mul" || op == "hip_matmul_bias";
+    }
     instrs.push_back(std::move(instr));
   }
   int device_count = 0;

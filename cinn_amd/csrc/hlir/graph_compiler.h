@@ -120,6 +120,8 @@ class Instruction {
   std::vector<const void*> ArgAddresses(bool outputs) const;
   // runs once ahead of the first execution instead of in every one (cinn/hlir/framework/instruction.h:129)
   bool pre_run{false};
+  // one matrix product through cinn_call_cublas or cinn_call_hip_matmul_bias and nothing else
+  bool product{false};
 
  private:
   void UpdateArgsCache();
@@ -169,6 +171,8 @@ class Program {
   bool prerun_done_{false};
   void* graph_exec_{nullptr};
   void* graph_{nullptr};
+  // Runs all instructions in order, consecutive matrix products as a group (kernels/product_group.h).
+  void RunInOrder(void* stream);
   // two-lane schedule of a graph replay
   void PlanLanes();
   void RunLanes(void* stream);

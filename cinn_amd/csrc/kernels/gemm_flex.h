@@ -37,4 +37,9 @@ struct FlexPlan {
 bool PlanFlexGemm(const FlexGemm& g, hipStream_t stream, FlexPlan* plan);
 void RunFlexGemm(const FlexGemm& g, FlexPlan plan, hipStream_t stream);
 
+// Up to kFlexGroup unbatched products of one type in one launch; `alone` is how each would run by itself.  false when that is
+// estimated to be faster.
+constexpr int kFlexGroup = 4;
+bool TryFlexGroup(const FlexGemm* g, const FlexPlan* alone, int count, hipStream_t stream);
+
 }  // namespace cinn_hip_kernels

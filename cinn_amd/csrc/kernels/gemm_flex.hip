@@ -56,21 +56,20 @@ __device__ __forceinline__ float Finish(float v, float alpha, float shift, float
 
 // KG groups of four wavefronts (2 x 2 over the tile) share the block's tiles and take a K step's slices in turn; their
 // sums meet in the epilogue.
+// Block `bid` of the tiles, `z` of the splits, batch entry `entry` of `entries`.
 template <typename T, bool A_KC, bool B_KC, int BM, int BN, int KG>
-__global__ void __launch_bounds__(256 * KG, 2)
-flex_gemm_kernel(FlexParams p) {
-  __shared__ __attribute__((aligned(256))) char lds[2 * (BM + BN) * 128];
+__device__ __forceinline__ void FlexBlock(const FlexParams& p, char* lds, int bid, int z, int entry, int entries) {
   const int tid = threadIdx.x;
   int tm, tn;
-  flex::TileOf(blockIdx.x, p.tiles_m, p.tiles_n, &tm, &tn);
+  flex::TileOf(bid, p.tiles_m, p.tiles_n, &tm, &tn);
   const int m0 = tm * BM, n0 = tn * BN;
 
   flex::Tile<T, A_KC, BM, 256 * KG> ta;
   flex::Tile<T, B_KC, BN, 256 * KG> tb;
-  ta.Init(static_cast<const T*>(p.a) + blockIdx.y * p.stride_a, p.lda, m0, p.m, p.k, tid);
-  tb.Init(static_cast<const T*>(p.b) + blockIdx.y * p.stride_b, p.ldb, n0, p.n, p.k, tid);
+  ta.Init(static_cast<const T*>(p.a) + entry * p.stride_a, p.lda, m0, p.m, p.k, tid);
+  tb.Init(static_cast<const T*>(p.b) + entry * p.stride_b, p.ldb, n0, p.n, p.k, tid);
   typename flex::Mma<T, A_KC, B_KC, BM, BN>::acc_t acc;
-  const int s0 = blockIdx.z * p.steps_per_split;
+  const int s0 = z * p.steps_per_split;
   flex::KLoop<T, A_KC, B_KC, BM, BN, KG>(lds, ta, tb, s0, min(s0 + p.steps_per_split, p.steps), p.full_steps, p.k, tid, acc);
 
   const int col0 = n0 + tid % (BN / 8) * 8;  // the eight columns this thread finishes
@@ -84,9 +83,9 @@ flex_gemm_kernel(FlexParams p) {
       for (int e = 0; e < 8; ++e) sh[e] = (float)static_cast<const T*>(p.shift16)[min(col0 + e, p.n - 1)];
     }
   }
-  T* c              = static_cast<T*>(p.c) + blockIdx.y * p.stride_c;
-  const T* residual = p.residual ? static_cast<const T*>(p.residual) + blockIdx.y * p.stride_c : nullptr;
-  float* plane      = p.partials + ((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * p.m * p.n;
+  T* c              = static_cast<T*>(p.c) + entry * p.stride_c;
+  const T* residual = p.residual ? static_cast<const T*>(p.residual) + entry * p.stride_c : nullptr;
+  float* plane      = p.partials + ((int64_t)z * entries + entry) * p.m * p.n;
   flex::EachRowGroup<T, A_KC, B_KC, BM, BN, KG>(lds, acc, tid, [&](int row, int, const float (&v)[8]) {
     const int m = m0 + row;
     if (m >= p.m || cols <= 0) return;
@@ -117,12 +116,55 @@ flex_gemm_kernel(FlexParams p) {
   });
 }
 
+template <typename T, bool A_KC, bool B_KC, int BM, int BN, int KG>
+__global__ void __launch_bounds__(256 * KG, 2)
+flex_gemm_kernel(FlexParams p) {
+  __shared__ __attribute__((aligned(256))) char lds[2 * (BM + BN) * 128];
+  FlexBlock<T, A_KC, B_KC, BM, BN, KG>(p, lds, blockIdx.x, blockIdx.z, blockIdx.y, gridDim.y);
+}
+
+// Several products on 64x64 tiles.  A layer's y, dx and dW are three products of the same volume, which each took a launch and
+// mostly one more to add the partial sums of a split K, because none has the tiles for all CUs by itself: small ones are bound by
+// those launches (about 3 us each), larger ones by their nearly empty rounds.  Together they share the CUs and one addition.  us of
+// the step with its two column sums, one by one | together: 37 x 75 -> 247 fp16 19.8 | 9.4, 665 x 233 -> 670 bf16 28.5 | 13.9,
+// 874 x 1237 -> 440 fp32 68 | 50, 630 x 2558 -> 1999 bf16 88 | 67.
+// Blocks [first[i], first[i + 1]) are product i's, split by split, the tiles of each in whole rounds of the XCDs (what is beyond
+// them returns at once): TileOf's neighbours stay on one XCD.
+struct GroupParams {
+  FlexParams p[kFlexGroup];
+  int first[kFlexGroup + 1];
+  int layout[kFlexGroup];  // bit 0: a_kc, bit 1: b_kc
+  int count;
+};
+
+__device__ __forceinline__ int MemberOf(const int* first, int count, int bid) {
+  int i = 0;
+  while (i + 1 < count && bid >= first[i + 1]) ++i;
+  return i;
+}
+
+template <typename T>
+__global__ void __launch_bounds__(256, 2)
+flex_group_kernel(GroupParams g) {
+  __shared__ __attribute__((aligned(256))) char lds[2 * 128 * 128];
+  const int i         = MemberOf(g.first, g.count, blockIdx.x);
+  const FlexParams& p = g.p[i];
+  const int tiles = p.tiles_m * p.tiles_n, round = (tiles + 7) & ~7, at = (int)blockIdx.x - g.first[i];
+  const int z = at / round, bid = at - z * round;
+  if (bid >= tiles) return;
+  switch (g.layout[i]) {
+    case 0: FlexBlock<T, false, false, 64, 64, 1>(p, lds, bid, z, 0, 1); break;
+    case 1: FlexBlock<T, true, false, 64, 64, 1>(p, lds, bid, z, 0, 1); break;
+    case 2: FlexBlock<T, false, true, 64, 64, 1>(p, lds, bid, z, 0, 1); break;
+    default: FlexBlock<T, true, true, 64, 64, 1>(p, lds, bid, z, 0, 1); break;
+  }
+}
+
 // Adds the planes of a split reduction and applies the epilogue: one thread per V consecutive elements of a plane row
 // (V divides n), planes in ascending order.
 template <typename T, int V>
-__global__ void __launch_bounds__(256)
-flex_reduce_kernel(FlexParams p, int splits, int64_t plane) {
-  const int64_t at = ((int64_t)blockIdx.x * 256 + threadIdx.x) * V;
+__device__ __forceinline__ void ReduceBlock(const FlexParams& p, int splits, int64_t plane, int bid) {
+  const int64_t at = ((int64_t)bid * 256 + threadIdx.x) * V;
   if (at >= plane) return;
   float v[V];
   __builtin_memcpy(v, p.partials + at, V * 4);
@@ -148,6 +190,25 @@ flex_reduce_kernel(FlexParams p, int splits, int64_t plane) {
   for (int e = 0; e < V; ++e)
     out[e] = (T)Finish(v[e], p.alpha, sh[e], p.residual_scale, (float)res[e]);
   __builtin_memcpy(static_cast<T*>(p.c) + at, out, V * sizeof(T));
+}
+
+template <typename T, int V>
+__global__ void __launch_bounds__(256)
+flex_reduce_kernel(FlexParams p, int splits, int64_t plane) {
+  ReduceBlock<T, V>(p, splits, plane, blockIdx.x);
+}
+
+template <typename T>
+__global__ void __launch_bounds__(256)
+flex_group_reduce_kernel(GroupParams g) {
+  const int i         = MemberOf(g.first, g.count, blockIdx.x);
+  const FlexParams& p = g.p[i];
+  const int splits = (p.steps + p.steps_per_split - 1) / p.steps_per_split, bid = (int)blockIdx.x - g.first[i];
+  if (p.n % 4 == 0) {
+    ReduceBlock<T, 4>(p, splits, (int64_t)p.m * p.n, bid);
+  } else {
+    ReduceBlock<T, 1>(p, splits, (int64_t)p.m * p.n, bid);
+  }
 }
 
 // K steps that neither loader has to guard
@@ -230,8 +291,9 @@ void LaunchTiles(const FlexPlan& plan, dim3 grid, const FlexParams& p, hipStream
   }
 }
 
+// everything but the partial sums' place; `plan.splits` becomes the splits that there are
 template <typename T>
-void Launch(const FlexGemm& g, FlexPlan plan, hipStream_t stream) {
+FlexParams ParamsOf(const FlexGemm& g, FlexPlan* plan) {
   FlexParams p;
   p.a = g.a, p.b = g.b, p.c = g.c;
   p.m = g.m, p.n = g.n, p.k = g.k;
@@ -241,12 +303,19 @@ void Launch(const FlexGemm& g, FlexPlan plan, hipStream_t stream) {
   p.full_steps = std::min(FullSteps<T>(g.a_kc, g.lda, g.m, g.k), FullSteps<T>(g.b_kc, g.ldb, g.n, g.k));
   p.shift = g.shift, p.shift16 = g.shift16, p.residual = g.residual;
   p.alpha = g.alpha, p.residual_scale = g.residual_scale;
+  p.steps_per_split = (p.steps + plan->splits - 1) / plan->splits;
+  plan->splits      = (p.steps + p.steps_per_split - 1) / p.steps_per_split;
+  p.tiles_m         = (g.m + plan->tile - 1) / plan->tile;
+  p.tiles_n         = (g.n + plan->tile - 1) / plan->tile;
+  p.partials        = nullptr;
+  return p;
+}
+
+template <typename T>
+void Launch(const FlexGemm& g, FlexPlan plan, hipStream_t stream) {
+  FlexParams p        = ParamsOf<T>(g, &plan);
   const int64_t plane = (int64_t)g.batch * g.m * g.n;
-  p.steps_per_split = (p.steps + plan.splits - 1) / plan.splits;
-  plan.splits       = (p.steps + p.steps_per_split - 1) / p.steps_per_split;
-  p.tiles_m         = (g.m + plan.tile - 1) / plan.tile;
-  p.tiles_n         = (g.n + plan.tile - 1) / plan.tile;
-  p.partials = plan.splits > 1 ? static_cast<float*>(Scratch(ScratchKind::kSplitK, PlaneBytes(g, plan.splits), stream)) : nullptr;
+  if (plan.splits > 1) p.partials = static_cast<float*>(Scratch(ScratchKind::kSplitK, PlaneBytes(g, plan.splits), stream));
   const dim3 grid((unsigned)(p.tiles_m * p.tiles_n), g.batch, plan.splits);
   if (g.a_kc && g.b_kc) LaunchTiles<T, true, true>(plan, grid, p, stream);
   if (g.a_kc && !g.b_kc) LaunchTiles<T, true, false>(plan, grid, p, stream);
@@ -260,6 +329,45 @@ void Launch(const FlexGemm& g, FlexPlan plan, hipStream_t stream) {
       hipLaunchKernelGGL((flex_reduce_kernel<T, 1>), dim3((unsigned)((plane + 255) / 256)), dim3(256), 0, stream, p, plan.splits,
                          plane);
     }
+  }
+  CINN_HIP_CALL(hipGetLastError());
+}
+
+template <typename T>
+void LaunchGroup(const FlexGemm* g, const int* splits, int count, hipStream_t stream) {
+  GroupParams group;
+  group.count = count;
+  size_t bytes = 0, at[kFlexGroup];
+  int blocks = 0;
+  for (int i = 0; i < count; ++i) {
+    FlexPlan plan{64, 1, splits[i], 0.0};
+    group.p[i]      = ParamsOf<T>(g[i], &plan);
+    group.layout[i] = (g[i].a_kc ? 1 : 0) | (g[i].b_kc ? 2 : 0);
+    group.first[i]  = blocks;
+    blocks += (group.p[i].tiles_m * group.p[i].tiles_n + 7) / 8 * 8 * plan.splits;
+    at[i] = SIZE_MAX;
+    if (plan.splits > 1) at[i] = bytes, bytes += (PlaneBytes(g[i], plan.splits) + 255) / 256 * 256;
+  }
+  group.first[count] = blocks;
+  if (bytes) {
+    char* planes = static_cast<char*>(Scratch(ScratchKind::kSplitK, bytes, stream));
+    for (int i = 0; i < count; ++i)
+      if (at[i] != SIZE_MAX) group.p[i].partials = reinterpret_cast<float*>(planes + at[i]);
+  }
+  hipLaunchKernelGGL((flex_group_kernel<T>), dim3((unsigned)blocks), dim3(256), 0, stream, group);
+  if (bytes) {
+    GroupParams reduce;
+    reduce.count = 0;
+    blocks       = 0;
+    for (int i = 0; i < count; ++i) {
+      if (!group.p[i].partials) continue;
+      reduce.p[reduce.count]       = group.p[i];
+      reduce.first[reduce.count++] = blocks;
+      const int64_t threads = (int64_t)g[i].m * g[i].n / (g[i].n % 4 == 0 ? 4 : 1);
+      blocks += (int)((threads + 255) / 256);
+    }
+    reduce.first[reduce.count] = blocks;
+    hipLaunchKernelGGL((flex_group_reduce_kernel<T>), dim3((unsigned)blocks), dim3(256), 0, stream, reduce);
   }
   CINN_HIP_CALL(hipGetLastError());
 }
@@ -278,6 +386,65 @@ void RunFlexGemm(const FlexGemm& g, FlexPlan plan, hipStream_t stream) {
     case FlexType::kBF16: Launch<__bf16>(g, plan, stream); break;
     case FlexType::kF32: Launch<float>(g, plan, stream); break;
   }
+}
+
+// The split of a group: all products with at most the same number of K steps in a block, the number that the model of ChoosePlan
+// likes best.  Against the sum of the separate estimates one tenth is asked for.  Over 70 linear layers' steps (y, dx and dW; 32 to
+// 12950 rows of 65 to 3989 values, the three types) all whose estimate was that far below were faster together, by 1.17 to 2.1.
+// Those above it were about even (68 | 65 us at 12950 x 108 -> 1200 in fp16, 91 | 81 at 7863 x 1533 -> 116) or slower (96 | 119 at
+// 4887 x 301 -> 2123): large products have 128x128 tiles by themselves.
+bool TryFlexGroup(const FlexGemm* g, const FlexPlan* alone, int count, hipStream_t stream) {
+  static const bool enabled = !(getenv("FLAGS_cinn_hip_gemm_group") && atoi(getenv("FLAGS_cinn_hip_gemm_group")) == 0);
+  if (!enabled || count < 2 || count > kFlexGroup) return false;
+  const bool fp32 = g[0].type == FlexType::kF32;
+  int longest = 0;
+  double sum = 0.0;
+  for (int i = 0; i < count; ++i) {
+    if (g[i].type != g[0].type || g[i].batch != 1 || !Fits(g[i])) return false;
+    longest = std::max(longest, Steps(g[i]));
+    sum += alone[i].us;
+  }
+  const double one = fp32 ? 0.62 : 0.42, shared = fp32 ? 0.50 : 0.245, start = fp32 ? 2.0 : 3.0;  // as in ChoosePlan
+  const size_t room = ScratchLimit(ScratchKind::kSplitK, stream);
+  int splits[kFlexGroup] = {1, 1, 1, 1};
+  double best = 1e30;
+  for (int most = longest;;) {
+    int s[kFlexGroup], block = 0;
+    double steps = 0.0, bytes = 0.0, blocks = 0.0;
+    size_t planes = 0;
+    for (int i = 0; i < count; ++i) {
+      const int all = Steps(g[i]);
+      const double tiles = (double)((g[i].m + 63) / 64) * ((g[i].n + 63) / 64);
+      s[i]            = std::min(16, (all + most - 1) / most);
+      const int share = (all + s[i] - 1) / s[i];
+      block = std::max(block, share);
+      blocks += (tiles + 7) * s[i];
+      steps += tiles * s[i] * (share + start);
+      if (s[i] > 1) bytes += 8.0 * s[i] * g[i].m * g[i].n, planes += (PlaneBytes(g[i], s[i]) + 255) / 256 * 256;
+    }
+    // the CUs' throughput and half of the last round, or the longest block by itself
+    double us = std::max(steps / 256 * shared + 0.5 * block * shared, (block + start) * one);
+    if (bytes > 0.0) us += 4.0 + bytes / 4e6;
+    if (planes <= room && blocks < 1e9 && us < best) {
+      best = us;
+      std::copy(s, s + count, splits);
+    }
+    if (most <= 4) break;
+    most = std::max(4, most > 8 ? most * 3 / 4 : most - 1);
+  }
+  if (best >= 0.9 * sum) return false;
+  // the longest blocks first
+  FlexGemm ordered[kFlexGroup];
+  int order[kFlexGroup] = {0, 1, 2, 3}, ordered_splits[kFlexGroup];
+  auto share = [&](int i) { return (Steps(g[i]) + splits[i] - 1) / splits[i]; };
+  std::stable_sort(order, order + count, [&](int x, int y) { return share(x) > share(y); });
+  for (int i = 0; i < count; ++i) ordered[i] = g[order[i]], ordered_splits[i] = splits[order[i]];
+  switch (g[0].type) {
+    case FlexType::kF16: LaunchGroup<_Float16>(ordered, ordered_splits, count, stream); break;
+    case FlexType::kBF16: LaunchGroup<__bf16>(ordered, ordered_splits, count, stream); break;
+    case FlexType::kF32: LaunchGroup<float>(ordered, ordered_splits, count, stream); break;
+  }
+  return true;
 }
 
 }  // namespace cinn_hip_kernels

@@ -29,6 +29,7 @@
 #include "kernels/conv_nhwc.h"
 #include "kernels/gemm_flex.h"
 #include "kernels/gemm_rows.h"
+#include "kernels/product_group.h"
 #include "runtime/hip_check.h"
 
 namespace {
@@ -1327,6 +1328,8 @@ struct GemmProblem {
   bool keep_in_cache{false};
   // a split that the scratch has no room for while the stream is captured stays whole, instead of aborting
   bool whole_without_scratch{false};
+  // only whether a kernel of this file takes the product is asked: nothing is launched
+  bool dry{false};
 };
 
 // Sum of the fp32 partial tiles of a split reduction, then the epilogue of gemm16_dma_kernel: 8 columns per thread
@@ -1414,6 +1417,7 @@ template <typename T, bool B_KC, int BM, int BN, int WAVES_M, int WAVES_N, bool 
           bool PAIR = false, bool A_KC = true>
 void LaunchDma16(const GemmProblem& p, hipStream_t stream, int splits = 1) {
   using cinn_hip_kernels::ScratchKind;
+  if (p.dry) return;
   if (p.whole_without_scratch && splits > 1 &&
       (size_t)splits * p.m * p.n * sizeof(float) > cinn_hip_kernels::ScratchLimit(ScratchKind::kSplitK, stream))
     splits = 1;
@@ -1460,6 +1464,7 @@ void LaunchDma16(const GemmProblem& p, hipStream_t stream, int splits = 1) {
 // FLAGS_cinn_hip_gemm_shortk=0 switches it off.
 template <typename T, int NT, int KH>
 void LaunchShortK(const GemmProblem& p, hipStream_t stream) {
+  if (p.dry) return;
   const int ny     = p.n / (NT * 16);
   const int groups = (p.m + 15) / 16;
   // two blocks of four wavefronts per CU, spread evenly over the XCDs and the column panels
@@ -1534,7 +1539,7 @@ bool TrySkinny(const GemmProblem& p, hipStream_t stream) {
   r.residual       = p.residual ? p.residual : (p.beta != 0.0f ? p.c : nullptr);
   r.residual_scale = p.residual ? p.residual_scale : p.beta;
   if (!cinn_hip_kernels::RowProductSupported(r) || !cinn_hip_kernels::RowProductPays(p.m, p.n, p.k, false, p.scale == nullptr)) return false;
-  cinn_hip_kernels::RunRowProduct(r, stream);
+  if (!p.dry) cinn_hip_kernels::RunRowProduct(r, stream);
   return true;
 }
 
@@ -1834,11 +1839,40 @@ bool ForceGeneric() {
   return force;
 }
 
+// The plan with which gemm_flex.hip would run the product; false when another kernel takes it.
+bool RunsFlexible(const GemmProblem& product, hipStream_t stream, cinn_hip_kernels::FlexPlan* plan) {
+  GemmProblem p = product;
+  p.dry         = true;
+  if (ForceGeneric() || p.type == GemmType::kF64 || p.batch != 1 || !cinn_hip_kernels::PlanFlexGemm(FlexOf(p), stream, plan)) return false;
+  if (p.type == GemmType::kF32) {
+    const bool aligned16 = reinterpret_cast<uintptr_t>(p.a) % 16 == 0 && reinterpret_cast<uintptr_t>(p.b) % 16 == 0;
+    return !aligned16 || p.m % kF32Tile != 0 || p.n % kF32Tile != 0 || p.k % kF32K != 0;
+  }
+  const bool bf16 = p.type == GemmType::kBF16;
+  if (p.trans_a) return !(bf16 ? TryDmaTransposedA<__bf16>(p, plan->us, stream) : TryDmaTransposedA<_Float16>(p, plan->us, stream));
+  return !(bf16 ? TryDma16<__bf16>(p, stream) : TryDma16<_Float16>(p, stream));
+}
+
+// the products that wait in this thread's ProductGroup
+struct WaitingProducts {
+  bool open{false};
+  int count{0};
+  hipStream_t stream{nullptr};
+  GemmProblem p[cinn_hip_kernels::kFlexGroup];
+};
+thread_local WaitingProducts t_waiting;
+
+void WaitInGroup(const GemmProblem& p, hipStream_t stream);
+
 void RunGemm(const GemmProblem& p, hipStream_t stream) {
   CINN_RT_CHECK(p.m > 0 && p.n > 0 && p.k > 0 && p.batch > 0, "gemm: dimensions must be positive, got m=%d n=%d k=%d batch=%d",
                 p.m, p.n, p.k, p.batch);
   CINN_RT_CHECK(p.a && p.b && p.c, "gemm: null operand");
   CINN_RT_CHECK(p.batch <= 65535, "gemm: batch %d exceeds the grid limit", p.batch);
+  if (t_waiting.open) {
+    WaitInGroup(p, stream);
+    return;
+  }
   const bool aligned16 = reinterpret_cast<uintptr_t>(p.a) % 16 == 0 && reinterpret_cast<uintptr_t>(p.b) % 16 == 0 &&
                          p.stride_a % 8 == 0 && p.stride_b % 8 == 0;
   const bool whole32 = !ForceGeneric() && aligned16 && p.m % kF32Tile == 0 && p.n % kF32Tile == 0 && p.k % kF32K == 0;
@@ -1893,6 +1927,59 @@ void RunGemm(const GemmProblem& p, hipStream_t stream) {
   CINN_HIP_CALL(hipGetLastError());
 }
 
+// Launches what waits: the products that gemm_flex.hip would run in one launch where that is faster, the others one by one.
+void RunWaiting() {
+  using namespace cinn_hip_kernels;
+  WaitingProducts& w = t_waiting;
+  w.open = false;  // the products are launched now
+  bool done[kFlexGroup] = {};
+  if (w.count > 1) {
+    FlexGemm g[kFlexGroup];
+    FlexPlan plans[kFlexGroup];
+    int members[kFlexGroup], count = 0;
+    for (int i = 0; i < w.count; ++i) {
+      if ((count > 0 && w.p[i].type != w.p[members[0]].type) || !RunsFlexible(w.p[i], w.stream, &plans[count])) continue;
+      g[count]         = FlexOf(w.p[i]);
+      members[count++] = i;
+    }
+    if (TryFlexGroup(g, plans, count, w.stream))
+      for (int i = 0; i < count; ++i) done[members[i]] = true;
+  }
+  for (int i = 0; i < w.count; ++i)
+    if (!done[i]) RunGemm(w.p[i], w.stream);
+  w.count = 0;
+  w.open  = true;
+}
+
+struct Range {
+  uintptr_t begin, end;
+};
+
+Range Memory(const void* at, int64_t elements, GemmType type) {
+  const uintptr_t begin = reinterpret_cast<uintptr_t>(at);
+  const int bytes = type == GemmType::kF64 ? 8 : type == GemmType::kF32 ? 4 : 2;
+  return {begin, begin + (at ? elements * bytes : 0)};
+}
+
+bool Overlap(const Range& x, const Range& y) { return x.begin < y.end && y.begin < x.end; }
+
+Range Written(const GemmProblem& p) { return Memory(p.c, (p.batch - 1) * p.stride_c + (int64_t)p.m * p.n, p.type); }
+
+bool Touches(const GemmProblem& p, const Range& r) {
+  return Overlap(r, Written(p)) || Overlap(r, Memory(p.a, (p.batch - 1) * p.stride_a + (int64_t)p.m * p.k, p.type)) ||
+         Overlap(r, Memory(p.b, (p.batch - 1) * p.stride_b + (int64_t)p.k * p.n, p.type)) ||
+         Overlap(r, Memory(p.shift, p.n, GemmType::kF32)) || Overlap(r, Memory(p.shift16, p.n, p.type));
+}
+
+void WaitInGroup(const GemmProblem& p, hipStream_t stream) {
+  WaitingProducts& w = t_waiting;
+  bool apart = w.count == cinn_hip_kernels::kFlexGroup || (w.count > 0 && w.stream != stream);
+  for (int i = 0; i < w.count && !apart; ++i) apart = Touches(p, Written(w.p[i])) || Touches(w.p[i], Written(p));
+  if (apart) RunWaiting();
+  w.stream       = stream;
+  w.p[w.count++] = p;
+}
+
 GemmType TypeOf(const cinn_buffer_t* buf) {
   int bytes = buf->type.bits / CHAR_BIT;
   if (buf->type.code == cinn_type_float && bytes == 2) return GemmType::kF16;
@@ -1912,6 +1999,13 @@ cinn_buffer_t* BufferArg(void* v_args, int index) {
 }  // namespace
 
 namespace cinn_hip_kernels {
+
+ProductGroup::ProductGroup() {
+  CINN_RT_CHECK(!t_waiting.open, "a thread has one group of products at a time");
+  t_waiting.open = true;
+}
+ProductGroup::~ProductGroup() { t_waiting.open = false, t_waiting.count = 0; }
+void ProductGroup::Run() { RunWaiting(); }
 
 bool ConvPairShape(int64_t m, int c1, int c2, int oc) {
   if (m <= 0 || m >= INT_MAX || c1 <= 0 || c2 <= 0 || oc <= 0 || c1 % kD64BK != 0 || c2 % kD64BK != 0 || oc % 8 != 0) return false;
