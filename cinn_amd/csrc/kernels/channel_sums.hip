@@ -60,7 +60,12 @@ __device__ __forceinline__ void LoadChannels(const T* p, float (&v)[E]) {
     v[0] = (float)*p;
   } else {
     typedef T chunk_t __attribute__((ext_vector_type(E)));
-    const chunk_t c = __builtin_bit_cast(chunk_t, LoadAny<T>(reinterpret_cast<const char*>(p)));
+    chunk_t c;
+    if constexpr (sizeof(chunk_t) == 16) {
+      c = __builtin_bit_cast(chunk_t, LoadAny<T>(reinterpret_cast<const char*>(p)));
+    } else {
+      __builtin_memcpy(&c, __builtin_assume_aligned(p, sizeof(chunk_t)), sizeof(chunk_t));
+    }
 #pragma unroll
     for (int e = 0; e < E; ++e) v[e] = (float)c[e];
   }
@@ -262,6 +267,14 @@ channel_apply_kernel(ApplyParams p) {
   }
 }
 
+// Channels of a thread: 16 bytes where the tensors allow it, and 4 where that would not give 256 CUs a block each at two pixels a
+// thread.  Blocks by themselves on a CU are bound by one thread's instructions (eight channels' conversions, divisions and
+// square roots, one after the other), not by loads: 525 pixels of 48 channels in fp16 took, sums 3.9, normalisation
+// 4.2, gradient's sums 4.8, gradient 5.7 us with 2 to 4 blocks of wide threads, and 3.0, 3.6, 3.2 and 3.1 with 16 to 31 of
+// narrow ones.  A line four times as high changes nothing for these kernels (60 convolutions' training steps: within 0.1% in the
+// geometric mean), one a quarter as high loses 0.4%.
+bool Few(int64_t pixels, int channels, int chunk) { return pixels * (channels / chunk) < 256 * 512; }
+
 // lanes of a block side by side over channel chunks: a power of two, at most 64
 int ChunkLanes(int chunks) {
   int lanes = 1;
@@ -274,23 +287,29 @@ void Apply(ApplyParams p, bool grad, hipStream_t stream) {
   constexpr int E = 16 / (int)sizeof(T);
   auto aligned    = [](const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; };
   const bool wide  = p.channels % E == 0 && aligned(p.a) && aligned(p.x) && aligned(p.out) && aligned(p.result);
-  const int chunks = p.channels / (wide ? E : 1);
+  constexpr int F  = 4 / (int)sizeof(T);
+  const bool few   = wide && Few(p.pixels, p.channels, E);
+  const int chunks = p.channels / (few ? F : wide ? E : 1);
   p.chunk_lanes    = ChunkLanes(chunks);
   const int column_blocks = (chunks + p.chunk_lanes - 1) / p.chunk_lanes, rows = 256 / p.chunk_lanes;
-  // four pixels per thread, more where that would be over 4096 blocks
-  int64_t blocks = std::max<int64_t>(1, std::min<int64_t>(4096 / column_blocks, p.pixels / (4 * rows)));
+  // four pixels per thread, more where that would be over 4096 blocks; two, one trip to memory, up to two blocks for every CU
+  int64_t blocks = std::min<int64_t>(4096 / column_blocks, p.pixels / (4 * rows));
+  blocks         = std::max<int64_t>({1, blocks, std::min<int64_t>(512 / column_blocks, p.pixels / (2 * rows))});
   p.pixels_per_block = (int)((p.pixels + blocks - 1) / blocks);
   blocks             = (p.pixels + p.pixels_per_block - 1) / p.pixels_per_block;
   const dim3 grid(column_blocks, (unsigned)blocks);
 #define CINN_APPLY(E, GRAD, MASKED) hipLaunchKernelGGL((channel_apply_kernel<T, E, GRAD, MASKED>), grid, dim3(256), 0, stream, p)
   if (!grad) {
-    if (wide) CINN_APPLY(E, false, false);
+    if (few) CINN_APPLY(F, false, false);
+    else if (wide) CINN_APPLY(E, false, false);
     else CINN_APPLY(1, false, false);
   } else if (p.out) {
-    if (wide) CINN_APPLY(E, true, true);
+    if (few) CINN_APPLY(F, true, true);
+    else if (wide) CINN_APPLY(E, true, true);
     else CINN_APPLY(1, true, true);
   } else {
-    if (wide) CINN_APPLY(E, true, false);
+    if (few) CINN_APPLY(F, true, false);
+    else if (wide) CINN_APPLY(E, true, false);
     else CINN_APPLY(1, true, false);
   }
 #undef CINN_APPLY
@@ -313,12 +332,17 @@ void Sums(SumsParams p, bool grad, float* first, float* second, hipStream_t stre
   constexpr int E = 16 / (int)sizeof(T);
   auto aligned    = [](const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; };
   const bool wide = p.channels % E == 0 && aligned(p.a) && aligned(p.x) && aligned(p.out);
-  const int chunks = p.channels / (wide ? E : 1);
+  constexpr int F = 4 / (int)sizeof(T);
+  bool few        = wide && Few(p.pixels, p.channels, E);
+  int chunks      = p.channels / (few ? F : wide ? E : 1);
   p.chunk_lanes    = ChunkLanes(chunks);
   const int column_blocks = (chunks + p.chunk_lanes - 1) / p.chunk_lanes;
   const int rows          = 256 / p.chunk_lanes;
-  // two blocks for every CU, at least eight pixels for every thread
-  int64_t splits = std::max<int64_t>(1, std::min<int64_t>(512 / column_blocks, p.pixels / (8 * rows)));
+  // Two blocks for every CU, at least eight pixels for every thread; or as many as it loads at a time, one trip to memory, while
+  // there are no more planes than channel_planes_kernel loads at a time (with two trips and more 5.5 us instead of 4.2 for the
+  // gradient's sums of 3915 pixels of 16 channels in fp32).
+  int64_t splits = std::min<int64_t>(512 / column_blocks, p.pixels / (8 * rows));
+  splits = std::max<int64_t>({1, splits, std::min<int64_t>({64, 512 / column_blocks, p.pixels / ((grad ? 2 : 4) * rows)})});
   p.pixels_per_split = (int)((p.pixels + splits - 1) / splits);
   splits             = (p.pixels + p.pixels_per_split - 1) / p.pixels_per_split;
   p.splits = (int)splits, p.first = first, p.second = second;
@@ -327,14 +351,17 @@ void Sums(SumsParams p, bool grad, float* first, float* second, hipStream_t stre
   if (plane_bytes > ScratchLimit(ScratchKind::kSplitK, stream)) {
     // under capture without an eager run or a reservation: a block walks all splits of its channels, four chunks of them,
     // and needs no planes
-    p.chunk_lanes = std::min(p.chunk_lanes, 4);
+    few           = false;
+    chunks        = p.channels / (wide ? E : 1);
+    p.chunk_lanes = std::min(ChunkLanes(chunks), 4);
     grid          = dim3((chunks + p.chunk_lanes - 1) / p.chunk_lanes);
   } else {
     p.planes = static_cast<float*>(Scratch(ScratchKind::kSplitK, plane_bytes, stream));
   }
   if (!p.planes && wide) LaunchSums<T, E, true>(p, grid, grad, stream);
   if (!p.planes && !wide) LaunchSums<T, 1, true>(p, grid, grad, stream);
-  if (p.planes && wide) LaunchSums<T, E, false>(p, grid, grad, stream);
+  if (p.planes && few) LaunchSums<T, F, false>(p, grid, grad, stream);
+  if (p.planes && wide && !few) LaunchSums<T, E, false>(p, grid, grad, stream);
   if (p.planes && !wide) LaunchSums<T, 1, false>(p, grid, grad, stream);
   if (p.planes) {
     hipLaunchKernelGGL(channel_planes_kernel, dim3((p.channels + 15) / 16), dim3(256), 0, stream, p.planes, first, second, p.channels,
