@@ -475,6 +475,19 @@ ir::Module GraphCompiler::LowerGraph(const CompileOptions& options) {
   KernelMergeOptions merge;
   const char* flag = getenv("FLAGS_cinn_hip_merge_kernels");
   merge.enabled    = options.merge_independent_kernels && !(flag && flag[0] == '0');
+  if (merge.enabled) {
+    std::vector<std::unique_ptr<Group>> groups;
+    std::vector<ir::LoweredFuncRef> ordered;
+    std::vector<bool> ordered_barrier;
+    for (size_t i : OrderForMerging(graph_->groups, funcs, barrier, merge)) {
+      groups.push_back(std::move(graph_->groups[i]));
+      ordered.push_back(funcs[i]);
+      ordered_barrier.push_back(barrier[i]);
+    }
+    graph_->groups = std::move(groups);
+    funcs.swap(ordered);
+    barrier.swap(ordered_barrier);
+  }
   if (merge.enabled && options.lowering.merged_rows_per_wave > 1) {
     // Which groups will share a launch is known once every kernel exists; row-reduce members are then lowered again
     // with that knowledge (a member's schedule may differ from the one it has alone, its block shape does not).

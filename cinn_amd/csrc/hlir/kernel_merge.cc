@@ -26,12 +26,6 @@ bool Mergeable(const ir::LoweredFunc& f) {
   return true;
 }
 
-bool SameBlock(const ir::LoweredFunc& a, const ir::LoweredFunc& b) {
-  for (int d = 0; d < 3; ++d)
-    if (a.axis_info.block[d] != b.axis_info.block[d]) return false;
-  return true;
-}
-
 // A block of bx x by threads whose body can run in a flat block of bx * by threads, with threadIdx.x and threadIdx.y
 // recovered from the flat index: bx a power of two, no third axis, no use of the block's extents (the device library's
 // wave and block reductions work on the linear thread index; the column reduction walks blockDim.y and is excluded
@@ -47,6 +41,92 @@ bool Flattenable(const Group& g, const ir::LoweredFunc& f) {
 
 int Threads(const ir::LoweredFunc& f) { return f.axis_info.block[0] * f.axis_info.block[1] * f.axis_info.block[2]; }
 
+// what decides which groups share a launch
+struct MergeTraits {
+  const Group* group;
+  bool mergeable{false}, flattenable{false};
+  int block[3]{0, 0, 0}, threads{0};
+  int64_t grid{0};
+};
+
+std::vector<MergeTraits> TraitsOf(const std::vector<std::unique_ptr<Group>>& groups, const std::vector<ir::LoweredFuncRef>& funcs,
+                                  const std::vector<bool>& barrier, const KernelMergeOptions& options) {
+  std::vector<MergeTraits> traits;
+  for (size_t i = 0; i < groups.size(); ++i) {
+    MergeTraits t;
+    t.group     = groups[i].get();
+    t.mergeable = options.enabled && !barrier[i] && Mergeable(*funcs[i]);
+    if (t.mergeable) {
+      t.flattenable = Flattenable(*groups[i], *funcs[i]);
+      for (int d = 0; d < 3; ++d) t.block[d] = funcs[i]->axis_info.block[d];
+      t.threads = Threads(*funcs[i]);
+      t.grid    = funcs[i]->axis_info.grid[0];
+    }
+    traits.push_back(t);
+  }
+  return traits;
+}
+
+bool SameBlock(const MergeTraits& a, const MergeTraits& b) { return std::equal(a.block, a.block + 3, b.block); }
+
+bool Reads(const Group& g, const Group& writer) {
+  for (auto* in : g.inputs)
+    for (auto* out : writer.outputs)
+      if (in == out) return true;
+  return false;
+}
+
+// One behind the last group of the run that begins at t[i]: the longest run of consecutive kernels none of which reads what an
+// earlier one of the run writes; the run is consecutive in execution order, so a dependence through other groups would
+// pass through a member as well.
+size_t RunEnd(const std::vector<MergeTraits>& t, size_t i, const KernelMergeOptions& options) {
+  if (!t[i].mergeable) return i + 1;
+  int64_t blocks = t[i].grid;
+  size_t end     = i + 1;
+  // A run keeps one block shape, or - once a member of another shape joins - every member must be able to run in a
+  // flat block of the same number of threads (a member that cannot, e.g. a column reduction, shares launches only
+  // with kernels of its own shape).
+  bool run_flat        = false;
+  bool all_flattenable = t[i].flattenable;
+  while (end < t.size() && static_cast<int>(end - i) < options.max_members) {
+    if (!t[end].mergeable || t[end].group->pre_run != t[i].group->pre_run) break;
+    const bool same = SameBlock(t[i], t[end]);
+    if ((run_flat || !same) && (!all_flattenable || !t[end].flattenable || t[i].threads != t[end].threads)) break;
+    bool depends = false;
+    for (size_t k = i; k < end; ++k) depends |= Reads(*t[end].group, *t[k].group);
+    if (depends) break;
+    if (blocks + t[end].grid > 0x7fffffff) break;
+    blocks += t[end].grid;
+    run_flat        = run_flat || !same;
+    all_flattenable = all_flattenable && t[end].flattenable;
+    ++end;
+  }
+  return end;
+}
+
+int Launches(const std::vector<MergeTraits>& t, const KernelMergeOptions& options) {
+  int n = 0;
+  for (size_t i = 0; i < t.size(); i = RunEnd(t, i, options)) ++n;
+  return n;
+}
+
+// `g` reads a program input and writes a result of its size: a caller may have bound both to the same memory
+bool MayUpdate(const Group& g, const NodeData& input) {
+  if (input.producer || std::find(g.inputs.begin(), g.inputs.end(), &input) == g.inputs.end()) return false;
+  for (auto* out : g.outputs)
+    if ((out->is_fetch || out->consumers.empty()) && out->dtype == input.dtype && out->numel() == input.numel()) return true;
+  return false;
+}
+
+// whether two groups that are not ordered by a value may change places
+bool MayPass(const Group& a, const Group& b) {
+  for (auto* in : a.inputs)
+    if (MayUpdate(b, *in)) return false;
+  for (auto* in : b.inputs)
+    if (MayUpdate(a, *in)) return false;
+  return !Reads(a, b) && !Reads(b, a);
+}
+
 LaunchUnit UnitOf(const Group& g) {
   LaunchUnit u;
   u.func_name = g.func_name;
@@ -59,49 +139,58 @@ LaunchUnit UnitOf(const Group& g) {
 
 }  // namespace
 
+std::vector<size_t> OrderForMerging(const std::vector<std::unique_ptr<Group>>& groups, const std::vector<ir::LoweredFuncRef>& funcs,
+                                    const std::vector<bool>& barrier, const KernelMergeOptions& options) {
+  CINN_CHECK_EQ(groups.size(), funcs.size());
+  std::vector<size_t> order(groups.size());
+  for (size_t i = 0; i < order.size(); ++i) order[i] = i;
+  std::vector<MergeTraits> t = TraitsOf(groups, funcs, barrier, options);
+  auto small = [&](const MergeTraits& m) {
+    int64_t bytes = 0;
+    for (auto* list : {&m.group->inputs, &m.group->outputs})
+      for (auto* v : *list) bytes += v->numel() * v->dtype.bytes();
+    return m.mergeable && !m.group->pre_run && bytes <= options.max_moved_bytes;
+  };
+  auto move = [](auto* list, size_t from, size_t to) {
+    if (from < to) std::rotate(list->begin() + from, list->begin() + from + 1, list->begin() + to + 1);
+    if (to < from) std::rotate(list->begin() + to, list->begin() + from, list->begin() + from + 1);
+  };
+  int launches = Launches(t, options);
+  for (size_t group = 0; group < order.size(); ++group) {
+    size_t at = std::find(order.begin(), order.end(), group) - order.begin();
+    if (!small(t[at])) continue;
+    // the nearest place, later or earlier, that saves a launch: next to a kernel, past groups that it may change places with
+    bool moved = false;
+    auto attempt = [&](size_t to) {
+      move(&t, at, to);
+      const int now = Launches(t, options);
+      moved = now < launches;
+      if (moved) {
+        move(&order, at, to);
+        launches = now;
+      } else {
+        move(&t, to, at);
+      }
+    };
+    for (size_t to = at + 1; to < t.size() && !moved && MayPass(*t[at].group, *t[to].group); ++to)
+      if (to + 1 < t.size() && t[to + 1].mergeable) attempt(to);
+    for (size_t to = at; to-- > 0 && !moved && MayPass(*t[at].group, *t[to].group);)
+      if (to > 0 && t[to - 1].mergeable) attempt(to);
+  }
+  return order;
+}
+
 std::vector<LaunchUnit> MergeIndependentKernels(const std::vector<std::unique_ptr<Group>>& groups,
                                                 const std::vector<ir::LoweredFuncRef>& funcs, const std::vector<bool>& barrier,
                                                 const KernelMergeOptions& options, std::vector<ir::LoweredFuncRef>* funcs_out) {
   CINN_CHECK_EQ(groups.size(), funcs.size());
+  const std::vector<MergeTraits> traits = TraitsOf(groups, funcs, barrier, options);
   std::vector<LaunchUnit> units;
   size_t i = 0;
   while (i < groups.size()) {
     const Group& first = *groups[i];
-    if (!options.enabled || barrier[i] || !Mergeable(*funcs[i])) {
-      units.push_back(UnitOf(first));
-      funcs_out->push_back(funcs[i]);
-      ++i;
-      continue;
-    }
-    // the longest run of consecutive kernels none of which reads what an earlier one of the run writes; the run is
-    // consecutive in execution order, so a dependence through other groups would pass through a member as well
-    std::set<const NodeData*> written(first.outputs.begin(), first.outputs.end());
-    int64_t blocks = funcs[i]->axis_info.grid[0];
-    size_t end     = i + 1;
-    // A run keeps one block shape, or - once a member of another shape joins - every member must be able to run in a
-    // flat block of the same number of threads (a member that cannot, e.g. a column reduction, shares launches only
-    // with kernels of its own shape).
-    bool run_flat        = false;
-    bool all_flattenable = Flattenable(first, *funcs[i]);
-    while (end < groups.size() && static_cast<int>(end - i) < options.max_members) {
-      const Group& g = *groups[end];
-      if (barrier[end] || !Mergeable(*funcs[end]) || g.pre_run != first.pre_run) break;
-      const bool same   = SameBlock(*funcs[i], *funcs[end]);
-      const bool g_flat = Flattenable(g, *funcs[end]);
-      if (run_flat || !same) {
-        if (!all_flattenable || !g_flat || Threads(*funcs[i]) != Threads(*funcs[end])) break;
-      }
-      bool depends = false;
-      for (auto* in : g.inputs) depends |= written.count(in) > 0;
-      if (depends) break;
-      if (blocks + funcs[end]->axis_info.grid[0] > 0x7fffffff) break;
-      blocks += funcs[end]->axis_info.grid[0];
-      written.insert(g.outputs.begin(), g.outputs.end());
-      run_flat        = run_flat || !same;
-      all_flattenable = all_flattenable && g_flat;
-      ++end;
-    }
-    if (end - i < 2) {
+    const size_t end = RunEnd(traits, i, options);
+    if (end - i < 2) {  // not mergeable, or alone
       units.push_back(UnitOf(first));
       funcs_out->push_back(funcs[i]);
       ++i;
@@ -113,10 +202,12 @@ std::vector<LaunchUnit> MergeIndependentKernels(const std::vector<std::unique_pt
     auto merged  = std::make_shared<ir::LoweredFunc>();
     merged->is_device = true;
     merged->axis_info = funcs[i]->axis_info;
+    int64_t blocks = 0;
+    for (size_t k = i; k < end; ++k) blocks += traits[k].grid;
     merged->axis_info.grid[0] = static_cast<int>(blocks);
     // members of different block shapes: the launch is a flat block and every member recovers its own threadIdx.x / y
     bool flat = false;
-    for (size_t k = i + 1; k < end; ++k) flat = flat || !SameBlock(*funcs[i], *funcs[k]);
+    for (size_t k = i + 1; k < end; ++k) flat = flat || !SameBlock(traits[i], traits[k]);
     if (flat) {
       merged->axis_info.block[0] = funcs[i]->axis_info.block[0] * funcs[i]->axis_info.block[1];
       merged->axis_info.block[1] = 1;
