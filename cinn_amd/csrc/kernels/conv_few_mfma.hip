@@ -1,4 +1,5 @@
-// Channels-last convolutions of few output tiles for gfx950: one image, or a few, through a network's deeper stages.
+// Channels-last convolutions of few output tiles for gfx950: one image, or a few, through a network's deeper stages; and layers
+// of few filters, whose tiles of 64 columns would be mostly padding.
 //
 //   y[pixel][oc] = act( sum_k im2col(x)[pixel][k] w[oc][k] * scale + shift + residual ),  fp16 / bf16 / fp32
 //
@@ -13,7 +14,9 @@
 // 512 -> 512 3x3 on 7x7 10.5 | 5.2; fp32 15.1 | 6.5, 12.3 | 4.6, 20.9 | 9.7.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <climits>
+#include <cmath>
 #include <cstdint>
 #include <cstdlib>
 
@@ -157,23 +160,44 @@ void Launch(const FewParams& p_in, hipStream_t stream) {
   CINN_HIP_CALL(hipGetLastError());
 }
 
-template <typename T>
-void Run(const FewParams& p, hipStream_t stream) {
-  struct Tile {
-    int tm, tn, nw;
-    void (*launch)(const FewParams&, hipStream_t);
-  };
-  // (four K steps in flight, or eight wavefronts for the larger tiles, leave room for one block on a CU: slower with
-  // more blocks than CUs and no faster with fewer; 64x64 tiles lose to the tiled kernels wherever they beat the others)
-  static const Tile tiles[] = {{1, 1, 8, Launch<T, 1, 1, 8>}, {1, 1, 4, Launch<T, 1, 1, 4>}, {1, 2, 4, Launch<T, 1, 2, 4>},
-                               {2, 2, 4, Launch<T, 2, 2, 4>}, {2, 4, 4, Launch<T, 2, 4, 4>}};
-  const Tile* best = nullptr;
-  double best_us   = 0.0;
-  for (const Tile& t : tiles) {
-    const double us = few::Estimate(p.pixels, p.oc, p.steps, sizeof(T) == 4, t.tm, t.tn, t.nw);
-    if (!best || us < best_us) best = &t, best_us = us;
+struct Tile {
+  int tm, tn, nw;
+};
+// (four K steps in flight, or eight wavefronts for the larger tiles, leave room for one block on a CU: slower with
+// more blocks than CUs and no faster with fewer; 64x64 tiles lose to the tiled kernels wherever they beat the others)
+constexpr Tile kTiles[] = {{1, 1, 8}, {1, 1, 4}, {1, 2, 4}, {2, 2, 4}, {2, 4, 4}};
+
+// index of the fastest tile, and its estimate
+int Choose(const FewParams& p, bool fp32, double* us) {
+  int best = 0;
+  for (int i = 0; i < (int)(sizeof(kTiles) / sizeof(Tile)); ++i) {
+    const double t = few::Estimate(p.pixels, p.oc, p.steps, fp32, kTiles[i].tm, kTiles[i].tn, kTiles[i].nw);
+    if (i == 0 || t < *us) best = i, *us = t;
   }
-  best->launch(p, stream);
+  return best;
+}
+
+template <typename T>
+void Run(const FewParams& p, int tile, hipStream_t stream) {
+  switch (tile) {
+    case 0: Launch<T, 1, 1, 8>(p, stream); break;
+    case 1: Launch<T, 1, 1, 4>(p, stream); break;
+    case 2: Launch<T, 1, 2, 4>(p, stream); break;
+    case 3: Launch<T, 2, 2, 4>(p, stream); break;
+    default: Launch<T, 2, 4, 4>(p, stream); break;
+  }
+}
+
+// us of the tiled kernels; fitted to 140 layers in fp32, 1x1 to 7x7 (9% off on average), and 62 of more than 128 tiles in 16 bits (17%)
+double TiledMicroseconds(const FewParams& p, bool fp32) {
+  const int tiles  = (int)std::min<int64_t>((int64_t)((p.pixels + 63) / 64) * ((p.oc + 63) / 64), 1 << 24);
+  const int splits = ConvSplits(tiles, p.steps, fp32), share = (p.steps + splits - 1) / splits;
+  const double cus = (double)tiles * splits / 256, mb = (double)p.pixels * p.oc * (fp32 ? 4e-6 : 2e-6);
+  if (fp32) {
+    const double per_cu = tiles < 256 ? std::ceil(cus) : cus;
+    return 4.0 + (per_cu <= 1.0 ? 0.65 : 0.6 * per_cu) * share + 0.4 * mb + (splits > 1 ? 2.4 + 0.25 * splits * mb : 0.0);
+  }
+  return 4.45 + 0.266 * std::max(cus, 1.0) * share + 0.14 * mb + (splits > 1 ? 3.7 + 0.39 * splits * mb : 0.0);
 }
 
 }  // namespace
@@ -185,9 +209,6 @@ bool TryConvFew(const ConvNhwcArgs& a, hipStream_t stream) {
   const bool is_float = a.type.code == cinn_type_float && (a.type.bits == 32 || a.type.bits == 16);
   const bool is_bf16  = a.type.code == cinn_type_bfloat && a.type.bits == 16;
   if (!is_float && !is_bf16) return false;
-  // A convolution in fp32 without a layer's scale stays with the tiled kernels: the K
-  // that they split for it is what the tests of scratch memory under graph replay hold on to.
-  if (a.type.bits == 32 && !a.scale) return false;
   // whole K steps inside a filter tap, whole groups of four channels of a result
   const int elem = a.type.bits / 8, lanes = few::kStepBytes / elem;
   if (a.c % lanes != 0 || a.oc % 4 != 0) return false;
@@ -197,10 +218,20 @@ bool TryConvFew(const ConvNhwcArgs& a, hipStream_t stream) {
   constexpr int64_t kLimit = (int64_t)1 << 31;
   const int64_t k_total = (int64_t)a.kh * a.kw * a.c, pixels = (int64_t)a.n * a.oh * a.ow;
   if ((int64_t)a.n * a.h * a.w_in * a.c * elem >= kLimit || a.oc * k_total * elem >= kLimit) return false;
-  // Up to half as many tiles of 64x64 as CUs: beyond that the tiled kernels' larger tiles pull in less.  us, tiled | here: 98 tiles
-  // (fp16, 256 -> 256 3x3 on 14x14, 8 images) 10.9 | 8.4, 104 (fp32, 512 -> 512 3x3 on 7x7, 16 images) 52.0 | 44.2, 112 (512 -> 1024 1x1 on
-  // 14x14, 2 images) 6.1 | 5.1; 154 (192 -> 40 7x7) 28.8 | 33.2, 180 (960 -> 332 3x3) 34.0 | 36.7, 196 (256 -> 128 1x1 on 56x56, 2 images) 4.6 | 6.2.
-  if (((pixels + 63) / 64) * ((a.oc + 63) / 64) > 128 || pixels < 1) return false;
+  // (512 threads for each tile of 16x16: fewer than 2^32 of a launch)
+  if (pixels < 1 || pixels >= (1 << 24) || pixels * a.oc >= (1 << 30)) return false;
+  // Up to half as many tiles of 64x64 as CUs.  us, tiled | here: 98 tiles (fp16, 256 -> 256 3x3 on 14x14, 8 images) 10.9 | 8.4, 104 (fp32,
+  // 512 -> 512 3x3 on 7x7, 16 images) 52.0 | 44.2, 112 (512 -> 1024 1x1 on 14x14, 2 images) 6.1 | 5.1.
+  // Beyond, the tiled kernels' larger tiles pull in less, but a tile's columns are 64: layers of 8 to 60 filters, or a few more than
+  // a multiple of 64, multiply mostly padding there.  Those go by the two estimates, a fifth apart.  60 layers in fp16 of 132 to 1168
+  // tiles: 23 taken, 1.17 to 2.3 times faster (64 -> 16 7x7 on 38x22, 24 images, 25.1 | 11.4; 512 -> 12 5x5 on 57x56, 3 images, 16.3 | 7.8), none slower;
+  // of those not taken 316 tiles (384 -> 72 5x5) 33.3 | 43.9, 485 (256 -> 304 1x1) 6.3 | 11.2, 945 (128 -> 192 3x3) 22.6 | 34.4.
+  // 140 in fp32, where these tiles are bound by the matrix pipe and padding costs most: 85 taken, 1.19 to 3.8 times faster (480 -> 16
+  // 1x1 / 2 on 16x11, 27 images, 12.9 | 3.4, 96 -> 200 3x3 / 2 on 35x41, 8 images, 22.5 | 18.4).  A multiple of 64 has no such columns: in 16 bits 196 tiles (256 -> 128 1x1
+  // on 56x56, 2 images) 4.6 | 6.2.  (In fp32 a convolution of such filters without a layer's scale stays with the tiled kernels at any size:
+  // the K that they split for it is what the tests of scratch memory under graph replay hold on to.)
+  const bool few_tiles = ((pixels + 63) / 64) * ((a.oc + 63) / 64) <= 128 && (elem == 2 || a.scale);
+  if (!few_tiles && a.oc % 64 == 0 && (elem == 2 || !a.scale)) return false;
   // (a single K step of few rows has nothing to share: 1 x 64 -> 4096 2.4 | 3.0, 8 x 64 -> 4096 2.9 | 3.0; 3136 x 64 -> 64 and more gain)
   if (k_total == lanes && pixels <= 16) return false;
   const bool outside = a.pad_h > 0 || a.pad_w > 0 || (int64_t)(a.oh - 1) * a.stride_h - a.pad_h + (int64_t)(a.kh - 1) * a.dil_h >= a.h ||
@@ -219,12 +250,15 @@ bool TryConvFew(const ConvNhwcArgs& a, hipStream_t stream) {
   p.relu = a.relu, p.alpha = a.alpha, p.residual_scale = a.residual_scale;
   // the larger operand is read from memory once: its rows go to one XCD
   p.pixels_outer = (int64_t)a.n * a.h * a.w_in * a.c > a.oc * k_total;
+  double us;
+  const int tile = Choose(p, elem == 4, &us);
+  if (!few_tiles && us >= 0.8 * TiledMicroseconds(p, elem == 4)) return false;
   if (is_bf16) {
-    Run<__bf16>(p, stream);
+    Run<__bf16>(p, tile, stream);
   } else if (elem == 2) {
-    Run<_Float16>(p, stream);
+    Run<_Float16>(p, tile, stream);
   } else {
-    Run<float>(p, stream);
+    Run<float>(p, tile, stream);
   }
   return true;
 }

@@ -51,9 +51,11 @@ bool TryPointwiseConvAsGemm(const ConvNhwcArgs& a, hipStream_t stream);
 // rows fit LDS (conv_patch_mfma.hip): the input patch of a band of output rows stays resident in LDS, only the filter
 // streams; same epilogue.  false when the shape does not qualify.
 bool TryConvPatch(const ConvNhwcArgs& a, hipStream_t stream);
-// few pixels (conv_few_mfma.hip): whole K steps of 128 bytes in every tap, same epilogue; one launch of
+// few output tiles, or many that are mostly padding (conv_few_mfma.hip): whole K steps of 128 bytes in every tap, same epilogue; one launch of
 // small tiles whose wavefronts share K.  false when the shape does not qualify or the tiled kernels are faster.
 bool TryConvFew(const ConvNhwcArgs& a, hipStream_t stream);
+// into how many parts the tiled kernel splits the K steps of a convolution of `tiles` tiles of 64x64
+int ConvSplits(int tiles, int steps, bool fp32);
 // Two 1x1, stride 1, unpadded convolutions in a row on channels-last 16-bit tensors, seen as matrix products over the
 // m = N * H * W pixels: e = act1(x w1^T * scale1 + shift1 + residual) [m][n1], y = act2(e w2^T * scale2 + shift2)
 // [m][n2], with x [m][k1], w1 [n1][k1], w2 [n2][n1]; both e and y are written (conv_chain_mfma.hip).

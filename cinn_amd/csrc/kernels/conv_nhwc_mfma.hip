@@ -941,6 +941,8 @@ bool ConvNhwcSupported(const ConvNhwcArgs& a) {
   return a.c % ChunkElems(a.type) == 0;
 }
 
+int ConvSplits(int tiles, int steps, bool fp32) { return ChooseSplits(tiles, steps, fp32, 0, 0); }
+
 void RunConvNhwc(const ConvNhwcArgs& a, hipStream_t stream) {
   CINN_RT_CHECK(ConvNhwcSupported(a), "conv2d (channels-last): unsupported type or channel count %d", a.c);
   CINN_RT_CHECK((int64_t)a.n * a.h * a.w_in * a.c < INT_MAX && (int64_t)a.n * a.oh * a.ow * a.oc < INT_MAX,

@@ -73,3 +73,38 @@ def test_layer(gpu, n, h, w, c, oc, k, stride, pad, dil, residual, relu, dtype):
     want = np.maximum(want, 0) if relu else want
     bound = (c * k * k + 2) * 2.0 ** -24 * size + UNIT[dtype] * np.abs(want) + 2.0 ** -25
     assert np.all(np.abs(got.astype(np.float64) - want) <= 1.01 * bound)
+
+
+# more than 128 tiles of 64x64 whose columns are mostly padding: one group of four channels, one below and above a tile of 16 and
+# of 64, a split that the tiled kernels would have, a K of one step
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16", "float32"])
+@pytest.mark.parametrize("n,h,w,c,oc,k,stride,pad,dil,residual,relu", [
+    (9, 31, 37, 128, 4, 3, 1, 1, 1, False, False),
+    (3, 57, 56, 64, 12, 5, 1, 2, 1, True, True),
+    (5, 91, 97, 64, 20, 1, 1, 0, 1, False, True),
+    (2, 70, 71, 192, 68, 3, 1, 1, 1, True, False),
+    (1, 129, 127, 64, 16, 7, 2, 3, 1, False, True),
+    (7, 40, 41, 320, 60, 3, 1, 1, 1, False, False),
+])
+def test_narrow_layer(gpu, n, h, w, c, oc, k, stride, pad, dil, residual, relu, dtype):
+    test_layer(gpu, n, h, w, c, oc, k, stride, pad, dil, residual, relu, dtype)
+
+
+@pytest.mark.parametrize("shape,oc,k", [((1, 1, 1, 32), 4, 1), ((2, 13, 11, 96), 36, 3), ((8, 35, 41, 96), 200, 3), ((4, 33, 31, 160), 12, 5)])
+def test_fp32_without_a_scale(gpu, shape, oc, k):
+    from cinn_amd.common import DefaultAMDGPUTarget, Float
+    from cinn_amd.frontend import Computation, NetBuilder
+    rng = np.random.default_rng(oc)
+    x = rng.standard_normal(shape).astype(np.float32)
+    w = (rng.standard_normal((oc, k, k, shape[3])) * 0.05).astype(np.float32)
+    b = NetBuilder("plain")
+    X, W = b.create_input(Float(32), list(x.shape), "x"), b.create_input(Float(32), list(w.shape), "w")
+    y = b.conv2d(X, W, [2, 2], [k // 2] * 2, data_format="NHWC")
+    comp = Computation.build_and_compile(DefaultAMDGPUTarget(), b, outputs=[y])
+    comp.get_tensor("x").from_numpy(x)
+    comp.get_tensor("w").from_numpy(w)
+    comp.execute()
+    got = comp.get_tensor(y.id).numpy().astype(np.float64)
+    x, w = x.astype(np.float64), w.astype(np.float64)
+    want, size = _conv64(x, w, 2, k // 2, 1), _conv64(np.abs(x), np.abs(w), 2, k // 2, 1)
+    assert np.all(np.abs(got - want) <= (shape[3] * k * k + 2) * 2.0 ** -24 * size + 2.0 ** -25)
