@@ -202,24 +202,26 @@ double TiledMicroseconds(const FewParams& p, bool fp32) {
 
 }  // namespace
 
-// FLAGS_cinn_hip_conv_few=0 switches the kernel off.
-bool TryConvFew(const ConvNhwcArgs& a, hipStream_t stream) {
+namespace {
+
+// TryProductFew, and TryConvFew with other_us < 0
+double TryFew(const ConvNhwcArgs& a, double other_us, bool dry, hipStream_t stream) {
   static const bool enabled = !(getenv("FLAGS_cinn_hip_conv_few") && atoi(getenv("FLAGS_cinn_hip_conv_few")) == 0);
-  if (!enabled || a.nchw_input || a.pool_after || a.x2) return false;
+  if (!enabled || a.nchw_input || a.pool_after || a.x2) return 0.0;
   const bool is_float = a.type.code == cinn_type_float && (a.type.bits == 32 || a.type.bits == 16);
   const bool is_bf16  = a.type.code == cinn_type_bfloat && a.type.bits == 16;
-  if (!is_float && !is_bf16) return false;
+  if (!is_float && !is_bf16) return 0.0;
   // whole K steps inside a filter tap, whole groups of four channels of a result
   const int elem = a.type.bits / 8, lanes = few::kStepBytes / elem;
-  if (a.c % lanes != 0 || a.oc % 4 != 0) return false;
+  if (a.c % lanes != 0 || a.oc % 4 != 0) return 0.0;
   for (const void* ptr : {a.x, a.w, static_cast<const void*>(a.y), static_cast<const void*>(a.scale), static_cast<const void*>(a.shift), a.residual})
-    if (reinterpret_cast<uintptr_t>(ptr) % 16 != 0) return false;
+    if (reinterpret_cast<uintptr_t>(ptr) % 16 != 0) return 0.0;
   // byte offsets are 32 bits wide, positions in the image are signed
   constexpr int64_t kLimit = (int64_t)1 << 31;
   const int64_t k_total = (int64_t)a.kh * a.kw * a.c, pixels = (int64_t)a.n * a.oh * a.ow;
-  if ((int64_t)a.n * a.h * a.w_in * a.c * elem >= kLimit || a.oc * k_total * elem >= kLimit) return false;
+  if ((int64_t)a.n * a.h * a.w_in * a.c * elem >= kLimit || a.oc * k_total * elem >= kLimit) return 0.0;
   // (512 threads for each tile of 16x16: fewer than 2^32 of a launch)
-  if (pixels < 1 || pixels >= (1 << 24) || pixels * a.oc >= (1 << 30)) return false;
+  if (pixels < 1 || pixels >= (1 << 24) || pixels * a.oc >= (1 << 30)) return 0.0;
   // Up to half as many tiles of 64x64 as CUs.  us, tiled | here: 98 tiles (fp16, 256 -> 256 3x3 on 14x14, 8 images) 10.9 | 8.4, 104 (fp32,
   // 512 -> 512 3x3 on 7x7, 16 images) 52.0 | 44.2, 112 (512 -> 1024 1x1 on 14x14, 2 images) 6.1 | 5.1.
   // Beyond, the tiled kernels' larger tiles pull in less, but a tile's columns are 64: layers of 8 to 60 filters, or a few more than
@@ -231,12 +233,12 @@ bool TryConvFew(const ConvNhwcArgs& a, hipStream_t stream) {
   // on 56x56, 2 images) 4.6 | 6.2.  (In fp32 a convolution of such filters without a layer's scale stays with the tiled kernels at any size:
   // the K that they split for it is what the tests of scratch memory under graph replay hold on to.)
   const bool few_tiles = ((pixels + 63) / 64) * ((a.oc + 63) / 64) <= 128 && (elem == 2 || a.scale);
-  if (!few_tiles && a.oc % 64 == 0 && (elem == 2 || !a.scale)) return false;
+  if (other_us < 0.0 && !few_tiles && a.oc % 64 == 0 && (elem == 2 || !a.scale)) return 0.0;
   // (a single K step of few rows has nothing to share: 1 x 64 -> 4096 2.4 | 3.0, 8 x 64 -> 4096 2.9 | 3.0; 3136 x 64 -> 64 and more gain)
-  if (k_total == lanes && pixels <= 16) return false;
+  if (k_total == lanes && pixels <= 16) return 0.0;
   const bool outside = a.pad_h > 0 || a.pad_w > 0 || (int64_t)(a.oh - 1) * a.stride_h - a.pad_h + (int64_t)(a.kh - 1) * a.dil_h >= a.h ||
                        (int64_t)(a.ow - 1) * a.stride_w - a.pad_w + (int64_t)(a.kw - 1) * a.dil_w >= a.w_in;
-  if (outside && !HasZeroPage(stream)) return false;
+  if (outside && !HasZeroPage(stream)) return 0.0;
   FewParams p{};
   p.x = a.x, p.w = a.w, p.y = a.y, p.scale = a.scale, p.shift = a.shift, p.residual = a.residual;
   p.zeros = outside ? ConvZeroPage() : nullptr;
@@ -252,7 +254,8 @@ bool TryConvFew(const ConvNhwcArgs& a, hipStream_t stream) {
   p.pixels_outer = (int64_t)a.n * a.h * a.w_in * a.c > a.oc * k_total;
   double us;
   const int tile = Choose(p, elem == 4, &us);
-  if (!few_tiles && us >= 0.8 * TiledMicroseconds(p, elem == 4)) return false;
+  if (other_us >= 0.0 ? us >= (p.steps > 1 ? 0.9 : 0.83) * other_us : !few_tiles && us >= 0.8 * TiledMicroseconds(p, elem == 4)) return 0.0;
+  if (dry) return us;
   if (is_bf16) {
     Run<__bf16>(p, tile, stream);
   } else if (elem == 2) {
@@ -260,7 +263,14 @@ bool TryConvFew(const ConvNhwcArgs& a, hipStream_t stream) {
   } else {
     Run<float>(p, tile, stream);
   }
-  return true;
+  return us;
 }
+
+}  // namespace
+
+// FLAGS_cinn_hip_conv_few=0 switches the kernel off.
+bool TryConvFew(const ConvNhwcArgs& a, hipStream_t stream) { return TryFew(a, -1.0, false, stream) > 0.0; }
+
+double TryProductFew(const ConvNhwcArgs& a, double other_us, bool dry, hipStream_t stream) { return TryFew(a, other_us, dry, stream); }
 
 }  // namespace cinn_hip_kernels

@@ -1839,6 +1839,26 @@ bool ForceGeneric() {
   return force;
 }
 
+// Products in fp32 with both operands in runs of K, as a linear layer's on the weights of a network: the wavefronts of a block share
+// K (conv_few_mfma.hip) where that is estimated to be a tenth faster than gemm_flex.hip's plan (a sixth with one K step), whose
+// estimate leaves out the 2 us of a block's start and end.  A product of few rows took that kernel a launch of 64x64 tiles that are
+// mostly padding, split over K, and a second launch that adds the parts.  us, that kernel | here: 7 x 1152 -> 1792 8.9 | 4.8, 10 x 320 -> 3520
+// 9.2 | 3.5, 1 x 192 -> 1208 7.4 | 3.1, 92 x 3168 -> 576 13.3 | 8.4.  Of 150 products of 1 to 2683 rows, no multiples of 128, 129 are taken, 1.69
+// times faster in the geometric mean, the worst 0.99; not taken 1912 x 64 -> 3520 17.6 | 43.7, 466 x 3520 -> 576 28.9 | 33.6.  The result is that kernel's
+// estimate where it takes the product, in the other's terms, else 0.
+double TryFewProduct(const GemmProblem& p, double flex_us, bool dry, hipStream_t stream) {
+  if (p.type != GemmType::kF32 || p.trans_a || !p.trans_b || p.batch != 1 || p.shift16) return 0.0;
+  cinn_hip_kernels::ConvNhwcArgs a;
+  a.x = p.a, a.w = p.b, a.y = p.c, a.scale = nullptr, a.shift = p.shift;
+  a.alpha = p.alpha, a.residual = p.beta != 0.0f ? p.c : nullptr, a.residual_scale = p.beta;
+  a.relu = a.nchw_input = false;
+  a.n = a.h = a.oh = a.kh = a.kw = 1, a.w_in = a.ow = p.m, a.c = p.k, a.oc = p.n;
+  a.pad_h = a.pad_w = 0, a.stride_h = a.stride_w = a.dil_h = a.dil_w = 1;
+  a.type.code = cinn_type_float, a.type.bits = 32, a.type.lanes = 1, a.type.num_asterisks = 0;
+  const double us = cinn_hip_kernels::TryProductFew(a, flex_us + 2.0, dry, stream);
+  return us > 0.0 ? std::max(us - 2.0, 0.1) : 0.0;
+}
+
 // The plan with which gemm_flex.hip would run the product; false when another kernel takes it.
 bool RunsFlexible(const GemmProblem& product, hipStream_t stream, cinn_hip_kernels::FlexPlan* plan) {
   GemmProblem p = product;
@@ -1846,7 +1866,10 @@ bool RunsFlexible(const GemmProblem& product, hipStream_t stream, cinn_hip_kerne
   if (ForceGeneric() || p.type == GemmType::kF64 || p.batch != 1 || !cinn_hip_kernels::PlanFlexGemm(FlexOf(p), stream, plan)) return false;
   if (p.type == GemmType::kF32) {
     const bool aligned16 = reinterpret_cast<uintptr_t>(p.a) % 16 == 0 && reinterpret_cast<uintptr_t>(p.b) % 16 == 0;
-    return !aligned16 || p.m % kF32Tile != 0 || p.n % kF32Tile != 0 || p.k % kF32K != 0;
+    if (aligned16 && p.m % kF32Tile == 0 && p.n % kF32Tile == 0 && p.k % kF32K == 0) return false;
+    const double few = TryFewProduct(p, plan->us, true, stream);  // a group has to be faster than that
+    if (few > 0.0) plan->us = few;
+    return true;
   }
   const bool bf16 = p.type == GemmType::kBF16;
   if (p.trans_a) return !(bf16 ? TryDmaTransposedA<__bf16>(p, plan->us, stream) : TryDmaTransposedA<_Float16>(p, plan->us, stream));
@@ -1906,6 +1929,7 @@ void RunGemm(const GemmProblem& p, hipStream_t stream) {
     // nearly empty are better off split all the same: 1280x1024x4096 138 | 101, 768x3072x4096 207 | 172.)
     const bool fast32 = whole32 && ((int64_t)(p.m / 64) * (p.n / 64) * p.batch >= 256 || plan.splits <= 1);
     const bool whole  = !bias && p.type == GemmType::kF32 && fast32;
+    if (!whole32 && planned && TryFewProduct(p, plan.us, false, stream) > 0.0) return;
     if (!whole && planned) {
       cinn_hip_kernels::RunFlexGemm(g, plan, stream);
       return;
