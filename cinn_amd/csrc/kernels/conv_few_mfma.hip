@@ -228,8 +228,8 @@ double TryFew(const ConvNhwcArgs& a, double other_us, bool dry, hipStream_t stre
   // a multiple of 64, multiply mostly padding there.  Those go by the two estimates, a fifth apart.  60 layers in fp16 of 132 to 1168
   // tiles: 23 taken, 1.17 to 2.3 times faster (64 -> 16 7x7 on 38x22, 24 images, 25.1 | 11.4; 512 -> 12 5x5 on 57x56, 3 images, 16.3 | 7.8), none slower;
   // of those not taken 316 tiles (384 -> 72 5x5) 33.3 | 43.9, 485 (256 -> 304 1x1) 6.3 | 11.2, 945 (128 -> 192 3x3) 22.6 | 34.4.
-  // 140 in fp32, where these tiles are bound by the matrix pipe and padding costs most: 85 taken, 1.19 to 3.8 times faster (480 -> 16
-  // 1x1 / 2 on 16x11, 27 images, 12.9 | 3.4, 96 -> 200 3x3 / 2 on 35x41, 8 images, 22.5 | 18.4).  A multiple of 64 has no such columns: in 16 bits 196 tiles (256 -> 128 1x1
+  // 140 in fp32, where these tiles are bound by the matrix pipe and padding costs most: 85 taken, 1.16 to 3.8 times faster (480 -> 16
+  // 1x1 / 2 on 16x11, 27 images, 12.9 | 3.4, 96 -> 200 3x3 / 2 on 35x41, 8 images, 22.5 | 19.3).  A multiple of 64 has no such columns: in 16 bits 196 tiles (256 -> 128 1x1
   // on 56x56, 2 images) 4.6 | 6.2.  (In fp32 a convolution of such filters without a layer's scale stays with the tiled kernels at any size:
   // the K that they split for it is what the tests of scratch memory under graph replay hold on to.)
   const bool few_tiles = ((pixels + 63) / 64) * ((a.oc + 63) / 64) <= 128 && (elem == 2 || a.scale);

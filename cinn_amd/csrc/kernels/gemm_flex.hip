@@ -57,7 +57,7 @@ __device__ __forceinline__ float Finish(float v, float alpha, float shift, float
 // KG groups of four wavefronts (2 x 2 over the tile) share the block's tiles and take a K step's slices in turn; their
 // sums meet in the epilogue.
 // Block `bid` of the tiles, `z` of the splits, batch entry `entry` of `entries`.
-template <typename T, bool A_KC, bool B_KC, int BM, int BN, int KG>
+template <typename T, bool A_KC, bool B_KC, int BM, int BN, int KG, int PARTS = 0>
 __device__ __forceinline__ void FlexBlock(const FlexParams& p, char* lds, int bid, int z, int entry, int entries) {
   const int tid = threadIdx.x;
   int tm, tn;
@@ -70,7 +70,7 @@ __device__ __forceinline__ void FlexBlock(const FlexParams& p, char* lds, int bi
   tb.Init(static_cast<const T*>(p.b) + entry * p.stride_b, p.ldb, n0, p.n, p.k, tid);
   typename flex::Mma<T, A_KC, B_KC, BM, BN>::acc_t acc;
   const int s0 = z * p.steps_per_split;
-  flex::KLoop<T, A_KC, B_KC, BM, BN, KG>(lds, ta, tb, s0, min(s0 + p.steps_per_split, p.steps), p.full_steps, p.k, tid, acc);
+  flex::KLoop<T, A_KC, B_KC, BM, BN, KG, PARTS>(lds, ta, tb, s0, min(s0 + p.steps_per_split, p.steps), p.full_steps, p.k, tid, acc);
 
   const int col0 = n0 + tid % (BN / 8) * 8;  // the eight columns this thread finishes
   const int cols = min(p.n - col0, 8);
@@ -127,7 +127,7 @@ flex_gemm_kernel(FlexParams p) {
 // mostly one more to add the partial sums of a split K, because none has the tiles for all CUs by itself: small ones are bound by
 // those launches (about 3 us each), larger ones by their nearly empty rounds.  Together they share the CUs and one addition.  us of
 // the step with its two column sums, one by one | together: 37 x 75 -> 247 fp16 19.8 | 9.4, 665 x 233 -> 670 bf16 28.5 | 13.9,
-// 874 x 1237 -> 440 fp32 68 | 50, 630 x 2558 -> 1999 bf16 88 | 67.
+// 874 x 1237 -> 440 fp32 68 | 53, 630 x 2558 -> 1999 bf16 88 | 67.
 // Blocks [first[i], first[i + 1]) are product i's, split by split, the tiles of each in whole rounds of the XCDs (what is beyond
 // them returns at once): TileOf's neighbours stay on one XCD.
 struct GroupParams {
@@ -152,11 +152,15 @@ flex_group_kernel(GroupParams g) {
   const int tiles = p.tiles_m * p.tiles_n, round = (tiles + 7) & ~7, at = (int)blockIdx.x - g.first[i];
   const int z = at / round, bid = at - z * round;
   if (bid >= tiles) return;
+  // fp32: the sums of a K step before they are added to those of the others, as a block may have more steps here than alone.
+  // Relative error against float64, 27 products of small layers: up to 1.5 times of the separate ones' as one chain, 0.51 on average so and
+  // nowhere more.  50.2 -> 53.2 us at 874 x 1237 -> 440.
+  constexpr int kParts = sizeof(T) == 4 ? 1 : 0;
   switch (g.layout[i]) {
-    case 0: FlexBlock<T, false, false, 64, 64, 1>(p, lds, bid, z, 0, 1); break;
-    case 1: FlexBlock<T, true, false, 64, 64, 1>(p, lds, bid, z, 0, 1); break;
-    case 2: FlexBlock<T, false, true, 64, 64, 1>(p, lds, bid, z, 0, 1); break;
-    default: FlexBlock<T, true, true, 64, 64, 1>(p, lds, bid, z, 0, 1); break;
+    case 0: FlexBlock<T, false, false, 64, 64, 1, kParts>(p, lds, bid, z, 0, 1); break;
+    case 1: FlexBlock<T, true, false, 64, 64, 1, kParts>(p, lds, bid, z, 0, 1); break;
+    case 2: FlexBlock<T, false, true, 64, 64, 1, kParts>(p, lds, bid, z, 0, 1); break;
+    default: FlexBlock<T, true, true, 64, 64, 1, kParts>(p, lds, bid, z, 0, 1); break;
   }
 }
 
@@ -390,7 +394,7 @@ void RunFlexGemm(const FlexGemm& g, FlexPlan plan, hipStream_t stream) {
 
 // The split of a group: all products with at most the same number of K steps in a block, the number that the model of ChoosePlan
 // likes best.  Against the sum of the separate estimates one tenth is asked for.  Over 70 linear layers' steps (y, dx and dW; 32 to
-// 12950 rows of 65 to 3989 values, the three types) all whose estimate was that far below were faster together, by 1.17 to 2.1.
+// 12950 rows of 65 to 3989 values, the three types) all whose estimate was that far below were faster together, by 1.14 to 2.1.
 // Those above it were about even (68 | 65 us at 12950 x 108 -> 1200 in fp16, 91 | 81 at 7863 x 1533 -> 116) or slower (96 | 119 at
 // 4887 x 301 -> 2123): large products have 128x128 tiles by themselves.
 bool TryFlexGroup(const FlexGemm* g, const FlexPlan* alone, int count, hipStream_t stream) {

@@ -1843,8 +1843,8 @@ bool ForceGeneric() {
 // K (conv_few_mfma.hip) where that is estimated to be a tenth faster than gemm_flex.hip's plan (a sixth with one K step), whose
 // estimate leaves out the 2 us of a block's start and end.  A product of few rows took that kernel a launch of 64x64 tiles that are
 // mostly padding, split over K, and a second launch that adds the parts.  us, that kernel | here: 7 x 1152 -> 1792 8.9 | 4.8, 10 x 320 -> 3520
-// 9.2 | 3.5, 1 x 192 -> 1208 7.4 | 3.1, 92 x 3168 -> 576 13.3 | 8.4.  Of 150 products of 1 to 2683 rows, no multiples of 128, 129 are taken, 1.69
-// times faster in the geometric mean, the worst 0.99; not taken 1912 x 64 -> 3520 17.6 | 43.7, 466 x 3520 -> 576 28.9 | 33.6.  The result is that kernel's
+// 9.2 | 3.5, 1 x 224 -> 1208 7.4 | 3.1, 92 x 3168 -> 576 13.3 | 8.3.  Of 150 products of 1 to 2683 rows, no multiples of 128, 129 are taken, 1.70
+// times faster in the geometric mean, the worst 0.98; not taken 1912 x 64 -> 3520 17.6 | 43.7, 466 x 3520 -> 576 28.9 | 33.6.  The result is that kernel's
 // estimate where it takes the product, in the other's terms, else 0.
 double TryFewProduct(const GemmProblem& p, double flex_us, bool dry, hipStream_t stream) {
   if (p.type != GemmType::kF32 || p.trans_a || !p.trans_b || p.batch != 1 || p.shift16) return 0.0;
