@@ -104,9 +104,10 @@ size_t RunEnd(const std::vector<MergeTraits>& t, size_t i, const KernelMergeOpti
   return end;
 }
 
-int Launches(const std::vector<MergeTraits>& t, const KernelMergeOptions& options) {
+// launches of the groups from `first` to before `last`
+int Launches(const std::vector<MergeTraits>& t, size_t first, size_t last, const KernelMergeOptions& options) {
   int n = 0;
-  for (size_t i = 0; i < t.size(); i = RunEnd(t, i, options)) ++n;
+  for (size_t i = first; i < last; i = RunEnd(t, i, options)) ++n;
   return n;
 }
 
@@ -155,26 +156,34 @@ std::vector<size_t> OrderForMerging(const std::vector<std::unique_ptr<Group>>& g
     if (from < to) std::rotate(list->begin() + from, list->begin() + from + 1, list->begin() + to + 1);
     if (to < from) std::rotate(list->begin() + to, list->begin() + from, list->begin() + from + 1);
   };
-  int launches = Launches(t, options);
+  // how far a group looks, and how many places it tries in either direction: a program of thousands of groups is ordered in
+  // a time that grows with their number
+  constexpr size_t kReach = 64;
+  constexpr int kPlaces   = 8;
+  const size_t around     = options.max_members;
   for (size_t group = 0; group < order.size(); ++group) {
     size_t at = std::find(order.begin(), order.end(), group) - order.begin();
     if (!small(t[at])) continue;
     // the nearest place, later or earlier, that saves a launch: next to a kernel, past groups that it may change places with
     bool moved = false;
+    int places = 0;
     auto attempt = [&](size_t to) {
+      const size_t low = std::min(at, to), first = low > around ? low - around : 0, last = std::min(t.size(), std::max(at, to) + 1 + around);
+      const int before = Launches(t, first, last, options);
       move(&t, at, to);
-      const int now = Launches(t, options);
-      moved = now < launches;
+      moved = Launches(t, first, last, options) < before;
       if (moved) {
         move(&order, at, to);
-        launches = now;
       } else {
         move(&t, to, at);
       }
+      ++places;
     };
-    for (size_t to = at + 1; to < t.size() && !moved && MayPass(*t[at].group, *t[to].group); ++to)
+    const size_t end = std::min(t.size(), at + 1 + kReach), begin = at > kReach ? at - kReach : 0;
+    for (size_t to = at + 1; to < end && !moved && places < kPlaces && MayPass(*t[at].group, *t[to].group); ++to)
       if (to + 1 < t.size() && t[to + 1].mergeable) attempt(to);
-    for (size_t to = at; to-- > 0 && !moved && MayPass(*t[at].group, *t[to].group);)
+    places = 0;
+    for (size_t to = at; to-- > begin && !moved && places < kPlaces && MayPass(*t[at].group, *t[to].group);)
       if (to > 0 && t[to - 1].mergeable) attempt(to);
   }
   return order;
