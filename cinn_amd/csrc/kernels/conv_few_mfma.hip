@@ -15,6 +15,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <climits>
 #include <cmath>
 #include <cstdint>
@@ -22,10 +23,14 @@
 
 #include "kernels/conv_nhwc.h"
 #include "kernels/few_tile.h"
+#include "kernels/launch_count.h"
 #include "runtime/hip_check.h"
 #include "runtime/scratch.h"
 
 namespace cinn_hip_kernels {
+
+std::atomic<long long> g_launches[kCounted];
+
 namespace {
 
 using few::f32x4;
@@ -179,6 +184,7 @@ int Choose(const FewParams& p, bool fp32, double* us) {
 
 template <typename T>
 void Run(const FewParams& p, int tile, hipStream_t stream) {
+  CountLaunch(kCountConvFew + tile);
   switch (tile) {
     case 0: Launch<T, 1, 1, 8>(p, stream); break;
     case 1: Launch<T, 1, 1, 4>(p, stream); break;
@@ -204,10 +210,22 @@ double TiledMicroseconds(const FewParams& p, bool fp32) {
 
 namespace {
 
+// 1: by the rules below (default), 0: never; -1: not read yet
+std::atomic<int> g_few_mode{-1};
+
+int FewMode() {
+  int mode = g_few_mode.load(std::memory_order_relaxed);
+  if (mode < 0) {
+    const char* v = getenv("FLAGS_cinn_hip_conv_few");
+    mode          = v && *v ? (atoi(v) != 0) : 1;
+    g_few_mode.store(mode, std::memory_order_relaxed);
+  }
+  return mode;
+}
+
 // TryProductFew, and TryConvFew with other_us < 0
 double TryFew(const ConvNhwcArgs& a, double other_us, bool dry, hipStream_t stream) {
-  static const bool enabled = !(getenv("FLAGS_cinn_hip_conv_few") && atoi(getenv("FLAGS_cinn_hip_conv_few")) == 0);
-  if (!enabled || a.nchw_input || a.pool_after || a.x2) return 0.0;
+  if (FewMode() == 0 || a.nchw_input || a.pool_after || a.x2) return 0.0;
   const bool is_float = a.type.code == cinn_type_float && (a.type.bits == 32 || a.type.bits == 16);
   const bool is_bf16  = a.type.code == cinn_type_bfloat && a.type.bits == 16;
   if (!is_float && !is_bf16) return 0.0;
@@ -268,9 +286,19 @@ double TryFew(const ConvNhwcArgs& a, double other_us, bool dry, hipStream_t stre
 
 }  // namespace
 
-// FLAGS_cinn_hip_conv_few=0 switches the kernel off.
 bool TryConvFew(const ConvNhwcArgs& a, hipStream_t stream) { return TryFew(a, -1.0, false, stream) > 0.0; }
 
 double TryProductFew(const ConvNhwcArgs& a, double other_us, bool dry, hipStream_t stream) { return TryFew(a, other_us, dry, stream); }
 
 }  // namespace cinn_hip_kernels
+
+// FLAGS_cinn_hip_conv_few=0, or a mode of 0, switches the kernel off.
+extern "C" int cinn_hip_conv_few_mode(int mode) {
+  const int before = cinn_hip_kernels::FewMode();
+  if (mode == 0 || mode == 1) cinn_hip_kernels::g_few_mode.store(mode, std::memory_order_relaxed);
+  return before;
+}
+
+extern "C" long long cinn_hip_launches(int which) {
+  return which >= 0 && which < cinn_hip_kernels::kCounted ? cinn_hip_kernels::g_launches[which].load(std::memory_order_relaxed) : -1;
+}

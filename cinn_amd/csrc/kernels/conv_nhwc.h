@@ -51,6 +51,9 @@ bool TryPointwiseConvAsGemm(const ConvNhwcArgs& a, hipStream_t stream);
 // rows fit LDS (conv_patch_mfma.hip): the input patch of a band of output rows stays resident in LDS, only the filter
 // streams; same epilogue.  false when the shape does not qualify.
 bool TryConvPatch(const ConvNhwcArgs& a, hipStream_t stream);
+// whether a switch of either kernel that is not at its default is about this convolution
+bool ConvGemmForced(const ConvNhwcArgs& a);
+bool ConvPatchForced(const ConvNhwcArgs& a);
 // few output tiles, or many that are mostly padding (conv_few_mfma.hip): whole K steps of 128 bytes in every tap, same epilogue; one launch of
 // small tiles whose wavefronts share K.  false when the shape does not qualify or the tiled kernels are faster.
 bool TryConvFew(const ConvNhwcArgs& a, hipStream_t stream);

@@ -639,13 +639,17 @@ int LdsBytes(int bm, int bn, int wm) {
 // cent of the fastest everywhere: the kernel prefetches one K step ahead, so what hides the load latency is the number
 // of blocks resident on a CU, and the small tile (32 KiB of LDS) allows five.  The larger tiles stay selectable for
 // experiments (FLAGS_cinn_hip_conv_tile = 0: 128x128, 1: 128x64, 2: 64x64).
-TileChoice ChooseTile(int pixels, int oc) {
+int ForcedTile() {
   static const int forced = [] {
     const char* e = getenv("FLAGS_cinn_hip_conv_tile");
     return e ? atoi(e) : -1;
   }();
+  return forced >= 0 && forced < 4 ? forced : -1;
+}
+
+TileChoice ChooseTile(int pixels, int oc) {
   const TileChoice options[4] = {{128, 128, 4}, {128, 64, 4}, {64, 64, 4}, {128, 128, 8}};
-  if (forced >= 0 && forced < 4) return options[forced];
+  if (ForcedTile() >= 0) return options[ForcedTile()];
   (void)pixels;
   (void)oc;
   return options[2];
@@ -653,11 +657,16 @@ TileChoice ChooseTile(int pixels, int oc) {
 
 // K splits: layers whose tile grid cannot fill the 256 CUs spend their time waiting for one block's serial chain of
 // loads; splitting the reduction puts several blocks of the same tile on different CUs
-int ChooseSplits(int tiles, int steps, bool fp32, size_t bytes_per_split, size_t cap) {
+int ForcedSplits() {
   static const int forced = [] {
     const char* e = getenv("FLAGS_cinn_hip_conv_splits");
     return e ? atoi(e) : 0;
   }();
+  return forced;
+}
+
+int ChooseSplits(int tiles, int steps, bool fp32, size_t bytes_per_split, size_t cap) {
+  const int forced = ForcedSplits();
   if (forced > 0) return forced < steps ? forced : steps;
   static const bool balance = [] {  // FLAGS_cinn_hip_conv_split_balance=0: the powers of two below for fp32 as well
     const char* e = getenv("FLAGS_cinn_hip_conv_split_balance");
@@ -959,7 +968,9 @@ void RunConvNhwc(const ConvNhwcArgs& a, hipStream_t stream) {
     RunConvStem(a, stream);
     return;
   }
-  if (TryConvFew(a, stream)) return;
+  // (a tile, a split or a kernel that a switch asks for is what runs)
+  const bool forced = ForcedTile() >= 0 || ForcedSplits() > 0 || ConvPatchForced(a) || ConvGemmForced(a);
+  if (!forced && TryConvFew(a, stream)) return;
   if (TryConvPatch(a, stream)) return;
   if (TryPointwiseConvAsGemm(a, stream)) return;
   const Params p = MakeParams(a);

@@ -42,6 +42,7 @@
 #include <cstdlib>
 
 #include "kernels/conv_nhwc.h"
+#include "kernels/launch_count.h"
 #include "kernels/mfma_tile.h"
 #include "runtime/hip_check.h"
 
@@ -1093,18 +1094,25 @@ int PatchTiles() {
   return tiles;
 }
 
-}  // namespace
-
-bool TryConvPatch(const ConvNhwcArgs& a, hipStream_t stream) {
-  const int flag = PatchMode();
-  if (flag == 0) return false;
+// what the kernels of this file compute
+bool PatchLayer(const ConvNhwcArgs& a) {
   const bool is_f16  = a.type.code == cinn_type_float && a.type.bits == 16;
   const bool is_bf16 = a.type.code == cinn_type_bfloat && a.type.bits == 16;
   if ((!is_f16 && !is_bf16) || a.nchw_input) return false;
   if (a.kh != 3 || a.kw != 3 || a.stride_h != 1 || a.stride_w != 1 || a.pad_h != 1 || a.pad_w != 1 || a.dil_h != 1 ||
       a.dil_w != 1 || a.oh != a.h || a.ow != a.w_in)
     return false;
-  if (a.c % 64 != 0 || a.c > 2048 || a.oc % 64 != 0) return false;  // one chunk, or two and more
+  return a.c % 64 == 0 && a.c <= 2048 && a.oc % 64 == 0;  // one chunk, or two and more
+}
+
+}  // namespace
+
+bool ConvPatchForced(const ConvNhwcArgs& a) { return (PatchMode() != 1 || PatchTiles() != 0 || !PatchStream()) && PatchLayer(a); }
+
+bool TryConvPatch(const ConvNhwcArgs& a, hipStream_t stream) {
+  const int flag = PatchMode();
+  if (flag == 0 || !PatchLayer(a)) return false;
+  const bool is_bf16 = a.type.code == cinn_type_bfloat;
   if ((int64_t)a.n * a.h * a.w_in * a.c >= INT_MAX || (int64_t)a.n * a.h * a.w_in * a.oc >= INT_MAX) return false;
   if (reinterpret_cast<uintptr_t>(a.x) % 16 != 0 || reinterpret_cast<uintptr_t>(a.w) % 16 != 0 ||
       reinterpret_cast<uintptr_t>(a.y) % 16 != 0 || reinterpret_cast<uintptr_t>(a.residual) % 16 != 0)
@@ -1155,6 +1163,7 @@ bool TryConvPatch(const ConvNhwcArgs& a, hipStream_t stream) {
   p.probe       = g_patch_probe.load(std::memory_order_relaxed);
   MagicFor(chunked ? (a.w_in + 7) & ~7 : a.w_in, &p.w_magic, &p.w_shift);
   MagicFor(a.w_in + 2, &p.pw_magic, &p.pw_shift);
+  CountLaunch(kCountConvPatch);
   if (chunked && tiles == 2) {
     if (is_bf16) {
       LaunchChunks<__bf16, 2, 2>(p, plan, stream);

@@ -25,6 +25,7 @@
 #include <type_traits>
 
 #include "kernels/flex_tile.h"
+#include "kernels/launch_count.h"
 #include "runtime/hip_check.h"
 #include "runtime/scratch.h"
 
@@ -437,6 +438,7 @@ bool TryFlexGroup(const FlexGemm* g, const FlexPlan* alone, int count, hipStream
     most = std::max(4, most > 8 ? most * 3 / 4 : most - 1);
   }
   if (best >= 0.9 * sum) return false;
+  CountLaunch(kCountProductGroup);
   // the longest blocks first
   FlexGemm ordered[kFlexGroup];
   int order[kFlexGroup] = {0, 1, 2, 3}, ordered_splits[kFlexGroup];

@@ -2039,10 +2039,24 @@ bool ConvPairShape(int64_t m, int c1, int c2, int oc) {
   return tiles256 >= 192 || tiles128 >= 192 || (tiles128 >= 128 && c1 + c2 >= 4096);
 }
 
-bool TryPointwiseConvAsGemm(const ConvNhwcArgs& a, hipStream_t stream) {
-  // FLAGS_cinn_hip_conv_pointwise_gemm: 0 keeps 1x1 layers on the convolution kernel, 2 sends every one the GEMM
-  // kernels can take to them, whatever the grid (for measurements)
+// FLAGS_cinn_hip_conv_pointwise_gemm: 0 keeps 1x1 layers on the convolution kernel, 2 sends every one the GEMM
+// kernels can take to them, whatever the grid (for measurements)
+static int PointwiseMode() {
   static const int mode = getenv("FLAGS_cinn_hip_conv_pointwise_gemm") ? atoi(getenv("FLAGS_cinn_hip_conv_pointwise_gemm")) : 1;
+  return mode;
+}
+
+bool ConvGemmForced(const ConvNhwcArgs& a) {
+  // tile, stages or split of the direct-to-LDS kernel
+  static const bool form = [] {
+    const char *tile = getenv("FLAGS_cinn_hip_gemm_tile"), *stages = getenv("FLAGS_cinn_hip_gemm_stages"), *split = getenv("FLAGS_cinn_hip_gemm_split_k");
+    return (tile && atoi(tile) != 0) || (stages && atoi(stages) != 0) || (split && atoi(split) >= 2);
+  }();
+  return a.type.bits == 16 && (form || (PointwiseMode() == 2 && a.kh == 1 && a.kw == 1));
+}
+
+bool TryPointwiseConvAsGemm(const ConvNhwcArgs& a, hipStream_t stream) {
+  const int mode     = PointwiseMode();
   const bool enabled = mode != 0;
   // a second input has no other implementation: the measurement flags do not apply to it
   const bool pair = a.x2 != nullptr;

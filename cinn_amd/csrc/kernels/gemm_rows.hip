@@ -28,6 +28,7 @@
 
 #include "cinn_hip_runtime.h"
 #include "kernels/few_tile.h"
+#include "kernels/launch_count.h"
 #include "runtime/hip_check.h"
 
 namespace cinn_hip_kernels {
@@ -373,6 +374,7 @@ bool RingTakes(const RowProduct& p) {
 template <typename T>
 bool TryRing(const RowProduct& p, hipStream_t stream) {
   if (!RingTakes(p)) return false;
+  CountLaunch(kCountRowsRing);
   if (p.gamma) {
     // With a block for every CU twice the columns in each: 1 x 384 -> 6272 4.4 | 3.8, 32 x 768 -> 3072 5.5 | 4.5, 16 x 1280 -> 5120 8.8 |
     // 5.7 (its rings leave room for one block on a CU); 256 blocks 16 x 1024 -> 4096 4.7 | 5.0
@@ -405,6 +407,7 @@ void Launch(const RowProduct& p, hipStream_t stream) {
     CINN_HIP_CALL(hipGetLastError());
     return;
   }
+  CountLaunch(kCountRows);
   int mt = (p.m + 15) / 16;
   dim3 grid((unsigned)((p.n + 15) / 16));
   // Fewer column blocks than CUs: one block per 16 rows as well.  A block's traffic is its 16 columns of B plus the
