@@ -76,9 +76,35 @@ bool Reads(const Group& g, const Group& writer) {
   return false;
 }
 
+// the program input that a group sees in `v`: `v` itself, or what it is a reshape (a view) of; null for a computed value
+const NodeData* ProgramInput(const NodeData* v) {
+  while (v->producer && v->producer->op_type() == "reshape") v = v->producer->inputs[0];
+  return v->producer ? nullptr : v;
+}
+
+// a value that the program returns, itself or through reshapes
+bool IsResult(const NodeData* v) {
+  if (v->is_fetch || v->consumers.empty()) return true;
+  for (auto* n : v->consumers)
+    if (n->op_type() == "reshape" && IsResult(n->outputs[0])) return true;
+  return false;
+}
+
+// `g` reads a program input that `reader` reads and writes a result of its type and size: a caller may have bound that
+// result to the input's memory, an update in place, and what `reader` sees depends on which of the two comes first.
+bool MayUpdate(const Group& g, const Group& reader) {
+  for (auto* read : reader.inputs) {
+    const NodeData* input = ProgramInput(read);
+    if (!input || std::none_of(g.inputs.begin(), g.inputs.end(), [&](const NodeData* in) { return ProgramInput(in) == input; })) continue;
+    for (auto* out : g.outputs)
+      if (IsResult(out) && out->dtype == input->dtype && out->numel() == input->numel()) return true;
+  }
+  return false;
+}
+
 // One behind the last group of the run that begins at t[i]: the longest run of consecutive kernels none of which reads what an
-// earlier one of the run writes; the run is consecutive in execution order, so a dependence through other groups would
-// pass through a member as well.
+// earlier one of the run writes, or may update what another one reads (the blocks of a launch run in any order); the run is
+// consecutive in execution order, so a dependence through other groups would pass through a member as well.
 size_t RunEnd(const std::vector<MergeTraits>& t, size_t i, const KernelMergeOptions& options) {
   if (!t[i].mergeable) return i + 1;
   int64_t blocks = t[i].grid;
@@ -93,7 +119,8 @@ size_t RunEnd(const std::vector<MergeTraits>& t, size_t i, const KernelMergeOpti
     const bool same = SameBlock(t[i], t[end]);
     if ((run_flat || !same) && (!all_flattenable || !t[end].flattenable || t[i].threads != t[end].threads)) break;
     bool depends = false;
-    for (size_t k = i; k < end; ++k) depends |= Reads(*t[end].group, *t[k].group);
+    for (size_t k = i; k < end; ++k)
+      depends |= Reads(*t[end].group, *t[k].group) || MayUpdate(*t[end].group, *t[k].group) || MayUpdate(*t[k].group, *t[end].group);
     if (depends) break;
     if (blocks + t[end].grid > 0x7fffffff) break;
     blocks += t[end].grid;
@@ -111,21 +138,9 @@ int Launches(const std::vector<MergeTraits>& t, size_t first, size_t last, const
   return n;
 }
 
-// `g` reads a program input and writes a result of its size: a caller may have bound both to the same memory
-bool MayUpdate(const Group& g, const NodeData& input) {
-  if (input.producer || std::find(g.inputs.begin(), g.inputs.end(), &input) == g.inputs.end()) return false;
-  for (auto* out : g.outputs)
-    if ((out->is_fetch || out->consumers.empty()) && out->dtype == input.dtype && out->numel() == input.numel()) return true;
-  return false;
-}
-
 // whether two groups that are not ordered by a value may change places
 bool MayPass(const Group& a, const Group& b) {
-  for (auto* in : a.inputs)
-    if (MayUpdate(b, *in)) return false;
-  for (auto* in : b.inputs)
-    if (MayUpdate(a, *in)) return false;
-  return !Reads(a, b) && !Reads(b, a);
+  return !Reads(a, b) && !Reads(b, a) && !MayUpdate(a, b) && !MayUpdate(b, a);
 }
 
 LaunchUnit UnitOf(const Group& g) {
