@@ -61,6 +61,7 @@ struct Group {
   // kRowReduce: rows x cols of the reduction space
   int64_t rows{0}, cols{0};
   bool pre_run{false};  // every node of the group is a pre-run node
+  int program_run{-1};  // which run of kernels, that can share a launch, it stands in before OrderForMerging moves any
   std::string func_name;
 };
 

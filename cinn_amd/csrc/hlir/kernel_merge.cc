@@ -102,8 +102,17 @@ bool MayUpdate(const Group& g, const Group& reader) {
   return false;
 }
 
+// Whether two groups that are not ordered by a value still keep their order, so that no launch runs their blocks side by side:
+// one may update what the other reads, element by element; or in any way, unless the program itself has the two next to
+// each other (a softmax and a maximum of one input have always shared a launch there).
+bool KeepOrder(const Group& a, const Group& b) {
+  const bool updates = MayUpdate(a, b), updated = MayUpdate(b, a);
+  if (!updates && !updated) return false;
+  return (updates && a.kind == GroupKind::kElementwise) || (updated && b.kind == GroupKind::kElementwise) || a.program_run != b.program_run;
+}
+
 // One behind the last group of the run that begins at t[i]: the longest run of consecutive kernels none of which reads what an
-// earlier one of the run writes, or may update what another one reads (the blocks of a launch run in any order); the run is
+// earlier one of the run writes, or keeps its order for another reason; the run is
 // consecutive in execution order, so a dependence through other groups would pass through a member as well.
 size_t RunEnd(const std::vector<MergeTraits>& t, size_t i, const KernelMergeOptions& options) {
   if (!t[i].mergeable) return i + 1;
@@ -120,7 +129,7 @@ size_t RunEnd(const std::vector<MergeTraits>& t, size_t i, const KernelMergeOpti
     if ((run_flat || !same) && (!all_flattenable || !t[end].flattenable || t[i].threads != t[end].threads)) break;
     bool depends = false;
     for (size_t k = i; k < end; ++k)
-      depends |= Reads(*t[end].group, *t[k].group) || MayUpdate(*t[end].group, *t[k].group) || MayUpdate(*t[k].group, *t[end].group);
+      depends |= Reads(*t[end].group, *t[k].group) || KeepOrder(*t[end].group, *t[k].group);
     if (depends) break;
     if (blocks + t[end].grid > 0x7fffffff) break;
     blocks += t[end].grid;
@@ -161,6 +170,9 @@ std::vector<size_t> OrderForMerging(const std::vector<std::unique_ptr<Group>>& g
   std::vector<size_t> order(groups.size());
   for (size_t i = 0; i < order.size(); ++i) order[i] = i;
   std::vector<MergeTraits> t = TraitsOf(groups, funcs, barrier, options);
+  for (auto& g : groups) g->program_run = -1;
+  for (size_t i = 0, run = 0; i < t.size(); ++run)
+    for (const size_t end = RunEnd(t, i, options); i < end; ++i) groups[i]->program_run = static_cast<int>(run);
   auto small = [&](const MergeTraits& m) {
     int64_t bytes = 0;
     for (auto* list : {&m.group->inputs, &m.group->outputs})

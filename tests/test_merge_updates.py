@@ -41,6 +41,31 @@ def test_reader_and_update_have_launches_of_their_own(reader, between, result):
     assert len(reads) == 1 and updates and reads[0] < min(updates), args
 
 
+# an update that reads more than it writes over, as a softmax: kept apart by what stands between the two in the program, which no
+# move takes out of the way; next to each other they share a launch, as they always have
+@pytest.mark.parametrize("reader", sorted(set(READERS) - {"softmax", "sum"}))  # (those of whole rows are fused with the softmax, in one thread)
+@pytest.mark.parametrize("first", ["reader", "update"])
+@pytest.mark.parametrize("between", ["products", "nothing"])
+def test_update_by_rows(reader, first, between):
+    b = NetBuilder("rows")
+    x, w, state = (b.create_input(Float(32), [64, 64], name) for name in ("x", "w", "state"))
+    parts = {"reader": lambda: READERS[reader](b, state), "update": lambda: b.softmax(state, axes=[-1])}
+    second = "update" if first == "reader" else "reader"
+    outs = {first: parts[first]()}
+    if between == "products":
+        y = outs["y"] = b.matmul(x, w)
+    outs[second] = parts[second]()
+    if between == "products":
+        outs["z"] = b.matmul(y, w)
+    args = instructions(b, list(outs.values()))
+    at = {name: [i for i, a in enumerate(args) if outs[name].id in a] for name in ("reader", "update")}
+    assert len(at["reader"]) == len(at["update"]) == 1
+    if between == "products":
+        assert at[first][0] < at[second][0], args
+    else:
+        assert at[first] == at[second], args
+
+
 def test_readers_that_update_nothing_share_a_launch():
     b = NetBuilder("readers")
     x, w, state = (b.create_input(Float(32), [64, 64], name) for name in ("x", "w", "state"))
