@@ -225,7 +225,13 @@ class RowProductFuser {
     const int reader = OnlyReader(y);
     cinn_hip_kernels::RowFusion fuse{k <= cinn_hip_kernels::kRowProductMaxNormK && OnlyReader(x4) >= 0 && MatchNorm(x, &norm),
                                      reader >= 0 && instrs_[reader]->op_type == "gelu" && !dropped_[reader]};
-    fuse = cinn_hip_kernels::ChooseRowFusion(m, n, k, fuse);
+    std::vector<size_t> columns;
+    if (!fuse.gelu && !residual) columns = Columns(y);
+    cinn_hip_kernels::RowProduct product{};  // (a program's tensors are aligned)
+    product.m = m, product.n = n, product.k = k;
+    product.width   = columns.empty() ? n : n / static_cast<int>(columns.size());
+    const bool ring = cinn_hip_kernels::RowRingTakes(product);
+    fuse            = cinn_hip_kernels::ChooseRowFusion(m, n, k, ring, fuse);
     if (fuse.norm) {
       call->inputs[0] = norm.x;
       call->inputs.push_back(norm.gamma);
@@ -234,15 +240,12 @@ class RowProductFuser {
     }
     for (size_t j : {size_t(0), size_t(1), size_t(4)})  // the views as images
       if (j < conv->inputs.size() && OnlyReader(conv->inputs[j]) >= 0) drop.push_back(defined_at_.at(conv->inputs[j]->id));
-    std::vector<size_t> columns;
     if (fuse.gelu) {
       y    = instrs_[reader]->outputs[0];
       last = static_cast<size_t>(reader);
       drop.push_back(last);
-    } else if (!residual) {
-      columns = Columns(y);
     }
-    if (!fuse.norm && !fuse.gelu && !((plain || !columns.empty()) && cinn_hip_kernels::RowProductPays(m, n, k, !columns.empty(), false))) return;
+    if (!fuse.norm && !fuse.gelu && !((plain || !columns.empty()) && cinn_hip_kernels::RowProductPays(m, n, k, ring, !columns.empty(), false))) return;
     if (columns.empty()) {
       call->outputs = {y};
     } else {

@@ -1538,8 +1538,9 @@ bool TrySkinny(const GemmProblem& p, hipStream_t stream) {
   r.scale = p.scale, r.shift = p.shift, r.alpha = p.alpha, r.relu = p.relu;
   r.residual       = p.residual ? p.residual : (p.beta != 0.0f ? p.c : nullptr);
   r.residual_scale = p.residual ? p.residual_scale : p.beta;
-  if (!cinn_hip_kernels::RowProductSupported(r) || !cinn_hip_kernels::RowProductPays(p.m, p.n, p.k, false, p.scale == nullptr)) return false;
-  if (!p.dry) cinn_hip_kernels::RunRowProduct(r, stream);
+  using namespace cinn_hip_kernels;
+  if (!RowProductSupported(r) || !RowProductPays(p.m, p.n, p.k, RowRingTakes(r), false, p.scale == nullptr)) return false;
+  if (!p.dry) RunRowProduct(r, stream);
   return true;
 }
 
@@ -2090,7 +2091,10 @@ bool TryPointwiseConvAsGemm(const ConvNhwcArgs& a, hipStream_t stream) {
     const int64_t tiles64 = ((pixels + 63) / 64) * ((a.oc + 63) / 64), tiles128 = ((pixels + 127) / 128) * ((a.oc + 127) / 128);
     const bool one_round128 = forced_tile == 0 && a.c % 64 == 0 && tiles64 > 256 && tiles128 < 192 && (a.c >= 768 || (a.c >= 384 && tiles128 >= 128));
     // at most 64 pixels (a matmul with few rows written as a 1x1 layer, its bias as the shift): gemm_rows.hip
-    const bool few_rows = forced_tile == 0 && pixels <= 64 && a.c % 32 == 0 && cinn_hip_kernels::RowProductPays((int)pixels, a.oc, a.c, false, false);
+    RowProduct r{};
+    r.a = a.x, r.b = a.w, r.c[0] = a.y, r.scale = a.scale, r.shift = a.shift, r.residual = a.residual;
+    r.m = (int)pixels, r.n = r.width = a.oc, r.k = a.c;
+    const bool few_rows = forced_tile == 0 && pixels <= 64 && a.c % 32 == 0 && RowProductPays(r.m, r.n, r.k, RowRingTakes(r), false, false);
     if (mode != 2 && !shortk && !long_k && !few_rows && !one_round128 && (a.c < 128 || (!narrow && tiles128 < 192)))
       return false;
     p.k = a.c;

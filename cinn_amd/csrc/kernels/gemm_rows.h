@@ -34,14 +34,16 @@ constexpr int kRowProductMaxNormK = 1280;
 
 // false where the kernel does not take the extents; operands lie at any address of their type
 bool RowProductSupported(const RowProduct& p);
-// whether the kernel is ahead of the tiled ones for a product that it takes; `saves_launch`: several results, which would
+// which of the file's two kernels runs it: gemm_rows_ring_kernel, or gemm_rows_kernel; by the addresses as well where there are any
+bool RowRingTakes(const RowProduct& p);
+// whether the kernel (`ring`: which one, as above) is ahead of the tiled ones for a product that it takes; `saves_launch`: several results, which would
 // be copied out of one; `splits`: without a scale, which gemm_flex.hip would take and split its K
-bool RowProductPays(int m, int n, int k, bool saves_launch, bool splits);
+bool RowProductPays(int m, int n, int k, bool ring, bool saves_launch, bool splits);
 // which of a layer norm before the product and a gelu behind it (those that there are) are faster inside
 struct RowFusion {
   bool norm, gelu;
 };
-RowFusion ChooseRowFusion(int m, int n, int k, RowFusion there);
+RowFusion ChooseRowFusion(int m, int n, int k, bool ring, RowFusion there);
 void RunRowProduct(const RowProduct& p, hipStream_t stream);
 
 }  // namespace cinn_hip_kernels

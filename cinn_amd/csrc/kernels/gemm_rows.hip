@@ -363,17 +363,9 @@ void LaunchNorm(const RowProduct& p, hipStream_t stream) {
   }
 }
 
-// whole K steps in aligned rows, results in aligned groups of four columns
-bool RingTakes(const RowProduct& p) {
-  uintptr_t wide = 0, four = 0;
-  for (const void* q : {p.a, p.b, static_cast<const void*>(p.scale), static_cast<const void*>(p.shift), p.gamma, p.beta}) wide |= reinterpret_cast<uintptr_t>(q);
-  for (const void* q : {p.residual, static_cast<const void*>(p.c[0]), static_cast<const void*>(p.c[1]), static_cast<const void*>(p.c[2])}) four |= reinterpret_cast<uintptr_t>(q);
-  return p.k % 64 == 0 && p.n % 4 == 0 && p.width % 4 == 0 && wide % 16 == 0 && four % 8 == 0 && (int64_t)p.m * p.k < (1 << 30) && (int64_t)p.n * p.k < (1 << 30);
-}
-
 template <typename T>
 bool TryRing(const RowProduct& p, hipStream_t stream) {
-  if (!RingTakes(p)) return false;
+  if (!RowRingTakes(p)) return false;
   CountLaunch(kCountRowsRing);
   if (p.gamma) {
     // With a block for every CU twice the columns in each: 1 x 384 -> 6272 4.4 | 3.8, 32 x 768 -> 3072 5.5 | 4.5, 16 x 1280 -> 5120 8.8 |
@@ -445,6 +437,14 @@ bool RowProductSupported(const RowProduct& p) {
   return !p.gamma || (p.beta && p.k <= kRowProductMaxNormK);
 }
 
+// whole K steps in aligned rows, results in aligned groups of four columns
+bool RowRingTakes(const RowProduct& p) {
+  uintptr_t wide = 0, four = 0;
+  for (const void* q : {p.a, p.b, static_cast<const void*>(p.scale), static_cast<const void*>(p.shift), p.gamma, p.beta}) wide |= reinterpret_cast<uintptr_t>(q);
+  for (const void* q : {p.residual, static_cast<const void*>(p.c[0]), static_cast<const void*>(p.c[1]), static_cast<const void*>(p.c[2])}) four |= reinterpret_cast<uintptr_t>(q);
+  return p.k % 64 == 0 && p.n % 4 == 0 && p.width % 4 == 0 && wide % 16 == 0 && four % 8 == 0 && (int64_t)p.m * p.k < (1 << 30) && (int64_t)p.n * p.k < (1 << 30);
+}
+
 // For gemm_rows_kernel: every wavefront waits for its own rows of B: with one block per CU (16 columns each; 16 rows, or all of them from 256 blocks of
 // columns on) that hides the launch, further ones take about as long again, where the tiled kernels need a few hundred tiles for
 // the same result.  us, tiled | here, fp16, at most as many blocks as CUs: 16 x 192 -> 4096 3.9 | 3.8, 64 x 960 -> 1000 7.3 | 4.3, two row
@@ -457,8 +457,8 @@ bool RowProductSupported(const RowProduct& p) {
 // That kernel splits a long K over more blocks than there are columns, where it can take the product (a plain one: `splits`): 64 x 6112 -> 64
 // 9.1 | 9.7, 24 x 7968 -> 200 9.1 | 11.7 (but 1 x 6112 -> 1000 8.7 | 7.0), 64 x 5024 -> 2048 11.7 | 14.9, 24 x 3968 -> 25 7.2 | 8.7; a layer with its scale
 // and shift has a convolution's tiles instead, 8 x 6112 -> 4096 with gelu 18.7 | 10.0.
-bool RowProductPays(int m, int n, int k, bool saves_launch, bool splits) {
-  if (k % 64 == 0 && n % 4 == 0) {
+bool RowProductPays(int m, int n, int k, bool ring, bool saves_launch, bool splits) {
+  if (ring) {
     // More than two row tiles of many columns: the tiled kernels' larger tiles pull in less, until K is long enough to be shared.  us,
     // tiled | here, fp16: 64 x 64 -> 12288 3.7 | 5.3, 64 x 512 -> 12288 5.8 | 6.4, 64 x 512 -> 32768 8.7 | 12.8, 64 x 1024 -> 32768 14.5 | 18.8, 32 x 192 ->
     // 32768 5.8 | 6.6; 64 x 128 -> 8192 3.9 | 3.9, 64 x 2048 -> 16384 15.0 | 15.2, 32 x 320 -> 32768 6.8 | 6.9, 16 x 1024 -> 8192 7.9 | 3.4.
@@ -484,8 +484,8 @@ bool RowProductPays(int m, int n, int k, bool saves_launch, bool splits) {
 // 2048 -> 16384 17.1 | 14.0, but 32 x 8192 -> 4096 (alone one round of two row tiles) 26.8 | 31.5.  Both: one round
 // 64 x 320 -> 1024 9.9 | 6.2, two 16 x 128 -> 8192 8.3 | 8.9, 48 x 192 -> 2048 9.2 | 8.9, three 64 x 320 -> 3072 10.0 | 12.6, six 64 x 1280 -> 6144 28.1 |
 // 24.9, eight 64 x 1280 -> 8192 28.9 | 32.6, four 64 x 768 -> 4096 13.0 | 16.9; the same blocks alone 64 x 768 -> 3072 15.5 | 13.1.
-RowFusion ChooseRowFusion(int m, int n, int k, RowFusion there) {
-  if (k % 64 == 0 && n % 4 == 0) {
+RowFusion ChooseRowFusion(int m, int n, int k, bool ring, RowFusion there) {
+  if (ring) {
     // gemm_rows_ring_kernel, blocks of 16 or of 32 columns.  us, outside | inside, norm: 1 x 128 -> 4096 5.3 | 3.1, 16 x 1280 -> 5120 6.6 | 5.8,
     // 32 x 1024 -> 4096 (256 blocks of 32) 5.9 | 5.3, 32 x 512 -> 8192 (512) 5.7 | 5.1, 64 x 768 -> 3072 (384) 6.4 | 6.1; 64 x 384 -> 6272 (784)
     // 6.3 | 6.9, 8 x 1280 -> 9984 (312) 7.5 | 7.8, 64 x 1024 -> 4096 (512) 6.4 | 7.0, 48 x 1280 -> 5120 (480) 8.1 | 8.2.  gelu: 1 x 768 -> 3072 5.8 |
@@ -498,7 +498,7 @@ RowFusion ChooseRowFusion(int m, int n, int k, RowFusion there) {
   const int rounds = ((n + 15) / 16 * ((m + 15) / 16) + 255) / 256;
   const bool same  = k % 256 == 0 && n <= 4080;  // the blocks of the product alone
   if (there.norm && there.gelu && (same || rounds <= 1 || (rounds <= 2 && k >= 192) || (rounds <= 6 && k >= 1152))) return there;
-  if (there.gelu && ((rounds <= 2 && k < 3072) || ((n <= 4080 || m <= 16) && RowProductPays(m, n, k, false, false)))) return {false, true};
+  if (there.gelu && ((rounds <= 2 && k < 3072) || ((n <= 4080 || m <= 16) && RowProductPays(m, n, k, false, false, false)))) return {false, true};
   return {there.norm && (rounds <= 1 || (same && k >= (rounds <= 2 ? 512 : 768)) || (rounds <= 2 && k >= 896) || (rounds <= 3 && k >= 1152)), false};
 }
 

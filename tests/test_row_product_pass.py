@@ -86,6 +86,14 @@ def test_what_a_product_of_few_rows_takes_along(m, k, n, norm, gelu, calls):
     assert len(got) == calls, got
 
 
+# results in other than whole groups of four columns run on the kernel without rings, and go by its rule
+@pytest.mark.parametrize("width,calls", [(2050, 2), (2052, 1)])
+def test_what_a_product_of_several_results_takes_along(width, calls):
+    b, y = linear_layer(32, 384, 2 * width, True, False)
+    got = names(compile_only(b, [b.slice(y, [1], [0], [width]), b.slice(y, [1], [width], [2 * width])]))
+    assert len(got) == calls and any("matmul_rows" in e for e in got), got
+
+
 @pytest.mark.parametrize("flag,taken", [("0", False), ("1", True)])
 def test_switch_of_the_kernel(monkeypatch, flag, taken):
     monkeypatch.setenv("FLAGS_cinn_hip_gemm_skinny", flag)
