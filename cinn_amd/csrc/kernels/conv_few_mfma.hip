@@ -194,7 +194,8 @@ void Run(const FewParams& p, int tile, hipStream_t stream) {
   }
 }
 
-// us of the tiled kernels; fitted to 140 layers in fp32, 1x1 to 7x7 (9% off on average), and 62 of more than 128 tiles in 16 bits (17%)
+// us of the tiled kernels; fitted to 140 layers in fp32, 1x1 to 7x7 (9% off on average), and 62 of more than 128 tiles in 16 bits (17%;
+// 105 of up to 128 tiles: 10%)
 double TiledMicroseconds(const FewParams& p, bool fp32) {
   const int tiles  = (int)std::min<int64_t>((int64_t)((p.pixels + 63) / 64) * ((p.oc + 63) / 64), 1 << 24);
   const int splits = ConvSplits(tiles, p.steps, fp32), share = (p.steps + splits - 1) / splits;
@@ -223,8 +224,8 @@ int FewMode() {
   return mode;
 }
 
-// TryProductFew, and TryConvFew with other_us < 0
-double TryFew(const ConvNhwcArgs& a, double other_us, bool dry, hipStream_t stream) {
+// TryProductFew, and TryConvFew with limit_us < 0
+double TryFew(const ConvNhwcArgs& a, double limit_us, bool dry, hipStream_t stream) {
   if (FewMode() == 0 || a.nchw_input || a.pool_after || a.x2) return 0.0;
   const bool is_float = a.type.code == cinn_type_float && (a.type.bits == 32 || a.type.bits == 16);
   const bool is_bf16  = a.type.code == cinn_type_bfloat && a.type.bits == 16;
@@ -240,18 +241,24 @@ double TryFew(const ConvNhwcArgs& a, double other_us, bool dry, hipStream_t stre
   if ((int64_t)a.n * a.h * a.w_in * a.c * elem >= kLimit || a.oc * k_total * elem >= kLimit) return 0.0;
   // (512 threads for each tile of 16x16: fewer than 2^32 of a launch)
   if (pixels < 1 || pixels >= (1 << 24) || pixels * a.oc >= (1 << 30)) return 0.0;
-  // Up to half as many tiles of 64x64 as CUs.  us, tiled | here: 98 tiles (fp16, 256 -> 256 3x3 on 14x14, 8 images) 10.9 | 8.4, 104 (fp32,
-  // 512 -> 512 3x3 on 7x7, 16 images) 52.0 | 44.2, 112 (512 -> 1024 1x1 on 14x14, 2 images) 6.1 | 5.1.
+  // A convolution goes by the two estimates.  Up to half as many tiles of 64x64 as CUs most are far apart: us, tiled | here, in fp16
+  // 98 tiles (256 -> 256 3x3 on 14x14, 8 images) 14.0 | 7.9, in fp32 26 tiles (128 -> 128 3x3 on 28x28) 13.0 | 6.7, 49 (64 -> 64 3x3 on 56x56) 11.7 | 6.6.
+  // What is even or slower is a long K, shared by four or eight wavefronts instead of up to eight blocks of four.  In 16 bits, 105 layers of up
+  // to 128 tiles: below 0.97 of the tiled kernels' estimate 93 of 94 are faster or even (0.99 to 2.4; 320 -> 448 7x7 on 29x32 27.2 | 29.8 is the
+  // other one), above it 9 of 11 slower or even (512 -> 144 7x7 on 39x49 40.3 | 46.2).  In fp32, 70 layers: of less than 200 steps below 0.95 44 are 0.97 to 2.6
+  // times as fast, above it 6 0.86 to 1.02 (448 -> 64 3x3 on 45x28, 5 images, 39.6 | 45.5); of more below 0.9 5 1.05 to 1.2, above it 15 0.73 to 1.0 (384 ->
+  // 64 7x7 on 57x57 82.8 | 112.9).  The filters' scale has no part in it.
   // Beyond, the tiled kernels' larger tiles pull in less, but a tile's columns are 64: layers of 8 to 60 filters, or a few more than
-  // a multiple of 64, multiply mostly padding there.  Those go by the two estimates, a fifth apart.  60 layers in fp16 of 132 to 1168
-  // tiles: 23 taken, 1.17 to 2.3 times faster (64 -> 16 7x7 on 38x22, 24 images, 25.1 | 11.4; 512 -> 12 5x5 on 57x56, 3 images, 16.3 | 7.8), none slower;
-  // of those not taken 316 tiles (384 -> 72 5x5) 33.3 | 43.9, 485 (256 -> 304 1x1) 6.3 | 11.2, 945 (128 -> 192 3x3) 22.6 | 34.4.
-  // 140 in fp32, where these tiles are bound by the matrix pipe and padding costs most: 85 taken, 1.16 to 3.8 times faster (480 -> 16
-  // 1x1 / 2 on 16x11, 27 images, 12.9 | 3.4, 96 -> 200 3x3 / 2 on 35x41, 8 images, 22.5 | 19.3).  A multiple of 64 has no such columns: in 16 bits 196 tiles (256 -> 128 1x1
-  // on 56x56, 2 images) 4.6 | 6.2.  (In fp32 a convolution of such filters without a layer's scale stays with the tiled kernels at any size:
-  // the K that they split for it is what the tests of scratch memory under graph replay hold on to.)
-  const bool few_tiles = ((pixels + 63) / 64) * ((a.oc + 63) / 64) <= 128 && (elem == 2 || a.scale);
-  if (other_us < 0.0 && !few_tiles && a.oc % 64 == 0 && (elem == 2 || !a.scale)) return 0.0;
+  // a multiple of 64, multiply mostly padding there.  60 layers in fp16 of 132 to 1168
+  // tiles: 23 are a fifth below, 1.17 to 2.3 times faster (64 -> 16 7x7 on 38x22, 24 images, 25.1 | 11.4; 512 -> 12 5x5 on 57x56, 3 images, 16.3 | 7.8), none slower;
+  // of the others 316 tiles (384 -> 72 5x5) 33.3 | 43.9, 485 (256 -> 304 1x1) 6.3 | 11.2, 945 (128 -> 192 3x3) 22.6 | 34.4.  A multiple of 64 has no
+  // such columns: 196 tiles (256 -> 128 1x1 on 56x56, 2 images) 4.6 | 6.2.
+  // In fp32 these tiles are bound by the matrix pipe, and whole columns gain as well, but four steps and fewer are bound by what they
+  // store: 1 (32 -> 384 1x1 on 43x30, 2 images) 4.9 | 7.9, 3 (96 -> 192 1x1 on 14x46, 8 images) 6.5 | 8.2, 4 (128 -> 40 1x1 / 2) 6.5 | 6.7.  From 5 steps
+  // on a fifth below: 140 layers 1.16 to 3.8 times faster (480 -> 16 1x1 / 2 on 16x11, 27 images, 12.9 | 3.4), 37 of 129 to 426 tiles 0.97 to 1.8
+  // (64 -> 512 3x3 / 2 on 37x24, 5 images, 16.1 | 13.5); of those not taken 404 tiles (256 -> 128 1x1) 14.4 | 16.6, 836 (32 -> 256 3x3 / 2) 26.0 | 42.9.
+  const bool few_tiles = ((pixels + 63) / 64) * ((a.oc + 63) / 64) <= 128;
+  if (limit_us < 0.0 && !few_tiles && (elem == 2 ? a.oc % 64 == 0 : k_total <= 4 * lanes)) return 0.0;
   // (a single K step of few rows has nothing to share: 1 x 64 -> 4096 2.4 | 3.0, 8 x 64 -> 4096 2.9 | 3.0; 3136 x 64 -> 64 and more gain)
   if (k_total == lanes && pixels <= 16) return 0.0;
   const bool outside = a.pad_h > 0 || a.pad_w > 0 || (int64_t)(a.oh - 1) * a.stride_h - a.pad_h + (int64_t)(a.kh - 1) * a.dil_h >= a.h ||
@@ -272,7 +279,8 @@ double TryFew(const ConvNhwcArgs& a, double other_us, bool dry, hipStream_t stre
   p.pixels_outer = (int64_t)a.n * a.h * a.w_in * a.c > a.oc * k_total;
   double us;
   const int tile = Choose(p, elem == 4, &us);
-  if (other_us >= 0.0 ? us >= (p.steps > 1 ? 0.9 : 0.83) * other_us : !few_tiles && us >= 0.8 * TiledMicroseconds(p, elem == 4)) return 0.0;
+  const double share = !few_tiles ? 0.8 : elem == 2 ? 0.97 : p.steps < 200 ? 0.95 : 0.9;
+  if (us >= (limit_us < 0.0 ? share * TiledMicroseconds(p, elem == 4) : limit_us)) return 0.0;
   if (dry) return us;
   if (is_bf16) {
     Run<__bf16>(p, tile, stream);
@@ -288,7 +296,7 @@ double TryFew(const ConvNhwcArgs& a, double other_us, bool dry, hipStream_t stre
 
 bool TryConvFew(const ConvNhwcArgs& a, hipStream_t stream) { return TryFew(a, -1.0, false, stream) > 0.0; }
 
-double TryProductFew(const ConvNhwcArgs& a, double other_us, bool dry, hipStream_t stream) { return TryFew(a, other_us, dry, stream); }
+double TryProductFew(const ConvNhwcArgs& a, double limit_us, bool dry, hipStream_t stream) { return TryFew(a, limit_us, dry, stream); }
 
 }  // namespace cinn_hip_kernels
 

@@ -57,9 +57,9 @@ bool ConvPatchForced(const ConvNhwcArgs& a);
 // few output tiles, or many that are mostly padding (conv_few_mfma.hip): whole K steps of 128 bytes in every tap, same epilogue; one launch of
 // small tiles whose wavefronts share K.  false when the shape does not qualify or the tiled kernels are faster.
 bool TryConvFew(const ConvNhwcArgs& a, hipStream_t stream);
-// A matrix product written as a 1x1 layer on m pixels, whose alternative takes `other_us`: that kernel's estimate where it takes
-// the product (nothing is launched if `dry`), 0 where it does not.
-double TryProductFew(const ConvNhwcArgs& a, double other_us, bool dry, hipStream_t stream);
+// A matrix product written as a 1x1 layer on m pixels: that kernel's estimate where it takes the product and the estimate
+// is below `limit_us` (nothing is launched if `dry`), else 0.
+double TryProductFew(const ConvNhwcArgs& a, double limit_us, bool dry, hipStream_t stream);
 // into how many parts the tiled kernel splits the K steps of a convolution of `tiles` tiles of 64x64
 int ConvSplits(int tiles, int steps, bool fp32);
 // Two 1x1, stride 1, unpadded convolutions in a row on channels-last 16-bit tensors, seen as matrix products over the

@@ -1856,7 +1856,7 @@ double TryFewProduct(const GemmProblem& p, double flex_us, bool dry, hipStream_t
   a.n = a.h = a.oh = a.kh = a.kw = 1, a.w_in = a.ow = p.m, a.c = p.k, a.oc = p.n;
   a.pad_h = a.pad_w = 0, a.stride_h = a.stride_w = a.dil_h = a.dil_w = 1;
   a.type.code = cinn_type_float, a.type.bits = 32, a.type.lanes = 1, a.type.num_asterisks = 0;
-  const double us = cinn_hip_kernels::TryProductFew(a, flex_us + 2.0, dry, stream);
+  const double us = cinn_hip_kernels::TryProductFew(a, (p.k > 32 ? 0.9 : 0.83) * (flex_us + 2.0), dry, stream);
   return us > 0.0 ? std::max(us - 2.0, 0.1) : 0.0;
 }
 

@@ -219,7 +219,8 @@ void cinn_call_hip_conv2d_pair_chain(void* v_args, int num_args, int relu, int i
 
 /* cinn_call_cudnn_conv2d_forward for callers that cannot allocate.  No counterpart in the reference: it exists for
  * code that runs under HIP graph capture, tight serving loops and harnesses that forbid hipMalloc.  Same arguments and
- * results as the call above for format 1 and 2 with groups == 1 (always on the general channels-last MFMA kernel);
+ * results as the call above for format 1 and 2 with groups == 1 (always on the general channels-last MFMA kernel; where the
+ * call above runs another one, the same sums in another order);
  * it calls no hipMalloc / hipFree and no allocating library routine.  What the kernels need beyond x, w and y (a page
  * of zeros, the fp32 partial sums of a split reduction) lives in a static device array of
  * cinn_hip_conv2d_forward_noalloc_scratch_limit() = 16 MiB (+ 256 bytes) that every GPU the library runs on holds

@@ -23,5 +23,18 @@ def gpu():
 
 
 @pytest.fixture
+def tiled_kernels(gpu):
+    """for the length of a test, layers and products of few tiles stay with the kernels that split their K over blocks and add the
+    parts through scratch memory"""
+    import ctypes
+    from cinn_amd import _lib
+    mode = _lib.load().cinn_hip_conv_few_mode
+    mode.argtypes, mode.restype = [ctypes.c_int], ctypes.c_int
+    before = mode(0)
+    yield
+    mode(before)
+
+
+@pytest.fixture
 def rng():
     return np.random.default_rng(1234)

@@ -34,7 +34,7 @@ def conv_program(name, x, w, stream):
     return comp, y.id
 
 
-def test_replay_of_a_captured_program_survives_a_later_larger_scratch_request(gpu):
+def test_replay_of_a_captured_program_survives_a_later_larger_scratch_request(tiled_kernels):
     rng = np.random.default_rng(77)
     stream = runtime.Stream()
     # program A: 7 tiles of 64x64, 18 K steps -> split in two, 200 KB of partial sums

@@ -71,7 +71,7 @@ def check_oracle(got, x, w, stride, pad, tol):
         assert np.all(np.abs(got.astype(np.float64) - want) <= tol * np.maximum(np.abs(want), 1e-3 * scale) + 2.0 ** -24)
 
 
-def test_noalloc_matches_the_allocating_entry_point_on_two_calls_in_a_row(gpu):
+def test_noalloc_matches_the_allocating_entry_point_on_two_calls_in_a_row(tiled_kernels):
     lib = _lib.load()
     lib.cinn_hip_conv2d_forward_noalloc_scratch_limit.restype = ctypes.c_size_t
     assert lib.cinn_hip_conv2d_forward_noalloc_scratch_limit() == 16 << 20
