@@ -486,14 +486,13 @@ bool RowProductPays(int m, int n, int k, bool ring, bool saves_launch, bool spli
 // 24.9, eight 64 x 1280 -> 8192 28.9 | 32.6, four 64 x 768 -> 4096 13.0 | 16.9; the same blocks alone 64 x 768 -> 3072 15.5 | 13.1.
 RowFusion ChooseRowFusion(int m, int n, int k, bool ring, RowFusion there) {
   if (ring) {
-    // gemm_rows_ring_kernel, blocks of 16 or of 32 columns.  us, outside | inside, norm: 1 x 128 -> 4096 5.3 | 3.1, 16 x 1280 -> 5120 6.6 | 5.8,
-    // 32 x 1024 -> 4096 (256 blocks of 32) 5.9 | 5.3, 32 x 512 -> 8192 (512) 5.7 | 5.1, 64 x 768 -> 3072 (384) 6.4 | 6.1; 64 x 384 -> 6272 (784)
-    // 6.3 | 6.9, 8 x 1280 -> 9984 (312) 7.5 | 7.8, 64 x 1024 -> 4096 (512) 6.4 | 7.0, 48 x 1280 -> 5120 (480) 8.1 | 8.2.  gelu: 1 x 768 -> 3072 5.8 |
-    // 3.5, 64 x 512 -> 16384 9.4 | 8.3.  What lies beyond these lines stays as such layers have always been compiled: norm outside at 16 x
-    // 128 -> 8192, inside at 48 x 1280 -> 4096, gelu outside from 64 x 768 -> 8192 on (with K = 2048 10.8 | 9.2).
-    const int tiles = (m + 15) / 16, narrow = tiles * ((n + 15) / 16), wide = tiles * ((n + 31) / 32);
-    const bool norm = narrow <= 256 || ((k >= 192 || n < 8192) && (wide <= 256 || (wide <= 512 && (k < 1024 || (k > 1024 && tiles >= 3)))));
-    return {there.norm && norm, there.gelu && (narrow < 2048 || k < 768)};
+    // gemm_rows_ring_kernel, blocks of 16 or of 32 columns; 197 layers of a program, 1 to 64 rows, us with the one outside | inside, fp16.
+    // gelu is ahead everywhere, 1.09 to 1.76: 1 x 128 -> 4096 5.1 | 3.1, 64 x 768 -> 8192 9.3 | 7.4, 64 x 2048 -> 8192 12.0 | 10.3, 64 x 1280 -> 9984
+    // 13.6 | 11.7.  The norm, which every block repeats for its rows, is 1.00 to 1.6 up to 512 blocks of 32 columns: 16 x 128 -> 8192 (256) 5.0 | 3.8,
+    // 48 x 1280 -> 4096 (384) 9.8 | 9.3, 64 x 1024 -> 4096 (512) 8.0 | 7.8, 16 x 1280 -> 16384 (512) 13.2 | 11.3; beyond, 1.03 to 1.45 up to a K of 384 and
+    // 0.76 to 1.01 from 768 on: 48 x 384 -> 6272 (588) 7.4 | 6.0, 64 x 384 -> 9984 (1248) 9.2 | 8.7; 48 x 768 -> 6272 9.4 | 9.8, 64 x 1280 -> 8192 11.9 | 15.1.
+    const int wide = (m + 15) / 16 * ((n + 31) / 32);
+    return {there.norm && (wide <= 512 || k <= 384), there.gelu};
   }
   const int rounds = ((n + 15) / 16 * ((m + 15) / 16) + 255) / 256;
   const bool same  = k % 256 == 0 && n <= 4080;  // the blocks of the product alone

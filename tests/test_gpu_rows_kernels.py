@@ -23,6 +23,16 @@ def test_row_tiles_of_a_block(gpu, m, k, n, outputs, residual, dtype):
     assert count(ROWS) == 1 and count(ROWS_RING) == 0
 
 
+# normalising blocks beyond 512, and of a grid of many rounds
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("m,k,n,outputs", [(64, 384, 6276, 1), (50, 128, 16388, 1), (33, 320, 12300, 3)])
+@pytest.mark.parametrize("gelu", [False, True])
+def test_norm_in_many_blocks(gpu, m, k, n, outputs, gelu, dtype):
+    with launches() as count:
+        check_rows(gpu, m, k, n, outputs, True, gelu, False, dtype)
+    assert count(ROWS_RING) == 1 and count(ROWS) == 0
+
+
 @pytest.mark.parametrize("m,k,n,outputs,ring", [(8, 768, 768, 1, True), (40, 512, 4104, 3, True), (40, 512, 4100, 2, False), (12, 576, 12, 2, False), (8, 96, 768, 1, False)])
 def test_kernel(gpu, m, k, n, outputs, ring):
     with launches() as count:
