@@ -34,7 +34,8 @@ constexpr int kRowProductMaxNormK = 1280;
 
 // false where the kernel does not take the extents; operands lie at any address of their type
 bool RowProductSupported(const RowProduct& p);
-// which of the file's two kernels runs it: gemm_rows_ring_kernel, or gemm_rows_kernel; by the addresses as well where there are any
+// which of the file's two kernels runs it: gemm_rows_ring_kernel (but for some single rows), or gemm_rows_kernel; by the addresses as
+// well where there are any
 bool RowRingTakes(const RowProduct& p);
 // whether the kernel (`ring`: which one, as above) is ahead of the tiled ones for a product that it takes; `saves_launch`: several results, which would
 // be copied out of one; `splits`: without a scale, which gemm_flex.hip would take and split its K

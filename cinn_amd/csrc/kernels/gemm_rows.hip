@@ -5,7 +5,7 @@
 // here small tiles give most CUs a block and its wavefronts split K.
 //   * gemm_rows_ring_kernel: whole K steps of 64 in aligned rows, operands through rings in LDS in whole lines (few_tile.h: a CU
 //     pulls in three times as much that way);
-//   * gemm_rows_kernel: any other K of 32-deep blocks, operands at any address of their type.  A block owns 16 output columns of
+//   * gemm_rows_kernel: any other K of 32-deep blocks, operands at any address of their type, and some single rows (OneRow).  A block owns 16 output columns of
 //     MT row tiles, its eight wavefronts split K, fragments come straight from global memory, 2 U k-blocks of loads in flight.
 // us, the latter | the former, fp16: 8 x 768 -> 768 4.1 | 3.3, 8 x 3072 -> 768 7.2 | 4.7, 64 x 1280 -> 5120 24.7 | 6.4, 16 x 4096 -> 4096 with gelu 10.4 |
 // 6.1; norm inside 8 x 768 -> 3072 5.4 | 4.1, with gelu 6.0 | 4.6.
@@ -363,9 +363,22 @@ void LaunchNorm(const RowProduct& p, hipStream_t stream) {
   }
 }
 
+// A single row of up to 256 blocks is ahead on gemm_rows_kernel where little is left of the rings' gain: the sixteen lanes that ask for
+// the one row of A there ask for the same bytes, while a ring brings them as a whole fragment; and a lane has one value for gelu there
+// (0.1 us), four here (0.4 us).  us, that kernel | rings, fp16, plain: 64 -> 1024 2.3 | 2.6, 128 -> 512 2.5 | 2.6, 1024 -> 4096 3.8 | 4.1, but 384 -> 1536
+// 3.0 | 2.9, 1280 -> 4096 4.9 | 4.4, 4096 -> 1024 6.9 | 4.8; gelu 128 -> 2048 2.7 | 3.1, 384 -> 1536 3.1 | 3.3, 640 -> 2560 3.5 | 3.9, 1024 -> 4096 3.9 | 4.5, but 256 ->
+// 768 3.2 | 3.1, 1280 -> 3840 4.9 | 4.7; norm and gelu 1024 -> 3072 5.3 | 5.4, 1280 -> 3840 5.5 | 5.9, but 768 -> 3072 5.2 | 4.9, norm alone 1024 -> 4096 5.3 | 5.1.
+// (Two rows: gelu 640 -> 2560 3.9 | 3.9, 256 -> 4096 3.8 | 3.6.)
+bool OneRow(const RowProduct& p) {
+  if (p.m != 1 || p.n > 4096) return false;
+  if (p.gamma) return p.gelu && p.k >= 1024;
+  if (p.gelu) return p.k <= 1024 && p.k != 256;
+  return p.k <= 128 || (p.k > 768 && p.k <= 1024);
+}
+
 template <typename T>
 bool TryRing(const RowProduct& p, hipStream_t stream) {
-  if (!RowRingTakes(p)) return false;
+  if (!RowRingTakes(p) || OneRow(p)) return false;
   CountLaunch(kCountRowsRing);
   if (p.gamma) {
     // With a block for every CU twice the columns in each: 1 x 384 -> 6272 4.4 | 3.8, 32 x 768 -> 3072 5.5 | 4.5, 16 x 1280 -> 5120 8.8 |
