@@ -1845,9 +1845,14 @@ bool ForceGeneric() {
 // estimate leaves out the 2 us of a block's start and end.  A product of few rows took that kernel a launch of 64x64 tiles that are
 // mostly padding, split over K, and a second launch that adds the parts.  us, that kernel | here: 7 x 1152 -> 1792 8.9 | 4.8, 10 x 320 -> 3520
 // 9.2 | 3.5, 1 x 224 -> 1208 7.4 | 3.1, 92 x 3168 -> 576 13.3 | 8.3.  Of 150 products of 1 to 2683 rows, no multiples of 128, 129 are taken, 1.70
-// times faster in the geometric mean, the worst 0.98; not taken 1912 x 64 -> 3520 17.6 | 43.7, 466 x 3520 -> 576 28.9 | 33.6.  The result is that kernel's
-// estimate where it takes the product, in the other's terms, else 0.
-double TryFewProduct(const GemmProblem& p, double flex_us, bool dry, hipStream_t stream) {
+// times faster in the geometric mean, the worst 0.98; not taken 1912 x 64 -> 3520 17.6 | 43.7, 466 x 3520 -> 576 28.9 | 33.6.
+// `whole`: tiles of 128, which gemm32_mfma_kernel may run as well.  Below 0.85 22 of 30 of these are taken, 1.10 to 2.2 times faster: 128 x 128 -> 128
+// 5.2 | 3.3, 128 x 4096 -> 128 13.0 | 9.4, 512 x 512 -> 512 11.4 | 6.3, 4096 x 512 -> 128 13.2 | 9.3, 768 x 768 -> 768 18.4 | 16.7; not taken 256 x 768 ->
+// 3072 18.3 | 17.8, 768 x 2048 -> 1024 37.3 | 38.4, 1024 x 1024 -> 1024 24.2 | 28.0, and one K step, 3.4 | 3.1 but with 1.3 times the error against float64 (the
+// others 0.3 to 0.8 of it).
+// The result is that kernel's estimate where it takes the product, in the other's terms, else 0.
+double TryFewProduct(const GemmProblem& p, double flex_us, bool whole, bool dry, hipStream_t stream) {
+  if (whole && p.k <= 32) return 0.0;
   if (p.type != GemmType::kF32 || p.trans_a || !p.trans_b || p.batch != 1 || p.shift16) return 0.0;
   cinn_hip_kernels::ConvNhwcArgs a;
   a.x = p.a, a.w = p.b, a.y = p.c, a.scale = nullptr, a.shift = p.shift;
@@ -1856,7 +1861,7 @@ double TryFewProduct(const GemmProblem& p, double flex_us, bool dry, hipStream_t
   a.n = a.h = a.oh = a.kh = a.kw = 1, a.w_in = a.ow = p.m, a.c = p.k, a.oc = p.n;
   a.pad_h = a.pad_w = 0, a.stride_h = a.stride_w = a.dil_h = a.dil_w = 1;
   a.type.code = cinn_type_float, a.type.bits = 32, a.type.lanes = 1, a.type.num_asterisks = 0;
-  const double us = cinn_hip_kernels::TryProductFew(a, (p.k > 32 ? 0.9 : 0.83) * (flex_us + 2.0), dry, stream);
+  const double us = cinn_hip_kernels::TryProductFew(a, (whole ? 0.85 : p.k > 32 ? 0.9 : 0.83) * (flex_us + 2.0), dry, stream);
   return us > 0.0 ? std::max(us - 2.0, 0.1) : 0.0;
 }
 
@@ -1868,7 +1873,7 @@ bool RunsFlexible(const GemmProblem& product, hipStream_t stream, cinn_hip_kerne
   if (p.type == GemmType::kF32) {
     const bool aligned16 = reinterpret_cast<uintptr_t>(p.a) % 16 == 0 && reinterpret_cast<uintptr_t>(p.b) % 16 == 0;
     if (aligned16 && p.m % kF32Tile == 0 && p.n % kF32Tile == 0 && p.k % kF32K == 0) return false;
-    const double few = TryFewProduct(p, plan->us, true, stream);  // a group has to be faster than that
+    const double few = TryFewProduct(p, plan->us, false, true, stream);  // a group has to be faster than that
     if (few > 0.0) plan->us = few;
     return true;
   }
@@ -1930,7 +1935,7 @@ void RunGemm(const GemmProblem& p, hipStream_t stream) {
     // nearly empty are better off split all the same: 1280x1024x4096 138 | 101, 768x3072x4096 207 | 172.)
     const bool fast32 = whole32 && ((int64_t)(p.m / 64) * (p.n / 64) * p.batch >= 256 || plan.splits <= 1);
     const bool whole  = !bias && p.type == GemmType::kF32 && fast32;
-    if (!whole32 && planned && TryFewProduct(p, plan.us, false, stream) > 0.0) return;
+    if (planned && TryFewProduct(p, plan.us, whole32, false, stream) > 0.0) return;
     if (!whole && planned) {
       cinn_hip_kernels::RunFlexGemm(g, plan, stream);
       return;

@@ -10,6 +10,8 @@ from cinn_amd import _lib, runtime
 
 from launch_counts import FEW, launches
 from test_gpu_conv_few import _conv64, test_layer as check_layer
+from test_gpu_few_products import check as check_product
+from test_gpu_gemm import call_cublas
 
 pytestmark = pytest.mark.gpu
 
@@ -62,6 +64,20 @@ def test_kernel(gpu, shape, oc, k, stride, dtype, few, scale):
     want, size = (_conv64(a, b, stride, k // 2, 1)[:, rows] for a, b in ((x, w), (np.abs(x), np.abs(w))))
     unit = 2.0 ** -11 if dtype == "float16" else 2.0 ** -24
     assert np.all(np.abs(y[-1:, rows].astype(np.float64) - want) <= 1.01 * ((w[0].size + 2) * 2.0 ** -24 * size + unit * np.abs(want) + 2.0 ** -25))
+
+
+# fp32 products with both operands in runs of K; whole tiles of 128 as well
+@pytest.mark.parametrize("m,n,k,few", [
+    (7, 1792, 1152, True), (92, 576, 3168, True), (1, 1208, 192, True), (64, 60, 2048, True), (1912, 3520, 64, False), (466, 576, 3520, False),
+    (128, 128, 128, True), (128, 128, 4096, True), (512, 512, 512, True), (4096, 128, 512, True), (256, 128, 64, True), (768, 768, 768, True),
+    (128, 128, 32, False), (256, 3072, 768, False), (1024, 1024, 1024, False)])
+def test_product(gpu, m, n, k, few):
+    rng = np.random.default_rng(m + n + k)
+    a, b = (rng.standard_normal(s).astype(np.float32) for s in ((m, k), (n, k)))
+    with launches() as count:
+        got = call_cublas(a, b, (m, n), "float32", False, True)
+        assert count(*FEW) == few
+    check_product(got, a.astype(np.float64), b.astype(np.float64), 1.0, 0.0, k)
 
 
 def test_every_tile_is_reached(gpu):

@@ -71,7 +71,7 @@ def test_what_lies_beyond_k_is_not_multiplied(gpu, kind, ta, tb):
 @pytest.mark.parametrize("batch,m,n,k,split", [(1, 128, 128, 4096, True), (1, 256, 128, 2048, True), (3, 128, 256, 1024, True),
                                                (1, 512, 1024, 1024, True), (1, 1024, 1024, 96, False), (2, 128, 128, 32, False),
                                                (1, 896, 1152, 1024, False)])
-def test_whole_fp32_tiles_that_leave_cus_idle_split_k(gpu, batch, m, n, k, split, ta, tb):
+def test_whole_fp32_tiles_that_leave_cus_idle_split_k(tiled_kernels, batch, m, n, k, split, ta, tb):
     """extents that are whole 128x128 tiles: a K that is worth splitting over the CUs left idle uses partial sums (the stream
     has no scratch before), others do not"""
     rng = np.random.default_rng(k)
