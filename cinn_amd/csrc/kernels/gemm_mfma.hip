@@ -1998,7 +1998,8 @@ Range Written(const GemmProblem& p) { return Memory(p.c, (p.batch - 1) * p.strid
 bool Touches(const GemmProblem& p, const Range& r) {
   return Overlap(r, Written(p)) || Overlap(r, Memory(p.a, (p.batch - 1) * p.stride_a + (int64_t)p.m * p.k, p.type)) ||
          Overlap(r, Memory(p.b, (p.batch - 1) * p.stride_b + (int64_t)p.k * p.n, p.type)) ||
-         Overlap(r, Memory(p.shift, p.n, GemmType::kF32)) || Overlap(r, Memory(p.shift16, p.n, p.type));
+         Overlap(r, Memory(p.shift, p.n, GemmType::kF32)) || Overlap(r, Memory(p.shift16, p.n, p.type)) ||
+         Overlap(r, Memory(p.scale, p.n, GemmType::kF32)) || Overlap(r, Memory(p.residual, (p.batch - 1) * p.stride_c + (int64_t)p.m * p.n, p.type));
 }
 
 void WaitInGroup(const GemmProblem& p, hipStream_t stream) {
