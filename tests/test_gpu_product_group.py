@@ -10,6 +10,8 @@ from cinn_amd import runtime
 from cinn_amd.common import BFloat16, DefaultAMDGPUTarget, Float, bfloat16_bits_to_float32, float32_to_bfloat16_bits
 from cinn_amd.frontend import Computation, NetBuilder
 
+from launch_counts import GROUP, launches
+
 pytestmark = pytest.mark.gpu
 
 TYPES = {"float32": Float(32), "float16": Float(16), "bfloat16": BFloat16()}
@@ -65,6 +67,20 @@ def test_a_layers_three_products_and_two_more(gpu, rows, inp, out, kind):
         got = [net.get(comp, o) for o in outs]
         for at, (p, q, shift) in enumerate(((x, w, c), (dy, w.T, 0.0), (x.T, dy, 0.0), (x, v, 0.0), (dy, v.T, 0.0))):
             net.check(got[at], p, q, shift)
+
+
+# which of these are one launch: small ones are, and those of one small tile in all products, until a tile of 128 or the small tiles of
+# fp32 are estimated to be faster one by one
+@pytest.mark.parametrize("kind", ["float32", "float16", "bfloat16"])
+@pytest.mark.parametrize("rows,inp,out,groups", [(37, 75, 247, 1), (665, 233, 670, 1), (33, 17, 65, 1), (127, 1001, 62, 1), (4887, 301, 2123, 0)])
+def test_a_layers_three_products_in_one_launch(gpu, rows, inp, out, groups, kind):
+    net = Net(kind)
+    x, w, dy = (net.input(n, s) for n, s in (("x", (rows, inp)), ("w", (inp, out)), ("dy", (rows, out))))
+    comp = net.compile([net.b.matmul(x, w), net.b.matmul(dy, w, False, True), net.b.matmul(x, dy, True, False)])
+    with launches() as count:
+        comp.execute()
+        net.stream.synchronize()
+    assert count(GROUP) == groups
 
 
 @pytest.mark.parametrize("kind", ["float32", "float16", "bfloat16"])
