@@ -100,8 +100,8 @@ struct Ring {
   __device__ __forceinline__ void Mma() {
     // fp32: the products of a step in a chain of their own, so that acc is a chain of steps and not of products.  (The tiled kernels
     // split K over more blocks than there are wavefronts here.  Relative error against float64 over theirs, 35 convolutions and 40
-    // products: 0.83 and 0.79 in the geometric mean and up to 1.6 as one chain, 0.48 and 0.64 so and none above but a product of one
-    // step at 1.1e-7; as two chains a step 0.42 and 0.54.  Time 1.01 to 1.02 of one chain's, two chains 1.04.)
+    // products: 0.83 and 0.79 in the geometric mean and up to 1.6 as one chain, 0.48 and 0.64 so and none above (a product of one
+    // step is the same chain there: 0.98 to 1.01); as two chains a step 0.42 and 0.54.  Time 1.01 to 1.02 of one chain's, two chains 1.04.)
     if constexpr (sizeof(T) == 4) {
       f32x4 sum[TM][TN];
 #pragma unroll
@@ -195,8 +195,9 @@ __device__ __forceinline__ void TileOf(int bid, int tiles_m, int tiles_n, bool r
   *tn = rows_outer ? id % tiles_n : id / tiles_m;
 }
 
-// A tile's launch, in us: a block's start and end, what its CU pulls in (147 bytes per ns) and multiplies, rounds of blocks beyond
-// those that a CU holds.  Fitted to 330 layers of 1 to 32 images (0.14 in the logarithm, 2% from the best tile on average).
+// A tile's launch, in us: a block's start and end, what its CU pulls in and multiplies, rounds of blocks beyond
+// those that a CU holds.  The coefficients are fitted and not rates (147 bytes per ns, where a CU was seen to pull in 110 to 130, since part
+// of that lies under the constant), to 330 layers of 1 to 32 images (0.14 in the logarithm, 2% from the best tile on average).
 inline double Estimate(int rows, int cols, int steps, bool fp32, int tm, int tn, int nw) {
   const double blocks   = (double)((rows + 16 * tm - 1) / (16 * tm)) * ((cols + 16 * tn - 1) / (16 * tn)), per_cu = std::ceil(blocks / 256);
   const int resident    = std::min(160 / (nw * 2 * (tm + tn) * 2), 8);

@@ -500,7 +500,8 @@ __device__ __forceinline__ void SelectFirst(u64 (&w)[E], int keep, u64* candidat
 // The first `keep` (at most kSelect) elements of a row.  A row of more than 1024 elements has several wavefronts; each selects
 // the first `keep` of its part.  Of up to sixteen (C = 1) the first wavefront selects again, of more each looks up how many of
 // the other parts' are before it.
-// Bound by the launch and the read of the row for few elements (2048 rows of 1000 fp32 values, k = 1: 5.6 us), by the wave
+// Bound by the launch and the read of the row for few elements (2048 rows of 1000 fp32 values in the last-level cache, k = 1: 5.6 us; an empty
+// launch 3.3; rows from memory add 2.7, the one trip that all of a wavefront's work waits for), by the wave
 // reductions that find the bound for many.  Taking the elements one by one - a 64-bit look at all of the owner's words for
 // each - against this: k = 5 7.8 -> 6.3 us, k = 10 10.5 -> 7.0, k = 16 13.8 -> 7.9; 64 rows of 8000 fp16, k = 10 18.0 -> 8.7;
 // 600 rows of 3000, k = 5 9.2 -> 6.5.

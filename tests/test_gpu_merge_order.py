@@ -65,7 +65,8 @@ def test_a_kernel_stays_between_what_it_reads_and_what_reads_it(gpu):
 
 
 def test_an_update_does_not_pass_other_readers_of_its_input(gpu):
-    """new = 0.9 state + 0.1 u may be bound to state's memory: what reads the old state before it still does"""
+    """new = 0.9 state + 0.1 u may be bound to state's memory: what reads the old state element by element is in the same kernel (fused
+    with it, in one thread) or before it.  Readers of other elements: test_merge_updates"""
     b = NetBuilder("update")
     feeds, (x, w, state, u) = inputs(b, {"x": (64, 64), "w": (64, 64), "state": (64,), "u": (64,)})
     seen = b.multiply(state, state)
