@@ -365,15 +365,15 @@ void LaunchNorm(const RowProduct& p, hipStream_t stream) {
 
 // A single row of up to 256 blocks is ahead on gemm_rows_kernel where little is left of the rings' gain: the sixteen lanes that ask for
 // the one row of A there ask for the same bytes, while a ring brings them as a whole fragment; and a lane has one value for gelu there
-// (0.1 us), four here (0.4 us).  us, that kernel | rings, fp16, plain: 64 -> 1024 2.3 | 2.6, 128 -> 512 2.5 | 2.6, 1024 -> 4096 3.8 | 4.1, but 384 -> 1536
-// 3.0 | 2.9, 1280 -> 4096 4.9 | 4.4, 4096 -> 1024 6.9 | 4.8; gelu 128 -> 2048 2.7 | 3.1, 384 -> 1536 3.1 | 3.3, 640 -> 2560 3.5 | 3.9, 1024 -> 4096 3.9 | 4.5, but 256 ->
-// 768 3.2 | 3.1, 1280 -> 3840 4.9 | 4.7; norm and gelu 1024 -> 3072 5.3 | 5.4, 1280 -> 3840 5.5 | 5.9, but 768 -> 3072 5.2 | 4.9, norm alone 1024 -> 4096 5.3 | 5.1.
-// (Two rows: gelu 640 -> 2560 3.9 | 3.9, 256 -> 4096 3.8 | 3.6.)
+// (0.1 us), four here (0.4 us).  us, that kernel | rings, fp16, plain: 64 -> 1024 2.3 | 2.6, 128 -> 512 2.5 | 2.6, 1024 -> 4096 3.8 | 4.1, but 1024 -> 1024
+// 3.4 | 3.4, 384 -> 1536 3.0 | 2.9, 1280 -> 4096 4.9 | 4.4, 4096 -> 1024 6.9 | 4.8; gelu 128 -> 2048 2.7 | 3.1, 384 -> 1536 3.1 | 3.3, 640 -> 2560 3.5 | 3.9, 1024 -> 4096 3.9 | 4.5, but 256 ->
+// 768 3.2 | 3.1, 1280 -> 3840 4.9 | 4.7; norm and gelu 1152 -> 4096 5.5 | 5.9, 1280 -> 3840 5.5 | 5.9, but 768 -> 3072 5.2 | 4.9, norm alone 1024 -> 4096 5.3 | 5.1.
+// (With norm and gelu 1024 -> 4096, 5.4 | 5.5, is even: a decoding block of one row of 1024 takes 28.4 us with it there, 28.1 with it here.  Two rows: gelu 640 -> 2560 3.9 | 3.9, 256 -> 4096 3.8 | 3.6.)
 bool OneRow(const RowProduct& p) {
   if (p.m != 1 || p.n > 4096) return false;
-  if (p.gamma) return p.gelu && p.k >= 1024;
+  if (p.gamma) return p.gelu && p.k > 1024;
   if (p.gelu) return p.k <= 1024 && p.k != 256;
-  return p.k <= 128 || (p.k > 768 && p.k <= 1024);
+  return p.k <= 128 || (p.k > 768 && p.k <= 1024 && p.n > 2048);
 }
 
 template <typename T>
@@ -504,8 +504,11 @@ RowFusion ChooseRowFusion(int m, int n, int k, bool ring, RowFusion there) {
     // 13.6 | 11.7.  The norm, which every block repeats for its rows, is 1.00 to 1.6 up to 512 blocks of 32 columns: 16 x 128 -> 8192 (256) 5.0 | 3.8,
     // 48 x 1280 -> 4096 (384) 9.8 | 9.3, 64 x 1024 -> 4096 (512) 8.0 | 7.8, 16 x 1280 -> 16384 (512) 13.2 | 11.3; beyond, 1.03 to 1.45 up to a K of 384 and
     // 0.76 to 1.01 from 768 on: 48 x 384 -> 6272 (588) 7.4 | 6.0, 64 x 384 -> 9984 (1248) 9.2 | 8.7; 48 x 768 -> 6272 9.4 | 9.8, 64 x 1280 -> 8192 11.9 | 15.1.
-    const int wide = (m + 15) / 16 * ((n + 31) / 32);
-    return {there.norm && (wide <= 512 || k <= 384), there.gelu};
+    // Even are three and four row tiles of up to 4096 columns with a K of 1024, of which the product alone has whole pairs of steps for each of its
+    // wavefronts: 48 x 1024 -> 3072 7.6 | 7.6, 64 x 1024 -> 4096 8.0 | 7.8, a block of 48 tokens of 1024 31.8 | 32.2; they stay outside.
+    const int tiles = (m + 15) / 16, wide = tiles * ((n + 31) / 32);
+    const bool even = tiles >= 3 && n <= 4096 && k > 512 && k % 512 == 0;
+    return {there.norm && (k <= 384 || (wide <= 512 && !even)), there.gelu};
   }
   const int rounds = ((n + 15) / 16 * ((m + 15) / 16) + 255) / 256;
   const bool same  = k % 256 == 0 && n <= 4080;  // the blocks of the product alone

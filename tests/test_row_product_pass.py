@@ -80,7 +80,7 @@ def linear_layer(m, k, n, norm, gelu):
     (16, 960, 8192, True, False, 1),
     (48, 1280, 4096, True, True, 1),
     (64, 960, 8192, False, True, 1),
-    (64, 1280, 4096, True, False, 1), (64, 1280, 4128, True, False, 2), (64, 448, 4128, True, False, 2),
+    (64, 1280, 4096, True, False, 1), (64, 1024, 4096, True, False, 2), (32, 1024, 4096, True, False, 1), (64, 1280, 4128, True, False, 2), (64, 448, 4128, True, False, 2),
     (48, 416, 6272, True, False, 2), (64, 800, 8192, True, True, 3), (16, 160, 8192, True, True, 2), (8, 800, 3072, True, True, 1),
 ])
 def test_what_a_product_of_few_rows_takes_along(m, k, n, norm, gelu, calls):
